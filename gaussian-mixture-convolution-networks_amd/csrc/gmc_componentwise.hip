@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kBlock) void componentwise_bwd_kernel(const T* __re
         {
             const Derived<D> dv = derive<T, D>(mixture + (size_t(bl) * M + (valid ? m : 0)) * G, covariance_form);
             // amplitude for dL/dx as in the summed backward kernel: w norm / (0.5 log2 e)
-            store_record<T, D>(r, dv, true, dv.w * dv.norm / kHalfLog2e, 0);
+            store_record<T, D>(r, dv, true, dv.w * dv.norm * (1.0 / kHalfLog2e), 0);
         }
         T ua[kU];                                   // -amp * u: dL/dx takes k*y against it
 #pragma unroll

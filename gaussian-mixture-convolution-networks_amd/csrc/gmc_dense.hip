@@ -449,17 +449,17 @@ __device__ __forceinline__ void bwd_epilogue_one(const T* __restrict__ g, const 
         for (int q = 0; q < D; ++q) { U[r][q] = 0.0; V[r][q] = 0.0; }
     if constexpr (D == 2) {
         U[0][0] = dv.u[0]; U[0][1] = dv.u[1]; U[1][1] = dv.u[2];
-        V[0][0] = 1.0 / U[0][0]; V[1][1] = 1.0 / U[1][1];
+        V[0][0] = reciprocal<T>(U[0][0]); V[1][1] = reciprocal<T>(U[1][1]);
         V[0][1] = -U[0][1] * V[0][0] * V[1][1];
     } else {
         U[0][0] = dv.u[0]; U[0][1] = dv.u[1]; U[0][2] = dv.u[2]; U[1][1] = dv.u[3]; U[1][2] = dv.u[4]; U[2][2] = dv.u[5];
-        V[0][0] = 1.0 / U[0][0]; V[1][1] = 1.0 / U[1][1]; V[2][2] = 1.0 / U[2][2];
+        V[0][0] = reciprocal<T>(U[0][0]); V[1][1] = reciprocal<T>(U[1][1]); V[2][2] = reciprocal<T>(U[2][2]);
         V[0][1] = -U[0][1] * V[0][0] * V[1][1];
         V[1][2] = -U[1][2] * V[1][1] * V[2][2];
         V[0][2] = -(U[0][1] * V[1][2] + U[0][2] * V[2][2]) * V[0][0];
     }
     // db = k u^T R1
-    const double k = wn / kHalfLog2e;
+    const double k = wn * (1.0 / kHalfLog2e);
 #pragma unroll
     for (int r = 0; r < D; ++r) {
         double acc = 0.0;
@@ -495,7 +495,7 @@ __device__ __forceinline__ void bwd_epilogue_one(const T* __restrict__ g, const 
             a[r][q] = acc;
         }
     const double det = determinant<T, D>(c);
-    const double kd = dv.w * Kappa<D>::v * R0 / (2.0 * sqrt(det));
+    const double kd = 0.5 * over<T>(dv.w * Kappa<D>::v * R0, root<T>(det));
     double gc[D][D];
 #pragma unroll
     for (int r = 0; r < D; ++r)
