@@ -188,11 +188,11 @@ __device__ __forceinline__ double determinant(const double (&m)[D][D]) {
     }
 }
 
+// `cm` receives the inverse covariance
 template <typename T, int D>
-__device__ __forceinline__ Derived<D> derive(const T* __restrict__ g, bool covariance_form = false) {
+__device__ __forceinline__ Derived<D> derive(const T* __restrict__ g, bool covariance_form, double (&cm)[D][D]) {
     Derived<D> r;
     r.w = double(g[0]);
-    double cm[D][D];
     load_inverse_covariance<T, D>(g + 1 + D, covariance_form, cm);
     if constexpr (D == 2) {
         const double c00 = cm[0][0], c01 = cm[0][1], c10 = cm[1][0], c11 = cm[1][1];
@@ -232,6 +232,12 @@ __device__ __forceinline__ Derived<D> derive(const T* __restrict__ g, bool covar
     return r;
 }
 
+template <typename T, int D>
+__device__ __forceinline__ Derived<D> derive(const T* __restrict__ g, bool covariance_form = false) {
+    double cm[D][D];
+    return derive<T, D>(g, covariance_form, cm);
+}
+
 // LDS record of one Gaussian for the pair loop: u, then nd ("shifted" form) or b ("centred" form), the
 // amplitude, and the Gaussian's index within its tile; padded to a multiple of 16 bytes.
 //
@@ -259,7 +265,10 @@ __device__ __forceinline__ void store_record(T* rec, const Derived<D>& d, bool c
 #pragma unroll
     for (int i = 0; i < kU; ++i) rec[i] = T(d.u[i]);
 #pragma unroll
-    for (int i = 0; i < D; ++i) rec[kU + i] = T(centred ? d.b[i] : d.nd[i]);
+    for (int i = 0; i < D; ++i) {
+        const double near = d.nd[i], centre = d.b[i];        // (values: a choice between the elements would put d into memory)
+        rec[kU + i] = T(centred ? centre : near);
+    }
     rec[Rec<T, D>::kAmp] = T(amplitude);
     reinterpret_cast<int*>(rec + Rec<T, D>::kIdx)[0] = index;
 }
@@ -356,6 +365,50 @@ __device__ __forceinline__ void stage_tile(const T* __restrict__ gaussians, int 
     }
     if (tid == 0) { counts[8] = centred_start; counts[9] = padded_total; }
     __syncthreads();
+}
+
+// Orders the LDS accesses of one wavefront's lanes among themselves (the hardware keeps them in program order).
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// stage_tile for ONE wavefront and its own LDS tile: the Gaussian of every lane (already derived; none in lanes with
+// active == false) becomes a record, shifted-form ones first, both groups padded with null records to a multiple of
+// GROUP.  The index of a record is the lane its Gaussian belongs to.  No workgroup barriers; the tile needs room for
+// 64 + 2 (GROUP - 1) records.
+struct WaveTile { int centred_start, padded_total; };
+
+template <typename T, int D, int GROUP>
+__device__ __forceinline__ WaveTile stage_wave_tile(const Derived<D>& dv, bool active, double amp_scale, T* lds, int lane) {
+    constexpr int S = Rec<T, D>::kStride;
+    const bool centred = active && !(dv.bound <= ShiftedBound<T>::v);
+    const unsigned long long mc = __ballot(centred), ms = __ballot(active && !centred);
+    const int shifted_total = __popcll(ms);
+    WaveTile t;
+    t.centred_start = (shifted_total + GROUP - 1) / GROUP * GROUP;
+    const int centred_end = t.centred_start + __popcll(mc);
+    t.padded_total = (centred_end + GROUP - 1) / GROUP * GROUP;
+    wave_fence();                                            // the tile's previous records have been read
+    if (active) {
+        const unsigned long long below = (1ull << lane) - 1ull;
+        const int slot = centred ? t.centred_start + __popcll(mc & below) : __popcll(ms & below);
+        store_record<T, D>(lds + slot * S, dv, centred, dv.w * dv.norm * amp_scale, lane);
+    }
+    if constexpr (GROUP > 1) {
+        int slot = -1;
+        if (lane < t.centred_start - shifted_total) slot = shifted_total + lane;
+        else if (lane >= GROUP && lane - GROUP < t.padded_total - centred_end) slot = centred_end + (lane - GROUP);
+        if (slot >= 0) {
+            T* rec = lds + slot * S;
+#pragma unroll
+            for (int i = 0; i < Rec<T, D>::kUsed; ++i) rec[i] = T(0);
+            reinterpret_cast<int*>(rec + Rec<T, D>::kIdx)[0] = -1;
+        }
+    }
+    wave_fence();
+    return t;
 }
 
 // ---- wavefront (64 lanes) sum; the total arrives in lane 63 -------------------------------------------

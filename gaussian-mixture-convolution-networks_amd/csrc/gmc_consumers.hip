@@ -17,13 +17,13 @@ int check_shape(const gmc_shape* s);
 
 constexpr int kTileC = 256;
 
-enum { kEpiReluShift = 1, kEpiRatio = 2, kEpiMoments = 3 };
+enum { kEpiStore = 0, kEpiReluShift = 1, kEpiRatio = 2, kEpiMoments = 3 };
 
 template <typename T> struct EpiArgs {
     const T* constant;     // [B][L]                     kinds 1, 3
     const T* goal;         // [B][L][N]                  kind 2
     const T* weights;      // [B][L][M], M == N          kind 2: x of the iteration, evaluated as |x|
-    T* out;                // [B][L][N]                  kinds 1, 2
+    T* out;                // [B][L][N]                  kinds 0, 1, 2
     double* moments;       // [B L][chunks][3] count, mean, sum of squared deviations from that mean   kind 3
 };
 
@@ -139,15 +139,148 @@ __global__ __launch_bounds__(kBlock) void consumer_fwd_kernel(const T* __restric
     }
 }
 
+// The same for few points and many Gaussians (a layer's convolved mixtures at the 128 centres of the fitted ones or at
+// 100 sampling positions).  The kernel above gives every wavefront a quarter of the points and all Gaussians: at 128
+// points an LDS record serves two pairs of a lane, and all four wavefronts wait for the preparation of every tile.
+// Here every wavefront holds ALL points (16 P, at most 256) and takes every fourth group of 64 Gaussians through its own
+// LDS tile, without a barrier until the four partial values of a point are added at the end.  Kind 0 is the plain
+// evaluation (gmc_dense.hip calls it), the only one with its Gaussians dealt to several workgroups (`ts`); its points
+// may be shared by mixtures (Bx, Lx).
+template <typename T, int D, int P, int KIND>
+__global__ __launch_bounds__(kBlock) void few_points_fwd_kernel(const T* __restrict__ mixture, const T* __restrict__ points,
+                                                                size_t mixture_stride, int point_stride, EpiArgs<T> epi,
+                                                                int L, int M, int N, int Bx, int Lx, int n_mixtures,
+                                                                bool covariance_form, TileSlices ts) {
+    constexpr int G = 1 + D + D * D;
+    constexpr int S = Rec<T, D>::kStride;
+    constexpr int kWaves = kBlock / kWave;
+    static_assert(16 * P <= kBlock, "one lane per point at the end");
+    constexpr int kWaveScalars = (kWave + 6) * S > 16 * P ? (kWave + 6) * S : 16 * P;
+    __shared__ __attribute__((aligned(16))) T lds[kWaves * kWaveScalars];
+    __shared__ double wave_moments[kWaves][2];
+    const T* exp2_tab = exp2_table<T>();
+    if constexpr (sizeof(T) == 8) __syncthreads();
+
+    int bl, slice;
+    map_workgroup(blockIdx.x, ts.slices, n_mixtures, bl, slice);
+    if (bl >= n_mixtures) return;
+    const int g_begin = slice * ts.tiles_per_slice * kTileC;
+    const int g_end = (g_begin + ts.tiles_per_slice * kTileC) < M ? (g_begin + ts.tiles_per_slice * kTileC) : M;
+    const int b = bl / L, l = bl - b * L;
+    const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
+    const T* __restrict__ mix_bl = mixture + size_t(bl) * M * G;
+    const T* __restrict__ x_bl = points + (size_t(xb) * Lx + xl) * mixture_stride;
+
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int row = lane >> 4, col = lane & 15;
+    T* tile = lds + wave * kWaveScalars;
+    T x[P][D];
+    T acc[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        int n = col + p * 16;
+        n = n < N ? n : N - 1;
+#pragma unroll
+        for (int d = 0; d < D; ++d) x[p][d] = x_bl[size_t(n) * point_stride + d];
+        acc[p] = T(0);
+    }
+    for (int g0 = g_begin + wave * kWave; g0 < g_end; g0 += kBlock) {
+        const bool active = g0 + lane < g_end;
+        const int m = active ? g0 + lane : g0;
+        Derived<D> dv = derive<T, D>(mix_bl + size_t(m) * G, covariance_form);
+        if (KIND == kEpiRatio) dv.w = fabs(double(epi.weights[size_t(bl) * M + m]));
+        const WaveTile t = stage_wave_tile<T, D, 4>(dv, active, 1.0, tile, lane);
+        rc_pairs<T, D, P, false>(tile, exp2_tab, 0, t.centred_start, row, x, acc);
+        rc_pairs<T, D, P, true>(tile, exp2_tab, t.centred_start, t.padded_total, row, x, acc);
+    }
+    wave_fence();
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        T v = acc[p];
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        if (row == 0) tile[col + p * 16] = v;
+    }
+    __syncthreads();
+    const int n = threadIdx.x;
+    const bool mine = n < N;
+    T v = T(0);
+    if (mine) v = (lds[n] + lds[kWaveScalars + n]) + (lds[2 * kWaveScalars + n] + lds[3 * kWaveScalars + n]);
+    const size_t at = size_t(bl) * N + n;
+    if constexpr (KIND == kEpiStore) {
+        if (mine) { if (ts.slices > 1) atomic_add(&epi.out[at], v); else epi.out[at] = v; }
+    } else if constexpr (KIND == kEpiReluShift) {
+        if (mine) {
+            const T c = epi.constant[bl];
+            const T shifted = v + c;
+            epi.out[at] = (shifted > T(0) ? shifted : T(0)) - (c > T(0) ? c : T(0));
+        }
+    } else if constexpr (KIND == kEpiRatio) {
+        if (mine) {
+            const T xw = epi.weights[at];                           // M == N: point n is the centre of component n
+            epi.out[at] = (xw < T(0) ? -xw : xw) * (epi.goal[at] + T(0.05)) / (v + T(0.05));
+        }
+    } else {
+        // mean, then squared deviations from it, of the workgroup's values (see the kernel above)
+        const double value = mine ? double(v) + double(epi.constant[bl]) : 0.0;
+        const double s1 = wave_sum_to_lane63(value);
+        if (lane == 63) wave_moments[wave][0] = s1;
+        __syncthreads();
+        const double mean = ((wave_moments[0][0] + wave_moments[1][0]) + (wave_moments[2][0] + wave_moments[3][0])) / double(N);
+        const double dv = value - mean;
+        const double m2 = wave_sum_to_lane63(mine ? dv * dv : 0.0);
+        if (lane == 63) wave_moments[wave][1] = m2;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double* o = epi.moments + size_t(bl) * 3;               // one record per mixture: one workgroup has all points
+            o[0] = double(N);
+            o[1] = mean;
+            o[2] = (wave_moments[0][1] + wave_moments[1][1]) + (wave_moments[2][1] + wave_moments[3][1]);
+        }
+    }
+}
+
 // points per lane and workgroups per mixture for N points per mixture
 static int consumer_points_per_lane(int N) { return N <= 128 ? 2 : N <= 256 ? 4 : 8; }
 static int consumer_chunks(int N) { const int P = consumer_points_per_lane(N); return (N + 64 * P - 1) / (64 * P); }
+
+// As few_points_fwd in gmc_dense.hip: more than two groups of Gaussians for the four wavefronts.  One workgroup has all
+// points: 1600 mixtures of 5120 Gaussians at 128 points 311 us (kernel above) / 259 us.
+static bool few_points_consumer(int M, int N) { return N <= 128 && M > 128; }
+
+template <typename T, int D, int KIND>
+static void launch_few_points(const T* mixture, const T* points, size_t mixture_stride, int point_stride, const EpiArgs<T>& epi,
+                              int B, int L, int M, int N, int Bx, int Lx, bool cov, TileSlices ts, hipStream_t stream) {
+    const size_t BL = size_t(B) * L;
+    const dim3 grid(unsigned(grid_mixtures(BL) * ts.slices));
+    const int P = (N + 15) / 16;
+#define GMC_FEW(PP) few_points_fwd_kernel<T, D, PP, KIND><<<grid, dim3(kBlock), 0, stream>>>(mixture, points, mixture_stride, point_stride, epi, L, M, N, Bx, Lx, int(BL), cov, ts)
+    if (P <= 2) GMC_FEW(2); else if (P <= 4) GMC_FEW(4); else if (P <= 6) GMC_FEW(6); else if (P == 7) GMC_FEW(7);
+    else if (P == 8) GMC_FEW(8);
+    else if constexpr (KIND == kEpiStore) { if (P <= 10) GMC_FEW(10); else if (P <= 13) GMC_FEW(13); else GMC_FEW(16); }
+#undef GMC_FEW
+}
+
+// The plain evaluation of mixtures with at most 256 points (gmc_dense.hip; `out` was cleared if there are slices).
+void few_points_forward(const void* mixture, const void* xes, void* out, const gmc_shape& s, bool cov, TileSlices ts,
+                        hipStream_t stream) {
+#define GMC_GO(T, DD) do { EpiArgs<T> e{nullptr, nullptr, nullptr, (T*)out, nullptr}; \
+        launch_few_points<T, DD, kEpiStore>((const T*)mixture, (const T*)xes, size_t(s.N) * DD, DD, e, s.B, s.L, s.M, s.N, s.Bx, s.Lx, cov, ts, stream); } while (0)
+    if (s.dtype == GMC_F32) { if (s.D == 2) GMC_GO(float, 2); else GMC_GO(float, 3); }
+    else { if (s.D == 2) GMC_GO(double, 2); else GMC_GO(double, 3); }
+#undef GMC_GO
+}
 
 template <typename T, int D, int KIND>
 static int launch_consumer(const T* mixture, const T* points, size_t mixture_stride, int point_stride, const EpiArgs<T>& epi,
                            int B, int L, int M, int N, hipStream_t stream) {
     const size_t BL = size_t(B) * L;
     if (BL == 0 || N == 0) return GMC_OK;
+    if (few_points_consumer(M, N)) {
+        launch_few_points<T, D, KIND>(mixture, points, mixture_stride, point_stride, epi, B, L, M, N, B, L, true,
+                                      TileSlices{1, (M + kTileC - 1) / kTileC}, stream);
+        return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
+    }
     const int P = consumer_points_per_lane(N);
     const int chunks = consumer_chunks(N);
     const dim3 grid(unsigned(grid_mixtures(BL) * chunks));

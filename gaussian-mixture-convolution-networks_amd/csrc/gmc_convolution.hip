@@ -133,12 +133,6 @@ constexpr int kConvWaves = 4;
 constexpr int kConvBlock = kConvWaves * kWave;
 constexpr int kConvDepth = 4;
 
-__device__ __forceinline__ void conv_wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <typename T, int D, bool NEED_DATA, bool NEED_KERNELS>
 __global__ __launch_bounds__(kConvBlock) void conv_bwd_fused_kernel(const T* __restrict__ grad_out, const T* __restrict__ data,
                                                                    const T* __restrict__ kernels, T* __restrict__ grad_data,
@@ -188,11 +182,11 @@ __global__ __launch_bounds__(kConvBlock) void conv_bwd_fused_kernel(const T* __r
     auto work = [&](int i, const T (&v)[G]) {
 #pragma unroll
         for (int r = 0; r < G; ++r) mine[lane + r * kWave] = lane + r * kWave < scalars ? v[r] : T(0);
-        conv_wave_fence();
+        wave_fence();
         T g[G];
 #pragma unroll
         for (int el = 0; el < G; ++el) g[el] = mine[lane * G + el];
-        conv_wave_fence();
+        wave_fence();
         if (NEED_DATA) {
             acc[0] = fma_(g[0], kernel_weight[i], acc[0]);
 #pragma unroll

@@ -33,6 +33,10 @@ static std::atomic<void*> scratch_address[kMaxDevices];
 bool dense_forward_f32(const float* mixture, const float* xes, float* out, const gmc_shape& s, bool covariance_form,
                        hipStream_t stream);
 
+// few points, many Gaussians (gmc_consumers.hip)
+void few_points_forward(const void* mixture, const void* xes, void* out, const gmc_shape& s, bool cov, TileSlices ts,
+                        hipStream_t stream);
+
 constexpr int kTile = 256;   // Gaussians staged per LDS tile (one per lane)
 
 template <typename T, int D, int P, bool CENTRED>
@@ -188,7 +192,8 @@ __global__ __launch_bounds__(kBlock) void eval_fwd_rc_kernel(const T* __restrict
 // copies of a tile's per-Gaussian sums in LDS: one per wavefront in float, a shared one in double (80 KB otherwise)
 template <typename T> struct SumCopies { static constexpr int k = sizeof(T) == 4 ? 4 : 1; };
 
-template <typename T, int D, int P, bool NEED_GM, bool NEED_GX, bool CENTRED>
+// OWN_SUMS: block_sums belongs to this wavefront alone, which meets every Gaussian of it once (plain stores).
+template <typename T, int D, int P, bool NEED_GM, bool NEED_GX, bool CENTRED, bool OWN_SUMS = (SumCopies<T>::k > 1)>
 __device__ __forceinline__ void bwd_rc_pairs(const T* __restrict__ lds, const T* __restrict__ tab,
                                              T* __restrict__ block_sums, int begin, int end, int row, const T (&x)[P][D],
                                              const T (&go)[P], T (&gx)[P][D]) {
@@ -288,7 +293,7 @@ __device__ __forceinline__ void bwd_rc_pairs(const T* __restrict__ lds, const T*
                     for (int i = 0; i < NR / 2; ++i) {
                         // float: every wavefront meets every Gaussian of a tile once and has its own copy of the sums,
                         // so a plain store does (LDS float atomics are serialised lane by lane); double: one copy
-                        if constexpr (SumCopies<T>::k > 1) dst[i] = half[i]; else atomic_add(&dst[i], half[i]);
+                        if constexpr (OWN_SUMS) dst[i] = half[i]; else atomic_add(&dst[i], half[i]);
                     }
                 }
             }
@@ -299,6 +304,9 @@ __device__ __forceinline__ void bwd_rc_pairs(const T* __restrict__ lds, const T*
 template <typename T, int D>
 __device__ __forceinline__ void bwd_epilogue_one(const T* __restrict__ g, const T* __restrict__ rs, T* __restrict__ o,
                                                  bool covariance_form);
+template <typename T, int D>
+__device__ __forceinline__ void bwd_epilogue_derived(const Derived<D>& dv, const double (&c)[D][D], const T* __restrict__ rs,
+                                                     T* __restrict__ o, bool covariance_form);
 
 // SOLE: the workgroup covers all points of its mixture (one chunk).  Its per-Gaussian sums are then final: they go
 // to `sums` with plain stores (no zero fill before the launch, no atomics) and the workgroup itself carries them on
@@ -434,9 +442,14 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
 template <typename T, int D>
 __device__ __forceinline__ void bwd_epilogue_one(const T* __restrict__ g, const T* __restrict__ rs, T* __restrict__ o,
                                                  bool covariance_form) {
-    const Derived<D> dv = derive<T, D>(g, covariance_form);
     double c[D][D];
-    load_inverse_covariance<T, D>(g + 1 + D, covariance_form, c);
+    const Derived<D> dv = derive<T, D>(g, covariance_form, c);
+    bwd_epilogue_derived<T, D>(dv, c, rs, o, covariance_form);
+}
+
+template <typename T, int D>
+__device__ __forceinline__ void bwd_epilogue_derived(const Derived<D>& dv, const double (&c)[D][D], const T* __restrict__ rs,
+                                                     T* __restrict__ o, bool covariance_form) {
     const double R0 = double(rs[0]);
     const double wn = dv.w * dv.norm;
     o[0] = T(dv.norm * R0);
@@ -551,6 +564,97 @@ __global__ __launch_bounds__(kBlock) void eval_bwd_epilogue_kernel(const T* __re
     bwd_epilogue_one<T, D>(mixture + i * G, sums + i * NR, grad_mixture + i * G, covariance_form);
 }
 
+// Backward pass of mixtures with few points (N <= 16 P, one wavefront's worth) and many Gaussians: a layer's convolved
+// mixtures at the centres of the fitted ones.  The kernel above gives the four wavefronts of a workgroup a quarter of
+// the points each, so at 128 points a row reduction (24 instructions in 2-D) serves two pairs per lane and the sums of
+// a Gaussian meet in LDS and, with tiles dealt over workgroups, in global memory.  Here every wavefront holds ALL
+// points and the wavefronts share the Gaussians, 64 at a time: four times fewer reductions per pair, the lane that
+// prepared a Gaussian finishes its gradient from the wavefront's own sums (no workspace, no atomics, no workgroup
+// barrier, no second preparation), and only dL/dx is added over wavefronts and slices at the end.  Bound by instruction
+// issue: 1600 mixtures of 5120 Gaussians at 128 points in 2-D 674 us (1.05e9 pairs, 42 cycles per 64 pairs and SIMD;
+// 1030 us with zero fill, pair kernel and epilogue before).
+template <typename T, int D, int P, bool NEED_GX>
+__global__ __launch_bounds__(kBlock) void few_points_bwd_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
+                                                                const T* __restrict__ xes, T* __restrict__ grad_xes,
+                                                                T* __restrict__ grad_mixture, int L, int M, int N, int Bx, int Lx,
+                                                                int xes_shared, int n_mixtures, bool covariance_form,
+                                                                TileSlices ts) {
+    constexpr int G = 1 + D + D * D;
+    constexpr int S = Rec<T, D>::kStride;
+    constexpr int NR = Sums<D>::k;
+    constexpr int kWaves = kBlock / kWave;
+    constexpr int kTileScalars = (kWave + 6) * S, kSumScalars = kWave * NR;
+    constexpr int kPointScalars = 16 * P * D;
+    constexpr int kWaveScalars = kTileScalars + kSumScalars > kPointScalars ? kTileScalars + kSumScalars : kPointScalars;
+    __shared__ __attribute__((aligned(16))) T lds[kWaves * kWaveScalars];
+    const T* exp2_tab = exp2_table<T>();
+    if constexpr (sizeof(T) == 8) __syncthreads();
+
+    int bl, slice;
+    map_workgroup(blockIdx.x, ts.slices, n_mixtures, bl, slice);
+    if (bl >= n_mixtures) return;
+    const int g_begin = slice * ts.tiles_per_slice * kTile;
+    const int g_end = (g_begin + ts.tiles_per_slice * kTile) < M ? (g_begin + ts.tiles_per_slice * kTile) : M;
+    const int b = bl / L, l = bl - b * L;
+    const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
+    const size_t x_off = (size_t(xb) * Lx + xl) * N;
+    const T* __restrict__ x_bl = xes + x_off * D;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int row = lane >> 4, col = lane & 15;
+    T* tile = lds + wave * kWaveScalars;
+    T* wave_sums = tile + kTileScalars;
+
+    T x[P][D], go[P], gx[P][D];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int n = col + p * 16;
+        const int nc = n < N ? n : N - 1;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            x[p][d] = x_bl[size_t(nc) * D + d];
+            gx[p][d] = T(0);
+        }
+        go[p] = n < N ? grad_out[size_t(bl) * N + nc] : T(0);
+    }
+    for (int g0 = g_begin + wave * kWave; g0 < g_end; g0 += kBlock) {
+        const bool active = g0 + lane < g_end;
+        const size_t at = size_t(bl) * M + (active ? g0 + lane : g0);
+        double c[D][D];
+        const Derived<D> dv = derive<T, D>(mixture + at * G, covariance_form, c);
+        const WaveTile t = stage_wave_tile<T, D, 4>(dv, active, 1.0 / kHalfLog2e, tile, lane);
+        bwd_rc_pairs<T, D, P, true, NEED_GX, false, true>(tile, exp2_tab, wave_sums, 0, t.centred_start, row, x, go, gx);
+        bwd_rc_pairs<T, D, P, true, NEED_GX, true, true>(tile, exp2_tab, wave_sums, t.centred_start, t.padded_total, row, x, go, gx);
+        wave_fence();
+        if (active) {
+            T rs[NR];
+#pragma unroll
+            for (int k = 0; k < NR; ++k) rs[k] = wave_sums[lane * NR + (k >> 1) + ((k & 1) ? NR / 2 : 0)];
+            bwd_epilogue_derived<T, D>(dv, c, rs, grad_mixture + at * G, covariance_form);
+        }
+    }
+    if (NEED_GX) {
+        // dL/dx: over the four rows of the wavefront, then over the wavefronts through LDS
+        wave_fence();
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                T v = gx[p][d];
+                v += __shfl_xor(v, 16, 64);
+                v += __shfl_xor(v, 32, 64);
+                if (row == 0) tile[(col + p * 16) * D + d] = v;
+            }
+        __syncthreads();
+        for (int i = threadIdx.x; i < N * D; i += kBlock) {
+            T v = T(0);
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) v += lds[w * kWaveScalars + i];
+            T* dst = grad_xes + x_off * D + i;
+            if (xes_shared) atomic_add(dst, -v); else *dst = -v;
+        }
+    }
+}
+
 // ---- host-side launchers ------------------------------------------------------------------------------
 
 static int pick_points_per_lane(int N, int BL, int tiles) {
@@ -607,11 +711,39 @@ static FwdPlan plan_fwd(const gmc_shape& s, bool is_double) {
     return plan;
 }
 
+// Shapes of the kernels that give every wavefront all points of a mixture (few_points_fwd_kernel, few_points_bwd_kernel):
+// at most 16 points per lane (8 in double), and more than two groups of 64 Gaussians to share out.  Measured, kernels
+// above / few-points kernels in us (float32, 2-D):
+//   mixtures x M at N points      forward        backward
+//   1600 x 5120 at 128            749 / 261     1030 / 674    (forward: the matrix-core kernel, whose blocks hold 1024 points)
+//   1200 x 1280 at 100            225 /  56      209 / 129
+//   320 x 1000 at 128            18.6 / 16.7    53.5 / 35.7
+//   1024 x 256 at 250            35.5 / 21.8    54.0 / 47.8
+//   1 x 256 at 128                7.1 /  6.3    18.1 / 11.6
+//   6000 x 129 at 250             138 /  70      163 / 178    (two of the four wavefronts nearly idle; in 3-D 170 / 106, 272 / 341)
+//   64 x 150 at 128               6.1 /  6.5    13.7 / 12.0    (forward: the 4 x 16 kernel)
+// hence three full groups, fewer only against the matrix-core forward kernel or with few points in the backward pass.
+// float64, 256 x 256 at 128: forward 11.8 / 14.4, backward 33.7 / 20.8; 64 x 256 at 64: 11.2 / 8.8 and 32.0 / 13.6.
+bool dense_forward_f32_takes(const gmc_shape& s);
+static bool few_points_fwd(const gmc_shape& s) {
+    if (s.dtype == GMC_F64) return s.M > 128 && s.N <= 64;
+    return s.N <= 256 && (s.M >= 192 || dense_forward_f32_takes(s));
+}
+static bool few_points_bwd(const gmc_shape& s) {
+    return s.N <= (s.dtype == GMC_F64 ? 128 : 256) && (s.M >= 256 || (s.M > 128 && s.N <= 128));
+}
+
 template <typename T, int D>
 static int launch_fwd(const T* mixture, const T* xes, T* out, const gmc_shape& s, bool cov, hipStream_t stream) {
     const size_t BL = size_t(s.B) * s.L;
     if (BL == 0 || s.N == 0) return GMC_OK;
     if (s.M == 0) { zero_async(out, BL * s.N, stream); return GMC_OK; }
+    if (few_points_fwd(s)) {
+        const TileSlices ts = plan_tile_slices(grid_mixtures(BL), s.M, kTile);
+        if (ts.slices > 1) zero_async(out, BL * s.N, stream);
+        few_points_forward(mixture, xes, out, s, cov, ts, stream);
+        return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
+    }
     if constexpr (std::is_same<T, float>::value) {
         if (dense_forward_f32(mixture, xes, out, s, cov, stream)) return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
     }
@@ -715,6 +847,26 @@ static void launch_bwd_main(const T* grad_out, const T* mixture, const T* xes, T
 #undef GMC_BWD
 }
 
+template <typename T, int D, bool GX>
+static void launch_few_points_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad_xes, T* grad_mixture,
+                                  const gmc_shape& s, bool xes_shared, bool cov, hipStream_t stream) {
+    const size_t BL = size_t(s.B) * s.L;
+    const int P = (s.N + 15) / 16;
+    const TileSlices ts = plan_tile_slices(grid_mixtures(BL), s.M, kTile);
+    const int gx_shared = (xes_shared || ts.slices > 1) ? 1 : 0;
+    if (GX && gx_shared) zero_async(grad_xes, size_t(s.Bx) * s.Lx * s.N * D, stream);
+    const dim3 grid(unsigned(grid_mixtures(BL) * ts.slices));
+#define GMC_FEW(PP) few_points_bwd_kernel<T, D, PP, GX><<<grid, dim3(kBlock), 0, stream>>>(grad_out, mixture, xes, grad_xes, grad_mixture, s.L, s.M, s.N, s.Bx, s.Lx, gx_shared, int(BL), cov, ts)
+    if constexpr (sizeof(T) == 4) {
+        if (P > 8) {
+            if (P <= 10) GMC_FEW(10); else if (P <= 13) GMC_FEW(13); else GMC_FEW(16);
+            return;
+        }
+    }
+    if (P <= 2) GMC_FEW(2); else if (P <= 4) GMC_FEW(4); else if (P <= 6) GMC_FEW(6); else if (P == 7) GMC_FEW(7); else GMC_FEW(8);
+#undef GMC_FEW
+}
+
 template <typename T, int D>
 static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad_mixture, T* grad_xes, T* sums,
                       const gmc_shape& s, bool need_gm, bool need_gx, bool cov, hipStream_t stream) {
@@ -727,6 +879,11 @@ static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad
     if (s.N == 0 || s.M == 0) {
         if (need_gm) zero_async(grad_mixture, n_gauss * G, stream);
         if (need_gx) zero_async(grad_xes, n_x, stream);
+        return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
+    }
+    if (need_gm && few_points_bwd(s)) {
+        if (need_gx) launch_few_points_bwd<T, D, true>(grad_out, mixture, xes, grad_xes, grad_mixture, s, xes_shared != 0, cov, stream);
+        else launch_few_points_bwd<T, D, false>(grad_out, mixture, xes, grad_xes, grad_mixture, s, xes_shared != 0, cov, stream);
         return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
     }
     const int P = bwd_points_per_lane<T, D>(s);
@@ -770,10 +927,9 @@ int dense_forward(const void* mixture, const void* xes, void* out, const gmc_sha
     return launch_fwd<double, 3>((const double*)mixture, (const double*)xes, (double*)out, s, cov, stream);
 }
 
-bool dense_forward_f32_takes(const gmc_shape& s);
-
 // Names of the kernels a call of this shape launches (the pair kernels; fills and epilogues aside), for reports.
 const char* dense_forward_kernel_name(const gmc_shape& s) {
+    if (few_points_fwd(s)) return "few_points_fwd_kernel";
     if (s.dtype == GMC_F32 && dense_forward_f32_takes(s)) return "eval_fwd_mfma_kernel";
     return plan_fwd(s, s.dtype == GMC_F64).rc > 0 ? "eval_fwd_rc_kernel" : "eval_fwd_kernel";
 }

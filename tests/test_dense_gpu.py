@@ -219,6 +219,26 @@ def test_one_chunk_per_mixture(dtype):
 
 
 @pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_few_points_many_gaussians(dtype, D):
+    """mixtures whose points all fit into one wavefront (16 per lane, 8 in double; the shape one beyond takes the general
+    kernels), with groups of 64 Gaussians that are full, ragged, or one for every wavefront, and with centred-form
+    Gaussians mixed in (positions up to 10 with narrow components)"""
+    n_max = 256 if dtype == torch.float32 else 128
+    shapes = [(1, 1, 129, 1), (2, 1, 192, 16), (1, 3, 193, 17), (1, 1, 256, 33), (2, 2, 300, 64), (1, 1, 511, 65),
+              (1, 2, 257, 97), (3, 1, 200, 112), (1, 1, 1000, 128), (2, 1, 140, 129), (1, 2, 320, 160), (1, 1, 150, 208),
+              (70, 1, 131, 20), (1, 1, 2100, n_max), (1, 2, 130, n_max + 1)]
+    for i, (B, L, M, N) in enumerate(shapes):
+        mix, xes, gout = _case(B, L, M, N, D, 61000 + i, broadcast=i % 3 == 2)
+        _check(mix, xes, gout, dtype, tag=f"B{B} L{L} M{M} N{N}")
+        mt, xt = torch.tensor(mix, dtype=dtype, device=DEV), torch.tensor(xes, dtype=dtype, device=DEV)
+        gt = torch.tensor(gout, dtype=dtype, device=DEV)
+        both = _native.eval_bwd(gt, mt, xt, True, True)[0]
+        alone = _native.eval_bwd(gt, mt, xt, True, False)[0]
+        assert rel_l2(alone.cpu().numpy(), both.cpu().numpy()) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("D", [2, 3])
 def test_matrix_core_forward_shapes(D):
     """float32 shapes that take the wide matrix-core forward kernel (more than 128 components and either many
     mixtures or many points): several 512-component tiles with a ragged last one, point counts that are no multiple
