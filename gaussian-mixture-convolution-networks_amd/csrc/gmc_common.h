@@ -498,11 +498,12 @@ inline size_t grid_mixtures(size_t n_mixtures) {
 // A launch with few workgroups (one large mixture, few point chunks) leaves most compute units idle, or with a single
 // wavefront per SIMD.  The LDS tiles of Gaussians of a mixture are then dealt to several workgroups per point chunk
 // ("slices"), which add their partial results with atomics into outputs that were cleared before.
-struct TileSlices { int slices, tiles_per_slice; };
+struct TileSlices { int slices, per_slice; };      // per_slice: Gaussians of a slice (the last one may have fewer)
 
+// Slices of whole LDS tiles, evenly filled: 1280 Gaussians in tiles of 512 are three slices of 432, not 1024 and 256.
 inline TileSlices plan_tile_slices(size_t workgroups, int M, int tile) {
     const int tiles = (M + tile - 1) / tile;
-    TileSlices t{1, tiles > 0 ? tiles : 1};
+    TileSlices t{1, M > 0 ? M : 1};
     // sixteen workgroups per compute unit: several scheduling rounds, so that the last one is short (measured on one
     // mixture of 16384 components and 100000 points: 1024 -> 1.80 / 3.96 ms forward / backward in float64, 4096 ->
     // 1.61 / 3.25 ms, no gain beyond; 2.49 / 6.35 ms without slices)
@@ -510,8 +511,10 @@ inline TileSlices plan_tile_slices(size_t workgroups, int M, int tile) {
     if (tiles <= 1 || workgroups == 0 || workgroups >= kWanted) return t;
     size_t want = (kWanted + workgroups - 1) / workgroups;
     if (want > size_t(tiles)) want = size_t(tiles);
-    t.tiles_per_slice = int((tiles + want - 1) / want);
-    t.slices = (tiles + t.tiles_per_slice - 1) / t.tiles_per_slice;
+    const int tiles_per_slice = tiles / int(want);
+    const int slices = (tiles + tiles_per_slice - 1) / tiles_per_slice;
+    t.per_slice = ((M + slices - 1) / slices + 15) / 16 * 16;
+    t.slices = (M + t.per_slice - 1) / t.per_slice;
     return t;
 }
 

@@ -164,8 +164,8 @@ __global__ __launch_bounds__(kBlock) void few_points_fwd_kernel(const T* __restr
     int bl, slice;
     map_workgroup(blockIdx.x, ts.slices, n_mixtures, bl, slice);
     if (bl >= n_mixtures) return;
-    const int g_begin = slice * ts.tiles_per_slice * kTileC;
-    const int g_end = (g_begin + ts.tiles_per_slice * kTileC) < M ? (g_begin + ts.tiles_per_slice * kTileC) : M;
+    const int g_begin = slice * ts.per_slice;
+    const int g_end = (g_begin + ts.per_slice) < M ? (g_begin + ts.per_slice) : M;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     const T* __restrict__ mix_bl = mixture + size_t(bl) * M * G;
@@ -278,7 +278,7 @@ static int launch_consumer(const T* mixture, const T* points, size_t mixture_str
     if (BL == 0 || N == 0) return GMC_OK;
     if (few_points_consumer(M, N)) {
         launch_few_points<T, D, KIND>(mixture, points, mixture_stride, point_stride, epi, B, L, M, N, B, L, true,
-                                      TileSlices{1, (M + kTileC - 1) / kTileC}, stream);
+                                      TileSlices{1, M}, stream);
         return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
     }
     const int P = consumer_points_per_lane(N);

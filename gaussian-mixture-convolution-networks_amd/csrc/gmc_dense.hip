@@ -73,8 +73,8 @@ __global__ __launch_bounds__(kBlock) void eval_fwd_kernel(const T* __restrict__ 
     if (bl >= n_mixtures) return;
     const int slice = chunk / chunks;
     chunk -= slice * chunks;
-    const int g_begin = slice * ts.tiles_per_slice * kTile;
-    const int g_end = (g_begin + ts.tiles_per_slice * kTile) < M ? (g_begin + ts.tiles_per_slice * kTile) : M;
+    const int g_begin = slice * ts.per_slice;
+    const int g_end = (g_begin + ts.per_slice) < M ? (g_begin + ts.per_slice) : M;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     const T* __restrict__ mix_bl = mixture + size_t(bl) * M * G;
@@ -146,8 +146,8 @@ __global__ __launch_bounds__(kBlock) void eval_fwd_rc_kernel(const T* __restrict
     if (bl >= n_mixtures) return;
     const int slice = chunk / chunks;
     chunk -= slice * chunks;
-    const int g_begin = slice * ts.tiles_per_slice * kTile;
-    const int g_end = (g_begin + ts.tiles_per_slice * kTile) < M ? (g_begin + ts.tiles_per_slice * kTile) : M;
+    const int g_begin = slice * ts.per_slice;
+    const int g_end = (g_begin + ts.per_slice) < M ? (g_begin + ts.per_slice) : M;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     const T* __restrict__ mix_bl = mixture + size_t(bl) * M * G;
@@ -308,7 +308,7 @@ template <typename T, int D>
 __device__ __forceinline__ void bwd_epilogue_derived(const Derived<D>& dv, const double (&c)[D][D], const T* __restrict__ rs,
                                                      T* __restrict__ o, bool covariance_form);
 
-// SOLE: the workgroup covers all points of its mixture (one chunk).  Its per-Gaussian sums are then final: they go
+// SOLE: the workgroup covers all points of its mixture (one chunk).  The sums of its Gaussians are then final: they go
 // to `sums` with plain stores (no zero fill before the launch, no atomics) and the workgroup itself carries them on
 // to grad_mixture at the end, which saves the fill and the epilogue launch of small problems.
 template <typename T, int D, int P, bool NEED_GM, bool NEED_GX, bool SOLE>
@@ -335,8 +335,8 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
     // (with several slices the host passes xes_shared != 0: dL/dx of a point then comes from several workgroups)
     const int slice = chunk / chunks;
     chunk -= slice * chunks;
-    const int g_begin = slice * ts.tiles_per_slice * kTile;
-    const int g_end = (g_begin + ts.tiles_per_slice * kTile) < M ? (g_begin + ts.tiles_per_slice * kTile) : M;
+    const int g_begin = slice * ts.per_slice;
+    const int g_end = (g_begin + ts.per_slice) < M ? (g_begin + ts.per_slice) : M;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     const T* __restrict__ mix_bl = mixture + size_t(bl) * M * G;
@@ -423,7 +423,7 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
     }
     if (NEED_GM && SOLE) {
         __syncthreads();            // the sums this workgroup stored are visible to all of its lanes
-        for (int i = threadIdx.x; i < M; i += kBlock) {
+        for (int i = g_begin + threadIdx.x; i < g_end; i += kBlock) {
             const size_t at = size_t(bl) * M + i;
             bwd_epilogue_one<T, D>(mixture + at * G, sums + at * NR, grad_mixture + at * G, covariance_form);
         }
@@ -593,8 +593,8 @@ __global__ __launch_bounds__(kBlock) void few_points_bwd_kernel(const T* __restr
     int bl, slice;
     map_workgroup(blockIdx.x, ts.slices, n_mixtures, bl, slice);
     if (bl >= n_mixtures) return;
-    const int g_begin = slice * ts.tiles_per_slice * kTile;
-    const int g_end = (g_begin + ts.tiles_per_slice * kTile) < M ? (g_begin + ts.tiles_per_slice * kTile) : M;
+    const int g_begin = slice * ts.per_slice;
+    const int g_end = (g_begin + ts.per_slice) < M ? (g_begin + ts.per_slice) : M;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     const size_t x_off = (size_t(xb) * Lx + xl) * N;
@@ -685,9 +685,50 @@ void set_tuning(int fwd_points_per_lane, int bwd_points_per_lane) {
     forced_bwd_points.store(bwd_points_per_lane);
 }
 
+// Launches that would not fill the chip (fewer than 2048 workgroups): points per lane and slices of Gaussians are
+// chosen together by the modelled time of the launch, in vector instructions of a wavefront.  A workgroup costs its
+// staging (per tile) and its steps of four Gaussians, each `pair` instructions per point and lane and `per_step` for the
+// rest (row reductions); a compute unit runs two workgroups in the time of one (a lone wavefront issues every second
+// slot), then ceil(workgroups / 256) after each other.  `clear`: the zero fill that slices need; `several_chunks`: the
+// zero fill and the epilogue launch of a backward pass whose sums come from several workgroups; `contended`: one more
+// addition to every dL/dx of points that all mixtures share (about 45 ns for each that meets on an address).  The plan
+// for full launches stays unless the model gives at least a tenth (three tenths against the
+// one-Gaussian-per-step layout).  Measured, full-launch plan / this one in us:
+//   15 x 333 Gaussians, 2777 points, float64, 3-D: forward 38.7 / 22.1, backward 100.9 / 52.9 (tiles of 256 and 77 before)
+//   3 x 540, 1058 points, float32, 2-D: 9.5 / 7.0 and 24.1 / 13.5;   60 x 79, 422 points, 3-D: forward 9.3 / 5.5
+struct LaunchCost {
+    double pair, per_step, clear, several_chunks, contended;
+    static constexpr double kStage = 900.0;
+
+    double of(int P, size_t chunks, size_t mixtures, int slices, int per) const {
+        const size_t rounds = (chunks * mixtures * slices + 255) / 256;
+        const double one = kStage * ((per + kTile - 1) / kTile) + (per + 3) / 4 * (P * pair + per_step);
+        return one * double(rounds < 2 ? 2 : rounds) + (slices > 1 ? clear : 0.0) + (chunks > 1 ? several_chunks : 0.0) +
+               contended * slices;
+    }
+};
+struct SmallPlan { int P; TileSlices ts; };
+
+static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int M, int N, int p_max, SmallPlan full, double to_beat) {
+    constexpr int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+    SmallPlan best = full;
+    double best_cost = to_beat;
+    for (int P = p_max; P >= 2; --P) {
+        const size_t chunks = (size_t(N) + 64 * P - 1) / (64 * P);
+        for (int want : kSlices) {
+            const int per = ((M + want - 1) / want + 3) / 4 * 4;
+            if (want > 1 && per < 32) break;
+            const int slices = (M + per - 1) / per;
+            const double cost = model.of(P, chunks, mixtures, slices, per < M ? per : M);
+            if (cost < best_cost) { best_cost = cost; best = SmallPlan{P, TileSlices{slices, per}}; }
+        }
+    }
+    return best;
+}
+
 // Which all-vector forward kernel a shape takes: `rc` > 0: the 4 x 16 layout with that many points per lane,
 // otherwise the one-Gaussian-per-step layout with `P` points per lane.
-struct FwdPlan { int P, chunks, rc; };
+struct FwdPlan { int P, chunks, rc; TileSlices ts; };
 
 static FwdPlan plan_fwd(const gmc_shape& s, bool is_double) {
     const size_t BL = size_t(s.B) * s.L;
@@ -708,6 +749,22 @@ static FwdPlan plan_fwd(const gmc_shape& s, bool is_double) {
     plan.rc = q_best;
     const int forced = forced_fwd_points.load();
     if (forced >= 2 && forced <= q_max) plan.rc = forced;
+    if (plan.rc > 0) plan.chunks = (s.N + 64 * plan.rc - 1) / (64 * plan.rc);
+    plan.ts = plan_tile_slices(grid_mixtures(BL) * plan.chunks, s.M, kTile);
+    if (BL * plan.chunks * plan.ts.slices < 2048 && forced < 2) {
+        const LaunchCost model{(s.D == 2 ? 9.0 : 13.0) + (is_double ? 16.0 : 0.0), 12.0, 1500.0, 0.0, 0.0};
+        const int per = plan.ts.per_slice < s.M ? plan.ts.per_slice : s.M;
+        // (the other layout: one Gaussian a step, 256 points per point of a lane)
+        const double full_cost = plan.rc > 0 ? model.of(plan.rc, plan.chunks, BL, plan.ts.slices, per)
+                                             : model.of(4 * plan.P, plan.chunks, BL, plan.ts.slices, per);
+        const SmallPlan small = plan_small_launch(model, BL, s.M, s.N, q_max, SmallPlan{0, plan.ts},
+                                                  (plan.rc > 0 ? 0.9 : 0.7) * full_cost);
+        if (small.P > 0) {
+            plan.rc = small.P;
+            plan.chunks = (s.N + 64 * plan.rc - 1) / (64 * plan.rc);
+            plan.ts = small.ts;
+        }
+    }
     return plan;
 }
 
@@ -749,15 +806,14 @@ static int launch_fwd(const T* mixture, const T* xes, T* out, const gmc_shape& s
     }
     const FwdPlan plan = plan_fwd(s, sizeof(T) == 8);
     const int P = plan.P, chunks = plan.chunks;
+    const TileSlices ts = plan.ts;
+    if (ts.slices > 1) zero_async(out, BL * s.N, stream);
+    const dim3 grid(unsigned(grid_mixtures(BL) * chunks * ts.slices));
     {
         constexpr int q_max = sizeof(T) == 8 ? 8 : 16;
         const int q_best = plan.rc;
         if (q_best > 0) {
-            const int q_chunks = (s.N + 64 * q_best - 1) / (64 * q_best);
-            const TileSlices ts = plan_tile_slices(grid_mixtures(BL) * q_chunks, s.M, kTile);
-            if (ts.slices > 1) zero_async(out, BL * s.N, stream);
-            const dim3 q_grid(unsigned(grid_mixtures(BL) * q_chunks * ts.slices));
-#define GMC_FWD_RC(QQ) case QQ: eval_fwd_rc_kernel<T, D, QQ><<<q_grid, dim3(kBlock), 0, stream>>>(mixture, xes, out, s.L, s.M, s.N, s.Bx, s.Lx, q_chunks, int(BL), cov, ts); break
+#define GMC_FWD_RC(QQ) case QQ: eval_fwd_rc_kernel<T, D, QQ><<<grid, dim3(kBlock), 0, stream>>>(mixture, xes, out, s.L, s.M, s.N, s.Bx, s.Lx, chunks, int(BL), cov, ts); break
             switch (q_best) {
                 GMC_FWD_RC(2); GMC_FWD_RC(3); GMC_FWD_RC(4); GMC_FWD_RC(5); GMC_FWD_RC(6); GMC_FWD_RC(7); GMC_FWD_RC(8);
                 default:
@@ -774,9 +830,6 @@ static int launch_fwd(const T* mixture, const T* xes, T* out, const gmc_shape& s
             return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
         }
     }
-    const TileSlices ts = plan_tile_slices(grid_mixtures(BL) * chunks, s.M, kTile);
-    if (ts.slices > 1) zero_async(out, BL * s.N, stream);
-    const dim3 grid(unsigned(grid_mixtures(BL) * chunks * ts.slices));
 #define GMC_FWD(PP) eval_fwd_kernel<T, D, PP><<<grid, dim3(kBlock), 0, stream>>>(mixture, xes, out, s.L, s.M, s.N, s.Bx, s.Lx, chunks, int(BL), cov, ts)
     switch (P) {
         case 8: GMC_FWD(8); break;
@@ -886,13 +939,22 @@ static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad
         else launch_few_points_bwd<T, D, false>(grad_out, mixture, xes, grad_xes, grad_mixture, s, xes_shared != 0, cov, stream);
         return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
     }
-    const int P = bwd_points_per_lane<T, D>(s);
+    int P = bwd_points_per_lane<T, D>(s);
     const size_t chunks = (size_t(s.N) + 64 * P - 1) / (64 * P);
-    const TileSlices ts = plan_tile_slices(grid_mixtures(BL) * chunks, s.M, kTile);
+    TileSlices ts = plan_tile_slices(grid_mixtures(BL) * chunks, s.M, kTile);
+    if (BL * chunks * ts.slices < 2048 && forced_bwd_points.load() < 2) {
+        const LaunchCost model{(D == 2 ? 20.0 : 32.0) + (sizeof(T) == 8 ? 16.0 : 0.0), (sizeof(T) == 8 ? 12.0 : 5.0) * Sums<D>::k,
+                               need_gx ? 1500.0 : 0.0, need_gm ? 3500.0 : 0.0,
+                               need_gx ? 30.0 * double(BL / (size_t(s.Bx) * s.Lx) - 1) : 0.0};
+        const double full_cost = model.of(P, chunks, BL, ts.slices, ts.per_slice < s.M ? ts.per_slice : s.M);
+        const SmallPlan small = plan_small_launch(model, BL, s.M, s.N, sizeof(T) == 8 ? 8 : 16, SmallPlan{P, ts}, 0.9 * full_cost);
+        P = small.P;
+        ts = small.ts;
+    }
     // several slices of Gaussian tiles per point chunk: dL/dx of a point is then added up over workgroups
     const int gx_shared = (xes_shared || ts.slices > 1) ? 1 : 0;
     // one chunk per mixture: the pair kernel's workgroups finish the gradient of their mixture themselves
-    const bool sole = need_gm && s.N <= 64 * P && ts.slices == 1;
+    const bool sole = need_gm && s.N <= 64 * P;
     if (need_gm && !sole) zero_async(sums, n_gauss * Sums<D>::k, stream);
     if (need_gx && gx_shared) zero_async(grad_xes, n_x, stream);
     if (sole && need_gx) launch_bwd_main<T, D, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream);

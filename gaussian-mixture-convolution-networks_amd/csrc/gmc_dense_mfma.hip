@@ -254,8 +254,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     // every partial result is added
     const int slice = chunk / chunks;
     chunk -= slice * chunks;
-    const int g_begin = slice * ts.tiles_per_slice * T;
-    const int g_end = (g_begin + ts.tiles_per_slice * T) < M ? (g_begin + ts.tiles_per_slice * T) : M;
+    const int g_begin = slice * ts.per_slice;
+    const int g_end = (g_begin + ts.per_slice) < M ? (g_begin + ts.per_slice) : M;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     const float* __restrict__ mix_bl = mixture + size_t(bl) * M * G;

@@ -220,6 +220,20 @@ def test_one_chunk_per_mixture(dtype):
 
 @pytest.mark.parametrize("D", [2, 3])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_small_launches_split_gaussians_below_a_tile(dtype, D):
+    """launches of few workgroups deal slices of any multiple of four Gaussians to them: ragged last slices, a single
+    Gaussian in one, one chunk of points with several slices (the workgroups finish their own Gaussians' gradients and
+    add to dL/dx), points that all mixtures share"""
+    shapes = [(1, 3, 333, 700), (2, 2, 97, 1300), (1, 1, 65, 3000), (1, 1, 129, 300), (1, 2, 253, 270), (3, 5, 77, 2000),
+              (1, 1, 33, 9000), (8, 2, 130, 520), (1, 1, 1000, 511)]
+    for i, (B, L, M, N) in enumerate(shapes):
+        for broadcast in (False, True):
+            mix, xes, gout = _case(B, L, M, N, D, 63000 + i, broadcast)
+            _check(mix, xes, gout, dtype, tag=f"B{B} L{L} M{M} N{N} broadcast {broadcast}")
+
+
+@pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_few_points_many_gaussians(dtype, D):
     """mixtures whose points all fit into one wavefront (16 per lane, 8 in double; the shape one beyond takes the general
     kernels), with groups of 64 Gaussians that are full, ragged, or one for every wavefront, and with centred-form
