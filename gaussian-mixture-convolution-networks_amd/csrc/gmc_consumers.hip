@@ -342,32 +342,66 @@ __global__ __launch_bounds__(kBlock) void moments_finish_kernel(const double* __
 
 // Sampling positions of BatchNorm (src/gmc/modules.py:394-400): the uniform numbers u [B][L][N][D] become positions in
 // the box of all centres of batch entry b (over layers and components), widened in 2-D by u * 1.3 - 0.15.  The
-// numbers of a batch entry are dealt to `chunks` workgroups, each of which finds the box itself (the centres are few
-// against the numbers, and a second launch or a scratch buffer for the box would cost more than reading them again).
+// numbers of a batch entry are dealt to `chunks` workgroups, each of which finds the box itself (a second launch or a
+// scratch buffer for the box would cost more).  Bound by the latency of reading the centres, which are many behind a
+// convolution: sixteen wavefronts with eight centres per lane in flight (100 batch entries of 81920 centres: 177 us with
+// four wavefronts and one centre in flight).
+constexpr int kSampleBlock = 1024;
+
 template <typename T, int D>
-__global__ __launch_bounds__(kBlock) void sampling_positions_kernel(const T* __restrict__ mixture, T* __restrict__ u,
-                                                                    int centres, size_t samples, int chunks) {
+__global__ __launch_bounds__(kSampleBlock) void sampling_positions_kernel(const T* __restrict__ mixture, T* __restrict__ u,
+                                                                          int centres, size_t samples, int chunks) {
     constexpr int G = 1 + D + D * D;
-    __shared__ T red[2 * D][kBlock];
+    constexpr int kFlight = 8;
+    __shared__ T red[2 * D][kSampleBlock / kWave];
     const int b = blockIdx.x / chunks, chunk = blockIdx.x - b * chunks;
     const T* mix_b = mixture + size_t(b) * centres * G;
     T lo[D], hi[D];
     for (int d = 0; d < D; ++d) { lo[d] = T(INFINITY); hi[d] = T(-INFINITY); }
-    for (int i = threadIdx.x; i < centres; i += kBlock)
-        for (int d = 0; d < D; ++d) {
-            const T v = mix_b[size_t(i) * G + 1 + d];
-            lo[d] = v < lo[d] ? v : lo[d];
-            hi[d] = v > hi[d] ? v : hi[d];
+    for (int i = threadIdx.x; i < centres; i += kFlight * kSampleBlock) {
+        T v[kFlight][D];
+#pragma unroll
+        for (int k = 0; k < kFlight; ++k) {
+            const int at = i + k * kSampleBlock < centres ? i + k * kSampleBlock : i;
+#pragma unroll
+            for (int d = 0; d < D; ++d) v[k][d] = mix_b[size_t(at) * G + 1 + d];
         }
-    block_bounds<T, D>(lo, hi, red);                         // red[d][0], red[D + d][0]: lower and upper bound of axis d
+#pragma unroll
+        for (int k = 0; k < kFlight; ++k)
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                lo[d] = v[k][d] < lo[d] ? v[k][d] : lo[d];
+                hi[d] = v[k][d] > hi[d] ? v[k][d] : hi[d];
+            }
+    }
+    const int wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        for (int off = 1; off < kWave; off <<= 1) {
+            const T l2 = __shfl_xor(lo[d], off, kWave), h2 = __shfl_xor(hi[d], off, kWave);
+            lo[d] = l2 < lo[d] ? l2 : lo[d];
+            hi[d] = h2 > hi[d] ? h2 : hi[d];
+        }
+        if ((threadIdx.x & 63) == 0) { red[d][wave] = lo[d]; red[D + d][wave] = hi[d]; }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        for (int w = 0; w < kSampleBlock / kWave; ++w) {
+            lo[d] = red[d][w] < lo[d] ? red[d][w] : lo[d];
+            hi[d] = red[D + d][w] > hi[d] ? red[D + d][w] : hi[d];
+        }
     T* u_b = u + size_t(b) * samples * D;
     const size_t n = samples * D, per = (n + chunks - 1) / chunks;
     const size_t begin = per * chunk, end = begin + per < n ? begin + per : n;
-    for (size_t i = begin + threadIdx.x; i < end; i += kBlock) {
+    for (size_t i = begin + threadIdx.x; i < end; i += kSampleBlock) {
         const int d = int(i % D);
+        T l = lo[0], h = hi[0];
+#pragma unroll
+        for (int k = 1; k < D; ++k) { l = d == k ? lo[k] : l; h = d == k ? hi[k] : h; }
         T v = u_b[i];
         if (D == 2) v = v * T(1.3) - T(0.15);
-        u_b[i] = v * (red[D + d][0] - red[d][0]) + red[d][0];
+        u_b[i] = v * (h - l) + l;
     }
 }
 
@@ -494,7 +528,7 @@ int gmc_batch_norm_sampling_positions(const void* mixture, void* uniform_in_posi
     const size_t wanted = (samples * shape->D + 16383) / 16384;
     const int chunks = int(wanted < 1 ? 1 : (wanted > 64 ? 64 : wanted));
     const dim3 grid{unsigned(shape->B) * unsigned(chunks)};
-#define GMC_SP(T, DD) gmc::sampling_positions_kernel<T, DD><<<grid, dim3(gmc::kBlock), 0, st>>>((const T*)mixture, (T*)uniform_in_positions_out, centres, samples, chunks)
+#define GMC_SP(T, DD) gmc::sampling_positions_kernel<T, DD><<<grid, dim3(gmc::kSampleBlock), 0, st>>>((const T*)mixture, (T*)uniform_in_positions_out, centres, samples, chunks)
     if (shape->dtype == GMC_F32) { if (shape->D == 2) GMC_SP(float, 2); else GMC_SP(float, 3); }
     else { if (shape->D == 2) GMC_SP(double, 2); else GMC_SP(double, 3); }
 #undef GMC_SP
