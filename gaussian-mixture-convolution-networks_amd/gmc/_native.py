@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(CSRC_DIR, "libgmc_hip.so")
 
 GMC_F32, GMC_F64 = 0, 1
 GMC_AABB_REFERENCE, GMC_AABB_TIGHT = 0, 1
-ABI_VERSION = 11
+ABI_VERSION = 12
 STATIC_SCRATCH_BYTES = 64 << 20
 
 
@@ -78,6 +78,10 @@ def lib() -> ctypes.CDLL:
     l.gmc_eval_cov_moments_bytes.argtypes = [shp]
     l.gmc_eval_cov_moments.argtypes = [vp, vp, vp, vp, sz, vp, vp, vp, vp, vp, ctypes.c_double, shp, ci, vp]
     l.gmc_batch_norm_sampling_positions.argtypes = [vp, vp, shp, vp]
+    l.gmc_scale_weights_chunks.restype = sz
+    l.gmc_scale_weights_chunks.argtypes = [shp]
+    l.gmc_scale_weights.argtypes = [vp, vp, vp, shp, ci, vp]
+    l.gmc_scale_weights_bwd.argtypes = [vp, vp, vp, vp, vp, shp, ci, vp]
     l.gmc_validate_mixture.argtypes = [vp, vp, shp, vp]
     cshp = ctypes.POINTER(ConvShape)
     l.gmc_convolution_fwd.argtypes = [vp, vp, vp, cshp, vp]
@@ -360,6 +364,42 @@ def batch_norm_sampling_positions(mixture: torch.Tensor, uniform: torch.Tensor) 
     with _on(mixture.device):
         check(lib().gmc_batch_norm_sampling_positions(_p(mixture), _p(uniform), ctypes.byref(shape), _stream(mixture.device)))
     return uniform
+
+
+def _scale_of(scale: torch.Tensor, mixture: torch.Tensor, shape: Shape) -> torch.Tensor:
+    if scale.dim() != 2 or scale.shape[0] not in (1, shape.B) or scale.shape[1] != shape.L:
+        raise RuntimeError("the scale must have shape [batch or 1, layers]")
+    return _like(scale, mixture, scale.shape, "scale")
+
+
+def scale_weights(mixture: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+    """the mixture with the weights of every (batch entry and) channel times their factor; scale [B or 1, L]"""
+    shape = _mixture_shape(mixture, 0)
+    scale = _scale_of(scale, mixture, shape)
+    out = torch.empty_like(mixture)
+    with _on(mixture.device):
+        check(lib().gmc_scale_weights(_p(mixture), _p(scale), _p(out), ctypes.byref(shape), int(scale.shape[0] == shape.B),
+                                      _stream(mixture.device)))
+    return out
+
+
+def scale_weights_bwd(grad_out: torch.Tensor, mixture: torch.Tensor, scale: torch.Tensor, need_mixture: bool, need_scale: bool):
+    """gradients of scale_weights (None where not needed)"""
+    shape = _mixture_shape(mixture, 0)
+    scale = _scale_of(scale, mixture, shape)
+    grad_out = _like(grad_out, mixture, mixture.shape, "grad_out")
+    grad_mixture = torch.empty_like(mixture) if need_mixture else None
+    partial = None
+    with _on(mixture.device):
+        if need_scale:
+            partial = torch.empty((shape.B, shape.L, int(lib().gmc_scale_weights_chunks(ctypes.byref(shape)))),
+                                  dtype=torch.float64, device=mixture.device)
+        check(lib().gmc_scale_weights_bwd(_p(grad_out), _p(mixture), _p(scale), _p(grad_mixture), _p(partial),
+                                          ctypes.byref(shape), int(scale.shape[0] == shape.B), _stream(mixture.device)))
+    if partial is None:
+        return grad_mixture, None
+    grad_scale = partial.sum((0, 2)).unsqueeze(0) if scale.shape[0] == 1 else partial.sum(2)
+    return grad_mixture, grad_scale.to(mixture.dtype)
 
 
 # ---------------------------------------------------------------------------------------------------------------

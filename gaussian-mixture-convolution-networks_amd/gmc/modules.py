@@ -17,6 +17,47 @@ def convolve(x: Tensor, kernels: Tensor) -> Tensor:
     return cpp_convolution.apply(x, kernels)
 
 
+def _scale_weights_composed(x_gm: Tensor, scaling: Tensor) -> Tensor:
+    return torch.cat((gm.weights(x_gm).unsqueeze(-1) * scaling.unsqueeze(-1).unsqueeze(-1), x_gm[..., 1:]), dim=-1)
+
+
+class _ScaleWeights(torch.autograd.Function):
+    """_scale_weights_composed as one pass over the mixture in either direction; a backward pass that is itself
+    differentiated is composed of torch operations"""
+
+    @staticmethod
+    def forward(ctx, x_gm: Tensor, scaling: Tensor) -> Tensor:
+        ctx.save_for_backward(x_gm, scaling)
+        return _native.scale_weights(x_gm.contiguous(), scaling)
+
+    @staticmethod
+    def backward(ctx, grad_out: Tensor):
+        x_gm, scaling = ctx.saved_tensors
+        need_gm, need_scaling = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            grad_gm = _scale_weights_composed(grad_out, scaling) if need_gm else None
+            grad_scaling = None
+            if need_scaling:
+                grad_scaling = (grad_out[..., 0] * gm.weights(x_gm)).sum(-1)
+                if scaling.shape[0] == 1:
+                    grad_scaling = grad_scaling.sum(0, keepdim=True)
+            return grad_gm, grad_scaling
+        return _native.scale_weights_bwd(grad_out.contiguous(), x_gm.contiguous(), scaling, need_gm, need_scaling)
+
+
+def _scale_weights(x_gm: Tensor, scaling: Tensor) -> Tensor:
+    """x_gm with its weights times scaling [batch or 1, channels].  The kernels take plain device tensors; others (CPU
+    tensors, other types, subclasses, tracing, functorch and forward-mode transforms) go through torch operations."""
+    plain = not torch.compiler.is_compiling() and \
+        type(x_gm) in (Tensor, torch.nn.Parameter) and type(scaling) in (Tensor, torch.nn.Parameter) and \
+        x_gm.is_cuda and scaling.device == x_gm.device and x_gm.dtype in (torch.float32, torch.float64) and \
+        scaling.dtype == x_gm.dtype and x_gm.dim() == 4 and x_gm.shape[-1] in (7, 13) and \
+        not torch.jit.is_tracing() and \
+        not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0 and \
+        torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+    return _ScaleWeights.apply(x_gm, scaling) if plain else _scale_weights_composed(x_gm, scaling)
+
+
 class BatchNorm(torch.nn.Module):
     """Scales the weights of every channel such that the sampled values of the mixture (plus constant) have unit
     standard deviation, and takes the sampled mean off the constant.
@@ -90,5 +131,4 @@ class BatchNorm(torch.nn.Module):
         scaling = scaling.view(-1, n_channels, 1)
         if validate and not bool(torch.isfinite(scaling).all()):
             raise RuntimeError("BatchNorm: the scaling is not finite")
-        scaled = torch.cat((gm.weights(x_gm).unsqueeze(-1) * scaling.unsqueeze(-1), x_gm[..., 1:]), dim=-1)
-        return scaled, x_constant - mean
+        return _scale_weights(x_gm, scaling.squeeze(-1)), x_constant - mean

@@ -152,6 +152,15 @@ int gmc_eval_cov_moments(const void* mixture, const void* constant, const void* 
  * place, into positions inside the box of all centres of their batch entry (2-D: widened by u * 1.3 - 0.15). */
 int gmc_batch_norm_sampling_positions(const void* mixture, void* uniform_in_positions_out, const gmc_shape* shape, void* stream);
 
+/* BatchNorm's scaling of the weights, src/gmc/modules.py:417-421: out = mixture [B][L][M] with every weight times
+ * scale[l] (scale_per_batch 0) or scale[b][l]; shape->N, Bx, Lx as for a call with one set of points per mixture (N may
+ * be 0).  Backward: grad_mixture (may be NULL) and partial (may be NULL), double [B][L][gmc_scale_weights_chunks], whose
+ * sum over the last axis (and over b for a scale per channel) is the gradient of the scale. */
+size_t gmc_scale_weights_chunks(const gmc_shape* shape);
+int gmc_scale_weights(const void* mixture, const void* scale, void* out, const gmc_shape* shape, int scale_per_batch, void* stream);
+int gmc_scale_weights_bwd(const void* grad_out, const void* mixture, const void* scale, void* grad_mixture, double* partial,
+                          const gmc_shape* shape, int scale_per_batch, void* stream);
+
 /* Optional input check, the reference's check_mixture (src/gmc/cpp/extensions/util/mixture.h:85-93, called by its CUDA
  * backward): flags[0] (device int32, cleared inside) |= 1 if the mixture holds a NaN or an infinity, |= 2 if a
  * matrix has a determinant <= 0.  One small launch; the caller decides when to read the flag back. */

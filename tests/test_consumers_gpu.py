@@ -374,6 +374,35 @@ def test_batch_norm_sampling_positions_and_running_averages():
     assert torch.allclose(inv, torch.full((2, 2), 1000.0, device=DEV), rtol=1e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("D", [2, 3])
+def test_batch_norm_scaling_of_the_weights(D, dtype):
+    """one pass over the mixture in either direction against the torch composition: component counts whose mixtures
+    start at multiples of 16 bytes and ones that do not, several chunks of a mixture, factors per channel and per batch
+    entry, a mixture that starts off a 16-byte boundary, strided inputs, and a backward pass that is differentiated"""
+    gen = torch.Generator(device=DEV).manual_seed(17)
+    G = 1 + D + D * D
+    for B, L, M in ((1, 1, 1), (3, 2, 4), (2, 3, 7), (1, 2, 1501), (5, 1, 3000), (2, 2, 0)):
+        flat = torch.randn(B * L * M * G + 1, generator=gen, device=DEV, dtype=dtype)
+        for x0 in (flat[:-1].view(B, L, M, G), flat[1:].view(B, L, M, G), flat[:-1].view(L, B, M, G).transpose(0, 1)):
+            g = torch.randn(B, L, M, G, generator=gen, device=DEV, dtype=dtype)
+            for S in (1, B):
+                s0 = torch.randn(S, L, generator=gen, device=DEV, dtype=dtype)
+                results = []
+                for fn in (modules._scale_weights, modules._scale_weights_composed):
+                    x, s = x0.detach().requires_grad_(True), s0.clone().requires_grad_(True)
+                    out = fn(x, s)
+                    results.append((out, *torch.autograd.grad(out, (x, s), g)))
+                (out, gx, gs), (rout, rgx, rgs) = results
+                assert torch.equal(out, rout) and torch.equal(gx, rgx)          # one product per weight
+                assert rel_l2(gs.cpu().numpy(), rgs.double().cpu().numpy(), 1e-30) <= TOL[dtype]
+    x = torch.randn(2, 2, 5, G, generator=gen, device=DEV, dtype=torch.float64, requires_grad=True)
+    s = torch.randn(1, 2, generator=gen, device=DEV, dtype=torch.float64, requires_grad=True)
+    assert torch.autograd.gradgradcheck(modules._scale_weights, (x, s))
+    tangent = torch.func.jvp(lambda t: modules._scale_weights(x.detach(), t), (s.detach(),), (torch.ones_like(s),))[1]
+    assert torch.equal(tangent[..., 0], x[..., 0]) and not tangent[..., 1:].any()
+
+
 def test_validate_flag_raises_like_the_reference_check():
     """util/mixture.h:85-93 (called by the reference's CUDA backward), off by default here: with validate=True NaNs,
     infinities and matrices with a determinant <= 0 raise RuntimeError; without it nothing is checked (and nothing
