@@ -632,9 +632,9 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The leaves' sort for one large tree (kSmallTreeMax < M <= kBucketSortMax; two trees of up to half that size, whose
-// workgroups fit a compute unit in pairs: more would queue up) in ONE launch instead of four radix
-// passes at their latency floor: 256 workgroups per tree, one per value of the top 8 key bits.  Workgroup d reads all
+// The leaves' sort for a few large trees (kSmallTreeMax < M <= kBucketSortMax) in ONE launch instead of four radix
+// passes at their latency floor: 2^bits workgroups per tree, one per value of the top `bits` key bits (8 for one or two
+// trees, 7 for up to four, 6 for up to eight, so that the launch is resident at once).  Workgroup d reads all
 // keys of the tree (in component order, as the Morton kernel wrote them; 64 KB at most, from L2), keeps those whose top
 // bits are d as unique keys (Morton code << 32 | component) in LDS, counts those with smaller top bits -- the first
 // slot of its own --, sorts its keys (by counting ranks; more than kBucketRankMax: a bitonic network) and writes them out: ascending
@@ -648,12 +648,13 @@ constexpr int kBucketCrowded = 1024;       // expected keys of one value of the 
 
 template <int CAP>
 __global__ __launch_bounds__(kBucketSortLanes) void bucket_sort_kernel(const uint32_t* __restrict__ keys_in, uint32_t* __restrict__ keys_out,
-                                                                      uint32_t* __restrict__ vals_out, int count, int* __restrict__ err) {
+                                                                      uint32_t* __restrict__ vals_out, int count, int bits,
+                                                                      int* __restrict__ err) {
     constexpr int kPerLane = CAP / kBucketSortLanes;         // keys of the tree per lane, at most
     __shared__ unsigned long long k[CAP];
     __shared__ int n_mine, n_before;
-    const int seg = blockIdx.x >> 8, lane = threadIdx.x & 63;
-    const uint32_t digit = blockIdx.x & 255;
+    const int seg = blockIdx.x >> bits, lane = threadIdx.x & 63, shift = 30 - bits;
+    const uint32_t digit = blockIdx.x & ((1u << bits) - 1u);
     const uint32_t* in = keys_in + size_t(seg) * count;
     if (threadIdx.x == 0) { n_mine = 0; n_before = 0; }
     static_assert(kPerLane % 4 == 0 || kPerLane == 2, "keys are fetched four (two) at a time");
@@ -698,7 +699,7 @@ __global__ __launch_bounds__(kBucketSortLanes) void bucket_sort_kernel(const uin
         for (int r = 1; r < kPerLane; ++r)
             if (int(threadIdx.x >> 3) % kPerLane == r) { mine = key[r]; r_mine = r; }
         const int i = component(r_mine);
-        if (i < count) atomicAdd(&sample_bins[(mine >> 22) & 255u], 1u);
+        if (i < count) atomicAdd(&sample_bins[(mine >> shift) & 255u], 1u);
         if ((threadIdx.x & 3) == ((threadIdx.x >> 5) & 3))
             sample[threadIdx.x >> 2] = i < count ? ((unsigned long long)mine << 32) | uint32_t(i) : ~0ull;
     }
@@ -720,11 +721,11 @@ __global__ __launch_bounds__(kBucketSortLanes) void bucket_sort_kernel(const uin
 #pragma unroll
         for (int step = 128; step > 0; step >>= 1)
             lo = splitter[lo + step] <= x ? lo + step : lo;
-        return uint32_t(lo);
+        return uint32_t(lo) >> (8 - bits);
     };
     uint32_t top[kPerLane];
 #pragma unroll
-    for (int r = 0; r < kPerLane; ++r) top[r] = key[r] >> 22;
+    for (int r = 0; r < kPerLane; ++r) top[r] = key[r] >> shift;
     if (crowded) {                                           // (the searches of a lane's keys side by side)
 #pragma unroll
         for (int r = 0; r < kPerLane; ++r) {
@@ -2634,9 +2635,9 @@ static int bvh_build_t(const T* mixture, const T* xes, char* bvh, const gmc_shap
     SortJob jg0, jp0;
     jobs_of_pass(0, jg0, jp0);
     MortonJob<T> mg = {}, mp = {};
-    // one or two large trees: every value of the top 8 key bits gathered and sorted in LDS (bucket_sort_kernel)
-    const bool bucket_sort = have_g && g_build_path != 2 && M > kSmallTreeMax && M <= kBucketSortMax &&
-                             (BL == 1 || (BL == 2 && M <= kBucketSortMax / 2));
+    // a few large trees: every value of the top key bits gathered and sorted in LDS (bucket_sort_kernel)
+    const int bucket_bits = BL <= 2 ? 8 : BL <= 4 ? 7 : 6;
+    const bool bucket_sort = have_g && g_build_path != 2 && M > kSmallTreeMax && M <= kBucketSortMax && BL <= 8;
     // (a Morton workgroup per block of the first radix pass; without a radix sort behind it: 256 keys each)
     if (have_g) mg = MortonJob<T>{mixture, G, 1, M, bucket_sort ? 1 : jg0.items, bucket_sort ? bpm : jg0.blocks_per_seg, parts_g, bpm, ka, va,
                                   unsigned(BL * (bucket_sort ? bpm : jg0.blocks_per_seg)), bucket_sort ? nullptr : (uint32_t*)jg0.hist, jg0.shift};
@@ -2661,12 +2662,12 @@ static int bvh_build_t(const T* mixture, const T* xes, char* bvh, const gmc_shap
         radix_scatter_kernel<<<dim3(jg.blocks), dim3(kBlock), 0, st>>>(jg, none);
     }
     if (bucket_sort) {
-        const dim3 grid{unsigned(BL * 256)}, block{unsigned(kBucketSortLanes)};
+        const dim3 grid{unsigned(BL << bucket_bits)}, block{unsigned(kBucketSortLanes)};
         int* err = (int*)(bvh + lay.cand_ctl) + 2;
-        if (M <= 2048) bucket_sort_kernel<2048><<<grid, block, 0, st>>>(ka, g_keys, g_order, M, err);
-        else if (M <= 4096) bucket_sort_kernel<4096><<<grid, block, 0, st>>>(ka, g_keys, g_order, M, err);
-        else if (M <= 8192) bucket_sort_kernel<8192><<<grid, block, 0, st>>>(ka, g_keys, g_order, M, err);
-        else bucket_sort_kernel<16384><<<grid, block, 0, st>>>(ka, g_keys, g_order, M, err);
+        if (M <= 2048) bucket_sort_kernel<2048><<<grid, block, 0, st>>>(ka, g_keys, g_order, M, bucket_bits, err);
+        else if (M <= 4096) bucket_sort_kernel<4096><<<grid, block, 0, st>>>(ka, g_keys, g_order, M, bucket_bits, err);
+        else if (M <= 8192) bucket_sort_kernel<8192><<<grid, block, 0, st>>>(ka, g_keys, g_order, M, bucket_bits, err);
+        else bucket_sort_kernel<16384><<<grid, block, 0, st>>>(ka, g_keys, g_order, M, bucket_bits, err);
     }
     if (!have_g) {                                   // no trees to build: the points' passes are launches of their own
         if (jp_first.blocks > 0) radix_scatter_kernel<<<dim3(jp_first.blocks), dim3(kBlock), 0, st>>>(jp_first, none);
