@@ -405,6 +405,74 @@ __global__ __launch_bounds__(kSampleBlock) void sampling_positions_kernel(const 
     }
 }
 
+// Element-wise part of the gradient of one fixed-point iteration (src/gmc/fitting.py:296-311), which sits between the
+// evaluations: x1 = x0 (b + 0.05) / c with x0 = |w| + 0.1, b = relu(v + constant) - relu(constant) and
+// c = current + 0.05.  As torch operations these were about forty launches over [B][L][N] values (0.2 ms of a layer's
+// backward pass, all of it launch latency).
+//   prepare: the upstream gradients of both evaluations, d_v = d_b [v + constant > 0] with d_b = d_x1 x0 / c and
+//            d_current = -d_x1 x0 ((b + 0.05) / c) / c, and the gradient of the constant, one workgroup per mixture;
+//   finish:  grad_out + [sign(w) (d_x1 (b + 0.05) / c + g_weight), sum of the centres' gradients, covariance gradient].
+template <typename T, int D>
+__global__ __launch_bounds__(kBlock) void relu_fit_prepare_kernel(const T* __restrict__ grad_out, const T* __restrict__ fit,
+                                                                  const T* __restrict__ goal, const T* __restrict__ current,
+                                                                  const T* __restrict__ constant, T* __restrict__ d_v,
+                                                                  T* __restrict__ d_current, T* __restrict__ grad_constant, int N) {
+    constexpr int G = 1 + D + D * D;
+    __shared__ double wave_sums[kBlock / kWave];
+    const T c0 = constant[blockIdx.x];
+    const T relu_c = c0 > T(0) ? c0 : (c0 == c0 ? T(0) : c0);
+    double acc = 0.0;
+    for (int n = threadIdx.x; n < N; n += kBlock) {
+        const size_t at = size_t(blockIdx.x) * N + n;
+        const T w = fit[at * G], d_x1 = grad_out[at * G], b = goal[at];
+        const T x0 = fabs(w) + T(0.1), c = current[at] + T(0.05);
+        const T d_b = d_x1 * x0 / c;
+        const bool lifted = b + relu_c > T(0);
+        d_v[at] = d_b * T(lifted);                       // (a NaN stays one)
+        d_current[at] = -d_x1 * x0 * ((b + T(0.05)) / c) / c;
+        acc += double(d_b * (T(lifted) - T(c0 > T(0))));
+    }
+    if (!grad_constant) return;
+    acc = wave_sum_to_lane63(acc);
+    if ((threadIdx.x & 63) == 63) wave_sums[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) grad_constant[blockIdx.x] = T((wave_sums[0] + wave_sums[1]) + (wave_sums[2] + wave_sums[3]));
+}
+
+template <typename T, int D>
+__global__ __launch_bounds__(kBlock) void relu_fit_finish_kernel(const T* __restrict__ grad_out, const T* __restrict__ fit,
+                                                                 const T* __restrict__ goal, const T* __restrict__ current,
+                                                                 const T* __restrict__ g_abs, const T* __restrict__ g_centres,
+                                                                 const T* __restrict__ g_centres2, T* __restrict__ grad_fit, size_t n) {
+    constexpr int G = 1 + D + D * D;
+    const size_t i = size_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const T* go = grad_out + i * G;
+    const T* ga = g_abs + i * G;
+    T* o = grad_fit + i * G;
+    const T w = fit[i * G];
+    const T sign = w > T(0) ? T(1) : (w < T(0) ? T(-1) : w);
+    o[0] = sign * (go[0] * ((goal[i] + T(0.05)) / (current[i] + T(0.05))) + ga[0]);
+#pragma unroll
+    for (int d = 0; d < D; ++d) o[1 + d] = go[1 + d] + ((ga[1 + d] + g_centres[i * D + d]) + g_centres2[i * D + d]);
+#pragma unroll
+    for (int k = 1 + D; k < G; ++k) o[k] = go[k] + ga[k];
+}
+
+// The fitting mixture with the iteration's weights in front of it (|w| + 0.1) and, packed, its centres.
+template <typename T, int D>
+__global__ __launch_bounds__(kBlock) void relu_fit_start_kernel(const T* __restrict__ fit, T* __restrict__ fit_abs,
+                                                                T* __restrict__ centres, size_t n) {
+    constexpr int G = 1 + D + D * D;
+    const size_t i = size_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (i >= n) return;
+    fit_abs[i * G] = fabs(fit[i * G]) + T(0.1);
+#pragma unroll
+    for (int k = 1; k < G; ++k) fit_abs[i * G + k] = fit[i * G + k];
+#pragma unroll
+    for (int d = 0; d < D; ++d) centres[i * D + d] = fit[i * G + 1 + d];
+}
+
 // BatchNorm's scaling of the weights (src/gmc/modules.py:417-421): out = mixture with every weight times the factor of its
 // (batch entry and) channel, and its gradients.  One pass over the mixture each, bound by HBM: a workgroup walks over a
 // chunk of one mixture's scalars, so that the factor is uniform, VEC scalars at a time.  (As torch operations -- slice,
@@ -605,6 +673,49 @@ int gmc_batch_norm_sampling_positions(const void* mixture, void* uniform_in_posi
 #undef GMC_SP
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
 }
+
+#define GMC_FIT(KERNEL, GRID, ...) do { \
+        const dim3 grid{unsigned(GRID)}, block{gmc::kBlock}; \
+        if (shape->dtype == GMC_F32) { using T = float; if (shape->D == 2) gmc::KERNEL<T, 2><<<grid, block, 0, st>>>(__VA_ARGS__); else gmc::KERNEL<T, 3><<<grid, block, 0, st>>>(__VA_ARGS__); } \
+        else { using T = double; if (shape->D == 2) gmc::KERNEL<T, 2><<<grid, block, 0, st>>>(__VA_ARGS__); else gmc::KERNEL<T, 3><<<grid, block, 0, st>>>(__VA_ARGS__); } \
+        return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH; } while (0)
+
+int gmc_relu_fit_grad_start(const void* fitting_mixture, void* fitting_abs, void* centres, const gmc_shape* shape, void* stream) {
+    const int rc = consumer_shape(shape);
+    if (rc != GMC_OK) return rc;
+    const size_t n = size_t(shape->B) * shape->L * shape->N;
+    if (n == 0) return GMC_OK;
+    if (!fitting_mixture || !fitting_abs || !centres) return GMC_E_NULL;
+    hipStream_t st = (hipStream_t)stream;
+    GMC_FIT(relu_fit_start_kernel, (n + gmc::kBlock - 1) / gmc::kBlock, (const T*)fitting_mixture, (T*)fitting_abs, (T*)centres, n);
+}
+
+int gmc_relu_fit_grad_prepare(const void* grad_out, const void* fitting_mixture, const void* goal, const void* current,
+                              const void* constant, void* d_value, void* d_current, void* grad_constant, const gmc_shape* shape,
+                              void* stream) {
+    const int rc = consumer_shape(shape);
+    if (rc != GMC_OK) return rc;
+    const size_t BL = size_t(shape->B) * shape->L;
+    if (BL == 0) return GMC_OK;
+    if (!constant || (shape->N > 0 && (!grad_out || !fitting_mixture || !goal || !current || !d_value || !d_current))) return GMC_E_NULL;
+    hipStream_t st = (hipStream_t)stream;
+    GMC_FIT(relu_fit_prepare_kernel, BL, (const T*)grad_out, (const T*)fitting_mixture, (const T*)goal, (const T*)current,
+            (const T*)constant, (T*)d_value, (T*)d_current, (T*)grad_constant, shape->N);
+}
+
+int gmc_relu_fit_grad_finish(const void* grad_out, const void* fitting_mixture, const void* goal, const void* current,
+                             const void* grad_abs, const void* grad_centres, const void* grad_centres2, void* grad_fitting,
+                             const gmc_shape* shape, void* stream) {
+    const int rc = consumer_shape(shape);
+    if (rc != GMC_OK) return rc;
+    const size_t n = size_t(shape->B) * shape->L * shape->N;
+    if (n == 0) return GMC_OK;
+    if (!grad_out || !fitting_mixture || !goal || !current || !grad_abs || !grad_centres || !grad_centres2 || !grad_fitting) return GMC_E_NULL;
+    hipStream_t st = (hipStream_t)stream;
+    GMC_FIT(relu_fit_finish_kernel, (n + gmc::kBlock - 1) / gmc::kBlock, (const T*)grad_out, (const T*)fitting_mixture, (const T*)goal,
+            (const T*)current, (const T*)grad_abs, (const T*)grad_centres, (const T*)grad_centres2, (T*)grad_fitting, n);
+}
+#undef GMC_FIT
 
 size_t gmc_scale_weights_chunks(const gmc_shape* shape) {
     return consumer_shape(shape) == GMC_OK ? size_t(gmc::scale_weights_chunks(*shape)) : 0;

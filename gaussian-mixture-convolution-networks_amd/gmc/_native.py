@@ -78,6 +78,9 @@ def lib() -> ctypes.CDLL:
     l.gmc_eval_cov_moments_bytes.argtypes = [shp]
     l.gmc_eval_cov_moments.argtypes = [vp, vp, vp, vp, sz, vp, vp, vp, vp, vp, ctypes.c_double, shp, ci, vp]
     l.gmc_batch_norm_sampling_positions.argtypes = [vp, vp, shp, vp]
+    l.gmc_relu_fit_grad_start.argtypes = [vp, vp, vp, shp, vp]
+    l.gmc_relu_fit_grad_prepare.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, shp, vp]
+    l.gmc_relu_fit_grad_finish.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, shp, vp]
     l.gmc_scale_weights_chunks.restype = sz
     l.gmc_scale_weights_chunks.argtypes = [shp]
     l.gmc_scale_weights.argtypes = [vp, vp, vp, shp, ci, vp]
@@ -326,6 +329,40 @@ def relu_fit_step(fitting_mixture: torch.Tensor, x: torch.Tensor, goal: torch.Te
         check(lib().gmc_relu_fit_step(_p(fitting_mixture), _p(x), _p(goal), _p(out), ctypes.byref(shape),
                                       _stream(fitting_mixture.device)))
     return out
+
+
+def relu_fit_bwd(grad_out: torch.Tensor, target: torch.Tensor, constant: torch.Tensor, fit: torch.Tensor, goal: torch.Tensor,
+                 need_target: bool, need_constant: bool, need_fit: bool):
+    """Gradients of one fixed-point iteration, x1 = x0 (goal + 0.05) / (current + 0.05) with x0 = |w| + 0.1: the
+    element-wise parts in three small launches around the backward kernels of the two evaluations (covariance form),
+    whose gradients with respect to the query points come back to the centres.  None where not needed."""
+    shape = _mixture_shape(fit, fit.shape[2])
+    B, L, N = shape.B, shape.L, shape.N
+    dev = fit.device
+    grad_out = _like(grad_out, fit, fit.shape, "grad_out")
+    full_constant = _like(constant.expand(B, L), fit, (B, L), "constant")
+    fit_abs = torch.empty_like(fit)
+    centres = torch.empty((B, L, N, shape.D), dtype=fit.dtype, device=dev)
+    d_value, d_current = torch.empty_like(goal), torch.empty_like(goal)
+    grad_constant = torch.empty_like(full_constant) if need_constant else None
+    with _on(dev):
+        check(lib().gmc_relu_fit_grad_start(_p(fit), _p(fit_abs), _p(centres), ctypes.byref(shape), _stream(dev)))
+        current = eval_fwd(fit_abs, centres, covariance_form=True)
+        check(lib().gmc_relu_fit_grad_prepare(_p(grad_out), _p(fit), _p(goal), _p(current), _p(full_constant), _p(d_value),
+                                              _p(d_current), _p(grad_constant), ctypes.byref(shape), _stream(dev)))
+        grad_target = grad_fit = None
+        if need_target or need_fit:
+            grad_target, grad_centres = eval_bwd(d_value, target, centres, need_target, need_fit, covariance_form=True)
+        if need_fit:
+            grad_abs, grad_centres2 = eval_bwd(d_current, fit_abs, centres, True, True, covariance_form=True)
+            grad_fit = torch.empty_like(fit)
+            check(lib().gmc_relu_fit_grad_finish(_p(grad_out), _p(fit), _p(goal), _p(current), _p(grad_abs), _p(grad_centres),
+                                                 _p(grad_centres2), _p(grad_fit), ctypes.byref(shape), _stream(dev)))
+    if need_constant:
+        for dim in (0, 1):
+            if constant.shape[dim] == 1 and grad_constant.shape[dim] != 1:
+                grad_constant = grad_constant.sum(dim, keepdim=True)
+    return grad_target if need_target else None, grad_constant, grad_fit
 
 
 def eval_cov_moments(mixture: torch.Tensor, constant: torch.Tensor, xes: torch.Tensor, per_sample: bool,

@@ -152,6 +152,20 @@ int gmc_eval_cov_moments(const void* mixture, const void* constant, const void* 
  * place, into positions inside the box of all centres of their batch entry (2-D: widened by u * 1.3 - 0.15). */
 int gmc_batch_norm_sampling_positions(const void* mixture, void* uniform_in_positions_out, const gmc_shape* shape, void* stream);
 
+/* Element-wise parts of the gradient of one fixed-point iteration (src/gmc/fitting.py:296-311) around the evaluations; N is
+ * the number of fitting components, all tensors in the mixture's dtype.  start: fitting_abs = the fitting mixture with the
+ * weights |w| + 0.1, centres [B][L][N][D].  prepare: upstream gradients d_value and d_current [B][L][N] of the evaluations of the
+ * target and of fitting_abs at the centres, from grad_out (of the fitted mixture), the goal of gmc_relu_fit_goal and the
+ * values `current` of fitting_abs; grad_constant [B][L] (may be NULL).  finish: gradient of the fitting mixture from the
+ * evaluations' gradients grad_abs (of fitting_abs), grad_centres and grad_centres2. */
+int gmc_relu_fit_grad_start(const void* fitting_mixture, void* fitting_abs, void* centres, const gmc_shape* shape, void* stream);
+int gmc_relu_fit_grad_prepare(const void* grad_out, const void* fitting_mixture, const void* goal, const void* current,
+                              const void* constant, void* d_value, void* d_current, void* grad_constant, const gmc_shape* shape,
+                              void* stream);
+int gmc_relu_fit_grad_finish(const void* grad_out, const void* fitting_mixture, const void* goal, const void* current,
+                             const void* grad_abs, const void* grad_centres, const void* grad_centres2, void* grad_fitting,
+                             const gmc_shape* shape, void* stream);
+
 /* BatchNorm's scaling of the weights, src/gmc/modules.py:417-421: out = mixture [B][L][M] with every weight times
  * scale[l] (scale_per_batch 0) or scale[b][l]; shape->N, Bx, Lx as for a call with one set of points per mixture (N may
  * be 0).  Backward: grad_mixture (may be NULL) and partial (may be NULL), double [B][L][gmc_scale_weights_chunks], whose
