@@ -54,29 +54,85 @@ __global__ __launch_bounds__(kBlock) void componentwise_fwd_kernel(const T* __re
     }
 }
 
-// Backward: grad_out [B][L][N][M] weights every pair on its own and is read once (4 bytes per pair: the pass is
-// bound by these loads and by instruction issue together, about 40 vector instructions per 64 pairs fit under the
-// HBM rate).  A wavefront owns one slice of 64 Gaussians (lanes = Gaussians, coalesced loads along M) and a range
-// of the workgroup's points (up to kCwPointsMax: the more points, the fewer atomics on the per-Gaussian sums): with
-// fewer than four slices in the mixture the four wavefronts share the points of the chunk instead of idling.  It walks its points eight at a time with the eight grad_out loads in
-// flight.  Per-Gaussian sums stay in the owning lane's registers over the points, are added over the wavefronts
-// that share a slice through LDS, and leave with one atomic per scalar and workgroup; dL/dx of a point is reduced over the wavefront's 64 Gaussians (DPP) into the workgroup's
-// LDS copy, which leaves with one atomic (or, when one workgroup sees all Gaussians of the point, one store) per
-// scalar.
-constexpr int kCwUnroll = 8;
-constexpr int kCwPointsMax = 1024;  // points per workgroup of the backward pass (a multiple of kCwPoints, chosen per launch)
+// Layout of the backward pass: the 64 lanes of a wavefront are 4 rows (points) by 16 columns, a column holds Q Gaussians,
+// so that the coordinates of a point are fetched once for Q pairs.  Where every row of grad_out starts at a multiple of
+// the vector (`wide`), a column's Gaussians lie next to each other and one access per lane (16 bytes for 4 floats) fetches
+// the values of 16 Q Gaussians at 4 points; elsewhere they lie 16 apart and Q accesses fetch 64 bytes of a row each.  A wavefront owns one such slice of
+// Gaussians; with fewer than four slices in its group the four wavefronts of a workgroup share the points of the chunk.
+// (The forward pass, which only stores, is faster with lanes = Gaussians: 800 x 128 Gaussians at 784 points in 2-D 74 us
+// against 107 us in this layout.)
+constexpr int kCwPointsMax = 1024; // most points per workgroup of the backward pass (the size of its LDS copy of dL/dx)
+template <typename T, int Q> struct __align__(sizeof(T) * Q) CwVec { T v[Q]; };
+// Gaussians per lane: what a 16-byte access holds in 2-D, half as many in 3-D (record and sums of every one of them stay in
+// registers: 26 per Gaussian) and where there are no wide accesses to gain (400 x 45 Gaussians at 900 points in 2-D: four
+// 47 us, two 35 us).
+template <typename T, int D> constexpr int cw_most = (D == 2 ? 16 : 8) / int(sizeof(T));
 
-template <typename T, int D, bool NEED_GM, bool NEED_GX>
-__global__ __launch_bounds__(kBlock) void componentwise_bwd_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
+struct CwSlices { int slice, rep, reps; };
+
+// the share of a wavefront: slice of the Gaussians (group of four slices, -1: none) and repetition over the points
+__device__ __forceinline__ CwSlices cw_share(int M, int group, int per_slice, int wave) {
+    const int slices_total = (M + per_slice - 1) / per_slice;
+    const int here = slices_total - group * 4 < 4 ? slices_total - group * 4 : 4;
+    const int reps = 4 / here;
+    const int rep = wave / here;
+    return CwSlices{rep < reps ? wave % here : -1, rep, reps};
+}
+
+// Sums of 4 (or 8) values over the 16 lanes of a DPP row at once: in every step the halves of a group exchange the
+// values they do not keep.  Returns, in lane `lane` of the row, the total of value cw_sum_index(lane) (4 values: bits 3
+// and 2 of the lane choose; 8 values: bits 3, 2 and 1).
+template <typename T, int COUNT>
+__device__ __forceinline__ T cw_row_sums(const T (&v)[COUNT], int lane) {
+    static_assert(COUNT == 4 || COUNT == 8, "");
+    T a[COUNT / 2];
+    const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0, b1 = (lane & 2) != 0;
+#pragma unroll
+    for (int i = 0; i < COUNT / 2; ++i) {
+        const T low = v[2 * i], high = v[2 * i + 1];
+        a[i] = (b3 ? high : low) + dpp_mov<0x128>(b3 ? low : high);         // row_ror:8
+    }
+    T c[COUNT / 4];
+#pragma unroll
+    for (int i = 0; i < COUNT / 4; ++i) {
+        const T low = a[2 * i], high = a[2 * i + 1];
+        c[i] = (b2 ? high : low) + dpp_mov<0x141>(b2 ? low : high);         // row_half_mirror: the other half of eight
+    }
+    T s;
+    if constexpr (COUNT == 8) {
+        const T low = c[0], high = c[1];
+        s = (b1 ? high : low) + dpp_mov<0x4e>(b1 ? low : high);             // quad_perm 2 3 0 1
+    } else {
+        s = c[0] + dpp_mov<0x4e>(c[0]);
+    }
+    return s + dpp_mov<0xb1>(s);                                            // quad_perm 1 0 3 2
+}
+template <int COUNT> __device__ __forceinline__ int cw_sum_index(int lane) {
+    return ((lane >> 3) & 1) + 2 * ((lane >> 2) & 1) + (COUNT == 8 ? 4 * ((lane >> 1) & 1) : 0);
+}
+
+// Backward: grad_out [B][L][N][M] weights every pair on its own and is read once.  A row's point meets Q Gaussians per
+// lane before its dL/dx is reduced, over the 16 columns only; four points of a row (16 of the wavefront) go through that
+// reduction together, and their grad_out values are in flight together.  Per-Gaussian sums stay in the lane's
+// registers over the points, are added over the rows and over the wavefronts that share a slice at the end, and leave
+// with one atomic per scalar and workgroup; dL/dx of a point goes through the workgroup's LDS copy and leaves with one
+// atomic (or, when one workgroup sees all Gaussians of the point, one store) per scalar.  Before, a lane held one Gaussian
+// and every point's dL/dx was reduced over 64 lanes (us before / now, float32, both gradients): 800 x 128 Gaussians at 784 points in
+// 2-D 124 / 97 (3.3 TB/s of grad_out), in 3-D 196 / 123; 20 x 512 at 4096 points 117 / 53 and 273 / 69.  Bound by
+// instruction issue and, at 154 registers (2-D), three wavefronts per SIMD.
+constexpr int kCwSteps = 4;        // points of a row per round
+
+template <typename T, int D, int Q, bool NEED_GM, bool NEED_GX>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : Q == 4 || D == 3 ? 3 : 4))) void componentwise_bwd_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
                                                                   const T* __restrict__ xes, T* __restrict__ sums,
                                                                   T* __restrict__ grad_xes, int L, int M, int N, int Bx,
                                                                   int Lx, int m_groups, int chunks, int points_per_chunk,
-                                                                  bool shared_points, bool covariance_form) {
-    constexpr int G = 1 + D + D * D;
+                                                                  bool shared_points, bool wide, bool covariance_form) {
+    constexpr int G = 1 + D + D * D, U = kCwSteps;
     constexpr int NR = 1 + D + D * (D + 1) / 2;
     constexpr int kU = Rec<T, D>::kU;
     __shared__ T point_grad[NEED_GX ? kCwPointsMax * D : 1];
-    __shared__ T shared_sums[NEED_GM ? kBlock * NR : 1];
+    __shared__ T shared_sums[NEED_GM ? 4 * 16 * Q * NR : 1];
     const T* exp2_tab = exp2_table<T>();
     if constexpr (sizeof(T) == 8) __syncthreads();          // the table is complete
     int id = blockIdx.x;
@@ -85,121 +141,142 @@ __global__ __launch_bounds__(kBlock) void componentwise_bwd_kernel(const T* __re
     const int bl = id / m_groups;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
-    // (no readfirstlane here: with a provably uniform wavefront index the point coordinates arrive through scalar
-    // loads, whose waits also cover the LDS traffic of the loop -- measured 15 % slower)
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    // slices of 64 Gaussians in this workgroup's group of up to four, and how often the group fits into the
-    // workgroup's four wavefronts (each repetition takes its share of the points)
-    const int slices_total = (M + kWave - 1) / kWave;
-    const int slices_here = slices_total - group * 4 < 4 ? slices_total - group * 4 : 4;
-    const int reps = 4 / slices_here;
-    const int slice = wave % slices_here, rep = wave / slices_here;
-    const int m = (group * 4 + slice) * kWave + lane;
-    const bool valid = m < M;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane >> 4, col = lane & 15;
+    const CwSlices share = cw_share(M, group, 16 * Q, wave);
+    // Gaussian q of this lane is m0 + q * apart
+    const int apart = wide ? 1 : 16;
+    const int m0 = (group * 4 + share.slice) * 16 * Q + (wide ? col * Q : col);
     const size_t x_off = (size_t(xb) * Lx + xl) * N;
     const T* __restrict__ x_bl = xes + x_off * D;
     if (NEED_GX) {
         for (int i = threadIdx.x; i < points_per_chunk * D; i += kBlock) point_grad[i] = T(0);
         __syncthreads();
     }
-    T rs[NR];
+    T rs[Q][NR];
 #pragma unroll
-    for (int i = 0; i < NR; ++i) rs[i] = T(0);
-    if (rep < reps) {
-        T r[Rec<T, D>::kStride];
-        {
-            const Derived<D> dv = derive<T, D>(mixture + (size_t(bl) * M + (valid ? m : 0)) * G, covariance_form);
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int i = 0; i < NR; ++i) rs[q][i] = T(0);
+    const int chunk_begin = chunk * points_per_chunk;
+    if (share.slice >= 0) {
+        T r[Q][Rec<T, D>::kStride], ua[Q][kU];      // ua = -amp * u: dL/dx takes k*y against it
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const Derived<D> dv = derive<T, D>(mixture + (size_t(bl) * M + (m0 + q * apart < M ? m0 + q * apart : 0)) * G, covariance_form);
             // amplitude for dL/dx as in the summed backward kernel: w norm / (0.5 log2 e)
-            store_record<T, D>(r, dv, true, dv.w * dv.norm * (1.0 / kHalfLog2e), 0);
-        }
-        T ua[kU];                                   // -amp * u: dL/dx takes k*y against it
+            store_record<T, D>(r[q], dv, true, dv.w * dv.norm * (1.0 / kHalfLog2e), 0);
 #pragma unroll
-        for (int i = 0; i < kU; ++i) ua[i] = -r[Rec<T, D>::kAmp] * r[i];
-        const int per_rep = (points_per_chunk + reps - 1) / reps;
-        const int chunk_begin = chunk * points_per_chunk;
-        const int n_begin = chunk_begin + rep * per_rep;
+            for (int i = 0; i < kU; ++i) ua[q][i] = -r[q][Rec<T, D>::kAmp] * r[q][i];
+        }
+        const int per_rep = ((points_per_chunk + share.reps - 1) / share.reps + 4 * U - 1) / (4 * U) * (4 * U);
+        const int n_begin = chunk_begin + share.rep * per_rep;
         int n_end = n_begin + per_rep < chunk_begin + points_per_chunk ? n_begin + per_rep : chunk_begin + points_per_chunk;
         n_end = n_end < N ? n_end : N;
-        const T* __restrict__ go_col = grad_out + size_t(bl) * N * M + (valid ? m : 0);
-        for (int n0 = n_begin; n0 < n_end; n0 += kCwUnroll) {
-            T go[kCwUnroll], xs[kCwUnroll][D];
+        const T* __restrict__ go_bl = grad_out + size_t(bl) * N * M;
+        // values and coordinates of the row's next U points; beyond the end and beyond M: zeros, which add nothing
+        auto fetch = [&](int n0, CwVec<T, Q> (&go)[U], T (&xs)[U][D]) {
 #pragma unroll
-            for (int u = 0; u < kCwUnroll; ++u) {
-                const int n = n0 + u < n_end ? n0 + u : n_end - 1;
-                go[u] = go_col[size_t(n) * M];
+            for (int u = 0; u < U; ++u) {
+                const int at = n0 + u * 4 + row;
+                const int n = at < n_end ? at : n_end - 1;
+                const T* from = go_bl + size_t(n) * M + m0;
+                if (wide && m0 < M) {                       // (M is a multiple of Q)
+                    go[u] = *reinterpret_cast<const CwVec<T, Q>*>(from);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) go[u].v[q] = m0 + q * apart < M ? from[q * apart] : T(0);
+                }
 #pragma unroll
                 for (int d = 0; d < D; ++d) xs[u][d] = x_bl[size_t(n) * D + d];
             }
-            T vs[kCwUnroll][D];                                     // dL/dx terms of the eight points, this lane's Gaussian
+        };
+        for (int n0 = n_begin; n0 < n_end; n0 += 4 * U) {
+            CwVec<T, Q> go[U];
+            T xs[U][D];
+            fetch(n0, go, xs);
+            T vs[D][U];                                     // dL/dx of the row's points, this lane's Gaussians
 #pragma unroll
-            for (int u = 0; u < kCwUnroll; ++u) {
-                T y[D];
-                const T q = quad_form<T, D, true>(r, xs[u], y);
-                const T k = (valid && n0 + u < n_end) ? pair_exp2(-q, exp2_tab) * go[u] : T(0);
-                T ky[D];
+            for (int u = 0; u < U; ++u) {
+                const bool in = n0 + u * 4 + row < n_end;
+                T v[D];
 #pragma unroll
-                for (int d = 0; d < D; ++d) ky[d] = k * y[d];
-                if (NEED_GM) {
-                    rs[0] += k;
-                    int at = 1 + D;
+                for (int d = 0; d < D; ++d) v[d] = T(0);
 #pragma unroll
-                    for (int a = 0; a < D; ++a) {
-                        rs[1 + a] += ky[a];
+                for (int q = 0; q < Q; ++q) {
+                    T y[D];
+                    const T e = quad_form<T, D, true>(r[q], xs[u], y);
+                    const T k = (in && m0 + q * apart < M) ? pair_exp2(-e, exp2_tab) * go[u].v[q] : T(0);
+                    T ky[D];
 #pragma unroll
-                        for (int c = a; c < D; ++c) { rs[at] = fma_(ky[a], y[c], rs[at]); ++at; }
+                    for (int d = 0; d < D; ++d) ky[d] = k * y[d];
+                    if (NEED_GM) {
+                        rs[q][0] += k;
+                        int at = 1 + D;
+#pragma unroll
+                        for (int a = 0; a < D; ++a) {
+                            rs[q][1 + a] += ky[a];
+#pragma unroll
+                            for (int c = a; c < D; ++c) { rs[q][at] = fma_(ky[a], y[c], rs[q][at]); ++at; }
+                        }
+                    }
+                    if (NEED_GX) {
+                        // -(amp u)^T (k y)
+                        if constexpr (D == 2) {
+                            v[0] = fma_(ua[q][0], ky[0], v[0]);
+                            v[1] = fma_(ua[q][1], ky[0], fma_(ua[q][2], ky[1], v[1]));
+                        } else {
+                            v[0] = fma_(ua[q][0], ky[0], v[0]);
+                            v[1] = fma_(ua[q][1], ky[0], fma_(ua[q][3], ky[1], v[1]));
+                            v[2] = fma_(ua[q][2], ky[0], fma_(ua[q][4], ky[1], fma_(ua[q][5], ky[2], v[2])));
+                        }
                     }
                 }
-                if (NEED_GX) {
-                    // -(amp u)^T (k y)
-                    if constexpr (D == 2) {
-                        vs[u][0] = ua[0] * ky[0];
-                        vs[u][1] = fma_(ua[1], ky[0], ua[2] * ky[1]);
-                    } else {
-                        vs[u][0] = ua[0] * ky[0];
-                        vs[u][1] = fma_(ua[1], ky[0], ua[3] * ky[1]);
-                        vs[u][2] = fma_(ua[2], ky[0], fma_(ua[4], ky[1], ua[5] * ky[2]));
-                    }
-                }
+#pragma unroll
+                for (int d = 0; d < D; ++d) vs[d][u] = v[d];
             }
             if (NEED_GX) {
-                // summed over the wavefront's Gaussians, four points at a time; the lane at the end of row r holds
-                // the total of point {0, 2, 1, 3}[r] of the four
-                const int row = lane >> 4;
-                const int mine = ((row & 1) << 1) | (row >> 1);
+                static_assert(U == 4, "four points of a row are reduced together");
+                // 2 coordinates of the four points in one reduction of 8 values, a third one in a reduction of 4
+                T eight[8];
 #pragma unroll
-                for (int u0 = 0; u0 < kCwUnroll; u0 += 4) {
-                    T total[D];
-#pragma unroll
-                    for (int d = 0; d < D; ++d)
-                        total[d] = wave_sum4_to_row_ends(vs[u0][d], vs[u0 + 1][d], vs[u0 + 2][d], vs[u0 + 3][d], lane);
-                    const int n = n0 + u0 + mine;
-                    if ((lane & 15) == 15 && n < n_end) {
-#pragma unroll
-                        for (int d = 0; d < D; ++d) atomic_add(&point_grad[(n - chunk_begin) * D + d], total[d]);
-                    }
+                for (int u = 0; u < 4; ++u) { eight[u] = vs[0][u]; eight[4 + u] = vs[1][u]; }
+                const T s8 = cw_row_sums<T, 8>(eight, lane);
+                {
+                    const int i = cw_sum_index<8>(lane), n = n0 + (i & 3) * 4 + row;
+                    if ((lane & 1) == 0 && n < n_end) atomic_add(&point_grad[(n - chunk_begin) * D + (i >> 2)], s8);
+                }
+                if constexpr (D == 3) {
+                    const T s4 = cw_row_sums<T, 4>(vs[2], lane);
+                    const int n = n0 + cw_sum_index<4>(lane) * 4 + row;
+                    if ((lane & 3) == 0 && n < n_end) atomic_add(&point_grad[(n - chunk_begin) * D + 2], s4);
                 }
             }
         }
     }
     if (NEED_GM) {
-        // the wavefronts that shared a slice add their sums through LDS; the first of them sends the total
+        // over the rows of the wavefront, then over the wavefronts that shared the slice; one atomic per scalar
 #pragma unroll
-        for (int i = 0; i < NR; ++i) shared_sums[threadIdx.x * NR + i] = rs[i];
-        __syncthreads();
-        if (rep == 0 && valid) {
-            for (int other = 1; other < reps; ++other) {
-                const T* from = shared_sums + ((other * slices_here + slice) * kWave + lane) * NR;
+        for (int q = 0; q < Q; ++q)
 #pragma unroll
-                for (int i = 0; i < NR; ++i) rs[i] += from[i];
+            for (int i = 0; i < NR; ++i) {
+                T v = rs[q][i];
+                v += __shfl_xor(v, 16, 64);
+                v += __shfl_xor(v, 32, 64);
+                if (row == 0) shared_sums[(wave * 16 * Q + (wide ? col * Q : col) + q * apart) * NR + i] = v;
             }
-            T* dst = sums + (size_t(bl) * M + m) * NR;
-#pragma unroll
-            for (int i = 0; i < NR; ++i) atomic_add(&dst[i], rs[i]);
+        __syncthreads();
+        constexpr int kSlice = 16 * Q * NR;
+        const int first = group * 4 * 16 * Q;               // the group's first Gaussian
+        const int left = (M - first + 16 * Q - 1) / (16 * Q), slices_here = left < 4 ? left : 4;
+        for (int i = threadIdx.x; i < slices_here * kSlice; i += kBlock) {
+            if (first + i / NR >= M) break;
+            T v = shared_sums[i];
+            for (int other = 1; other < share.reps; ++other) v += shared_sums[other * slices_here * kSlice + i];
+            atomic_add(&sums[(size_t(bl) * M + first) * NR + i], v);
         }
     }
     if (NEED_GX) {
         __syncthreads();
-        const int chunk_begin = chunk * points_per_chunk;
         for (int i = threadIdx.x; i < points_per_chunk * D; i += kBlock) {
             const int n = chunk_begin + i / D;
             if (n >= N) continue;
@@ -214,6 +291,19 @@ void launch_bwd_epilogue(const void* mixture, const void* sums, void* grad_mixtu
                          bool covariance_form, hipStream_t stream);
 size_t dense_backward_workspace_bytes(const gmc_shape& s);
 
+// Points per workgroup: about `wanted` workgroups for the launch, with chunks of the same size (a last chunk of a few
+// points costs a workgroup's preparation), a multiple of 32 points within [kCwPoints, kCwPointsMax].
+constexpr size_t kCwWanted = 2048;
+struct CwChunks { int chunks, points; };
+static CwChunks cw_chunks(size_t workgroups, int N, size_t wanted) {
+    size_t chunks = (wanted + workgroups - 1) / workgroups;
+    const size_t most = (size_t(N) + kCwPoints - 1) / kCwPoints, least = (size_t(N) + kCwPointsMax - 1) / kCwPointsMax;
+    chunks = chunks > most ? most : chunks;
+    chunks = chunks < least ? least : chunks;
+    const int points = int(((size_t(N) + chunks - 1) / chunks + 31) / 32 * 32);
+    return CwChunks{(N + points - 1) / points, points};
+}
+
 template <typename T, int D>
 static int cw_forward(const T* mixture, const T* xes, T* out, const gmc_shape& s, bool cov, hipStream_t st) {
     const size_t BL = size_t(s.B) * s.L;
@@ -224,23 +314,20 @@ static int cw_forward(const T* mixture, const T* xes, T* out, const gmc_shape& s
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
 }
 
-template <typename T, int D>
-static int cw_backward(const T* grad_out, const T* mixture, const T* xes, T* grad_mixture, T* grad_xes, T* sums,
-                       const gmc_shape& s, bool gm, bool gx, bool cov, hipStream_t st) {
+template <typename T, int D, int Q>
+static int cw_backward_q(const T* grad_out, const T* mixture, const T* xes, T* grad_mixture, T* grad_xes, T* sums,
+                       const gmc_shape& s, bool gm, bool gx, bool wide, bool cov, hipStream_t st) {
     constexpr int G = 1 + D + D * D;
     constexpr int NR = 1 + D + D * (D + 1) / 2;
     const size_t BL = size_t(s.B) * s.L;
     const size_t n_g = BL * s.M, n_x = size_t(s.Bx) * s.Lx * s.N * D;
     if (BL == 0) return GMC_OK;
-    const int m_groups = (s.M + kBlock - 1) / kBlock;
-    // points per workgroup: as many as leave about two thousand workgroups for the launch, within [64, kCwPointsMax]
-    int points_per_chunk = kCwPointsMax;
-    while (points_per_chunk > kCwPoints &&
-           BL * m_groups * ((size_t(s.N) + points_per_chunk - 1) / points_per_chunk) < 2048)
-        points_per_chunk /= 2;
-    const int chunks = (s.N + points_per_chunk - 1) / points_per_chunk;
+    constexpr int kGroup = 4 * 16 * Q;
+    const int m_groups = (s.M + kGroup - 1) / kGroup;
+    const CwChunks c = cw_chunks(BL * (m_groups > 0 ? m_groups : 1), s.N > 0 ? s.N : 1, kCwWanted);
+    const int chunks = c.chunks, points_per_chunk = c.points;
     // dL/dx of a point is stored by the one workgroup that sees all its Gaussians, and added atomically to zeros when
-    // several do (more than 256 Gaussians, or points shared by several mixtures)
+    // several do (more than one group of four slices, or points shared by several mixtures)
     const bool shared_points = m_groups > 1 || size_t(s.Bx) * s.Lx != BL;
     if (gx && (shared_points || s.N == 0 || s.M == 0)) zero_async(grad_xes, n_x, st);
     if (s.N == 0 || s.M == 0) {
@@ -249,14 +336,24 @@ static int cw_backward(const T* grad_out, const T* mixture, const T* xes, T* gra
     }
     if (gm) zero_async(sums, n_g * NR, st);
     const dim3 grid(unsigned(BL * m_groups * chunks));
-#define GMC_CW(GM, GX) componentwise_bwd_kernel<T, D, GM, GX><<<grid, dim3(kBlock), 0, st>>>( \
-        grad_out, mixture, xes, sums, grad_xes, s.L, s.M, s.N, s.Bx, s.Lx, m_groups, chunks, points_per_chunk, shared_points, cov)
+#define GMC_CW(GM, GX) componentwise_bwd_kernel<T, D, Q, GM, GX><<<grid, dim3(kBlock), 0, st>>>( \
+        grad_out, mixture, xes, sums, grad_xes, s.L, s.M, s.N, s.Bx, s.Lx, m_groups, chunks, points_per_chunk, shared_points, wide, cov)
     if (gm && gx) GMC_CW(true, true);
     else if (gm) GMC_CW(true, false);
     else if (gx) GMC_CW(false, true);
 #undef GMC_CW
     if (gm) launch_bwd_epilogue(mixture, sums, grad_mixture, n_g, D, s.dtype, cov, st);
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
+}
+
+template <typename T, int D>
+static int cw_backward(const T* grad_out, const T* mixture, const T* xes, T* grad_mixture, T* grad_xes, T* sums,
+                       const gmc_shape& s, bool gm, bool gx, bool cov, hipStream_t st) {
+    constexpr int Q = cw_most<T, D>;
+    const bool wide = s.M % Q == 0 && (uintptr_t(grad_out) & (sizeof(T) * Q - 1)) == 0;
+    if constexpr (Q > 2)
+        if (!wide) return cw_backward_q<T, D, 2>(grad_out, mixture, xes, grad_mixture, grad_xes, sums, s, gm, gx, false, cov, st);
+    return cw_backward_q<T, D, Q>(grad_out, mixture, xes, grad_mixture, grad_xes, sums, s, gm, gx, wide, cov, st);
 }
 
 }  // namespace gmc

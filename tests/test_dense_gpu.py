@@ -576,6 +576,34 @@ def test_componentwise(dtype, D):
     assert rel_l2(v2.cpu().numpy(), ref, fl) <= 20 * tol
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("D", [2, 3])
+def test_componentwise_backward_edges(dtype, D):
+    """gradients at the edges of the backward kernel's layout: Gaussians per column, slice and group (4, 64, 256 floats in
+    2-D, half of that in 3-D or in double) and rounds and chunks of points, each gradient alone as well, rows of grad_out that
+    start off a multiple of 16 bytes; reference: autograd in float64 on the CPU"""
+    shapes = [(1, 1, 1, 1), (2, 1, 16, 3), (1, 2, 17, 4), (3, 1, 33, 17), (1, 1, 63, 63), (2, 2, 64, 65), (1, 1, 66, 130),
+              (1, 1, 130, 1025), (1, 1, 257, 100), (1, 2, 513, 33), (60, 40, 3, 70)]
+    for i, (B, L, M, N) in enumerate(shapes):
+        bc = i % 4 == 2
+        mix, xes, _ = _case(B, L, M, N, D, 900 + i, bc)
+        mix, xes = torch.tensor(mix).to(dtype), torch.tensor(xes).to(dtype) * 0.5
+        gout = torch.randn((B, L, N, M), generator=torch.Generator().manual_seed(i), dtype=torch.float64).to(dtype)
+        m64, x64 = mix.double().requires_grad_(True), xes.double().requires_grad_(True)
+        c = m64[..., 1 + D:].view(B, L, 1, M, D, D)
+        t = x64.unsqueeze(3) - m64[..., 1:1 + D].unsqueeze(2)
+        q = (t.unsqueeze(-2) @ c @ t.unsqueeze(-1)).squeeze(-1).squeeze(-1)
+        vals = m64[..., 0].unsqueeze(2) * o.kappa(D) * torch.linalg.det(c).sqrt() * torch.exp(-0.5 * q)
+        rgm, rgx = torch.autograd.grad(vals, (m64, x64), gout.double())
+        md, xd, gd = mix.to(DEV), xes.to(DEV), gout.to(DEV)
+        for need_m, need_x in ((True, True), (True, False), (False, True)):
+            gm_, gx_ = _native.eval_componentwise_bwd(gd, md, xd, need_m, need_x)
+            if need_m:
+                assert rel_l2(gm_.cpu().numpy(), rgm.numpy(), FLOOR[dtype]) <= TOL[dtype], (B, L, M, N)
+            if need_x:
+                assert rel_l2(gx_.cpu().numpy(), rgx.numpy(), FLOOR[dtype]) <= TOL[dtype], (B, L, M, N)
+
+
 def _workload_check(name, **kw):
     wl, mix, xes, gout = synthetic.make_workload(name, **kw)
     out, gmix, gxes = _run(mix.numpy(), xes.numpy(), gout.numpy(), wl.dtype)
