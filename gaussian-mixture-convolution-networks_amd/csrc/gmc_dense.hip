@@ -311,11 +311,16 @@ __device__ __forceinline__ void bwd_epilogue_derived(const Derived<D>& dv, const
 // SOLE: the workgroup covers all points of its mixture (one chunk).  The sums of its Gaussians are then final: they go
 // to `sums` with plain stores (no zero fill before the launch, no atomics) and the workgroup itself carries them on
 // to grad_mixture at the end, which saves the fill and the epilogue launch of small problems.
-template <typename T, int D, int P, bool NEED_GM, bool NEED_GX, bool SOLE>
+// SEVERAL: the points are shared by all mixtures, and the workgroup takes `per_group` mixtures one after the other, with
+// dL/dx of its points in registers throughout: the additions of all mixtures meet on the same addresses, and each costs
+// about 45 ns there (see plan_mixtures_per_group).
+template <typename T, int D, int P, bool NEED_GM, bool NEED_GX, bool SOLE, bool SEVERAL>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 1)))
 void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture, const T* __restrict__ xes,
                         T* __restrict__ sums, T* __restrict__ grad_xes, T* __restrict__ grad_mixture, int L, int M, int N,
-                        int Bx, int Lx, int chunks, int xes_shared, int n_mixtures, bool covariance_form, TileSlices ts) {
+                        int Bx, int Lx, int chunks, int xes_shared, int n_mixtures, int per_group, bool covariance_form,
+                        TileSlices ts) {
+    static_assert(!SEVERAL || (NEED_GM && NEED_GX), "dL/dx alone takes the upstream gradient at the very end");
     constexpr int G = 1 + D + D * D;
     constexpr int S = Rec<T, D>::kStride;
     constexpr int NR = Sums<D>::k;
@@ -330,8 +335,14 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
 
     const ClockProbe probe = clock_probe_begin();
     int bl, chunk;
-    map_workgroup(blockIdx.x, chunks * ts.slices, n_mixtures, bl, chunk);
+    if constexpr (SEVERAL) {
+        map_workgroup(blockIdx.x, chunks * ts.slices, (n_mixtures + per_group - 1) / per_group, bl, chunk);
+        bl *= per_group;
+    } else {
+        map_workgroup(blockIdx.x, chunks * ts.slices, n_mixtures, bl, chunk);
+    }
     if (bl >= n_mixtures) return;
+    const int bl_end = SEVERAL ? (bl + per_group < n_mixtures ? bl + per_group : n_mixtures) : bl + 1;
     // (with several slices the host passes xes_shared != 0: dL/dx of a point then comes from several workgroups)
     const int slice = chunk / chunks;
     chunk -= slice * chunks;
@@ -339,7 +350,6 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
     const int g_end = (g_begin + ts.per_slice) < M ? (g_begin + ts.per_slice) : M;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
-    const T* __restrict__ mix_bl = mixture + size_t(bl) * M * G;
     const size_t x_off = (size_t(xb) * Lx + xl) * N;
     const T* __restrict__ x_bl = xes + x_off * D;
 
@@ -358,7 +368,7 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
             x[p][d] = x_bl[size_t(nc) * D + d];
             gx[p][d] = T(0);
         }
-        go[p] = n < N ? grad_out[size_t(bl) * N + nc] : T(0);   // padding lanes contribute nothing
+        if constexpr (!SEVERAL) go[p] = n < N ? grad_out[size_t(bl) * N + nc] : T(0);   // padding lanes contribute nothing
     }
     if (NEED_GM) {
         // (the per-wavefront copies need no zero fill: a tile's entries are all written before they are read)
@@ -366,30 +376,49 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
             for (int i = threadIdx.x; i < kTile * NR; i += kBlock) block_sums[i] = T(0);
     }
 
-    for (int g0 = g_begin; g0 < g_end; g0 += kTile) {
-        const int cnt = (g_end - g0) < kTile ? (g_end - g0) : kTile;
-        stage_tile<T, D, 4>(mix_bl + size_t(g0) * G, cnt, 1.0 / kHalfLog2e, lds, counts, covariance_form);
-        const int centred_start = counts[8], padded_total = counts[9];
-        T* wave_sums = block_sums + (NEED_GM && SumCopies<T>::k > 1 ? wave * kTile * NR : 0);
-        bwd_rc_pairs<T, D, P, NEED_GM, NEED_GX, false>(lds, exp2_tab, wave_sums, 0, centred_start, row, x, go, gx);
-        bwd_rc_pairs<T, D, P, NEED_GM, NEED_GX, true>(lds, exp2_tab, wave_sums, centred_start, padded_total, row, x, go, gx);
-        if (NEED_GM) {
-            __syncthreads();
-            T* __restrict__ dst = sums + (size_t(bl) * M + g0) * NR;
-            for (int i = threadIdx.x; i < cnt * NR; i += kBlock) {
-                // entry i holds sum k of Gaussian j at [j][k / 2 + (k odd ? NR / 2 : 0)] of every wavefront's copy
-                const int j = i / NR, k = i - j * NR;
-                const int at = j * NR + (k >> 1) + ((k & 1) ? NR / 2 : 0);
-                T v = block_sums[at];
-                if constexpr (SumCopies<T>::k > 1) {
-                    v = (v + block_sums[kTile * NR + at]) + (block_sums[2 * kTile * NR + at] + block_sums[3 * kTile * NR + at]);
-                } else {
-                    block_sums[at] = T(0);
-                }
-                if (SOLE) dst[i] = v; else atomic_add(&dst[i], v);
+    do {
+        const T* __restrict__ mix_bl = mixture + size_t(bl) * M * G;
+        if constexpr (SEVERAL) {
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const int n = n0 + p * 16;
+                go[p] = n < N ? grad_out[size_t(bl) * N + n] : T(0);
             }
         }
-    }
+        for (int g0 = g_begin; g0 < g_end; g0 += kTile) {
+            const int cnt = (g_end - g0) < kTile ? (g_end - g0) : kTile;
+            stage_tile<T, D, 4>(mix_bl + size_t(g0) * G, cnt, 1.0 / kHalfLog2e, lds, counts, covariance_form);
+            const int centred_start = counts[8], padded_total = counts[9];
+            T* wave_sums = block_sums + (NEED_GM && SumCopies<T>::k > 1 ? wave * kTile * NR : 0);
+            bwd_rc_pairs<T, D, P, NEED_GM, NEED_GX, false>(lds, exp2_tab, wave_sums, 0, centred_start, row, x, go, gx);
+            bwd_rc_pairs<T, D, P, NEED_GM, NEED_GX, true>(lds, exp2_tab, wave_sums, centred_start, padded_total, row, x, go, gx);
+            if (NEED_GM) {
+                __syncthreads();
+                T* __restrict__ dst = sums + (size_t(bl) * M + g0) * NR;
+                for (int i = threadIdx.x; i < cnt * NR; i += kBlock) {
+                    // entry i holds sum k of Gaussian j at [j][k / 2 + (k odd ? NR / 2 : 0)] of every wavefront's copy
+                    const int j = i / NR, k = i - j * NR;
+                    const int at = j * NR + (k >> 1) + ((k & 1) ? NR / 2 : 0);
+                    T v = block_sums[at];
+                    if constexpr (SumCopies<T>::k > 1) {
+                        v = (v + block_sums[kTile * NR + at]) + (block_sums[2 * kTile * NR + at] + block_sums[3 * kTile * NR + at]);
+                    } else {
+                        block_sums[at] = T(0);
+                    }
+                    if (SOLE) dst[i] = v; else atomic_add(&dst[i], v);
+                }
+            }
+        }
+        if constexpr (SEVERAL) {
+            if (NEED_GM && SOLE) {
+                __syncthreads();            // the sums this workgroup stored are visible to all of its lanes
+                for (int i = g_begin + threadIdx.x; i < g_end; i += kBlock) {
+                    const size_t at = size_t(bl) * M + i;
+                    bwd_epilogue_one<T, D>(mixture + at * G, sums + at * NR, grad_mixture + at * G, covariance_form);
+                }
+            }
+        }
+    } while (SEVERAL && ++bl < bl_end);
     if (NEED_GX) {
 #pragma unroll
         for (int p = 0; p < P; ++p) {
@@ -421,7 +450,7 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
             }
         }
     }
-    if (NEED_GM && SOLE) {
+    if (NEED_GM && SOLE && !SEVERAL) {
         __syncthreads();            // the sums this workgroup stored are visible to all of its lanes
         for (int i = g_begin + threadIdx.x; i < g_end; i += kBlock) {
             const size_t at = size_t(bl) * M + i;
@@ -691,7 +720,8 @@ void set_tuning(int fwd_points_per_lane, int bwd_points_per_lane) {
 // rest (row reductions); a compute unit runs two workgroups in the time of one (a lone wavefront issues every second
 // slot), then ceil(workgroups / 256) after each other.  `clear`: the zero fill that slices need; `several_chunks`: the
 // zero fill and the epilogue launch of a backward pass whose sums come from several workgroups; `contended`: one more
-// addition to every dL/dx of points that all mixtures share (about 45 ns for each that meets on an address).  The plan
+// addition to every dL/dx of points that all mixtures share (about 45 ns for each that meets on an address in 2-D, 75 ns
+// in 3-D).  The plan
 // for full launches stays unless the model gives at least a tenth (three tenths against the
 // one-Gaussian-per-step layout).  Measured, full-launch plan / this one in us:
 //   15 x 333 Gaussians, 2777 points, float64, 3-D: forward 38.7 / 22.1, backward 100.9 / 52.9 (tiles of 256 and 77 before)
@@ -722,6 +752,30 @@ static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int
             const double cost = model.of(P, chunks, mixtures, slices, per < M ? per : M);
             if (cost < best_cost) { best_cost = cost; best = SmallPlan{P, TileSlices{slices, per}}; }
         }
+    }
+    return best;
+}
+
+// Mixtures that a workgroup of the backward kernel takes one after the other when all mixtures share their points: few
+// enough to leave the chip busy, many enough that their additions to dL/dx do not queue up.  Taken where the queue would
+// be as long as 0.7 of the modelled work (a shorter one hides behind it: 800 x 128 Gaussians at 784 points 70.5 us with one
+// mixture per workgroup, 82 us with several).  Measured, one mixture / several in us:
+//   6400 x 16 Gaussians at 100 points, 2-D: 317 / 67;  1353 x 36 at 361: 82 / 44, in 3-D 120 / 69;  2268 x 23 at 3049,
+//   3-D: 382 / 190;  1116 x 52 at 1547, 3-D: 134 / 113
+static int plan_mixtures_per_group(const LaunchCost& model, int P, size_t mixtures, int M, int N, TileSlices ts) {
+    constexpr int kGroup[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+    const size_t chunks = (size_t(N) + 64 * P - 1) / (64 * P);
+    const int per = ts.per_slice < M ? ts.per_slice : M;
+    const double one = 0.5 * (model.of(P, 1, 1, 1, per) - model.contended);       // a workgroup and mixture
+    const double queue = model.contended / double(mixtures > 1 ? mixtures - 1 : 1) * ts.slices;      // per group
+    int best = 1;
+    double best_cost = 1e300;
+    for (int k : kGroup) {
+        if (size_t(k) > mixtures) break;
+        const size_t groups = (mixtures + k - 1) / k, rounds = (groups * chunks * ts.slices + 255) / 256;
+        const double work = one * k * double(rounds < 2 ? 2 : rounds), cost = work + queue * double(groups);
+        if (k == 1 && queue * double(groups) < 0.7 * work) return 1;
+        if (cost < 0.95 * best_cost) { best_cost = cost; best = k; }
     }
     return best;
 }
@@ -866,15 +920,16 @@ static int bwd_points_per_lane(const gmc_shape& s) {
     return P;
 }
 
-template <typename T, int D, bool GM, bool GX, bool SOLE>
+template <typename T, int D, bool GM, bool GX, bool SOLE, bool SEVERAL = false>
 static void launch_bwd_main(const T* grad_out, const T* mixture, const T* xes, T* sums, T* grad_xes, T* grad_mixture,
-                            const gmc_shape& s, int P, int xes_shared, bool cov, TileSlices ts, hipStream_t stream) {
+                            const gmc_shape& s, int P, int xes_shared, bool cov, TileSlices ts, hipStream_t stream,
+                            int per_group = 1) {
     const size_t BL = size_t(s.B) * s.L;
     constexpr int p_max = sizeof(T) == 8 ? 8 : 16;
     const int span = 64 * P;
     const int chunks = (s.N + span - 1) / span;
-    const dim3 grid(unsigned(grid_mixtures(BL) * chunks * ts.slices));
-#define GMC_BWD(PP) eval_bwd_rc_kernel<T, D, PP, GM, GX, SOLE><<<grid, dim3(kBlock), 0, stream>>>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s.L, s.M, s.N, s.Bx, s.Lx, chunks, xes_shared, int(BL), cov, ts)
+    const dim3 grid(unsigned(grid_mixtures((BL + per_group - 1) / per_group) * chunks * ts.slices));
+#define GMC_BWD(PP) eval_bwd_rc_kernel<T, D, PP, GM, GX, SOLE, SEVERAL><<<grid, dim3(kBlock), 0, stream>>>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s.L, s.M, s.N, s.Bx, s.Lx, chunks, xes_shared, int(BL), per_group, cov, ts)
     if constexpr (p_max > 8) {
         switch (P) {
             case 16: GMC_BWD(16); return;
@@ -942,10 +997,10 @@ static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad
     int P = bwd_points_per_lane<T, D>(s);
     const size_t chunks = (size_t(s.N) + 64 * P - 1) / (64 * P);
     TileSlices ts = plan_tile_slices(grid_mixtures(BL) * chunks, s.M, kTile);
+    const LaunchCost model{(D == 2 ? 20.0 : 32.0) + (sizeof(T) == 8 ? 16.0 : 0.0), (sizeof(T) == 8 ? 12.0 : 5.0) * Sums<D>::k,
+                           need_gx ? 1500.0 : 0.0, need_gm ? 3500.0 : 0.0,
+                           need_gx ? (D == 2 ? 30.0 : 50.0) * double(BL / (size_t(s.Bx) * s.Lx) - 1) : 0.0};
     if (BL * chunks * ts.slices < 2048 && forced_bwd_points.load() < 2) {
-        const LaunchCost model{(D == 2 ? 20.0 : 32.0) + (sizeof(T) == 8 ? 16.0 : 0.0), (sizeof(T) == 8 ? 12.0 : 5.0) * Sums<D>::k,
-                               need_gx ? 1500.0 : 0.0, need_gm ? 3500.0 : 0.0,
-                               need_gx ? 30.0 * double(BL / (size_t(s.Bx) * s.Lx) - 1) : 0.0};
         const double full_cost = model.of(P, chunks, BL, ts.slices, ts.per_slice < s.M ? ts.per_slice : s.M);
         const SmallPlan small = plan_small_launch(model, BL, s.M, s.N, sizeof(T) == 8 ? 8 : 16, SmallPlan{P, ts}, 0.9 * full_cost);
         P = small.P;
@@ -957,7 +1012,10 @@ static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad
     const bool sole = need_gm && s.N <= 64 * P;
     if (need_gm && !sole) zero_async(sums, n_gauss * Sums<D>::k, stream);
     if (need_gx && gx_shared) zero_async(grad_xes, n_x, stream);
-    if (sole && need_gx) launch_bwd_main<T, D, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream);
+    const int per_group = need_gm && need_gx && s.Bx == 1 && s.Lx == 1 && BL > 1 ? plan_mixtures_per_group(model, P, BL, s.M, s.N, ts) : 1;
+    if (per_group > 1 && sole) launch_bwd_main<T, D, true, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream, per_group);
+    else if (per_group > 1) launch_bwd_main<T, D, true, true, false, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream, per_group);
+    else if (sole && need_gx) launch_bwd_main<T, D, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream);
     else if (sole) launch_bwd_main<T, D, true, false, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream);
     else if (need_gm && need_gx) launch_bwd_main<T, D, true, true, false>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream);
     else if (need_gm) launch_bwd_main<T, D, true, false, false>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream);

@@ -234,6 +234,23 @@ def test_small_launches_split_gaussians_below_a_tile(dtype, D):
 
 @pytest.mark.parametrize("D", [2, 3])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_many_mixtures_on_shared_points(dtype, D):
+    """a backward workgroup takes several mixtures one after the other when all of them share their points: a last group
+    with fewer mixtures, one chunk of points (gradients finished in the workgroup) and several, several tiles of Gaussians,
+    slices; against the oracle, and each gradient alone against both"""
+    for i, (B, L, M, N) in enumerate([(20, 20, 30, 100), (701, 1, 5, 65), (1, 67, 60, 700), (9, 11, 130, 300), (43, 3, 40, 1030),
+                                      (7, 5, 300, 270)]):
+        mix, xes, gout = _case(B, L, M, N, D, 65000 + i, broadcast=True)
+        _check(mix, xes, gout, dtype, tag=f"B{B} L{L} M{M} N{N} shared")
+        mt, xt = torch.tensor(mix, dtype=dtype, device=DEV), torch.tensor(xes, dtype=dtype, device=DEV)
+        gt = torch.tensor(gout, dtype=dtype, device=DEV)
+        gm_, gx_ = _native.eval_bwd(gt, mt, xt, True, True)
+        assert rel_l2(_native.eval_bwd(gt, mt, xt, True, False)[0].cpu().numpy(), gm_.cpu().numpy()) <= TOL[dtype]
+        assert rel_l2(_native.eval_bwd(gt, mt, xt, False, True)[1].cpu().numpy(), gx_.cpu().numpy()) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_few_points_many_gaussians(dtype, D):
     """mixtures whose points all fit into one wavefront (16 per lane, 8 in double; the shape one beyond takes the general
     kernels), with groups of 64 Gaussians that are full, ragged, or one for every wavefront, and with centred-form
