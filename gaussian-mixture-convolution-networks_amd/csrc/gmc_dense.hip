@@ -731,26 +731,36 @@ struct LaunchCost {
     static constexpr double kStage = 900.0;
 
     double of(int P, size_t chunks, size_t mixtures, int slices, int per) const {
-        const size_t rounds = (chunks * mixtures * slices + 255) / 256;
-        const double one = kStage * ((per + kTile - 1) / kTile) + (per + 3) / 4 * (P * pair + per_step);
+        return of(P, chunks, chunks * mixtures * slices, slices, kStage * ((per + kTile - 1) / kTile), (per + 3) / 4);
+    }
+    double of(int P, size_t chunks, size_t workgroups, int slices, double staging, double steps) const {
+        const size_t rounds = (workgroups + 255) / 256;
+        const double one = staging + steps * (P * pair + per_step);
         return one * double(rounds < 2 ? 2 : rounds) + (slices > 1 ? clear : 0.0) + (chunks > 1 ? several_chunks : 0.0) +
                contended * slices;
     }
 };
 struct SmallPlan { int P; TileSlices ts; };
 
+// (what depends on the slices alone is formed once: the search over some hundred plans takes well under a microsecond of
+// every small call)
 static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int M, int N, int p_max, SmallPlan full, double to_beat) {
     constexpr int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+    struct { int per, slices; double staging, steps; } cand[12];
+    int n = 0;
+    for (int want : kSlices) {
+        const int per = ((M + want - 1) / want + 3) / 4 * 4;
+        if (want > 1 && per < 32) break;
+        const int here = per < M ? per : M;
+        cand[n++] = {per, (M + per - 1) / per, LaunchCost::kStage * ((here + kTile - 1) / kTile), double((here + 3) / 4)};
+    }
     SmallPlan best = full;
     double best_cost = to_beat;
     for (int P = p_max; P >= 2; --P) {
-        const size_t chunks = (size_t(N) + 64 * P - 1) / (64 * P);
-        for (int want : kSlices) {
-            const int per = ((M + want - 1) / want + 3) / 4 * 4;
-            if (want > 1 && per < 32) break;
-            const int slices = (M + per - 1) / per;
-            const double cost = model.of(P, chunks, mixtures, slices, per < M ? per : M);
-            if (cost < best_cost) { best_cost = cost; best = SmallPlan{P, TileSlices{slices, per}}; }
+        const unsigned chunks = (unsigned(N) + 64u * P - 1u) / (64u * P);
+        for (int c = 0; c < n; ++c) {
+            const double cost = model.of(P, chunks, size_t(chunks) * mixtures * cand[c].slices, cand[c].slices, cand[c].staging, cand[c].steps);
+            if (cost < best_cost) { best_cost = cost; best = SmallPlan{P, TileSlices{cand[c].slices, cand[c].per}}; }
         }
     }
     return best;

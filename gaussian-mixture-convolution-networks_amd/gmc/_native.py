@@ -194,6 +194,12 @@ def _p(t):
     return t.data_ptr() if t is not None and t.numel() > 0 else None
 
 
+def _bwd_workspace_bytes(shape: Shape) -> int:
+    """gmc_eval_bwd_workspace_bytes without a call into the library (which refuses a smaller workspace): the
+    per-Gaussian sums, 6 scalars in 2-D and 10 in 3-D"""
+    return shape.B * shape.L * shape.M * (6 if shape.D == 2 else 10) * (4 if shape.dtype == GMC_F32 else 8)
+
+
 def eval_fwd(mixture: torch.Tensor, xes: torch.Tensor, covariance_form: bool = False) -> torch.Tensor:
     """`covariance_form`: the mixture holds covariances and the inversion happens inside the kernel"""
     shape = check_input(mixture, xes)
@@ -226,7 +232,7 @@ def eval_bwd(grad_output, mixture, xes, need_mixture: bool, need_xes: bool, cova
     if not (need_mixture or need_xes):
         return grad_mixture, grad_xes
     with _on(dev):
-        ws_bytes = lib().gmc_eval_bwd_workspace_bytes(ctypes.byref(shape)) if need_mixture else 0
+        ws_bytes = _bwd_workspace_bytes(shape) if need_mixture else 0
         ws = torch.empty((max(ws_bytes, 8) // 8,), dtype=torch.float64, device=dev)
         fn = lib().gmc_eval_cov_bwd if covariance_form else lib().gmc_eval_bwd
         check(fn(_p(grad_output), _p(mixture), _p(xes), _p(grad_mixture), _p(grad_xes), _p(ws), ws_bytes,
@@ -259,7 +265,7 @@ def eval_componentwise_bwd(grad_output, mixture, xes, need_mixture: bool, need_x
     if not (need_mixture or need_xes):
         return grad_mixture, grad_xes
     with _on(dev):
-        ws_bytes = lib().gmc_eval_bwd_workspace_bytes(ctypes.byref(shape)) if need_mixture else 0
+        ws_bytes = _bwd_workspace_bytes(shape) if need_mixture else 0
         ws = torch.empty((max(ws_bytes, 8) // 8,), dtype=torch.float64, device=dev)
         check(lib().gmc_eval_componentwise_bwd(_p(grad_output), _p(mixture), _p(xes), _p(grad_mixture), _p(grad_xes),
                                                _p(ws), ws_bytes, ctypes.byref(shape), int(need_mixture), int(need_xes),

@@ -1,5 +1,6 @@
 """Parity of the dense HIP path (through the C ABI, via the gmc.mixture API) against the CPU oracle.
 Tolerances: relative L2 <= 1e-5 (float32) and <= 1e-12 (float64) per output tensor."""
+import ctypes
 import itertools
 import json
 import math
@@ -439,6 +440,12 @@ def test_more_than_65535_mixtures():
     _check(mix, xes, gout, torch.float32, tag="B70000")
     mix, xes, gout = _case(300, 250, 2, 4, 3, 78, True)
     _check(mix, xes, gout, torch.float64, tag="B300 L250 broadcast")
+
+
+def test_workspace_size_is_the_librarys():
+    for D, dtype, M in itertools.product((2, 3), (_native.GMC_F32, _native.GMC_F64), (0, 1, 333)):
+        shape = _native.Shape(3, 2, M, 10, D, 3, 2, dtype)
+        assert _native._bwd_workspace_bytes(shape) == _native.lib().gmc_eval_bwd_workspace_bytes(ctypes.byref(shape))
 
 
 def test_empty_inputs():
