@@ -567,4 +567,18 @@ inline void zero_async(T* p, size_t n, hipStream_t stream) {
     fill_zero_kernel<T><<<dim3(unsigned(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream>>>(p, n);
 }
 
+// two arrays in one launch
+template <typename T>
+__global__ void fill_zero2_kernel(T* p, size_t n, T* q, size_t m) {
+    const size_t stride = size_t(gridDim.x) * blockDim.x;
+    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n + m; i += stride) (i < n ? p[i] : q[i - n]) = T(0);
+}
+template <typename T>
+inline void zero2_async(T* p, size_t n, T* q, size_t m, hipStream_t stream) {
+    if (n == 0) return zero_async(q, m, stream);
+    if (m == 0) return zero_async(p, n, stream);
+    const size_t blocks = (n + m + 255) / 256;
+    fill_zero2_kernel<T><<<dim3(unsigned(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream>>>(p, n, q, m);
+}
+
 }  // namespace gmc

@@ -1020,8 +1020,7 @@ static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad
     const int gx_shared = (xes_shared || ts.slices > 1) ? 1 : 0;
     // one chunk per mixture: the pair kernel's workgroups finish the gradient of their mixture themselves
     const bool sole = need_gm && s.N <= 64 * P;
-    if (need_gm && !sole) zero_async(sums, n_gauss * Sums<D>::k, stream);
-    if (need_gx && gx_shared) zero_async(grad_xes, n_x, stream);
+    zero2_async(sums, need_gm && !sole ? n_gauss * Sums<D>::k : 0, grad_xes, need_gx && gx_shared ? n_x : 0, stream);
     const int per_group = need_gm && need_gx && s.Bx == 1 && s.Lx == 1 && BL > 1 ? plan_mixtures_per_group(model, P, BL, s.M, s.N, ts) : 1;
     if (per_group > 1 && sole) launch_bwd_main<T, D, true, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream, per_group);
     else if (per_group > 1) launch_bwd_main<T, D, true, true, false, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream, per_group);
