@@ -771,7 +771,7 @@ static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int
 // be as long as 0.7 of the modelled work (a shorter one hides behind it: 800 x 128 Gaussians at 784 points 70.5 us with one
 // mixture per workgroup, 82 us with several).  Measured, one mixture / several in us:
 //   6400 x 16 Gaussians at 100 points, 2-D: 317 / 67;  1353 x 36 at 361: 82 / 44, in 3-D 120 / 69;  2268 x 23 at 3049,
-//   3-D: 382 / 190;  1116 x 52 at 1547, 3-D: 134 / 113
+//   3-D: 381 / 227;  1116 x 52 at 1547, 3-D: 134 / 113
 static int plan_mixtures_per_group(const LaunchCost& model, int P, size_t mixtures, int M, int N, TileSlices ts) {
     constexpr int kGroup[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
     const size_t chunks = (size_t(N) + 64 * P - 1) / (64 * P);
