@@ -745,6 +745,7 @@ struct SmallPlan { int P; TileSlices ts; };
 // (what depends on the slices alone is formed once: the search over some hundred plans takes well under a microsecond of
 // every small call)
 static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int M, int N, int p_max, SmallPlan full, double to_beat) {
+    if (mixtures == 0 || M == 0 || N == 0) return full;         // (nothing to launch: asked for by reports only)
     constexpr int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
     struct { int per, slices; double staging, steps; } cand[12];
     int n = 0;

@@ -4,6 +4,8 @@ src/gmc/cpp/extensions/util/mixture.h:37-45,107-127 and parallel_implementation.
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -68,6 +70,22 @@ def test_scratch_sizes_and_knobs_without_a_device():
         knob(0)
     lib.gmc_bvh_set_traversal_groups(2, 3)
     lib.gmc_bvh_set_traversal_groups(0, 0)
+
+
+def test_forward_kernel_name_of_empty_shapes():
+    """a report asks for any shape the calls accept, empty ones among them: a name and no division by zero (in a process
+    of its own, which that would end)"""
+    code = """
+import ctypes, itertools, sys
+sys.path.insert(0, {!r})
+from gmc import _native
+names = set()
+for B, M, N, D, dtype in itertools.product((0, 1, 40), (0, 1, 333), (0, 1, 500), (2, 3), (0, 1)):
+    names.add(_native.lib().gmc_eval_fwd_kernel_name(ctypes.byref(_native.Shape(B, 2, M, N, D, B, 2, dtype))))
+assert b"" not in names, names
+assert _native.lib().gmc_eval_fwd_kernel_name(ctypes.byref(_native.Shape(1, 2, 3, 4, 5, 1, 2, 0))) == b""
+""".format(os.path.join(ROOT, "gaussian-mixture-convolution-networks_amd"))
+    assert subprocess.run([sys.executable, "-c", code], timeout=120).returncode == 0
 
 
 def test_python_boundary_errors():
