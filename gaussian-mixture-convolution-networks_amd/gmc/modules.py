@@ -21,9 +21,17 @@ def _scale_weights_composed(x_gm: Tensor, scaling: Tensor) -> Tensor:
     return torch.cat((gm.weights(x_gm).unsqueeze(-1) * scaling.unsqueeze(-1).unsqueeze(-1), x_gm[..., 1:]), dim=-1)
 
 
+def _plain_device_tensors(*tensors: Tensor) -> bool:
+    """what the kernels take: device memory behind each tensor itself (no subclass, batched or traced tensor)"""
+    return torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0 and \
+        all(type(t) in (Tensor, torch.nn.Parameter) and t.is_cuda and
+            not torch._C._functorch.is_functorch_wrapped_tensor(t) and
+            not torch._C._functorch.is_legacy_batchedtensor(t) for t in tensors)
+
+
 class _ScaleWeights(torch.autograd.Function):
     """_scale_weights_composed as one pass over the mixture in either direction; a backward pass that is itself
-    differentiated is composed of torch operations"""
+    differentiated or batched (is_grads_batched, vmap) is composed of torch operations"""
 
     @staticmethod
     def forward(ctx, x_gm: Tensor, scaling: Tensor) -> Tensor:
@@ -34,7 +42,7 @@ class _ScaleWeights(torch.autograd.Function):
     def backward(ctx, grad_out: Tensor):
         x_gm, scaling = ctx.saved_tensors
         need_gm, need_scaling = ctx.needs_input_grad
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not _plain_device_tensors(grad_out, x_gm, scaling):
             grad_gm = _scale_weights_composed(grad_out, scaling) if need_gm else None
             grad_scaling = None
             if need_scaling:
@@ -48,13 +56,11 @@ class _ScaleWeights(torch.autograd.Function):
 def _scale_weights(x_gm: Tensor, scaling: Tensor) -> Tensor:
     """x_gm with its weights times scaling [batch or 1, channels].  The kernels take plain device tensors; others (CPU
     tensors, other types, subclasses, tracing, functorch and forward-mode transforms) go through torch operations."""
-    plain = not torch.compiler.is_compiling() and \
-        type(x_gm) in (Tensor, torch.nn.Parameter) and type(scaling) in (Tensor, torch.nn.Parameter) and \
-        x_gm.is_cuda and scaling.device == x_gm.device and x_gm.dtype in (torch.float32, torch.float64) and \
-        scaling.dtype == x_gm.dtype and x_gm.dim() == 4 and x_gm.shape[-1] in (7, 13) and \
-        not torch.jit.is_tracing() and \
-        not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0 and \
-        torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+    plain = not torch.compiler.is_compiling() and not torch.jit.is_tracing() and \
+        _plain_device_tensors(x_gm, scaling) and scaling.device == x_gm.device and \
+        x_gm.dtype in (torch.float32, torch.float64) and scaling.dtype == x_gm.dtype and \
+        x_gm.dim() == 4 and x_gm.shape[-1] in (7, 13) and \
+        not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
     return _ScaleWeights.apply(x_gm, scaling) if plain else _scale_weights_composed(x_gm, scaling)
 
 

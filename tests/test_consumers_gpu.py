@@ -403,6 +403,23 @@ def test_batch_norm_scaling_of_the_weights(D, dtype):
     assert torch.equal(tangent[..., 0], x[..., 0]) and not tangent[..., 1:].any()
 
 
+def test_batch_norm_batched_backward():
+    """a batched backward pass through the layer (vectorised Jacobian rows) against the rows one by one; the statistics
+    carry no gradient, so training and evaluation mode alike end in the scaling of the weights"""
+    gen = torch.Generator(device=DEV).manual_seed(23)
+    m = torch.tensor(_cov_mixture(np.random.default_rng(29), 2, 3, 5, 2), dtype=torch.float32, device=DEV, requires_grad=True)
+    bn = modules.BatchNorm(3).to(DEV)
+    for training in (True, False):
+        bn.train(training)
+        out, _ = bn((m, None))
+        up = torch.randn(4, *out.shape, generator=gen, device=DEV)
+        wrt = (m, bn.learnable_scaling)
+        batched = torch.autograd.grad(out, wrt, up, is_grads_batched=True, retain_graph=True)
+        for k in range(4):
+            for a, b in zip(batched, torch.autograd.grad(out, wrt, up[k], retain_graph=True)):
+                assert rel_l2(a[k].cpu().numpy(), b.cpu().numpy(), 1e-30) <= 1e-6
+
+
 def test_validate_flag_raises_like_the_reference_check():
     """util/mixture.h:85-93 (called by the reference's CUDA backward), off by default here: with validate=True NaNs,
     infinities and matrices with a determinant <= 0 raise RuntimeError; without it nothing is checked (and nothing

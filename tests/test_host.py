@@ -204,6 +204,28 @@ def test_ply_text_matches_the_reference_writer_byte_for_byte(tmp_path, golden_di
     assert torch.equal(back, gm.pack_mixture(w, p, c))
 
 
+def test_batched_backward_of_the_weight_scaling_stays_off_the_kernels(monkeypatch):
+    """BatchNorm's scaling of the weights under a batched backward pass (is_grads_batched, vectorised Jacobians, vmap): the
+    kernels take memory and must not be handed a batched tensor.  Host tensors stand in for device ones."""
+    from gmc import modules
+
+    def no_kernel(*args):
+        raise AssertionError("a batched gradient reached the kernel")
+    monkeypatch.setattr(_native, "scale_weights", modules._scale_weights_composed)
+    monkeypatch.setattr(_native, "scale_weights_bwd", no_kernel)
+    g = torch.Generator().manual_seed(5)
+    for S in (1, 2):
+        x = torch.randn(2, 3, 4, 7, generator=g, dtype=torch.float64, requires_grad=True)
+        s = torch.randn(S, 3, generator=g, dtype=torch.float64, requires_grad=True)
+        up = torch.randn(5, 2, 3, 4, 7, generator=g, dtype=torch.float64)
+        ref = torch.autograd.grad(modules._scale_weights_composed(x, s), (x, s), up, is_grads_batched=True)
+        out = modules._ScaleWeights.apply(x, s)
+        got = [torch.autograd.grad(out, (x, s), up, is_grads_batched=True, retain_graph=True),
+               torch.vmap(lambda u: torch.autograd.grad(out, (x, s), u, retain_graph=True))(up)]
+        for grads in got:
+            assert all(torch.allclose(a, b, rtol=1e-13, atol=1e-13) for a, b in zip(grads, ref))
+
+
 def test_check_valid_mixture_on_host_tensors():
     g = torch.Generator().manual_seed(4)
     a = torch.rand(2, 2, 3, 2, 2, generator=g)
