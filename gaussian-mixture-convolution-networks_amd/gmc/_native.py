@@ -427,22 +427,24 @@ def scale_weights(mixture: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
 
 
 def scale_weights_bwd(grad_out: torch.Tensor, mixture: torch.Tensor, scale: torch.Tensor, need_mixture: bool, need_scale: bool):
-    """gradients of scale_weights (None where not needed)"""
-    shape = _mixture_shape(mixture, 0)
-    scale = _scale_of(scale, mixture, shape)
-    grad_out = _like(grad_out, mixture, mixture.shape, "grad_out")
-    grad_mixture = torch.empty_like(mixture) if need_mixture else None
+    """gradients of scale_weights (None where not needed); the mixture is read for the scale's gradient only and may be
+    None without it"""
+    shape = _mixture_shape(grad_out, 0)
+    scale = _scale_of(scale, grad_out, shape)
+    if need_scale:
+        mixture = _like(mixture, grad_out, grad_out.shape, "mixture")
+    grad_mixture = torch.empty_like(grad_out) if need_mixture else None
     partial = None
-    with _on(mixture.device):
+    with _on(grad_out.device):
         if need_scale:
             partial = torch.empty((shape.B, shape.L, int(lib().gmc_scale_weights_chunks(ctypes.byref(shape)))),
-                                  dtype=torch.float64, device=mixture.device)
-        check(lib().gmc_scale_weights_bwd(_p(grad_out), _p(mixture), _p(scale), _p(grad_mixture), _p(partial),
-                                          ctypes.byref(shape), int(scale.shape[0] == shape.B), _stream(mixture.device)))
+                                  dtype=torch.float64, device=grad_out.device)
+        check(lib().gmc_scale_weights_bwd(_p(grad_out), _p(mixture) if need_scale else None, _p(scale), _p(grad_mixture), _p(partial),
+                                          ctypes.byref(shape), int(scale.shape[0] == shape.B), _stream(grad_out.device)))
     if partial is None:
         return grad_mixture, None
     grad_scale = partial.sum((0, 2)).unsqueeze(0) if scale.shape[0] == 1 else partial.sum(2)
-    return grad_mixture, grad_scale.to(mixture.dtype)
+    return grad_mixture, grad_scale.to(grad_out.dtype)
 
 
 # ---------------------------------------------------------------------------------------------------------------

@@ -35,14 +35,16 @@ class _ScaleWeights(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x_gm: Tensor, scaling: Tensor) -> Tensor:
-        ctx.save_for_backward(x_gm, scaling)
+        # (the mixture only for the scaling's gradient: without learnable scaling it need not live until the backward pass,
+        # and its owner may overwrite it)
+        ctx.save_for_backward(x_gm if ctx.needs_input_grad[1] else None, scaling)
         return _native.scale_weights(x_gm.contiguous(), scaling)
 
     @staticmethod
     def backward(ctx, grad_out: Tensor):
         x_gm, scaling = ctx.saved_tensors
         need_gm, need_scaling = ctx.needs_input_grad
-        if torch.is_grad_enabled() or not _plain_device_tensors(grad_out, x_gm, scaling):
+        if torch.is_grad_enabled() or not _plain_device_tensors(grad_out, scaling, *((x_gm,) if need_scaling else ())):
             grad_gm = _scale_weights_composed(grad_out, scaling) if need_gm else None
             grad_scaling = None
             if need_scaling:
@@ -50,7 +52,8 @@ class _ScaleWeights(torch.autograd.Function):
                 if scaling.shape[0] == 1:
                     grad_scaling = grad_scaling.sum(0, keepdim=True)
             return grad_gm, grad_scaling
-        return _native.scale_weights_bwd(grad_out.contiguous(), x_gm.contiguous(), scaling, need_gm, need_scaling)
+        return _native.scale_weights_bwd(grad_out.contiguous(), x_gm.contiguous() if need_scaling else None, scaling,
+                                         need_gm, need_scaling)
 
 
 def _scale_weights(x_gm: Tensor, scaling: Tensor) -> Tensor:

@@ -168,7 +168,8 @@ int gmc_relu_fit_grad_finish(const void* grad_out, const void* fitting_mixture, 
 
 /* BatchNorm's scaling of the weights, src/gmc/modules.py:417-421: out = mixture [B][L][M] with every weight times
  * scale[l] (scale_per_batch 0) or scale[b][l]; shape->N, Bx, Lx as for a call with one set of points per mixture (N may
- * be 0).  Backward: grad_mixture (may be NULL) and partial (may be NULL), double [B][L][gmc_scale_weights_chunks], whose
+ * be 0).  Backward: grad_mixture (may be NULL) and partial (may be NULL, `mixture` is then not read and may be NULL too),
+ * double [B][L][gmc_scale_weights_chunks], whose
  * sum over the last axis (and over b for a scale per channel) is the gradient of the scale. */
 size_t gmc_scale_weights_chunks(const gmc_shape* shape);
 int gmc_scale_weights(const void* mixture, const void* scale, void* out, const gmc_shape* shape, int scale_per_batch, void* stream);

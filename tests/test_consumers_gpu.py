@@ -420,6 +420,24 @@ def test_batch_norm_batched_backward():
                 assert rel_l2(a[k].cpu().numpy(), b.cpu().numpy(), 1e-30) <= 1e-6
 
 
+def test_batch_norm_without_learnable_scaling_keeps_no_mixture():
+    """without a gradient for the scaling the backward pass needs no mixture: none is kept for it, and the layer's input
+    may be overwritten before it"""
+    x = torch.tensor(_cov_mixture(np.random.default_rng(31), 2, 3, 50, 2), dtype=torch.float32, device=DEV, requires_grad=True)
+    up = torch.randn(2, 3, 50, 7, generator=torch.Generator(device=DEV).manual_seed(24), device=DEV)
+    bn = modules.BatchNorm(3, learn_scaling=False).to(DEV).eval()
+    bn.averaged_channel_sd.copy_(torch.tensor([0.5, 2.0, 3.0]))
+    inner = x * 1.0
+    out, _ = bn((inner, None))
+    assert not any(t is not None and t.numel() == x.numel() for t in out.grad_fn.saved_tensors)
+    with torch.no_grad():
+        inner.zero_()
+    grad, = torch.autograd.grad(out, x, up)
+    ref = up.clone()
+    ref[..., 0] *= (1 / bn.averaged_channel_sd).view(1, 3, 1)
+    assert torch.equal(grad, ref)
+
+
 def test_validate_flag_raises_like_the_reference_check():
     """util/mixture.h:85-93 (called by the reference's CUDA backward), off by default here: with validate=True NaNs,
     infinities and matrices with a determinant <= 0 raise RuntimeError; without it nothing is checked (and nothing
