@@ -619,6 +619,7 @@ __global__ __launch_bounds__(kBlock) void few_points_bwd_kernel(const T* __restr
     const T* exp2_tab = exp2_table<T>();
     if constexpr (sizeof(T) == 8) __syncthreads();
 
+    const ClockProbe probe = clock_probe_begin();
     int bl, slice;
     map_workgroup(blockIdx.x, ts.slices, n_mixtures, bl, slice);
     if (bl >= n_mixtures) return;
@@ -682,6 +683,7 @@ __global__ __launch_bounds__(kBlock) void few_points_bwd_kernel(const T* __restr
             if (xes_shared) atomic_add(dst, -v); else *dst = -v;
         }
     }
+    clock_probe_end(probe, backward_clocks);
 }
 
 // ---- host-side launchers ------------------------------------------------------------------------------

@@ -63,7 +63,7 @@ void gmc_set_tuning(int fwd_points_per_lane, int bwd_points_per_lane);
  * "eval_fwd_rc_kernel" or "eval_fwd_kernel" (all vector ALU, two layouts); "" for an invalid shape. */
 const char* gmc_eval_fwd_kernel_name(const gmc_shape* shape);
 /* Shader clock in MHz that one workgroup in the middle of the grid saw during the last launch of the float32
- * matrix-core forward kernel (shader_mhz[0]) and of the backward pair kernel (shader_mhz[1]) on the current device; 0
+ * matrix-core forward kernel (shader_mhz[0]) and of a dense backward kernel (shader_mhz[1]) on the current device; 0
  * before the first such launch.  For benchmark reports (no counterpart in the reference): with the vector ALUs busy
  * the clock settles below the peak engine clock that published peak rates assume.  `shader_mhz` is host memory
  * for two doubles; the call waits for the device like a plain copy from device memory (do not call it under graph
@@ -169,8 +169,8 @@ int gmc_relu_fit_grad_finish(const void* grad_out, const void* fitting_mixture, 
 /* BatchNorm's scaling of the weights, src/gmc/modules.py:417-421: out = mixture [B][L][M] with every weight times
  * scale[l] (scale_per_batch 0) or scale[b][l]; shape->N, Bx, Lx as for a call with one set of points per mixture (N may
  * be 0).  Backward: grad_mixture (may be NULL) and partial (may be NULL, `mixture` is then not read and may be NULL too),
- * double [B][L][gmc_scale_weights_chunks], whose
- * sum over the last axis (and over b for a scale per channel) is the gradient of the scale. */
+ * double [B][L][gmc_scale_weights_chunks], whose sum over the last axis (and over b for a scale per channel) is the
+ * gradient of the scale. */
 size_t gmc_scale_weights_chunks(const gmc_shape* shape);
 int gmc_scale_weights(const void* mixture, const void* scale, void* out, const gmc_shape* shape, int scale_per_batch, void* stream);
 int gmc_scale_weights_bwd(const void* grad_out, const void* mixture, const void* scale, void* grad_mixture, double* partial,

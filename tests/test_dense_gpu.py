@@ -270,6 +270,20 @@ def test_few_points_many_gaussians(dtype, D):
         assert rel_l2(alone.cpu().numpy(), both.cpu().numpy()) <= TOL[dtype]
 
 
+def test_every_backward_launch_leaves_its_clocks():
+    """the exported clock of the last backward launch, whichever kernel it took: 64 or 1024 points a mixture (the kernel for
+    few points, the general one) in turn; a reading that no launch changes would be an earlier launch's"""
+    mhz = (ctypes.c_double * 2)()
+    readings = []
+    for n_points in (1024, 64, 64, 64, 64):
+        mix, xes, gout = (torch.tensor(a, dtype=torch.float32, device=DEV) for a in _case(8, 8, 512, n_points, 2, 64000, False))
+        _native.eval_bwd(gout, mix, xes, True, True)
+        torch.cuda.synchronize()
+        assert _native.lib().gmc_export_launch_clocks(mhz) == 0
+        readings.append(mhz[1])
+    assert min(readings) > 0.0 and len(set(readings)) > 1, readings
+
+
 @pytest.mark.parametrize("D", [2, 3])
 def test_matrix_core_forward_shapes(D):
     """float32 shapes that take the wide matrix-core forward kernel (more than 128 components and either many
