@@ -67,8 +67,9 @@ template <> __device__ __forceinline__ double reciprocal<float>(double x) {
     const double e = __builtin_fma(-x, r, 1.0);
     return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
-template <typename T> __device__ __forceinline__ double quotient(double a, double b) {
-    if constexpr (sizeof(T) == 8) return a / b; else return a * reciprocal<T>(b);
+// a / kHalfLog2e, rounded once for float64 tensors
+template <typename T> __device__ __forceinline__ double over_half_log2e(double a) {
+    if constexpr (sizeof(T) == 8) return a / kHalfLog2e; else return a * (1.0 / kHalfLog2e);
 }
 struct Root { double value, inverse; };                 // sqrt(x); 1 / sqrt(x), float only
 template <typename T> __device__ __forceinline__ Root root(double x);

@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T
         for (int q = 0; q < Q; ++q) {
             const Derived<D> dv = derive<T, D>(mixture + (size_t(bl) * M + (m0 + q * apart < M ? m0 + q * apart : 0)) * G, covariance_form);
             // amplitude for dL/dx as in the summed backward kernel: w norm / (0.5 log2 e)
-            store_record<T, D>(r[q], dv, true, dv.w * dv.norm * (1.0 / kHalfLog2e), 0);
+            store_record<T, D>(r[q], dv, true, over_half_log2e<T>(dv.w * dv.norm), 0);
 #pragma unroll
             for (int i = 0; i < kU; ++i) ua[q][i] = -r[q][Rec<T, D>::kAmp] * r[q][i];
         }

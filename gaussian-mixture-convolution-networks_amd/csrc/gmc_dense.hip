@@ -501,7 +501,7 @@ __device__ __forceinline__ void bwd_epilogue_derived(const Derived<D>& dv, const
         V[0][2] = -(U[0][1] * V[1][2] + U[0][2] * V[2][2]) * V[0][0];
     }
     // db = k u^T R1
-    const double k = wn * (1.0 / kHalfLog2e);
+    const double k = over_half_log2e<T>(wn);
 #pragma unroll
     for (int r = 0; r < D; ++r) {
         double acc = 0.0;

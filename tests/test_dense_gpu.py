@@ -642,6 +642,28 @@ def test_componentwise_backward_edges(dtype, D):
                 assert rel_l2(gx_.cpu().numpy(), rgx.numpy(), FLOOR[dtype]) <= TOL[dtype], (B, L, M, N)
 
 
+def test_float64_centre_gradients_round_like_the_formula():
+    """the gradients of position and query point of single pairs in float64, bit for bit: with a diagonal matrix and the
+    point so close to the centre that exp() is 1 every step is one rounding, so numpy gives the same bits -- as long as the
+    factor 2 / log2(e) is divided by, not multiplied with a rounded reciprocal"""
+    rng = np.random.default_rng(77)
+    n = 2000
+    half_log2e = 0.5 * 1.4426950408889634
+    w, c = rng.uniform(0.5, 2.0, n), rng.uniform(0.5, 2.0, (n, 2))
+    b = rng.integers(-2 ** 20, 2 ** 20, (n, 2)) * 2.0 ** -20
+    t = rng.integers(1, 8, (n, 2)) * 2.0 ** -40
+    go = rng.normal(size=n)
+    mix = np.zeros((n, 1, 1, 7))
+    mix[:, 0, 0, 0], mix[:, 0, 0, 1:3], mix[:, 0, 0, 3], mix[:, 0, 0, 6] = w, b, c[:, 0], c[:, 1]
+    gm_, gx_ = _native.eval_componentwise_bwd(torch.tensor(go, device=DEV).view(n, 1, 1, 1), torch.tensor(mix, device=DEV),
+                                              torch.tensor(b + t, device=DEV).view(n, 1, 1, 2), True, True)
+    u = np.sqrt(half_log2e * c)
+    ky = (u * t) * go[:, None]
+    k = (w * (o.kappa(2) * np.sqrt(c[:, 0] * c[:, 1]))) / half_log2e
+    assert np.array_equal(gm_.cpu().numpy()[:, 0, 0, 1:3], k[:, None] * (u * ky))
+    assert np.array_equal(gx_.cpu().numpy()[:, 0, 0], (-k[:, None] * u) * ky)
+
+
 def _workload_check(name, **kw):
     wl, mix, xes, gout = synthetic.make_workload(name, **kw)
     out, gmix, gxes = _run(mix.numpy(), xes.numpy(), gout.numpy(), wl.dtype)
