@@ -52,36 +52,53 @@ __device__ __forceinline__ double pair_exp2(double x, const double* __restrict__
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// Reciprocals and roots of the per-Gaussian preparation, in double.  For float32 tensors they come from the hardware's
-// estimates (v_rcp_f64 / v_rsq_f64, at least 2^-23) and one third-order correction, 2^-50 or better before the result
-// is rounded to float: 5 and 8 instructions instead of about 15 for a double division and 20 for a square root, which
-// the staging of a Gaussian needs five to fifteen of.  A float's entries keep every intermediate far inside double's
-// range, so the scaling and the special cases of the full sequences have nothing to do; 0 keeps its root 0, negative
-// arguments give NaN.  float64 tensors use the correctly rounded operations.  Measured with the full sequences / now:
-// a convolution layer whose 8.2e6 Gaussians are each met by 100-128 points only 2.93 / 2.84 ms, 336 mixtures of 64
-// Gaussians at 4096 points forward and backward 121 / 119 us.
+// Reciprocals, quotients and roots of the per-Gaussian preparation, in double.  For float32 tensors they come from the
+// hardware's estimates (v_rcp_f64 / v_rsq_f64, at least 2^-23), one third-order correction and, for quotients and roots, the
+// remainder against the rounded result: correctly rounded but for cases within 2^-20 of an ulp of a tie, instead of about
+// 15 instructions for a double division and 20 for a square root, which the staging of a Gaussian needs five to fifteen of.
+// (The factor's a11 - u01^2 of a singular matrix is then what it is with the full sequences: without the remainders a
+// matrix of ones came out as NaN.)  A float's entries keep every intermediate far inside double's range, so the scaling of
+// the full sequences has nothing to do; zeros and infinities take the estimate, which is exact there, and roots of negative
+// arguments give NaN.  float64 tensors use the compiler's sequences.  Values and gradients of 1200 mixtures of 60 Gaussians
+// at 700 points are the same bit for bit as with the full sequences (2-D and 3-D, both forms).  Measured with those for float32 too / now, covariance
+// form: 1600 mixtures of 5120 Gaussians at 100 points in 3-D forward 341 / 312 us (every Gaussian meets few points),
+// 4000 of 64 at 64 points in 3-D backward 66.4 / 61.8 us, 800 of 10 at 784 points in 2-D 14.5 / 13.8 us; where a Gaussian
+// meets many points 0 to 2 % (84 of 4644 at 755 points in 2-D backward 241 / 239 us).
 template <typename T> __device__ __forceinline__ double reciprocal(double x);
 template <> __device__ __forceinline__ double reciprocal<double>(double x) { return 1.0 / x; }
 template <> __device__ __forceinline__ double reciprocal<float>(double x) {
+    constexpr int kZeroOrInfinity = 0x264;
     const double r = __builtin_amdgcn_rcp(x);
     const double e = __builtin_fma(-x, r, 1.0);
-    return __builtin_fma(r, __builtin_fma(e, e, e), r);
+    return __builtin_amdgcn_class(x, kZeroOrInfinity) ? r : __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+// a / x with r = reciprocal<T>(x), x neither 0 nor infinite
+__device__ __forceinline__ double quotient_of_reciprocal(double a, double x, double r) {
+    const double q = a * r;
+    return __builtin_fma(__builtin_fma(-q, x, a), r, q);
+}
+struct Root { double value, inverse; bool special; };       // sqrt(x); float only: 1 / sqrt(x), x is 0 or infinite
+template <typename T> __device__ __forceinline__ Root root(double x);
+template <> __device__ __forceinline__ Root root<double>(double x) { return {sqrt(x), 0.0, false}; }
+template <> __device__ __forceinline__ Root root<float>(double x) {
+    constexpr int kZeroOrPositiveInfinity = 0x260;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = __builtin_fma(-(x * y), y, 1.0);
+    const double inv = __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+    const double s = x * inv;
+    const double value = __builtin_fma(__builtin_fma(-s, s, x), 0.5 * inv, s);
+    const bool special = __builtin_amdgcn_class(x, kZeroOrPositiveInfinity);
+    return {special ? x : value, special ? y : inv, special};
+}
+// a / r.value
+template <typename T> __device__ __forceinline__ double over(double a, const Root& r) {
+    if constexpr (sizeof(T) == 8) return a / r.value;
+    const double q = a * r.inverse;
+    return r.special ? q : __builtin_fma(__builtin_fma(-q, r.value, a), r.inverse, q);
 }
 // a / kHalfLog2e, rounded once for float64 tensors
 template <typename T> __device__ __forceinline__ double over_half_log2e(double a) {
     if constexpr (sizeof(T) == 8) return a / kHalfLog2e; else return a * (1.0 / kHalfLog2e);
-}
-struct Root { double value, inverse; };                 // sqrt(x); 1 / sqrt(x), float only
-template <typename T> __device__ __forceinline__ Root root(double x);
-template <> __device__ __forceinline__ Root root<double>(double x) { return {sqrt(x), 0.0}; }
-template <> __device__ __forceinline__ Root root<float>(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = __builtin_fma(-(x * y), y, 1.0);
-    const double inv = __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
-    return {x == 0.0 ? 0.0 : x * inv, inv};
-}
-template <typename T> __device__ __forceinline__ double over(double a, const Root& r) {
-    if constexpr (sizeof(T) == 8) return a / r.value; else return a * r.inverse;
 }
 
 // Per-Gaussian quantities derived once from the stored record (weight, position b, inverse covariance C):
@@ -114,7 +131,12 @@ __device__ __forceinline__ void load_inverse_covariance(const T* __restrict__ c,
         // (S^-1)^T
         if constexpr (sizeof(T) == 4) {
             const double r = reciprocal<T>(det);
-            m[0][0] = d * r; m[0][1] = -cc * r; m[1][0] = -b * r; m[1][1] = a * r;
+            if (r == 0.0 || det == 0.0) {
+                m[0][0] = d * r; m[0][1] = -cc * r; m[1][0] = -b * r; m[1][1] = a * r;
+            } else {
+                m[0][0] = quotient_of_reciprocal(d, det, r); m[0][1] = -quotient_of_reciprocal(cc, det, r);
+                m[1][0] = -quotient_of_reciprocal(b, det, r); m[1][1] = quotient_of_reciprocal(a, det, r);
+            }
         } else {
             m[0][0] = d / det; m[0][1] = -cc / det; m[1][0] = -b / det; m[1][1] = a / det;
         }
@@ -133,10 +155,12 @@ __device__ __forceinline__ void load_inverse_covariance(const T* __restrict__ c,
         const double det = m[0][0] * k[0][0] + m[0][1] * k[0][1] + m[0][2] * k[0][2];
         // S^-1 = cofactor^T / det, hence (S^-1)^T = cofactor / det
         const double r = sizeof(T) == 4 ? reciprocal<T>(det) : 0.0;
+        const bool plain = sizeof(T) == 4 && (r == 0.0 || det == 0.0);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) m[i][j] = sizeof(T) == 4 ? k[i][j] * r : k[i][j] / det;
+            for (int j = 0; j < 3; ++j)
+                m[i][j] = sizeof(T) == 8 ? k[i][j] / det : plain ? k[i][j] * r : quotient_of_reciprocal(k[i][j], det, r);
     }
 }
 

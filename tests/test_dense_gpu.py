@@ -664,6 +664,30 @@ def test_float64_centre_gradients_round_like_the_formula():
     assert np.array_equal(gx_.cpu().numpy()[:, 0, 0], (-k[:, None] * u) * ky)
 
 
+@pytest.mark.parametrize("D", [2, 3])
+def test_singular_matrices_give_the_same_infinities_in_both_types(D):
+    """float32 tensors prepare their Gaussians with corrected hardware estimates, float64 ones with full divisions and
+    roots; where a matrix is singular, infinite or negative both must give a NaN or an infinity in the same places"""
+    inf, nan = float("inf"), float("nan")
+    mats = {2: [[0, 0, 0, 0], [1, 1, 1, 1], [4, 0, 0, 0], [0, 0, 0, 4], [inf, 0, 0, 4], [4, 0, 0, inf], [-1, 0, 0, 4], [nan, 0, 0, 1]],
+            3: [[0] * 9, [1] * 9, [4, 0, 0, 0, 4, 0, 0, 0, 0], [0, 0, 0, 0, 4, 0, 0, 0, 4], [1, 1, 0, 1, 1, 0, 0, 0, 4],
+                [4, 0, 0, 0, inf, 0, 0, 0, 4], [4, 0, 0, 0, 4, 0, 0, 0, -1]]}[D]
+
+    def classes(t):
+        t = t.cpu()
+        return torch.where(t.isnan(), 3, torch.where(t.isinf(), t.sign(), torch.zeros_like(t)).int())
+    for mat, covariance_form in itertools.product(mats, (False, True)):
+        results = []
+        for dtype in (torch.float32, torch.float64):
+            m = torch.tensor([1.0] + [0.25] * D + mat, dtype=dtype, device=DEV).view(1, 1, 1, -1)
+            x = torch.tensor([[0.25] * D, [0.5] * D, [0.25] * (D - 1) + [-1.0]], dtype=dtype, device=DEV).view(1, 1, 3, D)
+            ones = torch.ones(1, 1, 3, dtype=dtype, device=DEV)
+            results.append([_native.eval_fwd(m, x, covariance_form), *_native.eval_bwd(ones, m, x, True, True, covariance_form),
+                            *_native.eval_componentwise_bwd(ones.unsqueeze(-1), m, x, True, True, covariance_form)])
+        for single, double in zip(*results):
+            assert torch.equal(classes(single), classes(double)), (mat, covariance_form, single, double)
+
+
 def _workload_check(name, **kw):
     wl, mix, xes, gout = synthetic.make_workload(name, **kw)
     out, gmix, gxes = _run(mix.numpy(), xes.numpy(), gout.numpy(), wl.dtype)
