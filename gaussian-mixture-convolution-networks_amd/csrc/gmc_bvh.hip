@@ -632,15 +632,19 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The leaves' sort for a few large trees (kSmallTreeMax < M <= kBucketSortMax) in ONE launch instead of four radix
-// passes at their latency floor: 2^bits workgroups per tree, one per value of the top `bits` key bits (8 for one or two
-// trees, 7 for up to four, 6 for up to eight, so that the launch is resident at once).  Workgroup d reads all
-// keys of the tree (in component order, as the Morton kernel wrote them; 64 KB at most, from L2), keeps those whose top
-// bits are d as unique keys (Morton code << 32 | component) in LDS, counts those with smaller top bits -- the first
-// slot of its own --, sorts its keys (by counting ranks; more than kBucketRankMax: a bitonic network) and writes them out: ascending
-// unique keys are the stable order of the codes.  No histograms, no passes that wait for each other.  A digit that
-// holds most keys (all centres in one cell) is one long sort by a single workgroup: slower than the four passes, same
-// result.
+// The leaves' sort for one large tree (kSmallTreeMax < M <= kBucketSortMax) or two to eight of at most half that size in
+// ONE launch instead of four radix passes at their latency floor: 2^bits workgroups per tree, one per value of the top
+// `bits` key bits (8 for one or two trees, 7 for up to four, 6 for up to eight: at most 512 workgroups, of which two fit
+// a compute unit up to 8192 components, so that the launch is resident at once; beyond, a workgroup's keys fill a compute
+// unit's LDS and several trees would take two rounds).  Workgroup d reads all keys of the tree (in component order, as
+// the Morton kernel wrote them; 64 KB at most, from L2), keeps those whose top bits are d as unique keys (Morton
+// code << 32 | component) in LDS, counts those with smaller top bits -- the first slot of its own --, sorts its keys (by
+// counting ranks; more than kBucketRankMax: a bitonic network) and writes them out: ascending unique keys are the stable
+// order of the codes.  No histograms, no passes that wait for each other.  Where the centres crowd into a few cells the
+// workgroups take their shares between sampled splitters (below).
+// Build time, four radix passes / this launch in us (2000 points; centres uniform, half of them in a few cells, in eight
+// clusters): 2 trees of 8192 50 / 34, 65 / 53, 56 / 47; 8 of 2048 49 / 32, 66 / 45, 51 / 40; 8 of 8192 60 / 43, 74 / 59,
+// 66 / 61.  Not taken: 2 of 16384 53 / 41, 69 / 81, 58 / 73; 8 of 8193 55 / 66, 71 / 83, 59 / 77.
 constexpr int kBucketSortLanes = 1024;
 constexpr int kBucketSortMax = 16384;
 constexpr int kBucketRankMax = 256;        // keys of one digit up to which counting ranks beats the sorting network
@@ -680,12 +684,12 @@ __global__ __launch_bounds__(kBucketSortLanes) void bucket_sort_kernel(const uin
     }
     // the component of key r of this lane
     auto component = [&](int r) { return ((r / kVec) * kBucketSortLanes + int(threadIdx.x)) * kVec + r % kVec; };
-    // Which workgroup takes a key: the one numbered by its top 8 bits -- unless the centres crowd into a few Morton
+    // Which workgroup takes a key: the one numbered by its top bits -- unless the centres crowd into a few Morton
     // cells (a stray Gaussian far from the others is enough to stretch the bounds), when one workgroup would sort most
     // of the tree alone.  Every workgroup tests the same sample for that (every lane one of its keys: 1024 of the tree's),
     // and all take splitters instead when a value of the top bits is expected to hold more than kBucketCrowded keys:
-    // 256 sampled unique keys, sorted by counting; workgroup d takes the keys from splitter d up to splitter d + 1, found
-    // by bisection.  Same result either way; the choice is a function of the keys alone.
+    // 256 sampled unique keys, sorted by counting; workgroup d takes the keys from splitter d up to splitter d + 1 (with
+    // fewer than 8 bits: from every second or fourth one up to the next such), found by bisection.  Same result either way; the choice is a function of the keys alone.
     __shared__ uint32_t sample_bins[256];
     __shared__ unsigned long long sample[256], splitter[256];
     if (threadIdx.x < 256) sample_bins[threadIdx.x] = 0u;
@@ -760,7 +764,7 @@ __global__ __launch_bounds__(kBucketSortLanes) void bucket_sort_kernel(const uin
     }
     const size_t at = size_t(seg) * count + begin;
     if (n <= kBucketRankMax) {
-        // a few keys (the usual case: M / 256 on average): lane i counts the keys below key i and puts it there -- every
+        // a few keys (the usual case: M >> bits on average): lane i counts the keys below key i and puts it there -- every
         // read is a broadcast, no step waits for another
         if (int(threadIdx.x) < n) {
             const unsigned long long mine = k[threadIdx.x];
@@ -2637,7 +2641,8 @@ static int bvh_build_t(const T* mixture, const T* xes, char* bvh, const gmc_shap
     MortonJob<T> mg = {}, mp = {};
     // a few large trees: every value of the top key bits gathered and sorted in LDS (bucket_sort_kernel)
     const int bucket_bits = BL <= 2 ? 8 : BL <= 4 ? 7 : 6;
-    const bool bucket_sort = have_g && g_build_path != 2 && M > kSmallTreeMax && M <= kBucketSortMax && BL <= 8;
+    const bool bucket_sort = have_g && g_build_path != 2 && M > kSmallTreeMax &&
+                             (BL == 1 ? M <= kBucketSortMax : BL <= 8 && M <= kBucketSortMax / 2);
     // (a Morton workgroup per block of the first radix pass; without a radix sort behind it: 256 keys each)
     if (have_g) mg = MortonJob<T>{mixture, G, 1, M, bucket_sort ? 1 : jg0.items, bucket_sort ? bpm : jg0.blocks_per_seg, parts_g, bpm, ka, va,
                                   unsigned(BL * (bucket_sort ? bpm : jg0.blocks_per_seg)), bucket_sort ? nullptr : (uint32_t*)jg0.hist, jg0.shift};

@@ -657,7 +657,7 @@ def _same_object_by_both_paths(m, x, g, dtype, paths, tag):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_sort_by_digits_in_lds_gives_the_order_of_the_four_radix_passes(dtype):
-    """The leaves of one or two trees of 1025 ... 16384 components are sorted by one launch (256 workgroups
+    """The leaves of one tree of 1025 ... 16384 components (two of at most 8192) are sorted by one launch (256 workgroups
     per tree, each gathers and sorts its share of the keys in LDS: by the top 8 key bits, or between sampled splitters
     when the centres crowd into a few cells), all others by four radix passes; with the latter forced for the same
     inputs the objects must be identical.  Sizes at both ends of every LDS capacity, duplicate keys, and centres crowded into a
@@ -675,14 +675,15 @@ def test_sort_by_digits_in_lds_gives_the_order_of_the_four_radix_passes(dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_sort_in_lds_for_three_to_eight_trees(dtype):
-    """three and four trees are sorted by 128 workgroups each, five to eight by 64, nine by the radix passes: the objects of
-    the radix passes, with trees that start off a multiple of the vector width, equal keys and crowded centres"""
-    for k, (B, L, M, N, D) in enumerate(((3, 1, 1027, 300, 2), (2, 2, 4096, 100, 3), (4, 1, 8193, 100, 2), (5, 1, 2049, 200, 3),
-                                         (2, 4, 1500, 100, 2), (8, 1, 4097, 100, 3), (9, 1, 1100, 100, 2))):
+    """three and four trees of at most 8192 components are sorted by 128 workgroups each, five to eight by 64, nine and
+    larger trees by the radix passes: the objects of the radix passes, with trees that start off a multiple of the vector
+    width, equal keys and crowded centres"""
+    for k, (B, L, M, N, D) in enumerate(((3, 1, 1027, 300, 2), (2, 2, 4096, 100, 3), (4, 1, 8193, 100, 2), (4, 1, 8191, 100, 2),
+                                         (8, 1, 8192, 50, 2), (5, 1, 2049, 200, 3), (2, 4, 1500, 100, 2), (8, 1, 4097, 100, 3), (9, 1, 1100, 100, 2))):
         mix, xes, gout = _case(B, L, M, N, D, seed=7700 + k)
         mix[:, :, 40:300] = mix[:, :, 40:41]
         mix[-1, -1, 1::2, 1:1 + D] *= 1e-3
-        if k == 3:
+        if k in (4, 5):
             mix[0, 0, :, 1:1 + D] = mix[0, 0, :1, 1:1 + D]
         m, x = mix.to(dtype).to(DEV).contiguous(), xes.to(dtype).to(DEV).contiguous()
         _same_object_by_both_paths(m, x, gout.to(dtype).to(DEV), dtype, (0, 2), f"B{B} L{L} M{M} N{N} D{D}")
