@@ -345,24 +345,24 @@ __global__ __launch_bounds__(kBlock) void moments_finish_kernel(const double* __
 // numbers of a batch entry are dealt to `chunks` workgroups, each of which finds the box itself (a second launch or a
 // scratch buffer for the box would cost more).  Bound by the latency of reading the centres, which are many behind a
 // convolution: sixteen wavefronts with eight centres per lane in flight (100 batch entries of 81920 centres: 177 us with
-// four wavefronts and one centre in flight).
-constexpr int kSampleBlock = 1024;
+// four wavefronts and one centre in flight).  Few centres (kSampleFew): four wavefronts.
+constexpr int kSampleBlock = 1024, kSampleFew = 2048;
 
-template <typename T, int D>
-__global__ __launch_bounds__(kSampleBlock) void sampling_positions_kernel(const T* __restrict__ mixture, T* __restrict__ u,
-                                                                          int centres, size_t samples, int chunks) {
+template <typename T, int D, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void sampling_positions_kernel(const T* __restrict__ mixture, T* __restrict__ u,
+                                                                   int centres, size_t samples, int chunks) {
     constexpr int G = 1 + D + D * D;
-    constexpr int kFlight = 8;
-    __shared__ T red[2 * D][kSampleBlock / kWave];
+    constexpr int kFlight = BLOCK == kSampleBlock ? 8 : 1;
+    __shared__ T red[2 * D][BLOCK / kWave];
     const int b = blockIdx.x / chunks, chunk = blockIdx.x - b * chunks;
     const T* mix_b = mixture + size_t(b) * centres * G;
     T lo[D], hi[D];
     for (int d = 0; d < D; ++d) { lo[d] = T(INFINITY); hi[d] = T(-INFINITY); }
-    for (int i = threadIdx.x; i < centres; i += kFlight * kSampleBlock) {
+    for (int i = threadIdx.x; i < centres; i += kFlight * BLOCK) {
         T v[kFlight][D];
 #pragma unroll
         for (int k = 0; k < kFlight; ++k) {
-            const int at = i + k * kSampleBlock < centres ? i + k * kSampleBlock : i;
+            const int at = i + k * BLOCK < centres ? i + k * BLOCK : i;
 #pragma unroll
             for (int d = 0; d < D; ++d) v[k][d] = mix_b[size_t(at) * G + 1 + d];
         }
@@ -387,14 +387,15 @@ __global__ __launch_bounds__(kSampleBlock) void sampling_positions_kernel(const 
     __syncthreads();
 #pragma unroll
     for (int d = 0; d < D; ++d)
-        for (int w = 0; w < kSampleBlock / kWave; ++w) {
+#pragma unroll 4        // (all sixteen at once spilled 340 bytes a lane in double: 26 us where the kernel takes 6)
+        for (int w = 0; w < BLOCK / kWave; ++w) {
             lo[d] = red[d][w] < lo[d] ? red[d][w] : lo[d];
             hi[d] = red[D + d][w] > hi[d] ? red[D + d][w] : hi[d];
         }
     T* u_b = u + size_t(b) * samples * D;
     const size_t n = samples * D, per = (n + chunks - 1) / chunks;
     const size_t begin = per * chunk, end = begin + per < n ? begin + per : n;
-    for (size_t i = begin + threadIdx.x; i < end; i += kSampleBlock) {
+    for (size_t i = begin + threadIdx.x; i < end; i += BLOCK) {
         const int d = int(i % D);
         T l = lo[0], h = hi[0];
 #pragma unroll
@@ -667,10 +668,12 @@ int gmc_batch_norm_sampling_positions(const void* mixture, void* uniform_in_posi
     const size_t wanted = (samples * shape->D + 16383) / 16384;
     const int chunks = int(wanted < 1 ? 1 : (wanted > 64 ? 64 : wanted));
     const dim3 grid{unsigned(shape->B) * unsigned(chunks)};
-#define GMC_SP(T, DD) gmc::sampling_positions_kernel<T, DD><<<grid, dim3(gmc::kSampleBlock), 0, st>>>((const T*)mixture, (T*)uniform_in_positions_out, centres, samples, chunks)
+#define GMC_SPB(T, DD, BLOCK) gmc::sampling_positions_kernel<T, DD, BLOCK><<<grid, dim3(BLOCK), 0, st>>>((const T*)mixture, (T*)uniform_in_positions_out, centres, samples, chunks)
+#define GMC_SP(T, DD) do { if (centres <= gmc::kSampleFew) GMC_SPB(T, DD, gmc::kBlock); else GMC_SPB(T, DD, gmc::kSampleBlock); } while (0)
     if (shape->dtype == GMC_F32) { if (shape->D == 2) GMC_SP(float, 2); else GMC_SP(float, 3); }
     else { if (shape->D == 2) GMC_SP(double, 2); else GMC_SP(double, 3); }
 #undef GMC_SP
+#undef GMC_SPB
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
 }
 

@@ -403,6 +403,23 @@ def test_batch_norm_scaling_of_the_weights(D, dtype):
     assert torch.equal(tangent[..., 0], x[..., 0]) and not tangent[..., 1:].any()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("D", [2, 3])
+def test_batch_norm_sampling_positions_for_few_and_many_centres(D, dtype):
+    """the box of the centres by four or by sixteen wavefronts: centre counts around the line between them and around a
+    workgroup's stride, numbers dealt to several workgroups; against torch (a handful of roundings)"""
+    for B, L, M, N in ((2, 1, 1, 5), (1, 1, 257, 3), (2, 2, 1024, 40), (2, 1, 2049, 7), (1, 3, 2731, 6000), (1, 1, 8193, 1)):
+        gen = torch.Generator(device=DEV).manual_seed(M)
+        m = torch.randn(B, L, M, 1 + D + D * D, generator=gen, device=DEV, dtype=dtype)
+        u = torch.rand(B, L, N, D, generator=gen, device=DEV, dtype=dtype)
+        centres = m[..., 1:1 + D].reshape(B, -1, D)
+        lo, hi = centres.min(1).values.view(B, 1, 1, D), centres.max(1).values.view(B, 1, 1, D)
+        ref = (u * 1.3 - 0.15 if D == 2 else u) * (hi - lo) + lo
+        got = _native.batch_norm_sampling_positions(m, u.clone())
+        eps = torch.finfo(dtype).eps                                # four roundings of values up to 1.3 (hi - lo) + |lo|
+        assert ((got - ref).abs() <= 4 * eps * (1.3 * (hi - lo) + lo.abs())).all(), (B, L, M, N)
+
+
 def test_batch_norm_batched_backward():
     """a batched backward pass through the layer (vectorised Jacobian rows) against the rows one by one; the statistics
     carry no gradient, so training and evaluation mode alike end in the scaling of the weights"""
