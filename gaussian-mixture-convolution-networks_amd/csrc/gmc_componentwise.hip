@@ -56,25 +56,33 @@ __global__ __launch_bounds__(kBlock) void componentwise_fwd_kernel(const T* __re
 
 // Layout of the backward pass: the 64 lanes of a wavefront are 4 rows (points) by 16 columns, a column holds Q Gaussians,
 // so that the coordinates of a point are fetched once for Q pairs.  Where every row of grad_out starts at a multiple of
-// the vector (`wide`), a column's Gaussians lie next to each other and one access per lane (16 bytes for 4 floats) fetches
-// the values of 16 Q Gaussians at 4 points; elsewhere they lie 16 apart and Q accesses fetch 64 bytes of a row each.  A wavefront owns one such slice of
-// Gaussians; with fewer than four slices in its group the four wavefronts of a workgroup share the points of the chunk.
-// (The forward pass, which only stores, is faster with lanes = Gaussians: 800 x 128 Gaussians at 784 points in 2-D 74 us
-// against 107 us in this layout.)
+// the vector (`wide`), a column's Gaussians lie next to each other and one access per lane fetches the values of 16 Q
+// Gaussians at 4 points; elsewhere they lie 16 apart and Q accesses fetch 64 bytes of a row each.  A wavefront owns one
+// such slice of Gaussians; with fewer than four slices in its group the four wavefronts of a workgroup share the points of
+// the chunk.  (The forward pass, which only stores, is faster with lanes = Gaussians: 800 x 128 Gaussians at 784 points in
+// 2-D 74 us against 107 us in this layout.)
 constexpr int kCwPointsMax = 1024; // most points per workgroup of the backward pass (the size of its LDS copy of dL/dx)
 template <typename T, int Q> struct __align__(sizeof(T) * Q) CwVec { T v[Q]; };
-// Gaussians per lane: what a 16-byte access holds in 2-D, half as many in 3-D (record and sums of every one of them stay in
-// registers: 26 per Gaussian) and where there are no wide accesses to gain (400 x 45 Gaussians at 900 points in 2-D: four
-// 47 us, two 35 us).
-template <typename T, int D> constexpr int cw_most = (D == 2 ? 16 : 8) / int(sizeof(T));
+
+// Gaussians per lane: one or, in float32, two -- a lane prepares them one after the other and holds a record and sums for
+// each.  Two where the mixtures fill their slices (groups of 128 components cover at most a tenth more than groups of 64)
+// and the launch has work for the chip (512 pieces of 64 x 64 pairs).  Measured, both gradients, one / two / four a lane in
+// us (float32 2-D): 800 x 128 Gaussians at 784 points 107 / 95 / 100, 800 x 132 123 / 147 / 137, 20 x 512 at 4096
+// 52 / 47 / 52, 1000 x 16 at 1000 28 / 41 / 73, 64 x 4 at 1 8.7 / 9.8 / 11.5; 3-D: 800 x 128 132 / 122 / -, 1000 x 129 at
+// 128 46 / 66 / -; float64 (2-D): 400 x 128 at 784 111 / 111 / -, 1000 x 1200 at 16 161 / 174 / -.
+template <typename T> static bool cw_two_per_lane(const gmc_shape& s) {
+    if (sizeof(T) == 8) return false;
+    const size_t groups = (size_t(s.M) + 63) / 64, pairs_of_groups = (groups + 1) / 2;
+    return 20 * pairs_of_groups <= 11 * groups && size_t(s.B) * s.L * groups * ((size_t(s.N) + 63) / 64) >= 512;
+}
 
 struct CwSlices { int slice, rep, reps; };
 
-// the share of a wavefront: slice of the Gaussians (group of four slices, -1: none) and repetition over the points
-__device__ __forceinline__ CwSlices cw_share(int M, int group, int per_slice, int wave) {
-    const int slices_total = (M + per_slice - 1) / per_slice;
-    const int here = slices_total - group * 4 < 4 ? slices_total - group * 4 : 4;
-    const int reps = 4 / here;
+// the share of a wavefront: slice of the Gaussians (of a group of one per wavefront, -1: none) and repetition over the points
+__device__ __forceinline__ CwSlices cw_share(int M, int group, int per_slice, int waves, int wave) {
+    const int left = (M + per_slice - 1) / per_slice - group * waves;
+    const int here = left < waves ? left : waves;
+    const int reps = waves / here;
     const int rep = wave / here;
     return CwSlices{rep < reps ? wave % here : -1, rep, reps};
 }
@@ -116,23 +124,24 @@ template <int COUNT> __device__ __forceinline__ int cw_sum_index(int lane) {
 // reduction together, and their grad_out values are in flight together.  Per-Gaussian sums stay in the lane's
 // registers over the points, are added over the rows and over the wavefronts that share a slice at the end, and leave
 // with one atomic per scalar and workgroup; dL/dx of a point goes through the workgroup's LDS copy and leaves with one
-// atomic (or, when one workgroup sees all Gaussians of the point, one store) per scalar.  Before, a lane held one Gaussian
-// and every point's dL/dx was reduced over 64 lanes (us before / now, float32, both gradients): 800 x 128 Gaussians at 784 points in
-// 2-D 124 / 97 (3.3 TB/s of grad_out), in 3-D 196 / 123; 20 x 512 at 4096 points 117 / 53 and 273 / 69.  Bound by
-// instruction issue and, at 154 registers (2-D), three wavefronts per SIMD.
+// atomic (or, when one workgroup sees all Gaussians of the point, one store) per scalar.  With lanes = Gaussians and every
+// point's dL/dx reduced over 64 lanes / now (us, float32, both gradients): 800 x 128 Gaussians at 784 points in 2-D
+// 128 / 102 (3.2 TB/s of grad_out), in 3-D 199 / 130; 20 x 512 at 4096 points 118 / 49 and 272 / 66; 1 x 2 mixtures of 4 at
+// 2 points 8.3 / 7.9.  Bound by instruction issue.
 constexpr int kCwSteps = 4;        // points of a row per round
 
-template <typename T, int D, int Q, bool NEED_GM, bool NEED_GX>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : Q == 4 || D == 3 ? 3 : 4))) void componentwise_bwd_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
+template <typename T, int D, int Q, int WAVES, bool NEED_GM, bool NEED_GX>
+__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(WAVES > 4 ? 4 : sizeof(T) == 8 ? 2 : D == 3 ? 3 : 4)))
+void componentwise_bwd_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
                                                                   const T* __restrict__ xes, T* __restrict__ sums,
                                                                   T* __restrict__ grad_xes, int L, int M, int N, int Bx,
                                                                   int Lx, int m_groups, int chunks, int points_per_chunk,
                                                                   bool shared_points, bool wide, bool covariance_form) {
-    constexpr int G = 1 + D + D * D, U = kCwSteps;
+    constexpr int G = 1 + D + D * D, U = kCwSteps, kThreads = WAVES * kWave;
     constexpr int NR = 1 + D + D * (D + 1) / 2;
     constexpr int kU = Rec<T, D>::kU;
     __shared__ T point_grad[NEED_GX ? kCwPointsMax * D : 1];
-    __shared__ T shared_sums[NEED_GM ? 4 * 16 * Q * NR : 1];
+    __shared__ T shared_sums[NEED_GM ? WAVES * 16 * Q * NR : 1];
     const T* exp2_tab = exp2_table<T>();
     if constexpr (sizeof(T) == 8) __syncthreads();          // the table is complete
     int id = blockIdx.x;
@@ -142,22 +151,22 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane >> 4, col = lane & 15;
-    const CwSlices share = cw_share(M, group, 16 * Q, wave);
+    const CwSlices share = cw_share(M, group, 16 * Q, WAVES, wave);
     // Gaussian q of this lane is m0 + q * apart
     const int apart = wide ? 1 : 16;
-    const int m0 = (group * 4 + share.slice) * 16 * Q + (wide ? col * Q : col);
+    const int m0 = (group * WAVES + share.slice) * 16 * Q + (wide ? col * Q : col);
     const size_t x_off = (size_t(xb) * Lx + xl) * N;
     const T* __restrict__ x_bl = xes + x_off * D;
     if (NEED_GX) {
-        for (int i = threadIdx.x; i < points_per_chunk * D; i += kBlock) point_grad[i] = T(0);
+        for (int i = threadIdx.x; i < points_per_chunk * D; i += kThreads) point_grad[i] = T(0);
         __syncthreads();
     }
+    const int chunk_begin = chunk * points_per_chunk;
     T rs[Q][NR];
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
         for (int i = 0; i < NR; ++i) rs[q][i] = T(0);
-    const int chunk_begin = chunk * points_per_chunk;
     if (share.slice >= 0) {
         T r[Q][Rec<T, D>::kStride], ua[Q][kU];      // ua = -amp * u: dL/dx takes k*y against it
 #pragma unroll
@@ -266,9 +275,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T
             }
         __syncthreads();
         constexpr int kSlice = 16 * Q * NR;
-        const int first = group * 4 * 16 * Q;               // the group's first Gaussian
-        const int left = (M - first + 16 * Q - 1) / (16 * Q), slices_here = left < 4 ? left : 4;
-        for (int i = threadIdx.x; i < slices_here * kSlice; i += kBlock) {
+        const int first = group * WAVES * 16 * Q;               // the group's first Gaussian
+        const int left = (M - first + 16 * Q - 1) / (16 * Q), slices_here = left < WAVES ? left : WAVES;
+        for (int i = threadIdx.x; i < slices_here * kSlice; i += kThreads) {
             if (first + i / NR >= M) break;
             T v = shared_sums[i];
             for (int other = 1; other < share.reps; ++other) v += shared_sums[other * slices_here * kSlice + i];
@@ -277,12 +286,109 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T
     }
     if (NEED_GX) {
         __syncthreads();
-        for (int i = threadIdx.x; i < points_per_chunk * D; i += kBlock) {
+        for (int i = threadIdx.x; i < points_per_chunk * D; i += kThreads) {
             const int n = chunk_begin + i / D;
             if (n >= N) continue;
             T* dst = grad_xes + (x_off + chunk_begin) * D + i;
             if (shared_points) atomic_add(dst, point_grad[i]); else *dst = point_grad[i];
         }
+    }
+}
+
+// dL/dx alone, with lanes = Gaussians: every wavefront prepares 64 of them at once, where the kernel above prepares 16 Q in
+// all four rows, and a workgroup's 256 leave fewer additions to a point.  Against that the kernel above reduces over 16
+// lanes instead of 64: it is the faster one where preparation and additions are few (cw_backward).
+constexpr int kCwUnroll = 8;
+
+template <typename T, int D>
+__global__ __launch_bounds__(kBlock) void componentwise_bwd_points_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
+                                                                         const T* __restrict__ xes, T* __restrict__ grad_xes, int L,
+                                                                         int M, int N, int Bx, int Lx, int m_groups, int chunks,
+                                                                         int points_per_chunk, bool shared_points, bool covariance_form) {
+    constexpr int G = 1 + D + D * D;
+    constexpr int kU = Rec<T, D>::kU;
+    __shared__ T point_grad[kCwPointsMax * D];
+    const T* exp2_tab = exp2_table<T>();
+    int id = blockIdx.x;
+    const int chunk = id % chunks; id /= chunks;
+    const int group = id % m_groups;
+    const int bl = id / m_groups;
+    const int b = bl / L, l = bl - b * L;
+    const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
+    // (no readfirstlane here: with a provably uniform wavefront index the point coordinates arrive through scalar
+    // loads, whose waits also cover the LDS traffic of the loop -- measured 15 % slower)
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const CwSlices share = cw_share(M, group, kWave, 4, wave);
+    const int m = (group * 4 + share.slice) * kWave + lane;
+    const bool valid = m < M;
+    const size_t x_off = (size_t(xb) * Lx + xl) * N;
+    const T* __restrict__ x_bl = xes + x_off * D;
+    for (int i = threadIdx.x; i < points_per_chunk * D; i += kBlock) point_grad[i] = T(0);
+    __syncthreads();                                        // (the table is complete as well)
+    const int chunk_begin = chunk * points_per_chunk;
+    if (share.slice >= 0) {
+        T r[Rec<T, D>::kStride], ua[kU];            // ua = -amp * u: dL/dx takes k*y against it
+        {
+            const Derived<D> dv = derive<T, D>(mixture + (size_t(bl) * M + (valid ? m : 0)) * G, covariance_form);
+            store_record<T, D>(r, dv, true, over_half_log2e<T>(dv.w * dv.norm), 0);
+        }
+#pragma unroll
+        for (int i = 0; i < kU; ++i) ua[i] = -r[Rec<T, D>::kAmp] * r[i];
+        const int per_rep = (points_per_chunk + share.reps - 1) / share.reps;
+        const int n_begin = chunk_begin + share.rep * per_rep;
+        int n_end = n_begin + per_rep < chunk_begin + points_per_chunk ? n_begin + per_rep : chunk_begin + points_per_chunk;
+        n_end = n_end < N ? n_end : N;
+        const T* __restrict__ go_col = grad_out + size_t(bl) * N * M + (valid ? m : 0);
+        for (int n0 = n_begin; n0 < n_end; n0 += kCwUnroll) {
+            T go[kCwUnroll], xs[kCwUnroll][D];
+#pragma unroll
+            for (int u = 0; u < kCwUnroll; ++u) {           // eight values in flight
+                const int n = n0 + u < n_end ? n0 + u : n_end - 1;
+                go[u] = go_col[size_t(n) * M];
+#pragma unroll
+                for (int d = 0; d < D; ++d) xs[u][d] = x_bl[size_t(n) * D + d];
+            }
+            T vs[kCwUnroll][D];                             // dL/dx terms of the eight points, this lane's Gaussian
+#pragma unroll
+            for (int u = 0; u < kCwUnroll; ++u) {
+                T y[D], ky[D];
+                const T q = quad_form<T, D, true>(r, xs[u], y);
+                const T k = (valid && n0 + u < n_end) ? pair_exp2(-q, exp2_tab) * go[u] : T(0);
+#pragma unroll
+                for (int d = 0; d < D; ++d) ky[d] = k * y[d];
+                // -(amp u)^T (k y)
+                vs[u][0] = ua[0] * ky[0];
+                if constexpr (D == 2) {
+                    vs[u][1] = fma_(ua[1], ky[0], ua[2] * ky[1]);
+                } else {
+                    vs[u][1] = fma_(ua[1], ky[0], ua[3] * ky[1]);
+                    vs[u][2] = fma_(ua[2], ky[0], fma_(ua[4], ky[1], ua[5] * ky[2]));
+                }
+            }
+            // summed over the wavefront's Gaussians, four points at a time; the lane at the end of row r holds the total of
+            // point {0, 2, 1, 3}[r] of the four
+            const int row = lane >> 4;
+            const int mine = ((row & 1) << 1) | (row >> 1);
+#pragma unroll
+            for (int u0 = 0; u0 < kCwUnroll; u0 += 4) {
+                T total[D];
+#pragma unroll
+                for (int d = 0; d < D; ++d)
+                    total[d] = wave_sum4_to_row_ends(vs[u0][d], vs[u0 + 1][d], vs[u0 + 2][d], vs[u0 + 3][d], lane);
+                const int n = n0 + u0 + mine;
+                if ((lane & 15) == 15 && n < n_end) {
+#pragma unroll
+                    for (int d = 0; d < D; ++d) atomic_add(&point_grad[(n - chunk_begin) * D + d], total[d]);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < points_per_chunk * D; i += kBlock) {
+        const int n = chunk_begin + i / D;
+        if (n >= N) continue;
+        T* dst = grad_xes + (x_off + chunk_begin) * D + i;
+        if (shared_points) atomic_add(dst, point_grad[i]); else *dst = point_grad[i];
     }
 }
 
@@ -314,7 +420,7 @@ static int cw_forward(const T* mixture, const T* xes, T* out, const gmc_shape& s
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
 }
 
-template <typename T, int D, int Q>
+template <typename T, int D, int Q, int WAVES = 4>
 static int cw_backward_q(const T* grad_out, const T* mixture, const T* xes, T* grad_mixture, T* grad_xes, T* sums,
                        const gmc_shape& s, bool gm, bool gx, bool wide, bool cov, hipStream_t st) {
     constexpr int G = 1 + D + D * D;
@@ -322,38 +428,74 @@ static int cw_backward_q(const T* grad_out, const T* mixture, const T* xes, T* g
     const size_t BL = size_t(s.B) * s.L;
     const size_t n_g = BL * s.M, n_x = size_t(s.Bx) * s.Lx * s.N * D;
     if (BL == 0) return GMC_OK;
-    constexpr int kGroup = 4 * 16 * Q;
+    constexpr int kGroup = WAVES * 16 * Q;
     const int m_groups = (s.M + kGroup - 1) / kGroup;
     const CwChunks c = cw_chunks(BL * (m_groups > 0 ? m_groups : 1), s.N > 0 ? s.N : 1, kCwWanted);
     const int chunks = c.chunks, points_per_chunk = c.points;
     // dL/dx of a point is stored by the one workgroup that sees all its Gaussians, and added atomically to zeros when
     // several do (more than one group of four slices, or points shared by several mixtures)
     const bool shared_points = m_groups > 1 || size_t(s.Bx) * s.Lx != BL;
-    if (gx && (shared_points || s.N == 0 || s.M == 0)) zero_async(grad_xes, n_x, st);
     if (s.N == 0 || s.M == 0) {
-        if (gm) zero_async(grad_mixture, n_g * G, st);
+        zero2_async(grad_mixture, gm ? n_g * G : 0, grad_xes, gx ? n_x : 0, st);
         return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
     }
-    if (gm) zero_async(sums, n_g * NR, st);
+    zero2_async(sums, gm ? n_g * NR : 0, grad_xes, gx && shared_points ? n_x : 0, st);
     const dim3 grid(unsigned(BL * m_groups * chunks));
-#define GMC_CW(GM, GX) componentwise_bwd_kernel<T, D, Q, GM, GX><<<grid, dim3(kBlock), 0, st>>>( \
+#define GMC_CW(GM, GX) componentwise_bwd_kernel<T, D, Q, WAVES, GM, GX><<<grid, dim3(WAVES * kWave), 0, st>>>( \
         grad_out, mixture, xes, sums, grad_xes, s.L, s.M, s.N, s.Bx, s.Lx, m_groups, chunks, points_per_chunk, shared_points, wide, cov)
-    if (gm && gx) GMC_CW(true, true);
-    else if (gm) GMC_CW(true, false);
-    else if (gx) GMC_CW(false, true);
+    if constexpr (WAVES > 4) {
+        GMC_CW(true, true);
+    } else {
+        if (gm && gx) GMC_CW(true, true);
+        else if (gm) GMC_CW(true, false);
+        else if (gx) GMC_CW(false, true);
+    }
 #undef GMC_CW
     if (gm) launch_bwd_epilogue(mixture, sums, grad_mixture, n_g, D, s.dtype, cov, st);
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
 }
 
 template <typename T, int D>
+static int cw_backward_points(const T* grad_out, const T* mixture, const T* xes, T* grad_xes, const gmc_shape& s, bool cov,
+                              hipStream_t st) {
+    const size_t BL = size_t(s.B) * s.L, n_x = size_t(s.Bx) * s.Lx * s.N * D;
+    if (BL == 0 || s.N == 0) return GMC_OK;
+    const int m_groups = (s.M + kBlock - 1) / kBlock;
+    const CwChunks c = cw_chunks(BL * m_groups, s.N, kCwWanted);
+    const bool shared_points = m_groups > 1 || size_t(s.Bx) * s.Lx != BL;
+    if (shared_points) zero_async(grad_xes, n_x, st);
+    componentwise_bwd_points_kernel<T, D><<<dim3(unsigned(BL * m_groups * c.chunks)), dim3(kBlock), 0, st>>>(
+        grad_out, mixture, xes, grad_xes, s.L, s.M, s.N, s.Bx, s.Lx, m_groups, c.chunks, c.points, shared_points, cov);
+    return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
+}
+
+template <typename T, int D>
 static int cw_backward(const T* grad_out, const T* mixture, const T* xes, T* grad_mixture, T* grad_xes, T* sums,
                        const gmc_shape& s, bool gm, bool gx, bool cov, hipStream_t st) {
-    constexpr int Q = cw_most<T, D>;
-    const bool wide = s.M % Q == 0 && (uintptr_t(grad_out) & (sizeof(T) * Q - 1)) == 0;
-    if constexpr (Q > 2)
-        if (!wide) return cw_backward_q<T, D, 2>(grad_out, mixture, xes, grad_mixture, grad_xes, sums, s, gm, gx, false, cov, st);
-    return cw_backward_q<T, D, Q>(grad_out, mixture, xes, grad_mixture, grad_xes, sums, s, gm, gx, wide, cov, st);
+    const size_t BL = size_t(s.B) * s.L, groups = (size_t(s.M) + 63) / 64;
+    const bool shared = size_t(s.Bx) * s.Lx != BL;
+    // dL/dx alone: lanes = Gaussians where a Gaussian's preparation serves few points, where additions of several mixtures
+    // meet on a point, or where the launch is small (more than one group: a zero fill and additions instead of stores).
+    // Lanes = Gaussians / the 4 x 16 layout, us: 882 x 1179 Gaussians at 2 points, 3-D, float64 68 / 121; 2170 x 427 at 18
+    // points that all share 93 / 286; 9 x 120 at 900 8.7 / 10.1; but 800 x 128 at 784 114 / 88, and with at most 64
+    // Gaussians (one group) the 4 x 16 layout takes 0.65 to 1.05 of the time.
+    if (!gm && gx && groups > 1 && (s.N <= 128 || shared || BL * groups * ((size_t(s.N) + 63) / 64) < 512))
+        return cw_backward_points<T, D>(grad_out, mixture, xes, grad_xes, s, cov, st);
+    // Both gradients, points shared by many mixtures: sixteen wavefronts a workgroup, so that 256 Gaussians make one addition
+    // to a point.  Four / sixteen, us (2-D): 2170 x 427 Gaussians at 18 points 321 / 139, 728 x 153 at 17 53 / 29, float64
+    // 256 x 1432 at 19 166 / 84; where fewer than 256 additions meet on a point four are as fast or faster.  (3-D in double:
+    // the registers of sixteen wavefronts do not hold a Gaussian's sums.)
+    if constexpr (sizeof(T) == 4 || D == 2) {
+        if (gm && gx && shared && groups > 2 && BL * groups >= 256 * size_t(s.Bx) * s.Lx)
+            return cw_backward_q<T, D, 1, 16>(grad_out, mixture, xes, grad_mixture, grad_xes, sums, s, gm, gx, true, cov, st);
+    }
+    if constexpr (sizeof(T) == 4) {
+        if (cw_two_per_lane<T>(s)) {
+            const bool wide = s.M % 2 == 0 && (uintptr_t(grad_out) & (2 * sizeof(T) - 1)) == 0;
+            return cw_backward_q<T, D, 2>(grad_out, mixture, xes, grad_mixture, grad_xes, sums, s, gm, gx, wide, cov, st);
+        }
+    }
+    return cw_backward_q<T, D, 1>(grad_out, mixture, xes, grad_mixture, grad_xes, sums, s, gm, gx, true, cov, st);
 }
 
 }  // namespace gmc

@@ -617,11 +617,14 @@ def test_componentwise(dtype, D):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("D", [2, 3])
 def test_componentwise_backward_edges(dtype, D):
-    """gradients at the edges of the backward kernel's layout: Gaussians per column, slice and group (4, 64, 256 floats in
-    2-D, half of that in 3-D or in double) and rounds and chunks of points, each gradient alone as well, rows of grad_out that
-    start off a multiple of 16 bytes; reference: autograd in float64 on the CPU"""
+    """gradients at the edges of the backward kernels' layouts: Gaussians per column, slice and group (one or two a lane, 16
+    or 32 a slice, four or -- many mixtures on shared points -- sixteen slices a workgroup; dL/dx alone: 64 a slice), rounds
+    and chunks of points, each gradient alone as well, rows of grad_out that start off a multiple of the vector width;
+    reference: autograd in float64 on the CPU"""
     shapes = [(1, 1, 1, 1), (2, 1, 16, 3), (1, 2, 17, 4), (3, 1, 33, 17), (1, 1, 63, 63), (2, 2, 64, 65), (1, 1, 66, 130),
-              (1, 1, 130, 1025), (1, 1, 257, 100), (1, 2, 513, 33), (60, 40, 3, 70)]
+              (1, 1, 130, 1025), (1, 1, 257, 100), (1, 2, 513, 33), (60, 40, 3, 70), (130, 2, 128, 66), (130, 2, 127, 65),
+              (1, 260, 128, 65), (90, 1, 130, 20), (3, 2, 65, 200), (64, 2, 254, 129), (64, 2, 256, 130), (24, 1, 1100, 17),
+              (1, 2, 255, 3), (1, 3, 300, 700), (9, 1, 513, 129), (5, 30, 257, 9)]
     for i, (B, L, M, N) in enumerate(shapes):
         bc = i % 4 == 2
         mix, xes, _ = _case(B, L, M, N, D, 900 + i, bc)
@@ -634,6 +637,8 @@ def test_componentwise_backward_edges(dtype, D):
         vals = m64[..., 0].unsqueeze(2) * o.kappa(D) * torch.linalg.det(c).sqrt() * torch.exp(-0.5 * q)
         rgm, rgx = torch.autograd.grad(vals, (m64, x64), gout.double())
         md, xd, gd = mix.to(DEV), xes.to(DEV), gout.to(DEV)
+        if i % 6 == 1:                                                      # the tensor itself off the vector width
+            gd = torch.cat((gd.new_zeros(1), gd.flatten()))[1:].view(gd.shape)
         for need_m, need_x in ((True, True), (True, False), (False, True)):
             gm_, gx_ = _native.eval_componentwise_bwd(gd, md, xd, need_m, need_x)
             if need_m:
