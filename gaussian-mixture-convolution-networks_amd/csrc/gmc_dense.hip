@@ -717,19 +717,20 @@ void set_tuning(int fwd_points_per_lane, int bwd_points_per_lane) {
 }
 
 // Launches that would not fill the chip (fewer than 2048 workgroups): points per lane and slices of Gaussians are
-// chosen together by the modelled time of the launch, in vector instructions of a wavefront.  A workgroup costs its
-// staging (per tile) and its steps of four Gaussians, each `pair` instructions per point and lane and `per_step` for the
-// rest (row reductions); a compute unit runs two workgroups in the time of one (a lone wavefront issues every second
-// slot), then ceil(workgroups / 256) after each other.  `clear`: the zero fill that slices need; `several_chunks`: the
-// zero fill and the epilogue launch of a backward pass whose sums come from several workgroups; `contended`: one more
-// addition to every dL/dx of points that all mixtures share (about 45 ns for each that meets on an address in 2-D, 75 ns
-// in 3-D).  The plan
-// for full launches stays unless the model gives at least a tenth (three tenths against the
+// chosen together by the modelled time of the launch, in vector instructions of a wavefront (about 1.5 ns).  A workgroup
+// costs its staging (per tile), its points (`point` for each of a lane's: loading and writing them back) and its steps of
+// four Gaussians, each `pair` instructions per point and lane and `per_step` for the rest (row reductions); a compute unit
+// runs two workgroups in the time of one (a lone wavefront issues every second slot), then ceil(workgroups / 256) after
+// each other.  `clear`: the zero fill that slices need; `several_chunks`: the zero fill and the epilogue launch of a
+// backward pass whose sums come from several workgroups; `contended`: one more addition to every dL/dx (about 45 ns for
+// each that meets on an address in 2-D, 75 ns in 3-D; taken half as high again for dL/dx alone, whose workgroups end
+// together).  The plan for full launches stays unless the model gives a tenth to a fifth (three tenths against the
 // one-Gaussian-per-step layout).  Measured, full-launch plan / this one in us:
 //   15 x 333 Gaussians, 2777 points, float64, 3-D: forward 38.7 / 22.1, backward 100.9 / 52.9 (tiles of 256 and 77 before)
-//   3 x 540, 1058 points, float32, 2-D: 9.5 / 7.0 and 24.1 / 13.5;   60 x 79, 422 points, 3-D: forward 9.3 / 5.5
+//   3 x 540, 1058 points, float32, 2-D: 9.5 / 7.0 and 24.1 / 13.5
+//   dL/dx alone: 5 x 1404, 877 points, 3-D, 16.9 / 14.2;  12 x 1491, one point shared by two, 2-D, 14.4 / 13.8
 struct LaunchCost {
-    double pair, per_step, clear, several_chunks, contended;
+    double pair, per_step, point, clear, several_chunks, contended;
     static constexpr double kStage = 900.0;
 
     double of(int P, size_t chunks, size_t mixtures, int slices, int per) const {
@@ -737,7 +738,7 @@ struct LaunchCost {
     }
     double of(int P, size_t chunks, size_t workgroups, int slices, double staging, double steps) const {
         const size_t rounds = (workgroups + 255) / 256;
-        const double one = staging + steps * (P * pair + per_step);
+        const double one = staging + P * point + steps * (P * pair + per_step);
         return one * double(rounds < 2 ? 2 : rounds) + (slices > 1 ? clear : 0.0) + (chunks > 1 ? several_chunks : 0.0) +
                contended * slices;
     }
@@ -746,7 +747,8 @@ struct SmallPlan { int P; TileSlices ts; };
 
 // (what depends on the slices alone is formed once: the search over some hundred plans takes well under a microsecond of
 // every small call)
-static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int M, int N, int p_max, SmallPlan full, double to_beat) {
+static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int M, int N, int p_max, SmallPlan full, double to_beat,
+                                   int min_slices = 1) {
     if (mixtures == 0 || M == 0 || N == 0) return full;         // (nothing to launch: asked for by reports only)
     constexpr int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
     struct { int per, slices; double staging, steps; } cand[12];
@@ -754,6 +756,7 @@ static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int
     for (int want : kSlices) {
         const int per = ((M + want - 1) / want + 3) / 4 * 4;
         if (want > 1 && per < 32) break;
+        if ((M + per - 1) / per < min_slices) continue;
         const int here = per < M ? per : M;
         cand[n++] = {per, (M + per - 1) / per, LaunchCost::kStage * ((here + kTile - 1) / kTile), double((here + 3) / 4)};
     }
@@ -771,12 +774,14 @@ static SmallPlan plan_small_launch(const LaunchCost& model, size_t mixtures, int
 
 // Mixtures that a workgroup of the backward kernel takes one after the other when all mixtures share their points: few
 // enough to leave the chip busy, many enough that their additions to dL/dx do not queue up.  Taken where the queue would
-// be as long as 0.7 of the modelled work (a shorter one hides behind it: 800 x 128 Gaussians at 784 points 70.5 us with one
-// mixture per workgroup, 82 us with several).  Measured, one mixture / several in us:
+// be as long as the modelled work, in double 1.4 times (a shorter one hides behind it: 800 x 128 Gaussians at 784 points
+// 70.5 us with one mixture per workgroup, 82 us with several), and in double not where the lanes hold mostly padding and
+// the preparation of many Gaussians stays serial (1231 x 127 at 7 points, 2-D, 54 / 73).  Measured, one mixture / several in us:
 //   6400 x 16 Gaussians at 100 points, 2-D: 317 / 67;  1353 x 36 at 361: 82 / 44, in 3-D 120 / 69;  2268 x 23 at 3049,
 //   3-D: 381 / 227;  1116 x 52 at 1547, 3-D: 134 / 113
-static int plan_mixtures_per_group(const LaunchCost& model, int P, size_t mixtures, int M, int N, TileSlices ts) {
+static int plan_mixtures_per_group(const LaunchCost& model, int P, size_t mixtures, int M, int N, TileSlices ts, bool is_double) {
     constexpr int kGroup[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+    if (is_double && M > 64 && N < 64) return 1;
     const size_t chunks = (size_t(N) + 64 * P - 1) / (64 * P);
     const int per = ts.per_slice < M ? ts.per_slice : M;
     const double one = 0.5 * (model.of(P, 1, 1, 1, per) - model.contended);       // a workgroup and mixture
@@ -787,7 +792,7 @@ static int plan_mixtures_per_group(const LaunchCost& model, int P, size_t mixtur
         if (size_t(k) > mixtures) break;
         const size_t groups = (mixtures + k - 1) / k, rounds = (groups * chunks * ts.slices + 255) / 256;
         const double work = one * k * double(rounds < 2 ? 2 : rounds), cost = work + queue * double(groups);
-        if (k == 1 && queue * double(groups) < 0.7 * work) return 1;
+        if (k == 1 && queue * double(groups) < (is_double ? 1.4 : 1.0) * work) return 1;
         if (cost < 0.95 * best_cost) { best_cost = cost; best = k; }
     }
     return best;
@@ -818,14 +823,17 @@ static FwdPlan plan_fwd(const gmc_shape& s, bool is_double) {
     if (forced >= 2 && forced <= q_max) plan.rc = forced;
     if (plan.rc > 0) plan.chunks = (s.N + 64 * plan.rc - 1) / (64 * plan.rc);
     plan.ts = plan_tile_slices(grid_mixtures(BL) * plan.chunks, s.M, kTile);
-    if (BL * plan.chunks * plan.ts.slices < 2048 && forced < 2) {
-        const LaunchCost model{(s.D == 2 ? 9.0 : 13.0) + (is_double ? 16.0 : 0.0), 12.0, 1500.0, 0.0, 0.0};
+    // (few Gaussians: the launch's latency, which the model does not see, decides: 262 x 2 at 3542 points 6.3 us with the full
+    // plan, 9.5 with its choice; the 4 x 16 layout gains from slices beyond 128 Gaussians and 64 points only, 44 x 170 at
+    // one point 6.0 / 7.0)
+    if (BL * plan.chunks * plan.ts.slices < 2048 && forced < 2 && (plan.rc > 0 ? s.M > 128 && s.N > 64 : s.M > 64)) {
+        const LaunchCost model{(s.D == 2 ? 9.0 : 13.0) + (is_double ? 16.0 : 0.0), 12.0, 0.0, 1500.0, 0.0, 0.0};
         const int per = plan.ts.per_slice < s.M ? plan.ts.per_slice : s.M;
         // (the other layout: one Gaussian a step, 256 points per point of a lane)
         const double full_cost = plan.rc > 0 ? model.of(plan.rc, plan.chunks, BL, plan.ts.slices, per)
                                              : model.of(4 * plan.P, plan.chunks, BL, plan.ts.slices, per);
         const SmallPlan small = plan_small_launch(model, BL, s.M, s.N, q_max, SmallPlan{0, plan.ts},
-                                                  (plan.rc > 0 ? 0.9 : 0.7) * full_cost);
+                                                  (plan.rc == 0 ? 0.7 : s.M > 256 ? 0.9 : 0.8) * full_cost);
         if (small.P > 0) {
             plan.rc = small.P;
             plan.chunks = (s.N + 64 * plan.rc - 1) / (64 * plan.rc);
@@ -847,10 +855,11 @@ static FwdPlan plan_fwd(const gmc_shape& s, bool is_double) {
 //   6000 x 129 at 250             138 /  70      163 / 178    (two of the four wavefronts nearly idle; in 3-D 170 / 106, 272 / 341)
 //   64 x 150 at 128               6.1 /  6.5    13.7 / 12.0    (forward: the 4 x 16 kernel)
 // hence three full groups, fewer only against the matrix-core forward kernel or with few points in the backward pass.
-// float64, 256 x 256 at 128: forward 11.8 / 14.4, backward 33.7 / 20.8; 64 x 256 at 64: 11.2 / 8.8 and 32.0 / 13.6.
+// float64, 256 x 256 at 128: forward 11.8 / 14.4, backward 33.7 / 20.8; 64 x 256 at 64: 11.2 / 8.8 and 32.0 / 13.6;
+// 81 x 136 at 61: forward 8.0 / 8.8.
 bool dense_forward_f32_takes(const gmc_shape& s);
 static bool few_points_fwd(const gmc_shape& s) {
-    if (s.dtype == GMC_F64) return s.M > 128 && s.N <= 64;
+    if (s.dtype == GMC_F64) return s.N <= 32 ? s.M > 128 : s.N <= 64 && s.M >= 192;
     return s.N <= 256 && (s.M >= 192 || dense_forward_f32_takes(s));
 }
 static bool few_points_bwd(const gmc_shape& s) {
@@ -1009,13 +1018,19 @@ static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad
     }
     int P = bwd_points_per_lane<T, D>(s);
     const size_t chunks = (size_t(s.N) + 64 * P - 1) / (64 * P);
-    TileSlices ts = plan_tile_slices(grid_mixtures(BL) * chunks, s.M, kTile);
-    const LaunchCost model{(D == 2 ? 20.0 : 32.0) + (sizeof(T) == 8 ? 16.0 : 0.0), (sizeof(T) == 8 ? 12.0 : 5.0) * Sums<D>::k,
-                           need_gx ? 1500.0 : 0.0, need_gm ? 3500.0 : 0.0,
-                           need_gx ? (D == 2 ? 30.0 : 50.0) * double(BL / (size_t(s.Bx) * s.Lx) - 1) : 0.0};
-    if (BL * chunks * ts.slices < 2048 && forced_bwd_points.load() < 2) {
+    TileSlices ts = plan_tile_slices(grid_mixtures(BL) * chunks, s.M, kTile, !need_gm && xes_shared);
+    const double met = double(BL / (size_t(s.Bx) * s.Lx));               // mixtures whose additions meet on a point
+    const double type_cost = sizeof(T) == 8 ? 16.0 : 0.0;
+    const LaunchCost model = need_gm
+        ? LaunchCost{(D == 2 ? 20.0 : 32.0) + type_cost, (sizeof(T) == 8 ? 12.0 : 5.0) * Sums<D>::k, 60.0, need_gx ? 1500.0 : 0.0,
+                     3500.0, need_gx ? (D == 2 ? 30.0 : 50.0) * (met - 1.0) : 0.0}
+        : LaunchCost{(D == 2 ? 12.0 : 18.0) + type_cost, 20.0, 60.0, 1500.0, 0.0, (D == 2 ? 45.0 : 75.0) * met};
+    // (one or two Gaussians: the full plan, as in plan_fwd: 99 x 2 at 2256 points, float64, dL/dx 12.4 / 16.4; dL/dx alone of
+    // shared points: no fewer slices than that plan, whose workgroups end one after the other)
+    if (s.M > 2 && BL * chunks * ts.slices < 2048 && forced_bwd_points.load() < 2) {
         const double full_cost = model.of(P, chunks, BL, ts.slices, ts.per_slice < s.M ? ts.per_slice : s.M);
-        const SmallPlan small = plan_small_launch(model, BL, s.M, s.N, sizeof(T) == 8 ? 8 : 16, SmallPlan{P, ts}, 0.9 * full_cost);
+        const SmallPlan small = plan_small_launch(model, BL, s.M, s.N, sizeof(T) == 8 ? 8 : 16, SmallPlan{P, ts}, 0.85 * full_cost,
+                                                  !need_gm && xes_shared ? ts.slices : 1);
         P = small.P;
         ts = small.ts;
     }
@@ -1024,7 +1039,7 @@ static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad
     // one chunk per mixture: the pair kernel's workgroups finish the gradient of their mixture themselves
     const bool sole = need_gm && s.N <= 64 * P;
     zero2_async(sums, need_gm && !sole ? n_gauss * Sums<D>::k : 0, grad_xes, need_gx && gx_shared ? n_x : 0, stream);
-    const int per_group = need_gm && need_gx && s.Bx == 1 && s.Lx == 1 && BL > 1 ? plan_mixtures_per_group(model, P, BL, s.M, s.N, ts) : 1;
+    const int per_group = need_gm && need_gx && s.Bx == 1 && s.Lx == 1 && BL > 1 ? plan_mixtures_per_group(model, P, BL, s.M, s.N, ts, sizeof(T) == 8) : 1;
     if (per_group > 1 && sole) launch_bwd_main<T, D, true, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream, per_group);
     else if (per_group > 1) launch_bwd_main<T, D, true, true, false, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream, per_group);
     else if (sole && need_gx) launch_bwd_main<T, D, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream);
