@@ -154,6 +154,7 @@ __global__ __launch_bounds__(kBlock) void few_points_fwd_kernel(const T* __restr
     constexpr int G = 1 + D + D * D;
     constexpr int S = Rec<T, D>::kStride;
     constexpr int kWaves = kBlock / kWave;
+    static_assert(KIND != kEpiRatio, "its points are as many as its components");
     static_assert(16 * P <= kBlock, "one lane per point at the end");
     constexpr int kWaveScalars = (kWave + 6) * S > 16 * P ? (kWave + 6) * S : 16 * P;
     __shared__ __attribute__((aligned(16))) T lds[kWaves * kWaveScalars];
@@ -187,8 +188,7 @@ __global__ __launch_bounds__(kBlock) void few_points_fwd_kernel(const T* __restr
     for (int g0 = g_begin + wave * kWave; g0 < g_end; g0 += kBlock) {
         const bool active = g0 + lane < g_end;
         const int m = active ? g0 + lane : g0;
-        Derived<D> dv = derive<T, D>(mix_bl + size_t(m) * G, covariance_form);
-        if (KIND == kEpiRatio) dv.w = fabs(double(epi.weights[size_t(bl) * M + m]));
+        const Derived<D> dv = derive<T, D>(mix_bl + size_t(m) * G, covariance_form);
         const WaveTile t = stage_wave_tile<T, D, 4>(dv, active, 1.0, tile, lane);
         rc_pairs<T, D, P, false>(tile, exp2_tab, 0, t.centred_start, row, x, acc);
         rc_pairs<T, D, P, true>(tile, exp2_tab, t.centred_start, t.padded_total, row, x, acc);
@@ -215,11 +215,6 @@ __global__ __launch_bounds__(kBlock) void few_points_fwd_kernel(const T* __restr
             const T shifted = v + c;
             epi.out[at] = (shifted > T(0) ? shifted : T(0)) - (c > T(0) ? c : T(0));
         }
-    } else if constexpr (KIND == kEpiRatio) {
-        if (mine) {
-            const T xw = epi.weights[at];                           // M == N: point n is the centre of component n
-            epi.out[at] = (xw < T(0) ? -xw : xw) * (epi.goal[at] + T(0.05)) / (v + T(0.05));
-        }
     } else {
         // mean, then squared deviations from it, of the workgroup's values (see the kernel above)
         const double value = mine ? double(v) + double(epi.constant[bl]) : 0.0;
@@ -244,9 +239,13 @@ __global__ __launch_bounds__(kBlock) void few_points_fwd_kernel(const T* __restr
 static int consumer_points_per_lane(int N) { return N <= 128 ? 2 : N <= 256 ? 4 : 8; }
 static int consumer_chunks(int N) { const int P = consumer_points_per_lane(N); return (N + 64 * P - 1) / (64 * P); }
 
-// As few_points_fwd in gmc_dense.hip: more than two groups of Gaussians for the four wavefronts.  One workgroup has all
-// points: 1600 mixtures of 5120 Gaussians at 128 points 311 us (kernel above) / 259 us.
-static bool few_points_consumer(int M, int N) { return N <= 128 && M > 128; }
+// As few_points_fwd in gmc_dense.hip: more than two groups of Gaussians for the four wavefronts, three full ones above 96
+// points, in double at most 96 points.  One workgroup has all points.  Kernel above / this one in us: 1600 mixtures of 5120
+// Gaussians at 128 points 311 / 259; 50 x 129 at 122, 3-D, 6.6 / 7.3; float64 14 x 315 at 109 17.1 / 20.3, 3-D 3 x 166 at
+// 103 11.6 / 13.6.
+template <typename T> static bool few_points_consumer(int M, int N) {
+    return M > 128 && (N <= 96 || (sizeof(T) == 4 && N <= 128 && M >= 192));
+}
 
 template <typename T, int D, int KIND>
 static void launch_few_points(const T* mixture, const T* points, size_t mixture_stride, int point_stride, const EpiArgs<T>& epi,
@@ -255,9 +254,18 @@ static void launch_few_points(const T* mixture, const T* points, size_t mixture_
     const dim3 grid(unsigned(grid_mixtures(BL) * ts.slices));
     const int P = (N + 15) / 16;
 #define GMC_FEW(PP) few_points_fwd_kernel<T, D, PP, KIND><<<grid, dim3(kBlock), 0, stream>>>(mixture, points, mixture_stride, point_stride, epi, L, M, N, Bx, Lx, int(BL), cov, ts)
-    if (P <= 2) GMC_FEW(2); else if (P <= 4) GMC_FEW(4); else if (P <= 6) GMC_FEW(6); else if (P == 7) GMC_FEW(7);
-    else if (P == 8) GMC_FEW(8);
-    else if constexpr (KIND == kEpiStore) { if (P <= 10) GMC_FEW(10); else if (P <= 13) GMC_FEW(13); else GMC_FEW(16); }
+    // (the rules of the callers: at most 16 P = 64 points for the plain evaluation in double and 256 in float, 96 and 128
+    // for the reductions)
+    if (P <= 2) GMC_FEW(2); else if (P <= 4) GMC_FEW(4);
+    else if constexpr (sizeof(T) == 4 || KIND != kEpiStore) {
+        if (P <= 6) GMC_FEW(6);
+        else if constexpr (sizeof(T) == 4) {
+            if (P == 7) GMC_FEW(7); else if (P == 8) GMC_FEW(8);
+            else if constexpr (KIND == kEpiStore) {
+                if (P <= 10) GMC_FEW(10); else if (P <= 12) GMC_FEW(12); else if (P == 13) GMC_FEW(13); else GMC_FEW(16);
+            }
+        }
+    }
 #undef GMC_FEW
 }
 
@@ -276,10 +284,12 @@ static int launch_consumer(const T* mixture, const T* points, size_t mixture_str
                            int B, int L, int M, int N, hipStream_t stream) {
     const size_t BL = size_t(B) * L;
     if (BL == 0 || N == 0) return GMC_OK;
-    if (few_points_consumer(M, N)) {
-        launch_few_points<T, D, KIND>(mixture, points, mixture_stride, point_stride, epi, B, L, M, N, B, L, true,
-                                      TileSlices{1, M}, stream);
-        return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
+    if constexpr (KIND != kEpiRatio) {                  // (the ratio's points are the components themselves: not many against them)
+        if (few_points_consumer<T>(M, N)) {
+            launch_few_points<T, D, KIND>(mixture, points, mixture_stride, point_stride, epi, B, L, M, N, B, L, true,
+                                          TileSlices{1, M}, stream);
+            return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
+        }
     }
     const int P = consumer_points_per_lane(N);
     const int chunks = consumer_chunks(N);
@@ -345,8 +355,10 @@ __global__ __launch_bounds__(kBlock) void moments_finish_kernel(const double* __
 // numbers of a batch entry are dealt to `chunks` workgroups, each of which finds the box itself (a second launch or a
 // scratch buffer for the box would cost more).  Bound by the latency of reading the centres, which are many behind a
 // convolution: sixteen wavefronts with eight centres per lane in flight (100 batch entries of 81920 centres: 177 us with
-// four wavefronts and one centre in flight).  Few centres (kSampleFew): four wavefronts.
-constexpr int kSampleBlock = 1024, kSampleFew = 2048;
+// four wavefronts and one centre in flight).  Few centres: four wavefronts (the reduction over sixteen is longer, above all
+// in double: 3-D, 52 entries of 3019 centres 8.0 / 10.3 us).
+constexpr int kSampleBlock = 1024;
+template <typename T, int D> constexpr int kSampleFew = sizeof(T) == 4 ? 2048 : D == 2 ? 4096 : 12288;
 
 template <typename T, int D, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void sampling_positions_kernel(const T* __restrict__ mixture, T* __restrict__ u,
@@ -669,7 +681,7 @@ int gmc_batch_norm_sampling_positions(const void* mixture, void* uniform_in_posi
     const int chunks = int(wanted < 1 ? 1 : (wanted > 64 ? 64 : wanted));
     const dim3 grid{unsigned(shape->B) * unsigned(chunks)};
 #define GMC_SPB(T, DD, BLOCK) gmc::sampling_positions_kernel<T, DD, BLOCK><<<grid, dim3(BLOCK), 0, st>>>((const T*)mixture, (T*)uniform_in_positions_out, centres, samples, chunks)
-#define GMC_SP(T, DD) do { if (centres <= gmc::kSampleFew) GMC_SPB(T, DD, gmc::kBlock); else GMC_SPB(T, DD, gmc::kSampleBlock); } while (0)
+#define GMC_SP(T, DD) do { if (centres <= gmc::kSampleFew<T, DD>) GMC_SPB(T, DD, gmc::kBlock); else GMC_SPB(T, DD, gmc::kSampleBlock); } while (0)
     if (shape->dtype == GMC_F32) { if (shape->D == 2) GMC_SP(float, 2); else GMC_SP(float, 3); }
     else { if (shape->D == 2) GMC_SP(double, 2); else GMC_SP(double, 3); }
 #undef GMC_SP

@@ -59,7 +59,9 @@ int gmc_eval_fwd(const void* mixture, const void* xes, void* out, const gmc_shap
 void gmc_set_tuning(int fwd_points_per_lane, int bwd_points_per_lane);
 
 /* Name of the forward pair kernel a call of this shape launches (for benchmark reports; no counterpart in the
- * reference): "few_points_fwd_kernel" (at most 256 points, more than 128 components), "eval_fwd_mfma_kernel" (float32, more than 128 components, enough work for 512-component tiles),
+ * reference): "few_points_fwd_kernel" (float32: at most 256 points and 192 components or more, or more than 128
+ * where the matrix-core kernel would be taken; float64: at most 64 points and 192 components or more, 32 points and more
+ * than 128), "eval_fwd_mfma_kernel" (float32, more than 128 components, enough work for 512-component tiles),
  * "eval_fwd_rc_kernel" or "eval_fwd_kernel" (all vector ALU, two layouts); "" for an invalid shape. */
 const char* gmc_eval_fwd_kernel_name(const gmc_shape* shape);
 /* Shader clock in MHz that one workgroup in the middle of the grid saw during the last launch of the float32
