@@ -10,6 +10,7 @@ import typing
 
 import torch
 from torch import Tensor
+from torch.autograd.function import once_differentiable
 
 from . import _native
 from . import mixture as gm
@@ -45,48 +46,10 @@ class _FusedReluFit(torch.autograd.Function):
         return out
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, grad_out: Tensor):
         target, constant, fit, goal = ctx.saved_tensors
-        # (a backward pass under grad mode, create_graph=True, stays a composition that autograd records)
-        backward = _relu_fit_bwd_composed if torch.is_grad_enabled() else _native.relu_fit_bwd
-        return backward(grad_out, target, constant, fit, goal, *ctx.needs_input_grad)
-
-
-def _relu_fit_bwd_composed(grad_out, target, constant, fit, b, need_target, need_constant, need_fit):
-    """_native.relu_fit_bwd with torch operations around the backward kernels"""
-    D = gm.n_dimensions(fit)
-    grad_out = grad_out.contiguous()
-    w = fit[..., 0]
-    x0 = w.abs() + 0.1
-    centres = fit[..., 1:1 + D].contiguous()
-    fit_abs = fit.clone()
-    fit_abs[..., 0] = x0
-    cur = _native.eval_fwd(fit_abs, centres, covariance_form=True) + 0.05
-    d_x1 = grad_out[..., 0]
-    ratio = (b + 0.05) / cur
-    d_b = d_x1 * x0 / cur
-    d_cur = -d_x1 * x0 * ratio / cur
-    c = constant.expand(b.shape[0], b.shape[1]).unsqueeze(-1)
-    relu_c = torch.clamp(c, min=0)
-    lifted = (b + relu_c) > 0                                    # v + c > 0
-    d_v = (d_b * lifted).contiguous()
-    grad_target = grad_constant = grad_fit = None
-    g_target, g_centres = _native.eval_bwd(d_v, target, centres, need_target, need_fit, covariance_form=True)
-    if need_target:
-        grad_target = g_target
-    if need_constant:
-        g = (d_b * (lifted.to(d_b.dtype) - (c > 0).to(d_b.dtype))).sum(-1)
-        for dim in (0, 1):
-            if constant.shape[dim] == 1 and g.shape[dim] != 1:
-                g = g.sum(dim, keepdim=True)
-        grad_constant = g
-    if need_fit:
-        g_abs, g_centres2 = _native.eval_bwd(d_cur.contiguous(), fit_abs, centres, True, True, covariance_form=True)
-        grad_fit = grad_out.clone()
-        grad_fit[..., 0] = torch.sign(w) * (d_x1 * ratio + g_abs[..., 0])
-        grad_fit[..., 1:1 + D] += g_abs[..., 1:1 + D] + g_centres + g_centres2
-        grad_fit[..., 1 + D:] += g_abs[..., 1 + D:]
-    return grad_target, grad_constant, grad_fit
+        return _native.relu_fit_bwd(grad_out, target, constant, fit, goal, *ctx.needs_input_grad)
 
 
 def fixed_point_iteration_to_relu(target_mixture: Tensor, target_constant: Tensor, fitting_mixture: Tensor,

@@ -278,6 +278,22 @@ def test_fused_fitting_gradients(dims, dtype, broadcast_constant):
     assert np.array_equal(c.grad.cpu().numpy(), (const > 0).astype(npdt))
 
 
+def test_fused_fitting_gradient_is_not_differentiable_again():
+    """the backward kernels record nothing: a second derivative is refused, as that of the evaluation is, instead of lacking
+    every term through the evaluations; a first one under create_graph=True is what it is without"""
+    rng = np.random.default_rng(41)
+    t, c, f = (torch.tensor(a, dtype=torch.float32, device=DEV, requires_grad=True)
+               for a in (_cov_mixture(rng, 1, 2, 20, 2, cov=0.1), rng.normal(size=(1, 2)) * 0.3, _cov_mixture(rng, 1, 2, 9, 2, cov=0.1)))
+    out, _ = fitting.fixed_point_iteration_to_relu(t, c, f, 1)
+    loss = (out[..., 0] ** 2).sum()
+    first = torch.autograd.grad(loss, (t, c, f), retain_graph=True)
+    again = torch.autograd.grad(loss, (t, c, f), create_graph=True)
+    for a, b in zip(first, again):
+        assert rel_l2(b.detach().cpu().numpy(), a.cpu().numpy()) <= 1e-6
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        sum(g.square().sum() for g in again).backward()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("D", [2, 3])
 def test_fused_moments_are_std_mean_of_the_sampled_values(D, dtype):
