@@ -296,6 +296,65 @@ def test_fused_fitting_gradient_is_not_differentiable_again():
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("D", [2, 3])
+def test_fused_fitting_gradients_one_at_a_time(D, dtype):
+    """each gradient alone and any two together, with targets of many components at few fitting centres (the kernel for few
+    points), fitting weights of zero, and upstream gradients that are strided or expanded; against the differentiable
+    composition"""
+    npdt = np.float32 if dtype == torch.float32 else np.float64
+    for B, L, Mt, Mf in ((2, 2, 129, 33), (1, 3, 193, 97), (3, 1, 300, 128), (2, 1, 129, 1), (1, 2, 40, 300)):
+        rng = np.random.default_rng(Mt + Mf + D)
+        target, fit = (_cov_mixture(rng, B, L, M, D, cov=0.1).astype(npdt) for M in (Mt, Mf))
+        fit[..., ::5, 0] = 0.0
+        const = (rng.normal(size=(B, 1)) * 0.3).astype(npdt)
+        G = fit.shape[-1]
+        ups = [torch.tensor(rng.normal(size=(Mf, G, L, B)).astype(npdt), device=DEV).permute(3, 2, 0, 1),
+               torch.tensor(rng.normal(size=(1, 1, 1, G)).astype(npdt), device=DEV).expand(B, L, Mf, G)]
+        for up in ups:
+            tensors = [torch.tensor(a, device=DEV, requires_grad=True) for a in (target, const, fit)]
+            want = torch.autograd.grad(fitting._composed_fixed_point(*tensors, 1), tensors, up)
+            for subset in ((0,), (1,), (2,), (0, 1), (0, 2), (1, 2), (0, 1, 2)):
+                args = [v.detach().requires_grad_(i in subset) for i, v in enumerate(tensors)]
+                out, _ = fitting.fixed_point_iteration_to_relu(*args, 1)
+                got = torch.autograd.grad(out, [args[i] for i in subset], up)
+                for i, g in zip(subset, got):
+                    assert rel_l2(g.cpu().numpy(), want[i].cpu().numpy(), 1e-30) <= 20 * TOL[dtype], (B, L, Mt, Mf, subset, i)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("D", [2, 3])
+def test_reductions_with_few_points_and_many_gaussians(D, dtype):
+    """the fitting goal and the moments of mixtures whose points one workgroup holds: both sides of every line of the rule
+    (128 / 129 and 191 / 192 Gaussians, 96 / 97 and 128 / 129 points), one point, and points that leave most of a wavefront
+    or of its last round idle; against the oracle, the moments also behind a constant large against the spread"""
+    npdt = np.float32 if dtype == torch.float32 else np.float64
+    cases = [(M, N) for M in (128, 129, 191, 192, 300, 1000) for N in (1, 17, 33, 65, 96, 97, 100, 112, 128, 129)]
+    for k, (M, N) in enumerate(cases):
+        rng = np.random.default_rng(1000 * M + N + D)
+        B, L = (2, 2) if k % 3 else (1, 3)
+        m = _cov_mixture(rng, B, L, M, D, cov=0.1).astype(npdt)
+        fit = _cov_mixture(rng, B, L, N, D, cov=0.1).astype(npdt)
+        xes = np.ascontiguousarray(fit[..., 1:1 + D])
+        const = (rng.normal(size=(B, L)) * 0.3).astype(npdt)
+        values = o.evaluate(m.astype(np.float64), xes.astype(np.float64))
+        c0 = const.astype(np.float64)[..., None]
+        mt = torch.tensor(m, device=DEV)
+        goal = _native.relu_fit_goal(mt, torch.tensor(const, device=DEV), torch.tensor(fit, device=DEV)).cpu().numpy()
+        # (the values' error is relative to the values, the goal is what the two relus leave of them)
+        want = np.maximum(values + c0, 0) - np.maximum(c0, 0)
+        assert np.linalg.norm(goal - want) <= 2 * TOL[dtype] * np.linalg.norm(np.abs(values) + np.abs(c0)), (M, N)
+        for shift in (0.0, 1000.0):
+            c1 = (const + npdt(shift)).astype(npdt)
+            sd, mean = _native.eval_cov_moments(mt, torch.tensor(c1, device=DEV), torch.tensor(xes, device=DEV), per_sample=True)
+            shifted = values + c1.astype(np.float64)[..., None]
+            assert rel_l2(mean.cpu().numpy(), shifted.mean(-1)) <= TOL[dtype], (M, N, shift)
+            if N > 1:
+                assert rel_l2(sd.cpu().numpy(), values.std(-1, ddof=1)) <= 10 * TOL[dtype], (M, N, shift)
+            sd, mean = _native.eval_cov_moments(mt, torch.tensor(c1, device=DEV), torch.tensor(xes, device=DEV), per_sample=False)
+            assert rel_l2(mean.cpu().numpy(), shifted.mean((0, 2))) <= TOL[dtype], (M, N, shift)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("D", [2, 3])
 def test_fused_moments_are_std_mean_of_the_sampled_values(D, dtype):
     """gmc_eval_cov_moments against torch.std_mean of the values that gm.evaluate returns and against numpy on the
     oracle's values, per channel over batch and samples and per (b, l), for point counts that take the 128-, 256- and
