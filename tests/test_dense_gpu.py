@@ -184,13 +184,16 @@ def test_every_points_per_lane_instance(dtype):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_one_chunk_per_mixture(dtype):
     """When one chunk of points covers a mixture, the workgroups of the backward pair kernel finish grad_mixture
-    themselves (plain stores of the sums, no zero fill, no epilogue launch).  256 mixtures make a launch take one
-    chunk whenever that covers N.  Covered: two tiles of Gaussians, per-mixture and broadcast points, every
-    combination of the need flags, and the covariance form (gm.evaluate)."""
+    themselves (plain stores of the sums, no zero fill, no epilogue launch).  128 mixtures of two tiles make a launch take
+    one chunk whenever that covers N.  Covered: two tiles of Gaussians in one workgroup or in two slices, per-mixture and
+    broadcast points, every combination of the need flags, and the covariance form (gm.evaluate); the first two shapes have
+    more points than the kernel for few points takes, the others are its own."""
     npdt = np.float32 if dtype == torch.float32 else np.float64
     tol, fl = TOL[dtype], FLOOR[dtype]
-    for D, M, N, broadcast in ((2, 280, 150, False), (3, 270, 100, True)):
-        mix, xes, gout = _case(8, 32, M, N, D, 7100 + D, broadcast)
+    beyond = 260 if dtype == torch.float32 else 132
+    for L, D, M, N, broadcast in ((16, 2, 280, beyond, False), (16, 3, 260, beyond, True), (32, 2, 280, 150, False),
+                                  (32, 3, 270, 100, True)):
+        mix, xes, gout = _case(8, L, M, N, D, 7100 + D, broadcast)
         _check(mix, xes, gout, dtype, tag=f"one chunk D{D}")
         mix, xes, gout = mix.astype(npdt), xes.astype(npdt), gout.astype(npdt)
         rgm, rgx = o.evaluate_inversed_backward(gout, mix, xes)
@@ -226,11 +229,16 @@ def test_small_launches_split_gaussians_below_a_tile(dtype, D):
     Gaussian in one, one chunk of points with several slices (the workgroups finish their own Gaussians' gradients and
     add to dL/dx), points that all mixtures share"""
     shapes = [(1, 3, 333, 700), (2, 2, 97, 1300), (1, 1, 65, 3000), (1, 1, 129, 300), (1, 2, 253, 270), (3, 5, 77, 2000),
-              (1, 1, 33, 9000), (8, 2, 130, 520), (1, 1, 1000, 511)]
+              (1, 1, 33, 9000), (8, 2, 130, 520), (1, 1, 1000, 511),
+              (6, 4, 600, 300), (1, 70, 2, 700), (12, 1, 300, 70)]
     for i, (B, L, M, N) in enumerate(shapes):
         for broadcast in (False, True):
             mix, xes, gout = _case(B, L, M, N, D, 63000 + i, broadcast)
             _check(mix, xes, gout, dtype, tag=f"B{B} L{L} M{M} N{N} broadcast {broadcast}")
+            mt, xt, gt = (torch.tensor(a, dtype=dtype, device=DEV) for a in (mix, xes, gout))
+            gm_, gx_ = _native.eval_bwd(gt, mt, xt, True, True)              # each gradient alone has a plan of its own
+            assert rel_l2(_native.eval_bwd(gt, mt, xt, True, False)[0].cpu().numpy(), gm_.cpu().numpy()) <= TOL[dtype]
+            assert rel_l2(_native.eval_bwd(gt, mt, xt, False, True)[1].cpu().numpy(), gx_.cpu().numpy()) <= TOL[dtype]
 
 
 @pytest.mark.parametrize("D", [2, 3])
@@ -291,17 +299,29 @@ def test_matrix_core_forward_shapes(D):
     of the 16-point groups, almost empty point blocks, and components far from the origin in units of their width
     (those are evaluated with an explicit x - b next to the matrix-core ones)."""
     dtype = torch.float32
+
+    def name(mix, xes):
+        (B, L, M, _), (Bx, Lx, N, _) = mix.shape, xes.shape
+        return _native.lib().gmc_eval_fwd_kernel_name(ctypes.byref(_native.Shape(B, L, M, N, D, Bx, Lx, _native.GMC_F32)))
+
+    def check(mix, xes, gout, tag):
+        assert name(mix, xes) == b"eval_fwd_mfma_kernel", tag
+        _check(mix, xes, gout, dtype, tag=tag)
     mix, xes, gout = _case(1, 1, 700, 8200, D, 900 + D, False)
-    _check(mix, xes, gout, dtype, tag=f"wide M700 N8200 D{D}")
+    check(mix, xes, gout, tag=f"wide M700 N8200 D{D}")
     far = mix.copy()
     far[:, :, ::3, 1:1 + D] *= 9.0           # every third component: |u b| well above the shifted-form limit
     xes_far = xes.copy()
     xes_far[:, :, ::2] *= 9.0
-    _check(far, xes_far, gout, dtype, tag=f"wide far components D{D}")
-    mix, xes, gout = _case(40, 16, 130, 100, D, 910 + D, False)
-    _check(mix, xes, gout, dtype, tag=f"wide many mixtures few points D{D}")
+    check(far, xes_far, gout, tag=f"wide far components D{D}")
+    # many mixtures, one partly filled block of points
+    mix, xes, _ = (a.astype(np.float32) for a in _case(32, 16, 130, 260, D, 910 + D, False))
+    assert name(mix, xes) == b"eval_fwd_mfma_kernel"
+    out = gm.evaluate_inversed(torch.tensor(mix, device=DEV), torch.tensor(xes, device=DEV)).cpu().numpy()
+    ref = cpu_ref.forward(mix.astype(np.float64), xes.astype(np.float64), n_threads=16)
+    assert rel_l2(out, ref, FLOOR[dtype]) <= TOL[dtype]
     mix, xes, gout = _case(2, 1, 1030, 8192 + 17, D, 920 + D, True)
-    _check(mix, xes, gout, dtype, tag=f"wide broadcast three tiles D{D}")
+    check(mix, xes, gout, tag=f"wide broadcast three tiles D{D}")
     # covariance form on the same kernel: gm.evaluate inverts inside the staging
     mix, xes, gout = _case(1, 2, 300, 8200, D, 930 + D, False)
     B, L, M = mix.shape[:3]
