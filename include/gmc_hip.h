@@ -55,7 +55,8 @@ int gmc_eval_fwd(const void* mixture, const void* xes, void* out, const gmc_shap
 
 /* Tuning and test knob (no counterpart in the reference; process-wide): forces the points per lane of the all-vector
  * "4 x 16" kernels, forward and backward (2 ... 16, float64: 2 ... 8; a workgroup then covers 64 times as many points);
- * 0 returns to the automatic choice.  Results do not depend on it beyond the order of additions. */
+ * 0 returns to the automatic choice.  Shapes that the kernels for few points take are not concerned.  Results do not depend
+ * on it beyond the order of additions. */
 void gmc_set_tuning(int fwd_points_per_lane, int bwd_points_per_lane);
 
 /* Name of the forward pair kernel a call of this shape launches (for benchmark reports; no counterpart in the
