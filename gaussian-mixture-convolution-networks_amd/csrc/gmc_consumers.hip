@@ -241,7 +241,7 @@ static int consumer_chunks(int N) { const int P = consumer_points_per_lane(N); r
 
 // As few_points_fwd in gmc_dense.hip: more than two groups of Gaussians for the four wavefronts, three full ones above 96
 // points, in double at most 96 points.  One workgroup has all points.  Kernel above / this one in us: 1600 mixtures of 5120
-// Gaussians at 128 points 311 / 259; 50 x 129 at 122, 3-D, 6.6 / 7.3; float64 14 x 315 at 109 17.1 / 20.3, 3-D 3 x 166 at
+// Gaussians at 128 points 296 / 277; 50 x 129 at 122, 3-D, 6.6 / 7.3; float64 14 x 315 at 109 17.1 / 20.3, 3-D 3 x 166 at
 // 103 11.6 / 13.6.
 template <typename T> static bool few_points_consumer(int M, int N) {
     return M > 128 && (N <= 96 || (sizeof(T) == 4 && N <= 128 && M >= 192));

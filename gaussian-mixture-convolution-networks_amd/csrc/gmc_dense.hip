@@ -600,8 +600,8 @@ __global__ __launch_bounds__(kBlock) void eval_bwd_epilogue_kernel(const T* __re
 // points and the wavefronts share the Gaussians, 64 at a time: four times fewer reductions per pair, the lane that
 // prepared a Gaussian finishes its gradient from the wavefront's own sums (no workspace, no atomics, no workgroup
 // barrier, no second preparation), and only dL/dx is added over wavefronts and slices at the end.  Bound by instruction
-// issue: 1600 mixtures of 5120 Gaussians at 128 points in 2-D 674 us (1.05e9 pairs, 42 cycles per 64 pairs and SIMD;
-// 1030 us with zero fill, pair kernel and epilogue before).
+// issue: 1600 mixtures of 5120 Gaussians at 128 points in 2-D 626 us (1.05e9 pairs, 39 cycles per 64 pairs and SIMD;
+// 1029 us with zero fill, pair kernel and epilogue before).
 template <typename T, int D, int P, bool NEED_GX>
 __global__ __launch_bounds__(kBlock) void few_points_bwd_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
                                                                 const T* __restrict__ xes, T* __restrict__ grad_xes,
@@ -726,8 +726,9 @@ void set_tuning(int fwd_points_per_lane, int bwd_points_per_lane) {
 // each that meets on an address in 2-D, 75 ns in 3-D; taken half as high again for dL/dx alone, whose workgroups end
 // together).  The plan for full launches stays unless the model gives a tenth to a fifth (three tenths against the
 // one-Gaussian-per-step layout).  Measured, full-launch plan / this one in us:
-//   15 x 333 Gaussians, 2777 points, float64, 3-D: forward 38.7 / 22.1, backward 100.9 / 52.9 (tiles of 256 and 77 before)
-//   3 x 540, 1058 points, float32, 2-D: 9.5 / 7.0 and 24.1 / 13.5
+//   15 x 333 Gaussians, 2777 points, float64, 3-D: backward 100 / 50 (tiles of 256 and 77 before; the forward launch
+//   keeps the full plan, its slices evenly filled: 38.1 / 28.9)
+//   3 x 540, 1058 points, float32, 2-D: 9.3 / 6.8 and 23.6 / 11.6
 //   dL/dx alone: 5 x 1404, 877 points, 3-D, 16.9 / 14.2;  12 x 1491, one point shared by two, 2-D, 14.4 / 13.8
 struct LaunchCost {
     double pair, per_step, point, clear, several_chunks, contended;
@@ -847,15 +848,15 @@ static FwdPlan plan_fwd(const gmc_shape& s, bool is_double) {
 // at most 16 points per lane (8 in double), and more than two groups of 64 Gaussians to share out.  Measured, kernels
 // above / few-points kernels in us (float32, 2-D):
 //   mixtures x M at N points      forward        backward
-//   1600 x 5120 at 128            749 / 261     1030 / 674    (forward: the matrix-core kernel, whose blocks hold 1024 points)
-//   1200 x 1280 at 100            225 /  56      209 / 129
-//   320 x 1000 at 128            18.6 / 16.7    53.5 / 35.7
-//   1024 x 256 at 250            35.5 / 21.8    54.0 / 47.8
-//   1 x 256 at 128                7.1 /  6.3    18.1 / 11.6
-//   6000 x 129 at 250             138 /  70      163 / 178    (two of the four wavefronts nearly idle; in 3-D 170 / 106, 272 / 341)
+//   1600 x 5120 at 128            745 / 247     1029 / 626    (forward: the matrix-core kernel, whose blocks hold 1024 points)
+//   1200 x 1280 at 100            223 /  53      205 / 114
+//   320 x 1000 at 128            17.4 / 16.0    52.9 / 34.1
+//   1024 x 256 at 250            34.4 / 20.6    52.2 / 45.8
+//   1 x 256 at 128                6.8 /  6.0    17.8 / 11.3
+//   6000 x 129 at 250             137 /  65      163 / 178    (two of the four wavefronts nearly idle; in 3-D 170 / 99, 272 / 341)
 //   64 x 150 at 128               6.1 /  6.5    13.7 / 12.0    (forward: the 4 x 16 kernel)
 // hence three full groups, fewer only against the matrix-core forward kernel or with few points in the backward pass.
-// float64, 256 x 256 at 128: forward 11.8 / 14.4, backward 33.7 / 20.8; 64 x 256 at 64: 11.2 / 8.8 and 32.0 / 13.6;
+// float64, 256 x 256 at 128: forward 11.8 / 14.4, backward 33.0 / 20.2; 64 x 256 at 64: 11.2 / 8.7 and 32.0 / 13.7;
 // 81 x 136 at 61: forward 8.0 / 8.8.
 bool dense_forward_f32_takes(const gmc_shape& s);
 static bool few_points_fwd(const gmc_shape& s) {
