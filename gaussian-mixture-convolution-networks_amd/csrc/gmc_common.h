@@ -520,6 +520,9 @@ inline size_t grid_mixtures(size_t n_mixtures) {
     return n_mixtures >= size_t(kXcdAffineMin) ? (n_mixtures + 7) / 8 * 8 : n_mixtures;
 }
 
+// Workgroups of one launch: its threads are counted in 32 bits, and a launch of more starts fewer of them without an error.
+inline size_t max_workgroups(int threads) { return ((size_t(1) << 32) - 1) / size_t(threads); }
+
 // A launch with few workgroups (one large mixture, few point chunks) leaves most compute units idle, or with a single
 // wavefront per SIMD.  The LDS tiles of Gaussians of a mixture are then dealt to several workgroups per point chunk
 // ("slices"), which add their partial results with atomics into outputs that were cleared before.

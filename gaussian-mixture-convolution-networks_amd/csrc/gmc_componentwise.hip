@@ -14,14 +14,14 @@ constexpr int kCwPoints = 64;      // points per workgroup
 template <typename T, int D>
 __global__ __launch_bounds__(kBlock) void componentwise_fwd_kernel(const T* __restrict__ mixture, const T* __restrict__ xes,
                                                                   T* __restrict__ out, int L, int M, int N, int Bx, int Lx,
-                                                                  int m_tiles, int chunks, bool covariance_form) {
+                                                                  int m_tiles, int first_mixture, int chunks, bool covariance_form) {
     constexpr int G = 1 + D + D * D;
     const T* exp2_tab = exp2_table<T>();
     if constexpr (sizeof(T) == 8) __syncthreads();          // the table is complete (all wavefronts are still here)
     int id = blockIdx.x;
     const int chunk = id % chunks; id /= chunks;
     const int tile = id % m_tiles;
-    const int bl = id / m_tiles;
+    const int bl = first_mixture + id / m_tiles;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     // A wavefront owns one slice of 64 Gaussians; with fewer than four slices in this tile the four wavefronts share
@@ -135,8 +135,8 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(W
 void componentwise_bwd_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
                                                                   const T* __restrict__ xes, T* __restrict__ sums,
                                                                   T* __restrict__ grad_xes, int L, int M, int N, int Bx,
-                                                                  int Lx, int m_groups, int chunks, int points_per_chunk,
-                                                                  bool shared_points, bool wide, bool covariance_form) {
+                                                                  int Lx, int m_groups, int first_mixture, int chunks,
+                                                                  int points_per_chunk, bool shared_points, bool wide, bool covariance_form) {
     constexpr int G = 1 + D + D * D, U = kCwSteps, kThreads = WAVES * kWave;
     constexpr int NR = 1 + D + D * (D + 1) / 2;
     constexpr int kU = Rec<T, D>::kU;
@@ -147,7 +147,7 @@ void componentwise_bwd_kernel(const T* __restrict__ grad_out, const T* __restric
     int id = blockIdx.x;
     const int chunk = id % chunks; id /= chunks;
     const int group = id % m_groups;
-    const int bl = id / m_groups;
+    const int bl = first_mixture + id / m_groups;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane >> 4, col = lane & 15;
@@ -303,8 +303,9 @@ constexpr int kCwUnroll = 8;
 template <typename T, int D>
 __global__ __launch_bounds__(kBlock) void componentwise_bwd_points_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
                                                                          const T* __restrict__ xes, T* __restrict__ grad_xes, int L,
-                                                                         int M, int N, int Bx, int Lx, int m_groups, int chunks,
-                                                                         int points_per_chunk, bool shared_points, bool covariance_form) {
+                                                                         int M, int N, int Bx, int Lx, int m_groups, int first_mixture,
+                                                                         int chunks, int points_per_chunk, bool shared_points,
+                                                                         bool covariance_form) {
     constexpr int G = 1 + D + D * D;
     constexpr int kU = Rec<T, D>::kU;
     __shared__ T point_grad[kCwPointsMax * D];
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(kBlock) void componentwise_bwd_points_kernel(const 
     int id = blockIdx.x;
     const int chunk = id % chunks; id /= chunks;
     const int group = id % m_groups;
-    const int bl = id / m_groups;
+    const int bl = first_mixture + id / m_groups;
     const int b = bl / L, l = bl - b * L;
     const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
     // (no readfirstlane here: with a provably uniform wavefront index the point coordinates arrive through scalar
@@ -415,8 +416,11 @@ static int cw_forward(const T* mixture, const T* xes, T* out, const gmc_shape& s
     const size_t BL = size_t(s.B) * s.L;
     if (BL == 0 || s.N == 0 || s.M == 0) return GMC_OK;
     const int m_tiles = (s.M + kBlock - 1) / kBlock, chunks = (s.N + kCwPoints - 1) / kCwPoints;
-    componentwise_fwd_kernel<T, D><<<dim3(unsigned(BL * m_tiles * chunks)), dim3(kBlock), 0, st>>>(
-        mixture, xes, out, s.L, s.M, s.N, s.Bx, s.Lx, m_tiles, chunks, cov);
+    const size_t per_mixture = size_t(m_tiles) * chunks, at_once = max_workgroups(kBlock) / per_mixture;
+    if (at_once == 0) return GMC_E_SHAPE;
+    for (size_t first = 0; first < BL; first += at_once)
+        componentwise_fwd_kernel<T, D><<<dim3(unsigned((BL - first < at_once ? BL - first : at_once) * per_mixture)), dim3(kBlock), 0, st>>>(
+            mixture, xes, out, s.L, s.M, s.N, s.Bx, s.Lx, m_tiles, int(first), chunks, cov);
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
 }
 
@@ -440,17 +444,23 @@ static int cw_backward_q(const T* grad_out, const T* mixture, const T* xes, T* g
         return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
     }
     zero2_async(sums, gm ? n_g * NR : 0, grad_xes, gx && shared_points ? n_x : 0, st);
-    const dim3 grid(unsigned(BL * m_groups * chunks));
+    // (as many mixtures a launch as its threads allow: more than one launch from 2^24 groups of Gaussians and points on)
+    const size_t per_mixture = size_t(m_groups) * chunks, at_once = max_workgroups(WAVES * kWave) / per_mixture;
+    if (at_once == 0) return GMC_E_SHAPE;
+    for (size_t first = 0; first < BL; first += at_once) {
+        const dim3 grid(unsigned((BL - first < at_once ? BL - first : at_once) * per_mixture));
 #define GMC_CW(GM, GX) componentwise_bwd_kernel<T, D, Q, WAVES, GM, GX><<<grid, dim3(WAVES * kWave), 0, st>>>( \
-        grad_out, mixture, xes, sums, grad_xes, s.L, s.M, s.N, s.Bx, s.Lx, m_groups, chunks, points_per_chunk, shared_points, wide, cov)
-    if constexpr (WAVES > 4) {
-        GMC_CW(true, true);
-    } else {
-        if (gm && gx) GMC_CW(true, true);
-        else if (gm) GMC_CW(true, false);
-        else if (gx) GMC_CW(false, true);
-    }
+            grad_out, mixture, xes, sums, grad_xes, s.L, s.M, s.N, s.Bx, s.Lx, m_groups, int(first), chunks, points_per_chunk, \
+            shared_points, wide, cov)
+        if constexpr (WAVES > 4) {
+            GMC_CW(true, true);
+        } else {
+            if (gm && gx) GMC_CW(true, true);
+            else if (gm) GMC_CW(true, false);
+            else if (gx) GMC_CW(false, true);
+        }
 #undef GMC_CW
+    }
     if (gm) launch_bwd_epilogue(mixture, sums, grad_mixture, n_g, D, s.dtype, cov, st);
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
 }
@@ -464,8 +474,11 @@ static int cw_backward_points(const T* grad_out, const T* mixture, const T* xes,
     const CwChunks c = cw_chunks(BL * m_groups, s.N, kCwWanted);
     const bool shared_points = m_groups > 1 || size_t(s.Bx) * s.Lx != BL;
     if (shared_points) zero_async(grad_xes, n_x, st);
-    componentwise_bwd_points_kernel<T, D><<<dim3(unsigned(BL * m_groups * c.chunks)), dim3(kBlock), 0, st>>>(
-        grad_out, mixture, xes, grad_xes, s.L, s.M, s.N, s.Bx, s.Lx, m_groups, c.chunks, c.points, shared_points, cov);
+    const size_t per_mixture = size_t(m_groups) * c.chunks, at_once = max_workgroups(kBlock) / per_mixture;
+    if (at_once == 0) return GMC_E_SHAPE;
+    for (size_t first = 0; first < BL; first += at_once)
+        componentwise_bwd_points_kernel<T, D><<<dim3(unsigned((BL - first < at_once ? BL - first : at_once) * per_mixture)), dim3(kBlock), 0, st>>>(
+            grad_out, mixture, xes, grad_xes, s.L, s.M, s.N, s.Bx, s.Lx, m_groups, int(first), c.chunks, c.points, shared_points, cov);
     return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
 }
 

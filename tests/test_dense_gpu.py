@@ -667,6 +667,29 @@ def test_componentwise_backward_edges(dtype, D):
                 assert rel_l2(gx_.cpu().numpy(), rgx.numpy(), FLOOR[dtype]) <= TOL[dtype], (B, L, M, N)
 
 
+def test_componentwise_launches_beyond_32_bit_thread_counts():
+    """more than the 2^32 threads of one launch (the runtime starts fewer without an error): the forward pass over 2^24 + 2^18
+    pieces of 64 points, the backward pass over as many groups of 64 Gaussians; every mixture is one of a few, so that the
+    results repeat"""
+    if torch.cuda.mem_get_info()[0] < 120 << 30:
+        pytest.skip("needs 120 GB of device memory")
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    k, M, B = 128, 129, 128 * 44544                                  # three groups of Gaussians per mixture
+    few = torch.randn(k, 1, M, 7, generator=gen, device=DEV)
+    few[..., 3:] = torch.tensor([2.0, 0.3, 0.3, 1.0], device=DEV)
+    x = torch.zeros(1, 1, 1, 2, device=DEV)
+    want = _native.eval_componentwise_bwd(torch.ones(k, 1, 1, M, device=DEV), few, x, True, False)[0]
+    got = _native.eval_componentwise_bwd(torch.ones(B, 1, 1, M, device=DEV), few.repeat(B // k, 1, 1, 1), x, True, False)[0]
+    for at in range(0, B // k, 4096):
+        part = got.view(B // k, k, 1, M, 7)[at:at + 4096]
+        assert torch.allclose(part, want.expand_as(part), rtol=1e-6, atol=1e-7), at
+    del got, part
+    B, N = 1 << 10, 65 * ((1 << 14) + (1 << 7))                      # 17.2e6 pieces of 64 points
+    out = _native.eval_componentwise_fwd(few[:8, :, :1].repeat(B // 8, 1, 1, 1), torch.zeros(1, 1, N, 2, device=DEV))
+    want = _native.eval_componentwise_fwd(few[:8, :, :1].contiguous(), x).view(1, 8, 1, 1, 1)
+    assert (out.view(B // 8, 8, 1, N, 1) == want).all()
+
+
 def test_float64_centre_gradients_round_like_the_formula():
     """the gradients of position and query point of single pairs in float64, bit for bit: with a diagonal matrix and the
     point so close to the centre that exp() is 1 every step is one rounding, so numpy gives the same bits -- as long as the
