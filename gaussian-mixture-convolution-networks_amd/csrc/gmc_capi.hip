@@ -26,7 +26,9 @@ int check_shape(const gmc_shape* s) {
     if (s->Lx != 1 && s->Lx != s->L) return GMC_E_SHAPE;
     // per-(b,l) index arithmetic inside the kernels is 32-bit
     if (size_t(s->M) * 13 > 0x7fffffffull || size_t(s->N) * 3 > 0x7fffffffull) return GMC_E_SHAPE;
-    if (size_t(s->B) * s->L > 0x7fffffffull / 64) return GMC_E_SHAPE;
+    // every mixture takes a workgroup of 256 threads, and a launch of 2^32 threads or more starts fewer without an error
+    // (mixtures are dealt to launches in multiples of 8)
+    if (size_t(s->B) * s->L > (size_t(1) << 24) - 8) return GMC_E_SHAPE;
     // launch grids: at most one workgroup per mixture, 64 points and 256 components (such tensors exceed the
     // memory of the device long before; the bound keeps the 32-bit grid sizes honest)
     const size_t groups = size_t(s->B) * s->L * (size_t(s->N) / 64 + 1);

@@ -18,6 +18,8 @@ GMC_F32, GMC_F64 = 0, 1
 GMC_AABB_REFERENCE, GMC_AABB_TIGHT = 0, 1
 ABI_VERSION = 12
 STATIC_SCRATCH_BYTES = 64 << 20
+MAX_MIXTURES = (1 << 24) - 8               # of a call: one workgroup each, 2^32 threads a launch
+MAX_COMPONENTS = 0x7FFFFFFF // 13           # of a mixture: 32-bit indices
 
 
 class Shape(ctypes.Structure):

@@ -57,12 +57,14 @@ class _ScaleWeights(torch.autograd.Function):
 
 
 def _scale_weights(x_gm: Tensor, scaling: Tensor) -> Tensor:
-    """x_gm with its weights times scaling [batch or 1, channels].  The kernels take plain device tensors; others (CPU
-    tensors, other types, subclasses, tracing, functorch and forward-mode transforms) go through torch operations."""
+    """x_gm with its weights times scaling [batch or 1, channels].  The kernels take plain device tensors of
+    sizes that a launch covers; others (CPU tensors, other types, subclasses, tracing, functorch and forward-mode
+    transforms) go through torch operations."""
     plain = not torch.compiler.is_compiling() and not torch.jit.is_tracing() and \
         _plain_device_tensors(x_gm, scaling) and scaling.device == x_gm.device and \
         x_gm.dtype in (torch.float32, torch.float64) and scaling.dtype == x_gm.dtype and \
         x_gm.dim() == 4 and x_gm.shape[-1] in (7, 13) and \
+        x_gm.shape[0] * x_gm.shape[1] <= _native.MAX_MIXTURES and x_gm.shape[2] <= _native.MAX_COMPONENTS and \
         not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0
     return _ScaleWeights.apply(x_gm, scaling) if plain else _scale_weights_composed(x_gm, scaling)
 

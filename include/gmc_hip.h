@@ -27,7 +27,8 @@ enum {
     GMC_OK = 0,
     GMC_E_DIMS = -1,       /* D not in {2,3} */
     GMC_E_DTYPE = -2,      /* dtype not GMC_F32 / GMC_F64 */
-    GMC_E_SHAPE = -3,      /* negative size, Bx not in {1,B}, Lx not in {1,L}, size beyond 2^31-1 elements per (b,l) */
+    GMC_E_SHAPE = -3,      /* negative size, Bx not in {1,B}, Lx not in {1,L}, size beyond 2^31-1 elements per (b,l),
+                              more than 2^24 - 8 mixtures */
     GMC_E_NULL = -4,       /* a required pointer is NULL */
     GMC_E_WORKSPACE = -5,  /* workspace smaller than the matching *_workspace_bytes() */
     GMC_E_LAUNCH = -6,     /* the HIP runtime refused a launch (hipGetLastError) */

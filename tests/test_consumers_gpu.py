@@ -495,6 +495,20 @@ def test_batch_norm_sampling_positions_for_few_and_many_centres(D, dtype):
         assert ((got - ref).abs() <= 4 * eps * (1.3 * (hi - lo) + lo.abs())).all(), (B, L, M, N)
 
 
+def test_batch_norm_of_more_mixtures_than_a_launch_covers():
+    """evaluation mode scales weights only: with more mixtures than the kernels take it goes through torch operations, and the
+    largest number they do take is covered by one launch; a larger call of the library is refused"""
+    for B in (_native.MAX_MIXTURES, _native.MAX_MIXTURES + 1, 17_000_000):
+        x = torch.ones(B, 1, 1, 7, device=DEV)
+        scale = torch.full((1, 1), 3.0, device=DEV)
+        assert (modules._scale_weights(x, scale)[:, 0, 0, 0] == 3.0).all(), B
+        if B > _native.MAX_MIXTURES:
+            with pytest.raises(RuntimeError):
+                _native.scale_weights(x, scale)
+            with pytest.raises(RuntimeError):
+                gm.evaluate(x, torch.zeros(1, 1, 1, 2, device=DEV))
+
+
 def test_batch_norm_batched_backward():
     """a batched backward pass through the layer (vectorised Jacobian rows) against the rows one by one; the statistics
     carry no gradient, so training and evaluation mode alike end in the scaling of the weights"""

@@ -45,6 +45,10 @@ def test_c_abi_rejects_bad_shapes_without_launching():
     assert lib.gmc_eval_fwd(null, null, null, ctypes.byref(S(1, 1, 2 ** 30, 5, 3, 1, 1, 0)), null) == -3
     assert lib.gmc_eval_fwd(null, null, null, ctypes.byref(S(4096, 4096, 4, 2 ** 20, 3, 1, 1, 0)), null) == -3
     assert lib.gmc_eval_bwd_workspace_bytes(ctypes.byref(S(1, 1, 2 ** 30, 5, 3, 1, 1, 0))) == 0
+    assert lib.gmc_eval_fwd(null, null, null, ctypes.byref(S(_native.MAX_MIXTURES, 1, 1, 1, 2, 1, 1, 0)), null) == -4
+    assert lib.gmc_eval_fwd(null, null, null, ctypes.byref(S(_native.MAX_MIXTURES + 1, 1, 1, 1, 2, 1, 1, 0)), null) == -3
+    assert lib.gmc_eval_fwd(null, null, null, ctypes.byref(S(1, 1, _native.MAX_COMPONENTS, 1, 2, 1, 1, 0)), null) == -4
+    assert lib.gmc_eval_fwd(null, null, null, ctypes.byref(S(1, 1, _native.MAX_COMPONENTS + 1, 1, 2, 1, 1, 0)), null) == -3
     assert lib.gmc_eval_fwd(null, null, null, ctypes.byref(ok), null) == -4
     assert lib.gmc_eval_fwd(null, null, null, None, null) == -4
     assert lib.gmc_eval_bwd(null, null, null, null, null, null, 0, ctypes.byref(ok), 1, 1, null) == -4
