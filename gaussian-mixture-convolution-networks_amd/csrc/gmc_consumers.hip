@@ -293,6 +293,7 @@ static int launch_consumer(const T* mixture, const T* points, size_t mixture_str
     }
     const int P = consumer_points_per_lane(N);
     const int chunks = consumer_chunks(N);
+    if (grid_mixtures(BL) * chunks > max_workgroups(kBlock)) return GMC_E_SHAPE;
     const dim3 grid(unsigned(grid_mixtures(BL) * chunks));
 #define GMC_CONS(PP) consumer_fwd_kernel<T, D, PP, KIND><<<grid, dim3(kBlock), 0, stream>>>(mixture, points, mixture_stride, point_stride, epi, L, M, N, chunks, int(BL))
     if (P == 2) GMC_CONS(2); else if (P == 4) GMC_CONS(4); else GMC_CONS(8);

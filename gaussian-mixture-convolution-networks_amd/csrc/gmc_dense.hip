@@ -884,6 +884,7 @@ static int launch_fwd(const T* mixture, const T* xes, T* out, const gmc_shape& s
     const FwdPlan plan = plan_fwd(s, sizeof(T) == 8);
     const int P = plan.P, chunks = plan.chunks;
     const TileSlices ts = plan.ts;
+    if (grid_mixtures(BL) * chunks * ts.slices > max_workgroups(kBlock)) return GMC_E_SHAPE;
     if (ts.slices > 1) zero_async(out, BL * s.N, stream);
     const dim3 grid(unsigned(grid_mixtures(BL) * chunks * ts.slices));
     {
@@ -1039,8 +1040,10 @@ static int launch_bwd(const T* grad_out, const T* mixture, const T* xes, T* grad
     const int gx_shared = (xes_shared || ts.slices > 1) ? 1 : 0;
     // one chunk per mixture: the pair kernel's workgroups finish the gradient of their mixture themselves
     const bool sole = need_gm && s.N <= 64 * P;
-    zero2_async(sums, need_gm && !sole ? n_gauss * Sums<D>::k : 0, grad_xes, need_gx && gx_shared ? n_x : 0, stream);
     const int per_group = need_gm && need_gx && s.Bx == 1 && s.Lx == 1 && BL > 1 ? plan_mixtures_per_group(model, P, BL, s.M, s.N, ts, sizeof(T) == 8) : 1;
+    if (grid_mixtures((BL + per_group - 1) / per_group) * ((size_t(s.N) + 64 * P - 1) / (64 * P)) * ts.slices > max_workgroups(kBlock))
+        return GMC_E_SHAPE;
+    zero2_async(sums, need_gm && !sole ? n_gauss * Sums<D>::k : 0, grad_xes, need_gx && gx_shared ? n_x : 0, stream);
     if (per_group > 1 && sole) launch_bwd_main<T, D, true, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream, per_group);
     else if (per_group > 1) launch_bwd_main<T, D, true, true, false, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream, per_group);
     else if (sole && need_gx) launch_bwd_main<T, D, true, true, true>(grad_out, mixture, xes, sums, grad_xes, grad_mixture, s, P, gx_shared, cov, ts, stream);

@@ -378,8 +378,8 @@ static void launch_fwd_variant(const float* mixture, const float* xes, float* ou
 // the machine with 512-component tiles and 1024-point blocks); false: the caller uses the all-vector kernel, which
 // is as fast or faster below that (measured: within +-10 % for 64..128 components).
 bool dense_forward_f32_takes(const gmc_shape& s) {
-    const size_t BL = size_t(s.B) * s.L;
-    return s.M > 128 && (BL * size_t((s.N + 1023) / 1024) >= 512 || s.N >= 8192);
+    const size_t blocks = size_t(s.B) * s.L * size_t((s.N + 1023) / 1024);
+    return s.M > 128 && (blocks >= 512 || s.N >= 8192) && blocks + 8 <= max_workgroups(512);
 }
 
 bool dense_forward_f32(const float* mixture, const float* xes, float* out, const gmc_shape& s, bool covariance_form,

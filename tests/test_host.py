@@ -54,6 +54,20 @@ def test_c_abi_rejects_bad_shapes_without_launching():
     assert lib.gmc_eval_bwd(null, null, null, null, null, null, 0, ctypes.byref(ok), 1, 1, null) == -4
 
 
+def test_launches_of_more_threads_than_one_can_have_are_refused():
+    """2^24 workgroups of 256 threads are the most a launch can be; the runtime starts fewer of a larger one without an error, so
+    that it must not come to the launch (the pointers are never followed here)"""
+    lib, S, p = _native.lib(), _native.Shape, ctypes.c_void_p(1 << 12)
+    for D, dtype in ((2, 0), (3, 0), (2, 1), (3, 1)):
+        for M in (1, 200):
+            big = S(1000000, 1, M, 40000, D, 1, 1, dtype)
+            assert lib.gmc_eval_fwd(p, p, p, ctypes.byref(big), None) == -3
+            assert lib.gmc_eval_bwd(p, p, p, p, p, p, 1 << 40, ctypes.byref(big), 1, 0, None) == -3
+            assert lib.gmc_eval_bwd(p, p, p, p, p, p, 1 << 40, ctypes.byref(big), 0, 1, None) == -3
+            own = S(1000000, 1, M, 40000, D, 1000000, 1, dtype)
+            assert lib.gmc_relu_fit_goal(p, p, p, p, ctypes.byref(own), None) == -3
+
+
 def test_scratch_sizes_and_knobs_without_a_device():
     """Host-only entry points: the scratch of the fused BatchNorm moments (three doubles per workgroup: 128 points per
     workgroup up to 128 points per mixture, 256 up to 256, then 512), the size of the opaque BVH object (grows with
