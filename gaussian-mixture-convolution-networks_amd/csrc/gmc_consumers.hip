@@ -27,24 +27,6 @@ template <typename T> struct EpiArgs {
     double* moments;       // [B L][chunks][3] count, mean, sum of squared deviations from that mean   kind 3
 };
 
-template <typename T, int D, int P, bool CENTRED>
-__device__ __forceinline__ void rc_pairs(const T* __restrict__ lds, const T* __restrict__ tab, int begin, int end, int row,
-                                         const T (&x)[P][D], T (&acc)[P]) {
-    constexpr int S = Rec<T, D>::kStride;
-#pragma unroll 2
-    for (int g = begin + row; g < end; g += 4) {
-        T r[Rec<T, D>::kUsed];
-#pragma unroll
-        for (int i = 0; i < Rec<T, D>::kUsed; ++i) r[i] = lds[g * S + i];
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            T y[D];
-            const T q = quad_form<T, D, CENTRED>(r, x[p], y);
-            acc[p] = fma_(r[Rec<T, D>::kAmp], pair_exp2(-q, tab), acc[p]);
-        }
-    }
-}
-
 // points: point n of mixture bl is read from points[bl * mixture_stride + n * point_stride + d] (query tensor
 // [B][L][N][D]: strides N D and D; the centres of a mixture [B][L][N][G]: pointer to its first position, strides N G
 // and G).  `mixture` holds covariances.
@@ -83,8 +65,8 @@ __global__ __launch_bounds__(kBlock) void consumer_fwd_kernel(const T* __restric
         const T* over = KIND == kEpiRatio ? epi.weights + size_t(bl) * M + g0 : nullptr;
         stage_tile<T, D, 4>(mix_bl + size_t(g0) * G, cnt, 1.0, lds, counts, true, over);
         const int centred_start = counts[8], padded_total = counts[9];
-        rc_pairs<T, D, P, false>(lds, exp2_tab, 0, centred_start, row, x, acc);
-        rc_pairs<T, D, P, true>(lds, exp2_tab, centred_start, padded_total, row, x, acc);
+        add_pairs<T, D, P, 4, false>(lds, exp2_tab, row, centred_start, x, acc);
+        add_pairs<T, D, P, 4, true>(lds, exp2_tab, centred_start + row, padded_total, x, acc);
     }
     double vals[P];                                  // kind 3: this lane's values (rows other than 0 and points beyond N: none)
     double s1 = 0.0;
@@ -190,8 +172,8 @@ __global__ __launch_bounds__(kBlock) void few_points_fwd_kernel(const T* __restr
         const int m = active ? g0 + lane : g0;
         const Derived<D> dv = derive<T, D>(mix_bl + size_t(m) * G, covariance_form);
         const WaveTile t = stage_wave_tile<T, D, 4>(dv, active, 1.0, tile, lane);
-        rc_pairs<T, D, P, false>(tile, exp2_tab, 0, t.centred_start, row, x, acc);
-        rc_pairs<T, D, P, true>(tile, exp2_tab, t.centred_start, t.padded_total, row, x, acc);
+        add_pairs<T, D, P, 4, false>(tile, exp2_tab, row, t.centred_start, x, acc);
+        add_pairs<T, D, P, 4, true>(tile, exp2_tab, t.centred_start + row, t.padded_total, x, acc);
     }
     wave_fence();
 #pragma unroll

@@ -39,24 +39,6 @@ void few_points_forward(const void* mixture, const void* xes, void* out, const g
 
 constexpr int kTile = 256;   // Gaussians staged per LDS tile (one per lane)
 
-template <typename T, int D, int P, bool CENTRED>
-__device__ __forceinline__ void fwd_pairs(const T* __restrict__ lds, const T* __restrict__ tab, int begin, int end,
-                                          const T (&x)[P][D], T (&acc)[P]) {
-    constexpr int S = Rec<T, D>::kStride;
-#pragma unroll 2
-    for (int g = begin; g < end; ++g) {
-        T r[Rec<T, D>::kUsed];
-#pragma unroll
-        for (int i = 0; i < Rec<T, D>::kUsed; ++i) r[i] = lds[g * S + i];
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            T y[D];
-            const T q = quad_form<T, D, CENTRED>(r, x[p], y);
-            acc[p] = fma_(r[Rec<T, D>::kAmp], pair_exp2(-q, tab), acc[p]);
-        }
-    }
-}
-
 template <typename T, int D, int P>
 __global__ __launch_bounds__(kBlock) void eval_fwd_kernel(const T* __restrict__ mixture, const T* __restrict__ xes,
                                                           T* __restrict__ out, int L, int M, int N, int Bx, int Lx,
@@ -96,8 +78,8 @@ __global__ __launch_bounds__(kBlock) void eval_fwd_kernel(const T* __restrict__ 
         const int cnt = (g_end - g0) < kTile ? (g_end - g0) : kTile;
         stage_tile<T, D>(mix_bl + size_t(g0) * G, cnt, 1.0, lds, counts, covariance_form);
         const int n_shifted = counts[8];
-        fwd_pairs<T, D, P, false>(lds, exp2_tab, 0, n_shifted, x, acc);
-        fwd_pairs<T, D, P, true>(lds, exp2_tab, n_shifted, cnt, x, acc);
+        add_pairs<T, D, P, 1, false>(lds, exp2_tab, 0, n_shifted, x, acc);
+        add_pairs<T, D, P, 1, true>(lds, exp2_tab, n_shifted, cnt, x, acc);
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
@@ -112,24 +94,6 @@ __global__ __launch_bounds__(kBlock) void eval_fwd_kernel(const T* __restrict__ 
 // Gaussian 4k + r in step k, column c on the points {c, c + 16, ...} of the wavefront's 16 P points): a workgroup
 // covers 64 P points for any P from 2 to 16, where the kernel above covers 256 P with P a power of two.  Used when
 // that pads the last chunk less (784 points: 832 instead of 1024).
-template <typename T, int D, int P, bool CENTRED>
-__device__ __forceinline__ void fwd_rc_pairs(const T* __restrict__ lds, const T* __restrict__ tab, int begin, int end,
-                                             int row, const T (&x)[P][D], T (&acc)[P]) {
-    constexpr int S = Rec<T, D>::kStride;
-#pragma unroll 2
-    for (int g = begin + row; g < end; g += 4) {
-        T r[Rec<T, D>::kUsed];
-#pragma unroll
-        for (int i = 0; i < Rec<T, D>::kUsed; ++i) r[i] = lds[g * S + i];
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            T y[D];
-            const T q = quad_form<T, D, CENTRED>(r, x[p], y);
-            acc[p] = fma_(r[Rec<T, D>::kAmp], pair_exp2(-q, tab), acc[p]);
-        }
-    }
-}
-
 template <typename T, int D, int P>
 __global__ __launch_bounds__(kBlock) void eval_fwd_rc_kernel(const T* __restrict__ mixture, const T* __restrict__ xes,
                                                              T* __restrict__ out, int L, int M, int N, int Bx, int Lx,
@@ -170,8 +134,8 @@ __global__ __launch_bounds__(kBlock) void eval_fwd_rc_kernel(const T* __restrict
         const int cnt = (g_end - g0) < kTile ? (g_end - g0) : kTile;
         stage_tile<T, D, 4>(mix_bl + size_t(g0) * G, cnt, 1.0, lds, counts, covariance_form);
         const int centred_start = counts[8], padded_total = counts[9];
-        fwd_rc_pairs<T, D, P, false>(lds, exp2_tab, 0, centred_start, row, x, acc);
-        fwd_rc_pairs<T, D, P, true>(lds, exp2_tab, centred_start, padded_total, row, x, acc);
+        add_pairs<T, D, P, 4, false>(lds, exp2_tab, row, centred_start, x, acc);
+        add_pairs<T, D, P, 4, true>(lds, exp2_tab, centred_start + row, padded_total, x, acc);
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
@@ -199,6 +163,9 @@ __device__ __forceinline__ void bwd_rc_pairs(const T* __restrict__ lds, const T*
                                              const T (&go)[P], T (&gx)[P][D]) {
     constexpr int S = Rec<T, D>::kStride;
     constexpr int NR = Sums<D>::k;
+    // Points whose exponentials are issued together (float; double has no such instruction).  3-D, both gradients, 2048 x 512
+    // Gaussians at 8192 points: two 5290, three 5240, four 5244, five 5267, six 5650 us (spilled registers).
+    constexpr int kBatch = sizeof(T) == 8 ? 1 : P < 3 ? P : 3;
     for (int g = begin + row; g < end; g += 4) {
         T r[Rec<T, D>::kUsed];
 #pragma unroll
@@ -218,82 +185,97 @@ __device__ __forceinline__ void bwd_rc_pairs(const T* __restrict__ lds, const T*
             for (int i = 0; i < Rec<T, D>::kU; ++i) ua[i] = r[Rec<T, D>::kAmp] * r[i];
         }
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            T y[D];
-            const T q = quad_form<T, D, CENTRED>(r, x[p], y);
-            const T e = pair_exp2(-q, tab);
-            const T k = NEED_GM ? e * go[p] : e;
-            T ky[D];
+        for (int p0 = 0; p0 < P; p0 += kBatch) {
+            T ys[kBatch][D], q[kBatch], e[kBatch];
 #pragma unroll
-            for (int d = 0; d < D; ++d) ky[d] = k * y[d];
-            if (NEED_GX) {
-                if constexpr (D == 2) {
-                    gx[p][0] = fma_(ua[0], ky[0], gx[p][0]);
-                    gx[p][1] = fma_(ua[1], ky[0], fma_(ua[2], ky[1], gx[p][1]));
-                } else {
-                    gx[p][0] = fma_(ua[0], ky[0], gx[p][0]);
-                    gx[p][1] = fma_(ua[1], ky[0], fma_(ua[3], ky[1], gx[p][1]));
-                    gx[p][2] = fma_(ua[2], ky[0], fma_(ua[4], ky[1], fma_(ua[5], ky[2], gx[p][2])));
+            for (int i = 0; i < kBatch; ++i)
+                if (p0 + i < P) q[i] = quad_form<T, D, CENTRED>(r, x[p0 + i], ys[i]);
+            if constexpr (sizeof(T) == 4) pair_exp2_batch(q, e, P - p0); else e[0] = pair_exp2(-q[0], tab);
+#pragma unroll
+            for (int i = 0; i < kBatch; ++i) {
+                const int p = p0 + i;
+                if (p >= P) break;
+                const T (&y)[D] = ys[i];
+                const T k = NEED_GM ? e[i] * go[p] : e[i];
+                T ky[D];
+#pragma unroll
+                for (int d = 0; d < D; ++d) ky[d] = k * y[d];
+                if (NEED_GX) {
+                    if constexpr (D == 2) {
+                        gx[p][0] = fma_(ua[0], ky[0], gx[p][0]);
+                        gx[p][1] = fma_(ua[1], ky[0], fma_(ua[2], ky[1], gx[p][1]));
+                    } else {
+                        gx[p][0] = fma_(ua[0], ky[0], gx[p][0]);
+                        gx[p][1] = fma_(ua[1], ky[0], fma_(ua[3], ky[1], gx[p][1]));
+                        gx[p][2] = fma_(ua[2], ky[0], fma_(ua[4], ky[1], fma_(ua[5], ky[2], gx[p][2])));
+                    }
+                    if (NEED_GM) {
+                        // keeps these additions here: left alone they sink behind the branch of the row reduction below
+                        // (their results are not needed before the next step) and the products k*y of all P points stay
+                        // in registers until then
+#pragma unroll
+                        for (int d = 0; d < D; ++d) asm volatile("" : "+v"(gx[p][d]));
+                    }
                 }
                 if (NEED_GM) {
-                    // keeps these additions here: left alone they sink behind the branch of the row reduction below
-                    // (their results are not needed before the next step) and the products k*y of all P points stay
-                    // in registers until then
+                    if (p == 0) {
+                        // the first point starts the sums (no zero fill, no additions)
+                        rs[0] = k;
 #pragma unroll
-                    for (int d = 0; d < D; ++d) asm volatile("" : "+v"(gx[p][d]));
-                }
-            }
-            if (NEED_GM) {
-                if (p == 0) {
-                    // the first point starts the sums (no zero fill, no additions)
-                    rs[0] = k;
+                        for (int d = 0; d < D; ++d) rs[1 + d] = ky[d];
+                        int at = 1 + D;
 #pragma unroll
-                    for (int d = 0; d < D; ++d) rs[1 + d] = ky[d];
-                    int at = 1 + D;
+                        for (int a = 0; a < D; ++a)
 #pragma unroll
-                    for (int a = 0; a < D; ++a)
-#pragma unroll
-                        for (int c = a; c < D; ++c) rs[at++] = ky[a] * y[c];
-                } else {
-                    rs[0] += k;
-                    if constexpr (D == 2) {
-                        rs[1] += ky[0]; rs[2] += ky[1];
-                        rs[3] = fma_(ky[0], y[0], rs[3]); rs[4] = fma_(ky[0], y[1], rs[4]); rs[5] = fma_(ky[1], y[1], rs[5]);
+                            for (int c = a; c < D; ++c) rs[at++] = ky[a] * y[c];
                     } else {
-                        rs[1] += ky[0]; rs[2] += ky[1]; rs[3] += ky[2];
-                        rs[4] = fma_(ky[0], y[0], rs[4]); rs[5] = fma_(ky[0], y[1], rs[5]); rs[6] = fma_(ky[0], y[2], rs[6]);
-                        rs[7] = fma_(ky[1], y[1], rs[7]); rs[8] = fma_(ky[1], y[2], rs[8]); rs[9] = fma_(ky[2], y[2], rs[9]);
+                        rs[0] += k;
+                        if constexpr (D == 2) {
+                            rs[1] += ky[0]; rs[2] += ky[1];
+                            rs[3] = fma_(ky[0], y[0], rs[3]); rs[4] = fma_(ky[0], y[1], rs[4]); rs[5] = fma_(ky[1], y[1], rs[5]);
+                        } else {
+                            rs[1] += ky[0]; rs[2] += ky[1]; rs[3] += ky[2];
+                            rs[4] = fma_(ky[0], y[0], rs[4]); rs[5] = fma_(ky[0], y[1], rs[5]); rs[6] = fma_(ky[0], y[2], rs[6]);
+                            rs[7] = fma_(ky[1], y[1], rs[7]); rs[8] = fma_(ky[1], y[2], rs[8]); rs[9] = fma_(ky[2], y[2], rs[9]);
+                        }
                     }
                 }
             }
         }
         if (NEED_GM) {
-            // Row reduction of the NR sums, two at a time: the two halves of a row first exchange the sum they do not
-            // keep (lanes 0-7 keep the even one, lanes 8-15 the odd one), then three shifts are left; the totals
-            // arrive in lanes 7 and 15.  4 instructions per sum instead of 5 and half as many LDS atomics.
-            static_assert(NR % 2 == 0, "the sums are reduced in pairs");
-            const bool high = (threadIdx.x & 8) != 0;
-            T half[NR / 2];
+            if constexpr (sizeof(T) == 4) {
+                slow_issue_begin(rs);
+                float total[1] = {row_sums(rs, threadIdx.x)};
+                slow_issue_end(total);
+                const int k = row_sums_index<NR>(threadIdx.x & 15);
+                if (idx >= 0 && k >= 0) {
+                    // float: every wavefront meets every Gaussian of a tile once and has its own copy of the sums, so a
+                    // plain store does (LDS float atomics are serialised lane by lane); double: one copy
+                    if constexpr (OWN_SUMS) block_sums[idx * NR + k] = total[0]; else atomic_add(&block_sums[idx * NR + k], total[0]);
+                }
+            } else {
+                // two sums at a time: the halves of a row first exchange the sum they do not keep (lanes 0-7 keep the even
+                // one, lanes 8-15 the odd one), then three shifts are left; the totals arrive in lanes 7 and 15
+                static_assert(NR % 2 == 0, "the sums are reduced in pairs");
+                const bool high = (threadIdx.x & 8) != 0;
+                T half[NR / 2];
 #pragma unroll
-            for (int i = 0; i < NR / 2; ++i) {
-                const T keep = high ? rs[2 * i + 1] : rs[2 * i], send = high ? rs[2 * i] : rs[2 * i + 1];
-                T v = keep + dpp_mov<0x128>(send);          // row_ror:8
-                v += dpp_mov<0x111>(v);                     // row_shr:1
-                v += dpp_mov<0x112>(v);                     // row_shr:2
-                v += dpp_mov<0x114>(v);                     // row_shr:4 -> lanes 7 and 15 hold the sums of lanes 0-7, 8-15
-                // keeps the last addition in front of the branch below, where it stays one DPP instruction (sunk
-                // into the branch it becomes a zero fill, a DPP move and an addition)
-                asm volatile("" : "+v"(v));
-                half[i] = v;
-            }
-            if ((threadIdx.x & 7) == 7) {
-                if (idx >= 0) {
-                    T* dst = block_sums + idx * NR + (high ? NR / 2 : 0);
+                for (int i = 0; i < NR / 2; ++i) {
+                    const T keep = high ? rs[2 * i + 1] : rs[2 * i], send = high ? rs[2 * i] : rs[2 * i + 1];
+                    T v = keep + dpp_mov<0x128>(send);          // row_ror:8
+                    v += dpp_mov<0x111>(v);                     // row_shr:1
+                    v += dpp_mov<0x112>(v);                     // row_shr:2
+                    v += dpp_mov<0x114>(v);                     // row_shr:4 -> lanes 7 and 15 hold the sums of lanes 0-7, 8-15
+                    // keeps the last addition in front of the branch below, where it stays one DPP instruction (sunk
+                    // into the branch it becomes a zero fill, a DPP move and an addition)
+                    asm volatile("" : "+v"(v));
+                    half[i] = v;
+                }
+                if ((threadIdx.x & 7) == 7 && idx >= 0) {
+                    T* dst = block_sums + idx * NR + (high ? 1 : 0);
 #pragma unroll
                     for (int i = 0; i < NR / 2; ++i) {
-                        // float: every wavefront meets every Gaussian of a tile once and has its own copy of the sums,
-                        // so a plain store does (LDS float atomics are serialised lane by lane); double: one copy
-                        if constexpr (OWN_SUMS) dst[i] = half[i]; else atomic_add(&dst[i], half[i]);
+                        if constexpr (OWN_SUMS) dst[2 * i] = half[i]; else atomic_add(&dst[2 * i], half[i]);
                     }
                 }
             }
@@ -396,14 +378,11 @@ void eval_bwd_rc_kernel(const T* __restrict__ grad_out, const T* __restrict__ mi
                 __syncthreads();
                 T* __restrict__ dst = sums + (size_t(bl) * M + g0) * NR;
                 for (int i = threadIdx.x; i < cnt * NR; i += kBlock) {
-                    // entry i holds sum k of Gaussian j at [j][k / 2 + (k odd ? NR / 2 : 0)] of every wavefront's copy
-                    const int j = i / NR, k = i - j * NR;
-                    const int at = j * NR + (k >> 1) + ((k & 1) ? NR / 2 : 0);
-                    T v = block_sums[at];
+                    T v = block_sums[i];
                     if constexpr (SumCopies<T>::k > 1) {
-                        v = (v + block_sums[kTile * NR + at]) + (block_sums[2 * kTile * NR + at] + block_sums[3 * kTile * NR + at]);
+                        v = (v + block_sums[kTile * NR + i]) + (block_sums[2 * kTile * NR + i] + block_sums[3 * kTile * NR + i]);
                     } else {
-                        block_sums[at] = T(0);
+                        block_sums[i] = T(0);
                     }
                     if (SOLE) dst[i] = v; else atomic_add(&dst[i], v);
                 }
@@ -658,7 +637,7 @@ __global__ __launch_bounds__(kBlock) void few_points_bwd_kernel(const T* __restr
         if (active) {
             T rs[NR];
 #pragma unroll
-            for (int k = 0; k < NR; ++k) rs[k] = wave_sums[lane * NR + (k >> 1) + ((k & 1) ? NR / 2 : 0)];
+            for (int k = 0; k < NR; ++k) rs[k] = wave_sums[lane * NR + k];
             bwd_epilogue_derived<T, D>(dv, c, rs, grad_mixture + at * G, covariance_form);
         }
     }

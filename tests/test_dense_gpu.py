@@ -823,3 +823,19 @@ def test_c4_full_size_properties():
     assert _native.lib().gmc_export_launch_clocks(mhz) == 0
     assert 800.0 < mhz[0] < 3500.0 and 800.0 < mhz[1] < 3500.0, (mhz[0], mhz[1])
     assert _native.lib().gmc_export_launch_clocks(None) != 0
+
+
+@pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("points", range(2, 17))
+def test_batched_exponentials_at_every_points_per_lane(D, points):
+    """the pair loops issue the exponentials of several pairs together: of three points in the backward pass, of all points
+    of a lane and, with three to five points, of two Gaussians in the forward pass; every number of points per lane has its
+    remainder, and 1 ... 9 Gaussians leave one for some rows of a wavefront and none for others"""
+    lib = _native.lib()
+    lib.gmc_set_tuning(points, points)
+    try:
+        for M in (1, 4, 5, 7, 9):
+            mix, xes, gout = _case(2, 3, M, 64 * points + 5, D, 7000 + 100 * points + 10 * D + M, False)
+            _check(mix, xes, gout, torch.float32, tag=f"{points} points per lane, {M} components, {D}-D")
+    finally:
+        lib.gmc_set_tuning(0, 0)
