@@ -1578,22 +1578,28 @@ __device__ __forceinline__ T exp_neg_half(T q, const T* __restrict__ tab) {
     return pair_exp2(q * T(-0.72134752044448170368), tab);
 }
 
-// e = exp(-1/2 t^T C t), u = C t for the leaf record r
+// t^T C t, t = x - b and u = C t for the leaf record r
 template <typename T, int D>
-__device__ __forceinline__ T leaf_terms(const T* __restrict__ r, const T* __restrict__ tab, const T (&x)[D], T (&t)[D],
-                                        T (&u)[D]) {
+__device__ __forceinline__ T leaf_exponent(const T* __restrict__ r, const T (&x)[D], T (&t)[D], T (&u)[D]) {
     if constexpr (D == 2) {
         t[0] = x[0] - r[0]; t[1] = x[1] - r[1];
         u[0] = fma_(r[2], t[0], r[3] * t[1]);
         u[1] = fma_(r[3], t[0], r[4] * t[1]);
-        return exp_neg_half(fma_(t[0], u[0], t[1] * u[1]), tab);
+        return fma_(t[0], u[0], t[1] * u[1]);
     } else {
         t[0] = x[0] - r[0]; t[1] = x[1] - r[1]; t[2] = x[2] - r[2];
         u[0] = fma_(r[3], t[0], fma_(r[4], t[1], r[5] * t[2]));
         u[1] = fma_(r[4], t[0], fma_(r[6], t[1], r[7] * t[2]));
         u[2] = fma_(r[5], t[0], fma_(r[7], t[1], r[8] * t[2]));
-        return exp_neg_half(fma_(t[0], u[0], fma_(t[1], u[1], t[2] * u[2])), tab);
+        return fma_(t[0], u[0], fma_(t[1], u[1], t[2] * u[2]));
     }
+}
+
+// the same with e = exp(-1/2 t^T C t) as the result
+template <typename T, int D>
+__device__ __forceinline__ T leaf_terms(const T* __restrict__ r, const T* __restrict__ tab, const T (&x)[D], T (&t)[D],
+                                        T (&u)[D]) {
+    return exp_neg_half(leaf_exponent<T, D>(r, x, t, u), tab);
 }
 
 template <int D> struct BvhSums { static constexpr int k = 1 + D + D * (D + 1) / 2; };
@@ -1711,7 +1717,7 @@ __device__ __forceinline__ void group_boxes(const T (&x)[D], bool valid, int lan
 //   Overlapping internal children go back on the stack, overlapping leaves into the group's candidate list (ballot
 //   + prefix-popcount compaction).  The descents of the groups are independent chains of memory round trips (about
 //   one per tree level) and run side by side.
-//   Phase 2 (all wavefronts, group after group, lanes = points): the candidates of a group are dealt to the
+//   Phase 2 (all wavefronts, group after group, lanes = points; see MODE 1 below): the candidates of a group are dealt to the
 //   wavefronts; each stages kStageBatch of its candidates (own box + evaluation record, one contiguous leaf
 //   record) in LDS, the records of the next batch being fetched while the current one is worked on, tests every
 //   lane's point against all staged boxes (closed interval, lbvh/aabb.h:39-47; the lane keeps a bit mask of the
@@ -1720,12 +1726,15 @@ __device__ __forceinline__ void group_boxes(const T (&x)[D], bool valid, int lan
 //   wavefronts are added in wavefront order (deterministic).
 // Phase 1 only filters, phase 2 applies the per-point rule of lbvh/query.h:13-66, so the result is the sum over the
 // Gaussians whose own box contains the point.
-// MODE 0: forward.  MODE 1: backward (grad_out given): dL/dx stays in the lanes' registers.  The per-Gaussian sums
-// of a batch are collected in a per-wavefront LDS copy and flushed with one global atomic per non-zero scalar:
-// a leaf that contains many of the points is evaluated by all lanes at once and its sums are reduced over the
-// wavefront (DPP); the remaining hits go through the lane-by-lane loop and are added with LDS atomics (a few
-// cycles per instruction when the lanes of an instruction address different leaves, hence the lanes start at
-// different leaves of the batch).
+// MODE 0: forward.  MODE 1: backward (grad_out given).  dL/dx alone runs as the forward pass does.  With the gradient of the
+// mixture phase 2 turns round (evaluate_by_leaves, lanes = leaves): a lane keeps a candidate leaf and its ten sums in
+// registers and walks over the points, so a leaf's sums are reduced over four lanes once per 64 points instead of over
+// the wavefront or, hit by hit, with ten LDS atomics; about a quarter of the pairs of a candidate lie inside its box, and the
+// others are multiplied by zero.  Measured, backward pass, lanes = points with reductions and LDS atomics / lanes = leaves:
+//   63 trees of 500 leaves, 4001 points each, float32 165 / 118 us;  one tree of 16384, 100000 points, float64 75 / 62,
+//   float32 67 / 48;  800 trees of 128 at 784 points, 2-D float32 138 / 106;  25 trees of 200 at 2000, float64 42 / 38
+// Bound by vector issue (float32: 37 instructions and a row sum of six per four points and 16 leaves) and the fixed 5 us of a
+// workgroup.
 template <typename T, int D, int MODE, bool NEED_GM, bool NEED_GX>
 __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4))) void bvh_traverse_kernel(
         const T* __restrict__ xes, const int* __restrict__ p_order, const T* __restrict__ child_box,
@@ -1741,7 +1750,11 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     __shared__ int leaves[kGroupsMax][kLeafCap];
     __shared__ int state[kGroupsMax][2];                    // [0] candidates gathered, [1] nodes left on the stack
     __shared__ int pids[kGroupsMax][kWave];                 // index of every point, -1 beyond the end
-    __shared__ T pts[kGroupsMax][D + 1][kWave];             // coordinates and upstream gradient of every point
+    // coordinates and upstream gradient of every point: one array per component, or, for the pass that evaluates by leaves,
+    // one record per point.  (There, where a point outside the box is multiplied by zero, points beyond the end and points with
+    // infinite or NaN coordinates, which no box contains, lie far away at finite coordinates and have no upstream gradient.)
+    __shared__ __attribute__((aligned(16))) T pts[kGroupsMax][4 * kWave];
+    constexpr int kPointStep = NEED_GM ? 4 : 1, kComponentStep = NEED_GM ? 1 : kWave;
     __shared__ float gbox[kGroupsMax][4 * D];               // two boxes (lower, upper; rounded outwards) around every group's points
     // results per point, in double: the forward sums are added wavefront by wavefront (deterministic), dL/dx with
     // LDS atomics (cheap for doubles on distinct words, unlike floats)
@@ -1752,9 +1765,6 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     // groups of the round are through (one barrier per round; with a barrier pair per group the workgroup waited for
     // its slowest wavefront once per group)
     __shared__ T partial[MODE == 0 ? kGroupsMax : 1][MODE == 0 ? kTravWaves : 1][kWave];
-    // double in both precisions: LDS atomic adds of doubles on distinct addresses cost a few cycles per
-    // instruction, those of floats are serialised lane by lane
-    __shared__ double rsum_mem[kTravWaves][NEED_GM ? kStageBatch * NR : 1];
     __shared__ int2 pend[kGroupsMax][kPendMax];             // pieces of a group's list that wait to be published
     __shared__ int piece_valid;                             // helper workgroups: the piece still describes the group's points
     const T* exp2_tab = exp2_table<T>();                    // (published by the barrier in front of the first evaluation)
@@ -1781,7 +1791,6 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     const size_t xseg = size_t(xb) * Lx + xl;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     T* staged = staged_mem[wave];
-    double* rsum = rsum_mem[wave];
     const unsigned long long below = (1ull << lane) - 1ull;
 
     // wavefront i loads the points of group i and their bounding box
@@ -1835,9 +1844,12 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
         for (int d = 0; d < D; ++d) x[d] = xes[(xseg * N + pid) * D + d];
         T g = T(0);
         if (MODE == 1) g = valid ? grad_out[size_t(bl) * N + pid] : T(0);
+        bool near = valid;
 #pragma unroll
-        for (int d = 0; d < D; ++d) pts[wave][d][lane] = x[d];
-        pts[wave][D][lane] = g;
+        for (int d = 0; d < D; ++d) near = near & (x[d] - x[d] == T(0));
+#pragma unroll
+        for (int d = 0; d < D; ++d) pts[wave][lane * kPointStep + d * kComponentStep] = NEED_GM && !near ? T(1e18) : x[d];
+        pts[wave][lane * kPointStep + D * kComponentStep] = NEED_GM && !near ? T(0) : g;
         pids[wave][lane] = valid ? pid : -1;
         if (cache.count) my_stamp = points_stamp<T, D>(x, valid, lane);
         const bool any = group * kWave < N;
@@ -1907,12 +1919,21 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     // Phase 2 walks this wavefront's batches of the round, group after group, with a wave-uniform cursor; the
     // leaf records of the NEXT batch (possibly of the next group) are fetched into registers before the current
     // batch is tested and evaluated, so their memory round trip overlaps that work and the group's barriers.
-    constexpr int kPre = (kStageBatch * LS + kWave - 1) / kWave;
-    constexpr int kDenseHits = sizeof(T) == 8 ? 16 : 6;    // lanes per leaf from which the reduction is cheaper
+    constexpr int kBatch = NEED_GM ? 16 : kStageBatch;
+    constexpr int kPre = (kBatch * LS + kWave - 1) / kWave;
     int cur_group = -1, cur_base = 0, cur_end = 0;
     T pre[kPre];
     auto next_batch = [&]() {
-        cur_base += kStageBatch;
+        if constexpr (NEED_GM) {
+            // the batches of all groups, numbered through, are dealt to the wavefronts in turn
+            cur_base += kTravWaves * kBatch;
+            while (cur_base >= cur_end && cur_group < groups) {
+                cur_base -= (cur_end + kBatch - 1) / kBatch * kBatch;
+                if (++cur_group < groups) cur_end = __builtin_amdgcn_readfirstlane(state[cur_group][0]);
+            }
+            return;
+        }
+        cur_base += kBatch;
         while (cur_base >= cur_end && cur_group < groups) {
             ++cur_group;
             if (cur_group >= groups) break;
@@ -1924,7 +1945,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     };
     auto prefetch = [&]() {
         if (cur_group >= groups) return;
-        const int cnt = cur_end - cur_base < kStageBatch ? cur_end - cur_base : kStageBatch;
+        const int cnt = cur_end - cur_base < kBatch ? cur_end - cur_base : kBatch;
 #pragma unroll
         for (int r = 0; r < kPre; ++r) {
             const int s = lane + r * kWave;
@@ -1938,15 +1959,12 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     auto evaluate_share = [&](int gi) {
         T x[D];
 #pragma unroll
-        for (int d = 0; d < D; ++d) x[d] = pts[gi][d][lane];
-        const T g = pts[gi][D][lane];
+        for (int d = 0; d < D; ++d) x[d] = pts[gi][lane * kPointStep + d * kComponentStep];
         const bool valid = pids[gi][lane] >= 0;
         T acc = T(0);
         T gx[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) gx[d] = T(0);
-        // lanes start at different leaves of a batch, so that LDS atomics of one instruction spread over the leaves
-        const int rot = NEED_GM ? lane % kStageBatch : 0;
         while (cur_group == gi) {
             const int cnt = cur_end - cur_base < kStageBatch ? cur_end - cur_base : kStageBatch;
 #pragma unroll
@@ -1954,8 +1972,6 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
                 const int s = lane + r * kWave;
                 if (s < cnt * LS) staged[s] = pre[r];
             }
-            if (NEED_GM)
-                for (int s = lane; s < cnt * NR; s += kWave) rsum[s] = 0.0;
             wave_lds_fence();
             next_batch();
             prefetch();
@@ -1971,50 +1987,9 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
                 for (int q = 0; q < 2; ++q) mask |= (valid & inside_box<T, D>(x, box[q])) ? (1u << (i0 + q)) : 0u;
             }
             mask &= (1u << cnt) - 1u;                   // slots beyond the batch hold stale records
-            if (NEED_GM) {
-                // Leaves that contain many of the points: every lane evaluates the same leaf, the sums are
-                // reduced over the wavefront and lane 63 alone adds them to the LDS copy.  (LDS atomics serialise
-                // the lanes that add to the same address; a reduction costs the same however many lanes hit.)
-                for (int i = 0; i < cnt; ++i) {
-                    const bool has = (mask >> i) & 1u;
-                    if (__popcll(__ballot(has)) < kDenseHits) continue;
-                    mask &= ~(1u << i);
-                    const T* lf = staged + i * LS + 2 * D;
-                    T r[kAmp - 2 * D + 1];
-#pragma unroll
-                    for (int k = 0; k < kAmp - 2 * D + 1; ++k) r[k] = lf[k];
-                    T t[D], u[D];
-                    const T e = leaf_terms<T, D>(r, exp2_tab, x, t, u);
-                    if (NEED_GX) {
-                        const T s = has ? r[kAmp - 2 * D] * e : T(0);
-#pragma unroll
-                        for (int d = 0; d < D; ++d) gx[d] = fma_(s, u[d], gx[d]);
-                    }
-                    T rs[NR];
-                    rs[0] = has ? e * g : T(0);
-#pragma unroll
-                    for (int d = 0; d < D; ++d) rs[1 + d] = rs[0] * t[d];
-                    int k = 1 + D;
-#pragma unroll
-                    for (int a = 0; a < D; ++a)
-#pragma unroll
-                        for (int c = a; c < D; ++c) rs[k++] = rs[1 + a] * t[c];
-                    // four sums at a time; the lane at the end of row r receives sum {0, 2, 1, 3}[r] of the four
-                    const int row = lane >> 4, mine = ((row & 1) << 1) | (row >> 1);
-#pragma unroll
-                    for (int q0 = 0; q0 < NR; q0 += 4) {
-                        const T total = wave_sum4_to_row_ends(rs[q0], q0 + 1 < NR ? rs[q0 + 1] : T(0),
-                                                              q0 + 2 < NR ? rs[q0 + 2] : T(0),
-                                                              q0 + 3 < NR ? rs[q0 + 3] : T(0), lane);
-                        if ((lane & 15) == 15 && q0 + mine < NR) rsum[i * NR + q0 + mine] += double(total);
-                    }
-                }
-                mask = ((mask >> rot) | (mask << (kStageBatch - rot))) & ((1u << kStageBatch) - 1u);
-            }
             while (__ballot(mask != 0u) != 0ull) {
                 const bool has = mask != 0u;
-                int i = has ? __builtin_ctz(mask) + rot : 0;
-                i = i >= kStageBatch ? i - kStageBatch : i;
+                const int i = has ? __builtin_ctz(mask) : 0;
                 mask &= mask - 1u;
                 const T* lf = staged + i * LS + 2 * D;
                 T r[kAmp - 2 * D + 1];
@@ -2026,35 +2001,9 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
                 if (MODE == 0) {
                     acc += has ? amp * e : T(0);
                 } else {
-                    if (NEED_GX) {
-                        const T s = has ? amp * e : T(0);
+                    const T s = has ? amp * e : T(0);
 #pragma unroll
-                        for (int d = 0; d < D; ++d) gx[d] = fma_(s, u[d], gx[d]);
-                    }
-                    if (NEED_GM && has) {
-                        double* rs = rsum + i * NR;
-                        const T eg = e * g;
-                        atomic_add(&rs[0], double(eg));
-                        T rt[D];
-#pragma unroll
-                        for (int d = 0; d < D; ++d) { rt[d] = eg * t[d]; atomic_add(&rs[1 + d], double(rt[d])); }
-                        int k = 1 + D;
-#pragma unroll
-                        for (int a = 0; a < D; ++a)
-#pragma unroll
-                            for (int c = a; c < D; ++c) atomic_add(&rs[k++], double(rt[a] * t[c]));
-                    }
-                }
-            }
-            if (NEED_GM) {
-                wave_lds_fence();
-                for (int s = lane; s < cnt * NR; s += kWave) {
-                    const int c = s / NR, k = s - c * NR;
-                    const T v = T(rsum[s]);
-                    if (v != T(0)) {
-                        const int comp = reinterpret_cast<const int*>(staged + c * LS + kAmp + 1)[0];
-                        atomic_add(&sums[(size_t(bl) * M + comp) * NR + k], v);
-                    }
+                    for (int d = 0; d < D; ++d) gx[d] = fma_(s, u[d], gx[d]);
                 }
             }
             wave_lds_fence();
@@ -2064,6 +2013,121 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
         } else if (NEED_GX) {
 #pragma unroll
             for (int d = 0; d < D; ++d) atomic_add(&result[gi][d][lane], double(gx[d]));
+        }
+    };
+
+    // The backward pass with per-Gaussian sums: lanes = leaves.  The four rows of a wavefront hold the same 16 leaves of a
+    // batch and walk over the 64 points of the group, a point per row and step, so the ten sums of a leaf stay in the
+    // lane's registers (over rows and to memory once per batch), and only dL/dx of a point is added over the 16
+    // lanes of its row, four points at a time (row_sums_of_four).
+    auto evaluate_by_leaves = [&]() {
+        const int row = lane >> 4, col = lane & 15;
+        while (cur_group < groups) {
+            const int gi = cur_group;
+            const int cnt = cur_end - cur_base < kBatch ? cur_end - cur_base : kBatch;
+#pragma unroll
+            for (int r = 0; r < kPre; ++r) {
+                const int s = lane + r * kWave;
+                if (s < cnt * LS) staged[s] = pre[r];
+            }
+            wave_lds_fence();
+            next_batch();
+            prefetch();
+            const bool active = col < cnt;
+            int rec_at = (active ? col : 0) * LS;
+            T rec[kAmp + 1];
+#pragma unroll
+            for (int k = 0; k < kAmp + 1; ++k) rec[k] = staged[rec_at + k];
+            const int comp = reinterpret_cast<const int*>(staged + (active ? col : 0) * LS + kAmp + 1)[0];
+            T rs[NR];
+#pragma unroll
+            for (int k = 0; k < NR; ++k) rs[k] = T(0);
+            // kSteps points per row at a time (double: more would not fit into the registers); their exponentials are issued
+            // together
+            constexpr int kSteps = sizeof(T) == 4 ? 4 : 1;
+#pragma unroll 1
+            for (int s0 = 0; s0 < kWave; s0 += 4 * kSteps) {
+                const T* point = pts[gi] + 4 * (s0 + row);              // step i: point s0 + 4 i + row
+                T t[kSteps][D], u[kSteps][D], q[kSteps], e[kSteps], g[kSteps], part[NR];
+                bool in[kSteps];
+#pragma unroll
+                for (int i = 0; i < kSteps; ++i) {
+                    T x[D];
+#pragma unroll
+                    for (int d = 0; d < D; ++d) x[d] = point[16 * i + d];
+                    g[i] = point[16 * i + D];
+                    in[i] = active & inside_box<T, D>(x, rec);
+                    q[i] = T(0.72134752044448170368) * leaf_exponent<T, D>(rec + 2 * D, x, t[i], u[i]);
+                }
+                if constexpr (sizeof(T) == 4) pair_exp2_batch(q, e); else e[0] = pair_exp2(-q[0], exp2_tab);
+#pragma unroll
+                for (int i = 0; i < kSteps; ++i) {
+                    const T k = in[i] ? e[i] : T(0);
+                    if (NEED_GX) {
+                        const T s = k * rec[kAmp];
+#pragma unroll
+                        for (int d = 0; d < D; ++d) u[i][d] *= s;
+                    }
+                    const T kg = k * g[i];
+                    // (float: the four steps are summed on their own first, which halves the rounding error of the sums)
+                    if (i == 0 && kSteps > 1) {
+                        part[0] = kg;
+                        int at = 1 + D;
+#pragma unroll
+                        for (int a = 0; a < D; ++a) {
+                            part[1 + a] = kg * t[i][a];
+#pragma unroll
+                            for (int c = a; c < D; ++c) part[at++] = part[1 + a] * t[i][c];
+                        }
+                    } else {
+                        T* to = kSteps > 1 ? part : rs;
+                        to[0] += kg;
+                        int at = 1 + D;
+#pragma unroll
+                        for (int a = 0; a < D; ++a) {
+                            const T kt = kg * t[i][a];
+                            to[1 + a] += kt;
+#pragma unroll
+                            for (int c = a; c < D; ++c) { to[at] = fma_(kt, t[i][c], to[at]); ++at; }
+                        }
+                    }
+                }
+                if (kSteps > 1) {
+#pragma unroll
+                    for (int k = 0; k < NR; ++k) rs[k] += part[k];
+                }
+                if constexpr (NEED_GX && sizeof(T) == 4) {
+                    T sum[D];
+                    slow_issue_begin(u[kSteps - 1]);
+                    row_sums_of_four(u, sum);
+                    slow_issue_end(sum);
+                    // lane 4 b + d of row r adds component d of point s0 + 4 b + r
+                    const int d = lane & 3;
+                    const T v = D == 3 && d == 2 ? sum[D - 1] : d == 1 ? sum[1] : sum[0];
+                    if (d < D) atomic_add(&result[gi][d][s0 + (lane & 12) + row], double(v));
+                } else if constexpr (NEED_GX) {
+                    const T v = row_sum_of_point<D>(u[0], lane);
+                    const int d = col == 0 ? 0 : col == 8 ? 1 : D == 3 && col == 4 ? 2 : -1;
+                    if (d >= 0) atomic_add(&result[gi][d][s0 + row], v);
+                }
+            }
+            T w[NR / 4 + 1];
+            if constexpr (sizeof(T) == 4) {
+                slow_issue_begin(rs);
+                sums_over_rows(rs, w);
+                slow_issue_end(w);
+            } else {
+                sums_over_rows(rs, w);
+            }
+            if (active) {
+                T* dst = sums + (size_t(bl) * M + comp) * NR;
+                const int mine = (row >> 1) | ((row & 1) << 1);
+#pragma unroll
+                for (int q = 0; q < NR / 4; ++q)
+                    if (w[q] != T(0)) atomic_add(&dst[4 * q + mine], w[q]);
+                if ((row & 1) == 0 && w[NR / 4] != T(0)) atomic_add(&dst[NR - 2 + (row >> 1)], w[NR / 4]);
+            }
+            wave_lds_fence();
         }
     };
 
@@ -2175,15 +2239,16 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
         }
         __syncthreads();
         bool left_on_stack = false;
-        cur_group = -1; cur_base = 0; cur_end = 0;
+        cur_group = -1; cur_base = NEED_GM ? (wave - kTravWaves) * kBatch : 0; cur_end = 0;
         next_batch();
         prefetch();
         for (int gi = 0; gi < groups; ++gi) {
             const int n_leaf = state[gi][0];
             left_on_stack |= state[gi][1] > 0;
-            if (n_leaf == 0) continue;                                  // uniform over the workgroup
+            if (NEED_GM || n_leaf == 0) continue;                       // uniform over the workgroup
             evaluate_share(gi);
         }
+        if constexpr (NEED_GM) evaluate_by_leaves();
         if (MODE == 0) {
             // forward: the wavefronts' partial sums are added in a fixed order, by wavefront g for group g (the
             // backward pass has added its dL/dx with atomics)
@@ -2226,7 +2291,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     if (MODE == 0) {
         out[size_t(bl) * N + pid] = T(result[wave][0][lane]);
     } else if (NEED_GX) {
-        const T g = pts[wave][D][lane];
+        const T g = pts[wave][lane * kPointStep + D * kComponentStep];
         if (piece >= 0) {
 #pragma unroll
             for (int d = 0; d < D; ++d) piece_gx[(size_t(piece) * D + d) * kWave + lane] = -g * T(result[0][d][lane]);
@@ -2710,12 +2775,14 @@ static int bvh_build_t(const T* mixture, const T* xes, char* bvh, const gmc_shap
 // forward rule (64 trees of 512 leaves, 4096 groups: 72 us with 4 against 79 with 3 and 98 with 1; 256 trees of 200
 // leaves, 3328 groups: 44 us with 4, 46 with 2, 52 with 1).
 static int g_traversal_groups[2] = {0, 0};      // test knob (gmc_bvh_set_traversal_groups): forward, backward; 0 = automatic
-static int traversal_groups(size_t BL, int M, int N, bool backward) {
+static int traversal_groups(size_t BL, int M, int N, bool backward, bool by_leaves = false) {
     const size_t per_mixture = (size_t(N) + kWave - 1) / kWave;
     const size_t total = BL * per_mixture, slots = size_t(kTravSlots);
     size_t g;
     if (g_traversal_groups[backward ? 1 : 0] > 0) g = size_t(g_traversal_groups[backward ? 1 : 0]);
-    else if (backward && M > kSmallTreeMax) g = total < 4 * slots ? 1 : total < 8 * slots ? 2 : total < 16 * slots ? 3 : kGroupsMax;
+    // (lanes = leaves: few groups per workgroup leave wavefronts without a batch of leaves; one, two, three, four groups take 74,
+    // 69, 71, 62 us for 1563 groups of one tree of 16384 in float64, 82, 73, 81, 75 us for 1876 groups of four trees of 4096)
+    else if (backward && !by_leaves && M > kSmallTreeMax) g = total < 4 * slots ? 1 : total < 8 * slots ? 2 : total < 16 * slots ? 3 : kGroupsMax;
     else g = total <= slots ? 1 : total <= 2 * slots ? 2 : kGroupsMax;
     if (g > per_mixture) g = per_mixture;
     return g < 1 ? 1 : int(g);
@@ -2794,7 +2861,7 @@ static int bvh_bwd_t(const T* grad_out, const T* mixture, const T* xes, char* bv
         }
         return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
     }
-    const int groups = traversal_groups(BL, s.M, s.N, true);
+    const int groups = traversal_groups(BL, s.M, s.N, true, gm);
     int chunks = (s.N + kWave * groups - 1) / (kWave * groups);
     if (groups > 1 && BL * size_t(chunks) < size_t(kTravSlots)) {       // (as in the forward pass: no resident slot left empty)
         const size_t per_mixture = (size_t(s.N) + kWave - 1) / kWave, fill = size_t(kTravSlots) / BL;

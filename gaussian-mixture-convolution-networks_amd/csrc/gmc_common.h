@@ -373,7 +373,6 @@ __device__ __forceinline__ void add_pairs(const T* __restrict__ lds, const T* __
     constexpr int U = sizeof(T) == 4 && P >= 3 && P < 6 ? 2 : 1;       // Gaussians whose exponentials are batched
     int g = begin;
     if constexpr (sizeof(T) == 4 && P >= 3) {
-#pragma unroll 2
         for (; g + (U - 1) * STEP < end; g += U * STEP) {
             T r[U][Rec<T, D>::kUsed], q[U * P], e[U * P];
 #pragma unroll
@@ -585,6 +584,103 @@ __device__ __forceinline__ float row_sums(const float (&s)[6], int lane) {
 #undef GMC_ROR8
 #undef GMC_MIRROR
 #undef GMC_MIRROR1
+
+// ---- sums over the rows and over the lanes of a row, several values at once ------------------------------------------
+// D values of four points per lane, summed over the 16 lanes of a row: afterwards the lanes 4 b ... 4 b + 3 of a row hold
+// the sums of point b.  (As in row_sums: masked additions, two instructions between a write and its DPP read.)
+__device__ __forceinline__ void row_sums_of_four(const float (&v)[4][3], float (&sum)[3]) {
+    float h[6], k[3];
+#define GMC_ROR8(h, a, b) "v_add_f32_dpp " h ", " a ", " a " row_ror:8 row_mask:0xf bank_mask:0x3\n\t" \
+                          "v_add_f32_dpp " h ", " b ", " b " row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+#define GMC_MIRROR(k, a, b) "v_add_f32_dpp " k ", " a ", " a " row_half_mirror row_mask:0xf bank_mask:0x5\n\t" \
+                            "v_add_f32_dpp " k ", " b ", " b " row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+    asm volatile("s_nop 1\n\t"
+                 GMC_ROR8("%0", "%9", "%15") GMC_ROR8("%1", "%12", "%18") GMC_ROR8("%2", "%10", "%16")
+                 GMC_ROR8("%3", "%13", "%19") GMC_ROR8("%4", "%11", "%17") GMC_ROR8("%5", "%14", "%20")
+                 GMC_MIRROR("%6", "%0", "%1") GMC_MIRROR("%7", "%2", "%3") GMC_MIRROR("%8", "%4", "%5") "s_nop 1"
+                 : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(h[4]), "=&v"(h[5]), "=&v"(k[0]), "=&v"(k[1]), "=&v"(k[2])
+                 : "v"(v[0][0]), "v"(v[0][1]), "v"(v[0][2]), "v"(v[1][0]), "v"(v[1][1]), "v"(v[1][2]),
+                   "v"(v[2][0]), "v"(v[2][1]), "v"(v[2][2]), "v"(v[3][0]), "v"(v[3][1]), "v"(v[3][2]));
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        k[d] += dpp_mov<0x4e>(k[d]);                                       // quad_perm 2 3 0 1
+        sum[d] = k[d] + dpp_mov<0xb1>(k[d]);                               // quad_perm 1 0 3 2
+    }
+}
+__device__ __forceinline__ void row_sums_of_four(const float (&v)[4][2], float (&sum)[2]) {
+    float h[4], k[2];
+    asm volatile("s_nop 1\n\t"
+                 GMC_ROR8("%0", "%6", "%10") GMC_ROR8("%1", "%8", "%12") GMC_ROR8("%2", "%7", "%11") GMC_ROR8("%3", "%9", "%13")
+                 GMC_MIRROR("%4", "%0", "%1") GMC_MIRROR("%5", "%2", "%3") "s_nop 1"
+                 : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(k[0]), "=&v"(k[1])
+                 : "v"(v[0][0]), "v"(v[0][1]), "v"(v[1][0]), "v"(v[1][1]), "v"(v[2][0]), "v"(v[2][1]), "v"(v[3][0]), "v"(v[3][1]));
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+        k[d] += dpp_mov<0x4e>(k[d]);
+        sum[d] = k[d] + dpp_mov<0xb1>(k[d]);
+    }
+}
+#undef GMC_ROR8
+#undef GMC_MIRROR
+// double: the D values of one point; the lanes 0, 8 and (D = 3) 4 of a row receive the sums of component 0, 1 and 2
+template <int D>
+__device__ __forceinline__ double row_sum_of_point(const double (&v)[D], int lane) {
+    const bool b3 = (lane & 8) != 0;
+    double k = (b3 ? v[1] : v[0]) + dpp_mov<0x128>(b3 ? v[0] : v[1]);            // row_ror:8
+    if constexpr (D == 3) {
+        const bool b2 = (lane & 4) != 0;
+        const double h = v[2] + dpp_mov<0x128>(v[2]);
+        k = (b2 ? h : k) + dpp_mov<0x141>(b2 ? k : h);                           // row_half_mirror
+    } else {
+        k += dpp_mov<0x141>(k);
+    }
+    k += dpp_mov<0x4e>(k);
+    return k + dpp_mov<0xb1>(k);
+}
+
+// a and b hold one value per lane each: afterwards the even rows (ROWS = 16) or the lower half (32) hold the sums of a over
+// the pairs of rows (halves), the others those of b
+template <int ROWS>
+__device__ __forceinline__ float swap_sum(float a, float b) {
+    const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
+    if constexpr (ROWS == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
+        return __builtin_bit_cast(float, unsigned(r[0])) + __builtin_bit_cast(float, unsigned(r[1]));
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+        return __builtin_bit_cast(float, unsigned(r[0])) + __builtin_bit_cast(float, unsigned(r[1]));
+    }
+}
+template <int ROWS>
+__device__ __forceinline__ double swap_sum(double a, double b) {
+    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a), ub = __builtin_bit_cast(unsigned long long, b);
+    unsigned x[2], y[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const unsigned p = unsigned(ua >> (32 * i)), q = unsigned(ub >> (32 * i));
+        if constexpr (ROWS == 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap(p, q, false, false);
+            x[i] = r[0]; y[i] = r[1];
+        } else {
+            const auto r = __builtin_amdgcn_permlane16_swap(p, q, false, false);
+            x[i] = r[0]; y[i] = r[1];
+        }
+    }
+    return __builtin_bit_cast(double, (unsigned long long)(x[1]) << 32 | x[0]) + __builtin_bit_cast(double, (unsigned long long)(y[1]) << 32 | y[0]);
+}
+// NR = 10 or 6 values per lane summed over the four rows (lanes with the same lane & 15): row r holds the sums
+// 4 q + (r >> 1 | (r & 1) << 1) in w[q] for q < NR / 4; the last two sums are in w[NR / 4], the first of them in the rows 0 and 1
+// (the same in both), the second in the rows 2 and 3.
+template <typename T, int NR>
+__device__ __forceinline__ void sums_over_rows(const T (&v)[NR], T (&w)[NR / 4 + 1]) {
+    static_assert(NR % 4 == 2, "pairs of pairs and one pair");
+    T h[NR / 2];
+#pragma unroll
+    for (int i = 0; i < NR / 2; ++i) h[i] = swap_sum<32>(v[2 * i], v[2 * i + 1]);
+#pragma unroll
+    for (int q = 0; q < NR / 4; ++q) w[q] = swap_sum<16>(h[2 * q], h[2 * q + 1]);
+    w[NR / 4] = swap_sum<16>(h[NR / 2 - 1], h[NR / 2 - 1]);
+}
 
 // ---- sum over the 16 lanes of a DPP row; the total arrives in lane 15 of the row ---------------------------
 template <typename T>

@@ -927,3 +927,36 @@ def test_step_is_capturable_in_a_hip_graph():
         for got, want in zip(captured, eager):
             # sums over atomics differ in their last bits between runs; everything else is identical
             assert ((got - want).norm() / want.norm()).item() < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("D", [2, 3])
+def test_backward_by_leaves_at_the_edges_of_its_batches(dtype, D):
+    """the backward traversal keeps 16 candidate leaves per wavefront and walks over the 64 points of a group: leaf counts on
+    both sides of a batch, of the eight wavefronts and of several groups' batches dealt in turn; groups of 1 ... 64 points;
+    wide boxes, so that every leaf is a candidate of every group"""
+    lib = _native.lib()
+    lib.gmc_bvh_set_eval_path(1)
+    try:
+        for M, N in ((1, 1), (2, 65), (15, 64), (16, 63), (17, 130), (127, 64), (128, 257), (129, 300), (145, 1)):
+            mix, xes, gout = _case(2, 2, M, N, D, 5000 + 10 * M + D, cov_radius=2.0)
+            _check_culled(mix, xes, gout, dtype, "tight", tag=f"{M} leaves, {N} points, {D}-D")
+    finally:
+        lib.gmc_bvh_set_eval_path(0)
+
+
+def test_points_without_finite_coordinates_leave_the_gradients_of_the_others():
+    """a point with a NaN or infinite coordinate lies in no box: it adds nothing to any gradient"""
+    for dtype in (torch.float32, torch.float64):
+        mix, xes, gout = _case(1, 2, 300, 200, 3, 5200)
+        m, x, g = mix.to(dtype).to(DEV), xes.to(dtype).to(DEV), gout.to(dtype).to(DEV)
+        bad = x.clone()
+        bad[0, 0, 7, 1], bad[0, 1, 100, 0], bad[0, 1, 101, 2] = float("nan"), float("inf"), float("-inf")
+        keep = torch.isfinite(bad).all(-1)
+        bvh = _native.Bvh(m, x, 0.001, "tight")
+        _native.eval_bvh_fwd(m, x, bvh)
+        want, _ = _native.eval_bvh_bwd(g * keep, m, x, bvh, True, True)
+        _native.eval_bvh_fwd(m, bad, bvh)
+        got, gxes = _native.eval_bvh_bwd(g, m, bad, bvh, True, True)
+        assert rel_l2(got.cpu().numpy(), want.cpu().numpy(), FLOOR[dtype]) <= TOL[dtype]
+        assert bool((gxes[~keep] == 0).all())
