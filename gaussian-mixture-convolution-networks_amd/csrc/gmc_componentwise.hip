@@ -10,6 +10,7 @@ namespace gmc {
 int check_shape(const gmc_shape* s);
 
 constexpr int kCwPoints = 64;      // points per workgroup
+template <typename T, int Q> struct __align__(sizeof(T) * Q) CwVec { T v[Q]; };
 
 template <typename T, int D>
 __global__ __launch_bounds__(kBlock) void componentwise_fwd_kernel(const T* __restrict__ mixture, const T* __restrict__ xes,
@@ -54,6 +55,85 @@ __global__ __launch_bounds__(kBlock) void componentwise_fwd_kernel(const T* __re
     }
 }
 
+// The same with four Gaussians per lane (float32): a power of two of lanes holds a point's row, the others of a wavefront the
+// following points, so that few Gaussians leave no lanes idle.  WIDE, where every row starts at a multiple of 16 bytes: a
+// lane's Gaussians are neighbours and its values leave with one store; elsewhere they lie a row of lanes apart.  The workgroup
+// prepares the tile's Gaussians once, through LDS, and walks over `points_per_chunk` points; four steps of a wavefront are in
+// flight.  Taken (cw_wide_forward) for at most 64 Gaussians (32 without WIDE), where the kernel above leaves lanes or
+// wavefronts idle, and for launches of fewer than 512 of its workgroups; with more of both it takes between 0.8 and 1.3 of the
+// time, and in double, where a lane prepares two, small calls take up to 1.4 times as long.  Kernel above / this one, us: 1600 x
+// 16 Gaussians at 1000 points, 2-D, 65 / 20;  800 x 44 at 900, 3-D, 45 / 28;  320 x 32 at 4096 57 / 30 (167 MB of values,
+// 5.6 TB/s: bound by the stores);  1 x 300 at 3000, 3-D, 11.9 / 4.8;  1 x 32 at 784 3.8 / 2.6.  Over 11000 drawn calls the
+// median is 0.71 of the time, none slower.
+template <int D, bool WIDE>
+__global__ __launch_bounds__(kBlock) void componentwise_fwd_wide_kernel(const float* __restrict__ mixture, const float* __restrict__ xes,
+                                                                       float* __restrict__ out, int L, int M, int N, int Bx, int Lx,
+                                                                       int m_tiles, int first_mixture, int chunks,
+                                                                       int points_per_chunk, bool covariance_form) {
+    constexpr int G = 1 + D + D * D, S = Rec<float, D>::kStride, Q = 4, kTileG = kWave * Q, U = 4;
+    __shared__ __attribute__((aligned(16))) float lds[kTileG * S];
+    int id = blockIdx.x;
+    const int chunk = id % chunks; id /= chunks;
+    const int tile = id % m_tiles;
+    const int bl = first_mixture + id / m_tiles;
+    const int b = bl / L, l = bl - b * L;
+    const int xb = b < Bx ? b : Bx - 1, xl = l < Lx ? l : Lx - 1;
+    const float* __restrict__ x_bl = xes + (size_t(xb) * Lx + xl) * N * D;
+    const int here = M - tile * kTileG < kTileG ? M - tile * kTileG : kTileG;
+    if (int(threadIdx.x) < here) {
+        const Derived<D> dv = derive<float, D>(mixture + (size_t(bl) * M + tile * kTileG + threadIdx.x) * G, covariance_form);
+        store_record<float, D>(lds + threadIdx.x * S, dv, true, dv.w * dv.norm, 0);
+    }
+    __syncthreads();
+    int shift = 6;                                          // log2 of the lanes of a row
+    while (shift > 0 && (Q << (shift - 1)) >= here) --shift;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int slot = lane & ((1 << shift) - 1), rows = 64 >> shift;
+    // Gaussian q of this lane
+    const int first = WIDE ? slot * Q : slot, apart = WIDE ? 1 : 1 << shift;
+    const bool active = first < here;
+    float r[Q][Rec<float, D>::kUsed];
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int i = 0; i < Rec<float, D>::kUsed; ++i) r[q][i] = lds[(first + q * apart < here ? first + q * apart : 0) * S + i];
+    const int n_first = chunk * points_per_chunk;
+    const int n_end = n_first + points_per_chunk < N ? n_first + points_per_chunk : N;
+    float* __restrict__ to = out + size_t(bl) * N * M + tile * kTileG + first;
+    for (int n0 = n_first + wave * rows + (lane >> shift); n0 - (lane >> shift) < n_end; n0 += 4 * rows * U) {
+        float x[U][D];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int n = n0 + u * 4 * rows < n_end ? n0 + u * 4 * rows : n_end - 1;
+#pragma unroll
+            for (int d = 0; d < D; ++d) x[u][d] = x_bl[size_t(n) * D + d];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int n = n0 + u * 4 * rows;
+            float f[Q], e[Q];
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                float y[D];
+                f[q] = quad_form<float, D, true>(r[q], x[u], y);
+            }
+            pair_exp2_batch(f, e);
+            if (active && n < n_end) {
+                if constexpr (WIDE) {
+                    CwVec<float, Q> v;
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) v.v[q] = r[q][Rec<float, D>::kAmp] * e[q];
+                    *reinterpret_cast<CwVec<float, Q>*>(to + size_t(n) * M) = v;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < Q; ++q)
+                        if (first + q * apart < here) to[size_t(n) * M + q * apart] = r[q][Rec<float, D>::kAmp] * e[q];
+                }
+            }
+        }
+    }
+}
+
 // Layout of the backward pass: the 64 lanes of a wavefront are 4 rows (points) by 16 columns, a column holds Q Gaussians,
 // so that the coordinates of a point are fetched once for Q pairs.  Where every row of grad_out starts at a multiple of
 // the vector (`wide`), a column's Gaussians lie next to each other and one access per lane fetches the values of 16 Q
@@ -62,7 +142,6 @@ __global__ __launch_bounds__(kBlock) void componentwise_fwd_kernel(const T* __re
 // the chunk.  (The forward pass, which only stores, is faster with lanes = Gaussians: 800 x 128 Gaussians at 784 points in
 // 2-D 74 us against 107 us in this layout.)
 constexpr int kCwPointsMax = 1024; // most points per workgroup of the backward pass (the size of its LDS copy of dL/dx)
-template <typename T, int Q> struct __align__(sizeof(T) * Q) CwVec { T v[Q]; };
 
 // Gaussians per lane: one or, in float32, two -- a lane prepares them one after the other and holds a record and sums for
 // each.  Two where the mixtures fill their slices (groups of 128 components cover at most a tenth more than groups of 64)
@@ -411,6 +490,12 @@ static CwChunks cw_chunks(size_t workgroups, int N, size_t wanted) {
     return CwChunks{(N + points - 1) / points, points};
 }
 
+// (see componentwise_fwd_wide_kernel; `workgroups`: of the kernel with lanes = Gaussians)
+static bool cw_wide_forward(const gmc_shape& s, size_t workgroups, bool wide) {
+    if (s.dtype != GMC_F32) return false;
+    return s.M <= (wide ? 64 : 32) ? s.N >= 16 : s.M > 64 && workgroups < 512 && s.N >= (wide ? 96 : 128);
+}
+
 template <typename T, int D>
 static int cw_forward(const T* mixture, const T* xes, T* out, const gmc_shape& s, bool cov, hipStream_t st) {
     const size_t BL = size_t(s.B) * s.L;
@@ -418,6 +503,27 @@ static int cw_forward(const T* mixture, const T* xes, T* out, const gmc_shape& s
     const int m_tiles = (s.M + kBlock - 1) / kBlock, chunks = (s.N + kCwPoints - 1) / kCwPoints;
     const size_t per_mixture = size_t(m_tiles) * chunks, at_once = max_workgroups(kBlock) / per_mixture;
     if (at_once == 0) return GMC_E_SHAPE;
+    if constexpr (sizeof(T) == 4) {
+        constexpr int Q = 4, kTileG = kWave * Q;
+        const bool wide = s.M % Q == 0 && (uintptr_t(out) & 15) == 0;
+        if (cw_wide_forward(s, BL * per_mixture, wide)) {
+            const int tiles = (s.M + kTileG - 1) / kTileG;
+            size_t wide_chunks = (kCwWanted + BL * tiles - 1) / (BL * tiles);
+            const size_t most = s.N < 64 ? 1 : size_t(s.N) / 32;
+            if (wide_chunks > most) wide_chunks = most;
+            const int points = int(((s.N + wide_chunks - 1) / wide_chunks + 31) / 32 * 32);
+            wide_chunks = (size_t(s.N) + points - 1) / points;
+            const size_t per_wide = size_t(tiles) * wide_chunks, wide_at_once = max_workgroups(kBlock) / per_wide;
+            for (size_t first = 0; first < BL; first += wide_at_once) {
+                const dim3 grid(unsigned((BL - first < wide_at_once ? BL - first : wide_at_once) * per_wide));
+#define GMC_CW(W) componentwise_fwd_wide_kernel<D, W><<<grid, dim3(kBlock), 0, st>>>( \
+                    mixture, xes, out, s.L, s.M, s.N, s.Bx, s.Lx, tiles, int(first), int(wide_chunks), points, cov)
+                if (wide) GMC_CW(true); else GMC_CW(false);
+#undef GMC_CW
+            }
+            return hipGetLastError() == hipSuccess ? GMC_OK : GMC_E_LAUNCH;
+        }
+    }
     for (size_t first = 0; first < BL; first += at_once)
         componentwise_fwd_kernel<T, D><<<dim3(unsigned((BL - first < at_once ? BL - first : at_once) * per_mixture)), dim3(kBlock), 0, st>>>(
             mixture, xes, out, s.L, s.M, s.N, s.Bx, s.Lx, m_tiles, int(first), chunks, cov);

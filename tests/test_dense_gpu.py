@@ -839,3 +839,22 @@ def test_batched_exponentials_at_every_points_per_lane(D, points):
             _check(mix, xes, gout, torch.float32, tag=f"{points} points per lane, {M} components, {D}-D")
     finally:
         lib.gmc_set_tuning(0, 0)
+
+
+@pytest.mark.parametrize("D", [2, 3])
+def test_componentwise_forward_with_four_gaussians_per_lane(D):
+    """few Gaussians and small launches of the component-wise forward pass: Gaussian counts around every power of two of lanes
+    and around the tile of 256, rows on and off a multiple of 16 bytes, points around the steps of a wavefront and the chunks;
+    reference: float64 on the CPU"""
+    shapes = [(3, 2, M, N) for M in (1, 2, 3, 4, 5, 8, 12, 16, 17, 20, 31, 32, 36, 60, 64) for N in (16, 17, 64, 65, 131)]
+    shapes += [(1, 2, M, N) for M in (68, 101, 128, 252, 256, 257, 260, 300, 516) for N in (128, 129, 331)]
+    for i, (B, L, M, N) in enumerate(shapes):
+        mix, xes, _ = _case(B, L, M, N, D, 8100 + i, i % 4 == 2)
+        mix, xes = torch.tensor(mix).float(), torch.tensor(xes).float() * 0.5
+        m64, x64 = mix.double(), xes.double()
+        c = m64[..., 1 + D:].view(B, L, 1, M, D, D)
+        t = x64.unsqueeze(3) - m64[..., 1:1 + D].unsqueeze(2)
+        q = (t.unsqueeze(-2) @ c @ t.unsqueeze(-1)).squeeze(-1).squeeze(-1)
+        vals = m64[..., 0].unsqueeze(2) * o.kappa(D) * torch.linalg.det(c).sqrt() * torch.exp(-0.5 * q)
+        got = _native.eval_componentwise_fwd(mix.to(DEV), xes.to(DEV))
+        assert rel_l2(got.cpu().numpy(), vals.numpy(), FLOOR[torch.float32]) <= TOL[torch.float32], (B, L, M, N)
