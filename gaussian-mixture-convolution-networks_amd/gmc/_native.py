@@ -7,6 +7,7 @@ missing, or a tensor does not live on a HIP device, the call raises.
 import ctypes
 import os
 import subprocess
+import sys
 
 import torch
 
@@ -35,9 +36,11 @@ class BvhConfigC(ctypes.Structure):
 
 
 def build(verbose: bool = False) -> str:
-    """Compiles every HIP source of the library for gfx950 (hipcc cross-compiles without a GPU)."""
+    """Compiles every HIP source of the library for gfx950 (hipcc cross-compiles without a GPU) and the C++ autograd of the
+    dense evaluation for the torch of this interpreter."""
     out = None if verbose else subprocess.DEVNULL
-    subprocess.run(["make", "-B", "-j8", "-C", CSRC_DIR, "libgmc_hip.so"], check=True, stdout=out, stderr=out)
+    subprocess.run(["make", "-B", "-j8", "-C", CSRC_DIR, f"PYTHON={sys.executable}", "_gmc_autograd.so"], check=True, stdout=out,
+                   stderr=out)
     global _lib
     _lib = None
     return LIB_PATH

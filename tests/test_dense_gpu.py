@@ -858,3 +858,81 @@ def test_componentwise_forward_with_four_gaussians_per_lane(D):
         vals = m64[..., 0].unsqueeze(2) * o.kappa(D) * torch.linalg.det(c).sqrt() * torch.exp(-0.5 * q)
         got = _native.eval_componentwise_fwd(mix.to(DEV), xes.to(DEV))
         assert rel_l2(got.cpu().numpy(), vals.numpy(), FLOOR[torch.float32]) <= TOL[torch.float32], (B, L, M, N)
+
+
+def test_native_autograd_behaves_like_the_python_function():
+    """gm.evaluate(_inversed) hands plain device tensors to the C++ autograd of csrc/gmc_autograd.cpp: the same values and
+    gradients as through the Python classes, and the same answer or refusal to what autograd can be asked"""
+    from gmc.cpp.extensions.evaluate_inversed import evaluate_inversed as binding
+    import torch.autograd.forward_ad as fwad
+    mix, xes, gout = (torch.tensor(a, dtype=torch.float32, device=DEV) for a in _case(2, 3, 40, 100, 2, 9100, False))
+    assert "CppFunction" in type(binding.apply(mix.clone().requires_grad_(True), xes).grad_fn).__name__
+
+    def outcome(f):
+        try:
+            r = f()
+        except Exception as e:                                          # noqa: BLE001
+            return type(e).__name__, str(e)[:60]
+        return [None if t is None else t.detach() for t in (r if isinstance(r, tuple) else (r,))]
+
+    def questions(apply):
+        m, x = mix.clone().requires_grad_(True), xes.clone().requires_grad_(True)
+        # channels first in memory: the same values in another order of strides
+        strided = mix.transpose(0, 1).contiguous().transpose(0, 1).requires_grad_(True)
+        shared = xes[:1, :1].clone().requires_grad_(True)
+        packed = []
+
+        def second(go):
+            first = torch.autograd.grad(apply(m, x), (m, x), go, create_graph=True)
+            return torch.autograd.grad(first[0].sum() + first[1].sum(), go if go.requires_grad else m)
+
+        def hooked():
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(1), t * 2)[1], lambda t: t / 2):
+                out = apply(m, x)
+            return torch.autograd.grad(out, (m, x), gout)
+
+        def changed():
+            inner = m * 1.0
+            out = apply(inner, x)
+            inner.add_(1.0)
+            return torch.autograd.grad(out, m, gout)
+
+        def dual():
+            with fwad.dual_level():
+                return apply(fwad.make_dual(mix, mix), xes)
+
+        def on_a_stream():
+            side = torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                r = torch.autograd.grad(apply(m, x), (m, x), gout)
+            torch.cuda.current_stream().wait_stream(side)
+            return r
+
+        def without_grad():
+            with torch.no_grad():
+                return torch.tensor(float(apply(m, x).requires_grad))
+
+        return [outcome(f) for f in (
+            lambda: apply(m, x), lambda: torch.autograd.grad(apply(m, x), (m, x), gout),
+            lambda: torch.autograd.grad(apply(mix, x), x, gout), lambda: torch.autograd.grad(apply(m, xes), m, gout),
+            lambda: torch.autograd.grad(apply(strided, shared), (strided, shared), gout),
+            lambda: torch.autograd.grad(apply(torch.nn.Parameter(mix), x), x, gout),
+            lambda: torch.autograd.grad(apply(m.double(), x.double()), (m, x), gout.double()),
+            lambda: second(gout), lambda: second(gout.clone().requires_grad_(True)), hooked, changed, dual, on_a_stream, without_grad,
+            lambda: torch.vmap(lambda a: apply(a, xes))(mix.unsqueeze(0)), lambda: torch.func.grad(lambda a: apply(a, xes).sum())(mix),
+            lambda: torch.func.jvp(lambda a: apply(a, xes), (mix,), (mix,)), lambda: apply(mix.cpu(), xes.cpu()),
+            lambda: apply(mix[0], xes), lambda: apply(mix.half(), xes.half()), lambda: apply(mix.double(), xes),
+            lambda: apply(mix, xes[:, :2]), lambda: apply(mix, torch.zeros(2, 3, 5, 3, device=DEV)), lambda: apply(mix[:, :, :0], xes),
+            lambda: apply(mix, xes[:, :, :0]))] + [len(packed)]
+
+    for native, python in ((binding.apply, binding.EvaluateInversed.apply), (binding.apply_covariance, binding.EvaluateCovariance.apply)):
+        got, want = questions(native), questions(python)
+        assert len(got) == len(want)
+        for i, (a, b) in enumerate(zip(got, want)):
+            if isinstance(a, list):
+                assert isinstance(b, list) and len(a) == len(b), i
+                for s, t in zip(a, b):
+                    assert torch.allclose(s, t, rtol=1e-5, atol=1e-5 * float(t.abs().max()) if t.numel() else 0.0), i
+            else:
+                assert a == b, (i, a, b)

@@ -257,3 +257,14 @@ def test_check_valid_mixture_on_host_tensors():
     bad[1, 0, 0, 3:] = torch.tensor([1.0, 2.0, 2.0, 1.0])
     with pytest.raises(RuntimeError, match="non positive definite"):
         gm.check_valid_mixture(bad)
+
+
+def test_native_autograd_leaves_host_tensors_to_the_python_classes():
+    """csrc/gmc_autograd.cpp answers None to what is not a plain device tensor; the call is then refused as ever"""
+    from gmc.cpp.extensions.evaluate_inversed import evaluate_inversed as binding
+    m, x = torch.rand(1, 1, 2, 7), torch.rand(1, 1, 3, 2)
+    evaluate = binding._load_native_autograd()
+    assert evaluate(m, x, False) is None and evaluate(m.numpy(), x, True) is None
+    for apply in (binding.apply, binding.apply_covariance):
+        with pytest.raises(RuntimeError, match="AMD GPU only"):
+            apply(m, x)
