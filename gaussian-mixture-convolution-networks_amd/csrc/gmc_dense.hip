@@ -151,8 +151,8 @@ __global__ __launch_bounds__(kBlock) void eval_fwd_rc_kernel(const T* __restrict
 
 // Backward pair kernel, "4 x 16" wavefront layout.  The 64 lanes of a wavefront form 4 DPP rows of 16 lanes:
 // row r works on Gaussian 4k + r of the tile in step k, column c on the points {c, c + 16, ..., c + 16 (P-1)} of
-// the wavefront's 16 P points.  The per-Gaussian sums are then reduced over one DPP row only (4 shifts, no
-// cross-row traffic) once per step and Gaussian, and dL/dx is reduced over the 4 rows once per kernel.
+// the wavefront's 16 P points.  The per-Gaussian sums are then reduced over one DPP row only (row_sums, no cross-row
+// traffic) once per step and Gaussian, and dL/dx is reduced over the 4 rows once per kernel.
 // copies of a tile's per-Gaussian sums in LDS: one per wavefront in float, a shared one in double (80 KB otherwise)
 template <typename T> struct SumCopies { static constexpr int k = sizeof(T) == 4 ? 4 : 1; };
 
@@ -579,8 +579,9 @@ __global__ __launch_bounds__(kBlock) void eval_bwd_epilogue_kernel(const T* __re
 // points and the wavefronts share the Gaussians, 64 at a time: four times fewer reductions per pair, the lane that
 // prepared a Gaussian finishes its gradient from the wavefront's own sums (no workspace, no atomics, no workgroup
 // barrier, no second preparation), and only dL/dx is added over wavefronts and slices at the end.  Bound by instruction
-// issue: 1600 mixtures of 5120 Gaussians at 128 points in 2-D 626 us (1.05e9 pairs, 39 cycles per 64 pairs and SIMD;
-// 1029 us with zero fill, pair kernel and epilogue before).
+// issue: 1600 mixtures of 5120 Gaussians at 128 points in 2-D 519 us (1.05e9 pairs, 67 cycles per 64 pairs and SIMD
+// at 2.07 GHz, the clock the power limit leaves; 656 us with the exponentials among the other instructions, 1029 us with zero
+// fill, pair kernel and epilogue).
 template <typename T, int D, int P, bool NEED_GX>
 __global__ __launch_bounds__(kBlock) void few_points_bwd_kernel(const T* __restrict__ grad_out, const T* __restrict__ mixture,
                                                                 const T* __restrict__ xes, T* __restrict__ grad_xes,
@@ -825,7 +826,8 @@ static FwdPlan plan_fwd(const gmc_shape& s, bool is_double) {
 
 // Shapes of the kernels that give every wavefront all points of a mixture (few_points_fwd_kernel, few_points_bwd_kernel):
 // at most 16 points per lane (8 in double), and more than two groups of 64 Gaussians to share out.  Measured, kernels
-// above / few-points kernels in us (float32, 2-D):
+// above / few-points kernels in us (float32, 2-D; both before their exponentials were issued in batches, since when the first
+// row's few-points kernels take 215 and 519 us):
 //   mixtures x M at N points      forward        backward
 //   1600 x 5120 at 128            745 / 247     1029 / 626    (forward: the matrix-core kernel, whose blocks hold 1024 points)
 //   1200 x 1280 at 100            223 /  53      205 / 114
