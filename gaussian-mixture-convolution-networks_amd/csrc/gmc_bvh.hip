@@ -2314,8 +2314,8 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
 // 4096 points, forward / backward us without the tree against the traversal: 32 leaves 16 / 28 against 21 / 40 (6 % of
 // the pairs inside a box; the same ratio at 0.1 %), 64 leaves 25 / 44 against 23 / 49, and with a quarter of the pairs
 // inside (336 mixtures) 78 / 159 against 130 / 262; from 128 leaves on the traversal wins unless most boxes contain
-// most points (22 / 42 against 39 / 56 at 0.6 % inside).  With the traversal's backward pass on lanes = leaves, a quarter of
-// the pairs inside: 32 leaves in 3-D 14 / 33 against 20 / 33, 64 leaves 23 / 53 against 23 / 49 (336 mixtures: 72 / 127
+// most points (22 / 42 against 39 / 56 at 0.6 % inside).  With the traversal's backward pass on lanes = leaves, random
+// mixtures: 32 leaves in 3-D 14 / 33 against 20 / 33, 64 leaves 23 / 53 against 23 / 49 (336 mixtures: 72 / 127
 // against 88 / 170; in 2-D 46 / 78 against 74 / 110), 48 leaves (200 mixtures) 42 / 77 against 52 / 91: the line stays.  Mixtures of at most kAllPairsMax components are therefore
 // evaluated without the tree: the leaf records of the mixture (own box + evaluation record,
 // as the build left them) are staged in LDS, a wavefront owns P groups of 64 Morton-neighbouring points (lanes =
