@@ -1729,8 +1729,8 @@ __device__ __forceinline__ void group_boxes(const T (&x)[D], bool valid, int lan
 // MODE 0: forward.  MODE 1: backward (grad_out given).  dL/dx alone runs as the forward pass does.  With the gradient of the
 // mixture phase 2 turns round (evaluate_by_leaves, lanes = leaves): a lane keeps a candidate leaf and its ten sums in
 // registers and walks over the points, so a leaf's sums are reduced over four lanes once per 64 points instead of over
-// the wavefront or, hit by hit, with ten LDS atomics; about a quarter of the pairs of a candidate lie inside its box, and the
-// others are multiplied by zero.  Measured, backward pass, lanes = points with reductions and LDS atomics / lanes = leaves:
+// the wavefront or, hit by hit, with ten LDS atomics; of the pairs of a candidate a fifth (100000 points over
+// 16384 leaves on a surface) to a hundredth (1000 points) lie inside its box.  Measured, backward pass, lanes = points with reductions and LDS atomics / lanes = leaves:
 //   63 trees of 500 leaves, 4001 points each, float32 165 / 118 us;  one tree of 16384, 100000 points, float64 75 / 62,
 //   float32 67 / 48;  800 trees of 128 at 784 points, 2-D float32 138 / 106;  25 trees of 200 at 2000, float64 42 / 38
 // Bound by vector issue (float32: 37 instructions and a row sum of six per four points and 16 leaves) and the fixed 5 us of a
@@ -1751,8 +1751,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     __shared__ int state[kGroupsMax][2];                    // [0] candidates gathered, [1] nodes left on the stack
     __shared__ int pids[kGroupsMax][kWave];                 // index of every point, -1 beyond the end
     // coordinates and upstream gradient of every point: one array per component, or, for the pass that evaluates by leaves,
-    // one record per point.  (There, where a point outside the box is multiplied by zero, points beyond the end and points with
-    // infinite or NaN coordinates, which no box contains, lie far away at finite coordinates and have no upstream gradient.)
+    // one record per point (NaN coordinates beyond the end: in no box)
     __shared__ __attribute__((aligned(16))) T pts[kGroupsMax][4 * kWave];
     constexpr int kPointStep = NEED_GM ? 4 : 1, kComponentStep = NEED_GM ? 1 : kWave;
     __shared__ float gbox[kGroupsMax][4 * D];               // two boxes (lower, upper; rounded outwards) around every group's points
@@ -1844,12 +1843,9 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
         for (int d = 0; d < D; ++d) x[d] = xes[(xseg * N + pid) * D + d];
         T g = T(0);
         if (MODE == 1) g = valid ? grad_out[size_t(bl) * N + pid] : T(0);
-        bool near = valid;
 #pragma unroll
-        for (int d = 0; d < D; ++d) near = near & (x[d] - x[d] == T(0));
-#pragma unroll
-        for (int d = 0; d < D; ++d) pts[wave][lane * kPointStep + d * kComponentStep] = NEED_GM && !near ? T(1e18) : x[d];
-        pts[wave][lane * kPointStep + D * kComponentStep] = NEED_GM && !near ? T(0) : g;
+        for (int d = 0; d < D; ++d) pts[wave][lane * kPointStep + d * kComponentStep] = NEED_GM && !valid ? T(NAN) : x[d];
+        pts[wave][lane * kPointStep + D * kComponentStep] = g;
         pids[wave][lane] = valid ? pid : -1;
         if (cache.count) my_stamp = points_stamp<T, D>(x, valid, lane);
         const bool any = group * kWave < N;
@@ -2019,7 +2015,8 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     // The backward pass with per-Gaussian sums: lanes = leaves.  The four rows of a wavefront hold the same 16 leaves of a
     // batch and walk over the 64 points of the group, a point per row and step, so the ten sums of a leaf stay in the
     // lane's registers (over rows and to memory once per batch), and only dL/dx of a point is added over the 16
-    // lanes of its row, four points at a time (row_sums_of_four).
+    // lanes of its row, four points at a time (row_sums_of_four).  Only pairs inside a box enter anything: upstream gradients,
+    // amplitudes and, far away, t and u may be infinite or NaN, so the others are left out instead of multiplied by zero.
     auto evaluate_by_leaves = [&]() {
         const int row = lane >> 4, col = lane & 15;
         while (cur_group < groups) {
@@ -2034,81 +2031,93 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
             next_batch();
             prefetch();
             const bool active = col < cnt;
-            int rec_at = (active ? col : 0) * LS;
+            const T* from = staged + (active ? col : 0) * LS;
             T rec[kAmp + 1];
 #pragma unroll
-            for (int k = 0; k < kAmp + 1; ++k) rec[k] = staged[rec_at + k];
-            const int comp = reinterpret_cast<const int*>(staged + (active ? col : 0) * LS + kAmp + 1)[0];
+            for (int k = 0; k < kAmp + 1; ++k) rec[k] = from[k];
+            const int comp = reinterpret_cast<const int*>(from + kAmp + 1)[0];
             T rs[NR];
 #pragma unroll
             for (int k = 0; k < NR; ++k) rs[k] = T(0);
-            // kSteps points per row at a time (double: more would not fit into the registers); their exponentials are issued
-            // together
-            constexpr int kSteps = sizeof(T) == 4 ? 4 : 1;
+            // point 4 i + row of the group at points[16 i]
+            const T* points = pts[gi] + 4 * row;
+            if constexpr (sizeof(T) == 4) {
+                // four points per row at a time: their exponentials are issued together
 #pragma unroll 1
-            for (int s0 = 0; s0 < kWave; s0 += 4 * kSteps) {
-                const T* point = pts[gi] + 4 * (s0 + row);              // step i: point s0 + 4 i + row
-                T t[kSteps][D], u[kSteps][D], q[kSteps], e[kSteps], g[kSteps], part[NR];
-                bool in[kSteps];
+                for (int s0 = 0; s0 < kWave; s0 += 16) {
+                    T t[4][D], u[4][D], q[4], e[4], g[4], part[NR];
+                    bool in[4];
 #pragma unroll
-                for (int i = 0; i < kSteps; ++i) {
-                    T x[D];
+                    for (int i = 0; i < 4; ++i) {
+                        T x[D];
 #pragma unroll
-                    for (int d = 0; d < D; ++d) x[d] = point[16 * i + d];
-                    g[i] = point[16 * i + D];
-                    in[i] = active & inside_box<T, D>(x, rec);
-                    q[i] = T(0.72134752044448170368) * leaf_exponent<T, D>(rec + 2 * D, x, t[i], u[i]);
-                }
-                if constexpr (sizeof(T) == 4) pair_exp2_batch(q, e); else e[0] = pair_exp2(-q[0], exp2_tab);
-#pragma unroll
-                for (int i = 0; i < kSteps; ++i) {
-                    const T k = in[i] ? e[i] : T(0);
-                    if (NEED_GX) {
-                        const T s = k * rec[kAmp];
-#pragma unroll
-                        for (int d = 0; d < D; ++d) u[i][d] *= s;
+                        for (int d = 0; d < D; ++d) x[d] = points[4 * s0 + 16 * i + d];
+                        g[i] = points[4 * s0 + 16 * i + D];
+                        in[i] = active & inside_box<T, D>(x, rec);
+                        q[i] = T(0.72134752044448170368) * leaf_exponent<T, D>(rec + 2 * D, x, t[i], u[i]);
                     }
-                    const T kg = k * g[i];
-                    // (float: the four steps are summed on their own first, which halves the rounding error of the sums)
-                    if (i == 0 && kSteps > 1) {
-                        part[0] = kg;
+                    pair_exp2_batch(q, e);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const T s = e[i] * rec[kAmp];
+#pragma unroll
+                        for (int d = 0; d < D; ++d) {
+                            t[i][d] = in[i] ? t[i][d] : T(0);
+                            if (NEED_GX) u[i][d] = in[i] ? s * u[i][d] : T(0);
+                        }
+                        // (the four steps are summed on their own first, which halves the rounding error of the sums)
+                        const T k0 = in[i] ? e[i] * g[i] : T(0);
+                        part[0] = i == 0 ? k0 : part[0] + k0;
                         int at = 1 + D;
 #pragma unroll
                         for (int a = 0; a < D; ++a) {
-                            part[1 + a] = kg * t[i][a];
+                            const T kt = k0 * t[i][a];
+                            part[1 + a] = i == 0 ? kt : part[1 + a] + kt;
 #pragma unroll
-                            for (int c = a; c < D; ++c) part[at++] = part[1 + a] * t[i][c];
-                        }
-                    } else {
-                        T* to = kSteps > 1 ? part : rs;
-                        to[0] += kg;
-                        int at = 1 + D;
-#pragma unroll
-                        for (int a = 0; a < D; ++a) {
-                            const T kt = kg * t[i][a];
-                            to[1 + a] += kt;
-#pragma unroll
-                            for (int c = a; c < D; ++c) { to[at] = fma_(kt, t[i][c], to[at]); ++at; }
+                            for (int c = a; c < D; ++c) { part[at] = i == 0 ? kt * t[i][c] : fma_(kt, t[i][c], part[at]); ++at; }
                         }
                     }
-                }
-                if (kSteps > 1) {
 #pragma unroll
                     for (int k = 0; k < NR; ++k) rs[k] += part[k];
+                    if constexpr (NEED_GX) {
+                        T sum[D];
+                        slow_issue_begin(u[3]);
+                        row_sums_of_four(u, sum);
+                        slow_issue_end(sum);
+                        // lane 4 b + d of row r adds component d of point s0 + 4 b + r
+                        const int d = lane & 3;
+                        const T v = D == 3 && d == 2 ? sum[D - 1] : d == 1 ? sum[1] : sum[0];
+                        if (d < D) atomic_add(&result[gi][d][s0 + (lane & 12) + row], double(v));
+                    }
                 }
-                if constexpr (NEED_GX && sizeof(T) == 4) {
-                    T sum[D];
-                    slow_issue_begin(u[kSteps - 1]);
-                    row_sums_of_four(u, sum);
-                    slow_issue_end(sum);
-                    // lane 4 b + d of row r adds component d of point s0 + 4 b + r
-                    const int d = lane & 3;
-                    const T v = D == 3 && d == 2 ? sum[D - 1] : d == 1 ? sum[1] : sum[0];
-                    if (d < D) atomic_add(&result[gi][d][s0 + (lane & 12) + row], double(v));
-                } else if constexpr (NEED_GX) {
-                    const T v = row_sum_of_point<D>(u[0], lane);
-                    const int d = col == 0 ? 0 : col == 8 ? 1 : D == 3 && col == 4 ? 2 : -1;
-                    if (d >= 0) atomic_add(&result[gi][d][s0 + row], v);
+            } else {
+                // (more than one point at a time would not fit into the registers)
+#pragma unroll 1
+                for (int i = 0; i < kWave / 4; ++i) {
+                    T x[D], v[D];
+#pragma unroll
+                    for (int d = 0; d < D; ++d) { x[d] = points[16 * i + d]; v[d] = T(0); }
+                    if (active & inside_box<T, D>(x, rec)) {
+                        T t[D];
+                        const T e = leaf_terms<T, D>(rec + 2 * D, exp2_tab, x, t, v);
+                        const T s = e * rec[kAmp], k0 = e * points[16 * i + D];
+#pragma unroll
+                        for (int d = 0; d < D; ++d) v[d] *= s;
+                        rs[0] += k0;
+                        int at = 1 + D;
+#pragma unroll
+                        for (int a = 0; a < D; ++a) {
+                            const T kt = k0 * t[a];
+                            rs[1 + a] += kt;
+#pragma unroll
+                            for (int c = a; c < D; ++c) { rs[at] = fma_(kt, t[c], rs[at]); ++at; }
+                        }
+                    }
+                    if constexpr (NEED_GX) {
+                        const T w = row_sum_of_point<D>(v, lane);
+                        const int d = col == 0 ? 0 : col == 8 ? 1 : D == 3 && col == 4 ? 2 : -1;
+                        if (d >= 0) atomic_add(&result[gi][d][4 * i + row], w);
+                    }
                 }
             }
             T w[NR / 4 + 1];

@@ -960,3 +960,60 @@ def test_points_without_finite_coordinates_leave_the_gradients_of_the_others():
         got, gxes = _native.eval_bvh_bwd(g, m, bad, bvh, True, True)
         assert rel_l2(got.cpu().numpy(), want.cpu().numpy(), FLOOR[dtype]) <= TOL[dtype]
         assert bool((gxes[~keep] == 0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("D", [2, 3])
+@pytest.mark.parametrize("need", [(True, True), (True, False)])
+def test_pairs_outside_a_box_stay_out_of_the_gradients(dtype, D, need):
+    """points in no box with infinite and NaN upstream gradients (the value there is 0, and a logarithm or a root of it has
+    such a gradient), Gaussians with a NaN weight and points so far away that products with them overflow: the gradients of
+    everything outside the boxes concerned are those of the call without them"""
+    M, N = 150, 500
+    mix, xes, gout = _case(2, 2, M, N, D, 5300 + D, cov_radius=0.05 if D == 2 else 0.1)
+    mix, xes, gout = mix.to(dtype), xes.to(dtype), gout.to(dtype)
+    _, lo, up = _device_boxes(mix, xes, dtype, "tight")
+    inside = o.inside_mask(lo, up, xes.double().numpy())           # [B, L, M, N]
+    alone = torch.tensor(~inside.any(2))
+    assert 30 < int(alone[0, 0].sum()) < N // 2
+    m, x = mix.to(DEV), xes.to(DEV)
+
+    def grads(mixture, points, g):
+        b = _native.Bvh(mixture, x, 0.001, "tight")
+        _native.eval_bvh_fwd(mixture, points, b)
+        return [t.cpu() for t in _native.eval_bvh_bwd(g.to(DEV), mixture, points, b, *need)]
+
+    def same(got, want, keep):
+        assert int((~torch.isfinite(got[keep])).sum()) == 0
+        assert rel_l2(got[keep].numpy(), want[keep].numpy(), FLOOR[dtype]) <= TOL[dtype]
+
+    every_m = torch.ones(2, 2, M, dtype=torch.bool)
+    # upstream gradients of points in no box
+    bad = gout.clone()
+    at = alone.nonzero()
+    for i, value in enumerate((float("inf"), float("-inf"), float("nan"))):
+        b, l, n = at[i::3].unbind(1)
+        bad[b, l, n] = value
+    want, got = grads(m, x, gout.where(~alone, torch.zeros(()).to(dtype))), grads(m, x, bad)
+    same(got[0], want[0], every_m)
+    same(got[1], want[1], ~alone)
+    # Gaussians with a NaN weight (their boxes are finite): the gradients of the points outside of them are those of
+    # the call where they weigh nothing
+    heavy, light = mix.clone(), m.clone()
+    heavy[:, :, :60, 0], light[:, :, :60, 0] = float("nan"), 0
+    _, lo, up = _device_boxes(heavy, xes, dtype, "tight")
+    outside = torch.tensor(~o.inside_mask(lo, up, xes.double().numpy())[:, :, :60].any(2))
+    assert int(outside.sum()) > 4 * N // 2
+    same(grads(heavy.to(DEV), x, gout)[1], grads(light, x, gout)[1], outside)
+    # finite points far away: C t overflows, and then t t^T
+    far = x.clone()
+    scale = 1e38 if dtype == torch.float32 else 1e308
+    far[:, :, 45], far[:, :, 46, 0], far[:, :, 47] = scale, -scale, 0.01 * scale
+    gone = gout.clone()
+    gone[:, :, 45:48] = 0
+    want, got = grads(m, x, gone), grads(m, far, gout)
+    same(got[0], want[0], every_m)
+    near = torch.ones(2, 2, N, dtype=torch.bool)
+    near[:, :, 45:48] = False
+    same(got[1], want[1], near)
+    assert bool((got[1][:, :, 45:48] == 0).all())
