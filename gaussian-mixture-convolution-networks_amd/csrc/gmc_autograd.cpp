@@ -39,6 +39,34 @@ gmc_shape shape_of(const Tensor& mixture, const Tensor& xes) {
                      int(xes.size(0)), int(xes.size(1)), mixture.scalar_type() == at::kFloat ? GMC_F32 : GMC_F64};
 }
 
+// Rules and messages of check_input and eval_bwd in gmc/_native.py, for the backward pass: a hook on saved tensors may hand
+// back anything in their place.
+void check_saved(const Tensor& mixture, const Tensor& xes, const Tensor& grad_out) {
+    TORCH_CHECK(mixture.dim() == 4, "mixture must have 4 dimensions");
+    TORCH_CHECK(mixture.size(3) == 7 || mixture.size(3) == 13, "mixture must have 7 or 13 elements in the last dimension");
+    TORCH_CHECK(mixture.is_contiguous(), "mixture must be contiguous");
+    TORCH_CHECK(xes.is_contiguous(), "xes must be contiguous");
+    TORCH_CHECK(xes.dim() == 4, "xes must have 4 dimensions");
+    TORCH_CHECK(xes.scalar_type() == mixture.scalar_type(), "mixture and xes must have the same dtype");
+    TORCH_CHECK(xes.device() == mixture.device(), "mixture and xes must have the same device");
+    TORCH_CHECK(mixture.scalar_type() == at::kFloat || mixture.scalar_type() == at::kDouble,
+                "unsupported datatype: evaluate_inversed is implemented for float32 and float64");
+    TORCH_CHECK(xes.size(0) == 1 || xes.size(0) == mixture.size(0), "xes must have a batch dimension equal to one or the mixture");
+    TORCH_CHECK(xes.size(1) == 1 || xes.size(1) == mixture.size(1), "xes must have a layer dimension equal to one or the mixture");
+    TORCH_CHECK(xes.size(3) == (mixture.size(3) == 7 ? 2 : 3),
+                "xes must have the last dimension equal to the number of dimensions of the mixture");
+    TORCH_CHECK(mixture.is_cuda(), "gmc_hip evaluates on an AMD GPU only: mixture and xes must be HIP ('cuda') tensors; "
+                                   "this build has no CPU implementation");
+    for (int i = 0; i < 3; ++i)
+        TORCH_CHECK(mixture.size(i) <= INT_MAX && xes.size(i) <= INT_MAX, "gmc_hip: ", gmc_error_string(GMC_E_SHAPE));
+    TORCH_CHECK(grad_out.dim() == 3, "grad_output has wrong number of dimensions");
+    TORCH_CHECK(grad_out.size(0) == mixture.size(0), "grad_output has wrong batch dimension");
+    TORCH_CHECK(grad_out.size(1) == mixture.size(1), "grad_output has wrong layer dimension");
+    TORCH_CHECK(grad_out.size(2) == xes.size(2), "grad_output has wrong xes dimension");
+    TORCH_CHECK(grad_out.scalar_type() == mixture.scalar_type(), "grad_output dtype does not match with mixture dtype");
+    TORCH_CHECK(grad_out.device() == mixture.device(), "grad_output must live on the device of the mixture");
+}
+
 Tensor forward(const Tensor& mixture, const Tensor& xes, bool covariance_form) {
     const gmc_shape s = shape_of(mixture, xes);
     const c10::DeviceGuard guard(mixture.device());
@@ -62,6 +90,7 @@ struct Evaluate : public torch::autograd::Function<Evaluate<COVARIANCE>> {
         {
             const at::AutoGradMode off(false);
             const Tensor mixture = saved[0].detach(), xes = saved[1].detach(), grad_out = grads[0].detach().contiguous();
+            check_saved(mixture, xes, grad_out);
             const gmc_shape s = shape_of(mixture, xes);
             const c10::DeviceGuard guard(mixture.device());
             if (want_mixture) result[0] = at::empty_like(mixture);

@@ -891,6 +891,12 @@ def test_native_autograd_behaves_like_the_python_function():
                 out = apply(m, x)
             return torch.autograd.grad(out, (m, x), gout)
 
+        def replaced(change, which):
+            """saved tensors (0: mixture, 1: points) that come back as something else: refused before anything reads them"""
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: change(t) if which[t.shape[3] == 2] else t):
+                out = apply(m, x)
+            return torch.autograd.grad(out, (m, x), gout)
+
         def changed():
             inner = m * 1.0
             out = apply(inner, x)
@@ -920,6 +926,10 @@ def test_native_autograd_behaves_like_the_python_function():
             lambda: torch.autograd.grad(apply(torch.nn.Parameter(mix), x), x, gout),
             lambda: torch.autograd.grad(apply(m.double(), x.double()), (m, x), gout.double()),
             lambda: second(gout), lambda: second(gout.clone().requires_grad_(True)), hooked, changed, dual, on_a_stream, without_grad,
+            *[lambda f=f, w=w: replaced(f, w) for w in ((1, 0), (0, 1), (1, 1)) for f in (
+                lambda t: t.transpose(0, 1).contiguous().transpose(0, 1), lambda t: t.half(), lambda t: t.bfloat16(), lambda t: t.double(),
+                lambda t: t.cpu(), lambda t: t[0], lambda t: t[:, :2].contiguous(), lambda t: t[..., :1].contiguous(),
+                lambda t: t.expand(3, 2, *t.shape[1:])[:, 0], lambda t: torch.cat((t, t), 2) if t.shape[3] == 2 else t[0])],
             lambda: torch.vmap(lambda a: apply(a, xes))(mix.unsqueeze(0)), lambda: torch.func.grad(lambda a: apply(a, xes).sum())(mix),
             lambda: torch.func.jvp(lambda a: apply(a, xes), (mix,), (mix,)), lambda: apply(mix.cpu(), xes.cpu()),
             lambda: apply(mix[0], xes), lambda: apply(mix.half(), xes.half()), lambda: apply(mix.double(), xes),
