@@ -2014,7 +2014,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
 
     // The backward pass with per-Gaussian sums: lanes = leaves.  The four rows of a wavefront hold the same 16 leaves of a
     // batch and walk over the 64 points of the group, a point per row and step, so the ten sums of a leaf stay in the
-    // lane's registers (over rows and to memory once per batch), and only dL/dx of a point is added over the 16
+    // lane's registers, in double (over rows and, rounded, to memory once per batch), and only dL/dx of a point is added over the 16
     // lanes of its row, four points at a time (row_sums_of_four).  Only pairs inside a box enter anything: upstream gradients,
     // amplitudes and, far away, t and u may be infinite or NaN, so the others are left out instead of multiplied by zero.
     auto evaluate_by_leaves = [&]() {
@@ -2036,9 +2036,9 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
             for (int k = 0; k < kAmp + 1; ++k) rec[k] = from[k];
             const int comp = reinterpret_cast<const int*>(from + kAmp + 1)[0];
-            T rs[NR];
+            double rs[NR];
 #pragma unroll
-            for (int k = 0; k < NR; ++k) rs[k] = T(0);
+            for (int k = 0; k < NR; ++k) rs[k] = 0.0;
             // point 4 i + row of the group at points[16 i]
             const T* points = pts[gi] + 4 * row;
             if constexpr (sizeof(T) == 4) {
@@ -2065,7 +2065,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
                             t[i][d] = in[i] ? t[i][d] : T(0);
                             if (NEED_GX) u[i][d] = in[i] ? s * u[i][d] : T(0);
                         }
-                        // (the four steps are summed on their own first, which halves the rounding error of the sums)
+                        // (float sums of four points; everything beyond them is added in double)
                         const T k0 = in[i] ? e[i] * g[i] : T(0);
                         part[0] = i == 0 ? k0 : part[0] + k0;
                         int at = 1 + D;
@@ -2078,7 +2078,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
                         }
                     }
 #pragma unroll
-                    for (int k = 0; k < NR; ++k) rs[k] += part[k];
+                    for (int k = 0; k < NR; ++k) rs[k] += double(part[k]);
                     if constexpr (NEED_GX) {
                         T sum[D];
                         slow_issue_begin(u[3]);
@@ -2120,14 +2120,11 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
                     }
                 }
             }
+            double total[NR / 4 + 1];
+            sums_over_rows(rs, total);
             T w[NR / 4 + 1];
-            if constexpr (sizeof(T) == 4) {
-                slow_issue_begin(rs);
-                sums_over_rows(rs, w);
-                slow_issue_end(w);
-            } else {
-                sums_over_rows(rs, w);
-            }
+#pragma unroll
+            for (int q = 0; q < NR / 4 + 1; ++q) w[q] = T(total[q]);
             if (active) {
                 T* dst = sums + (size_t(bl) * M + comp) * NR;
                 const int mine = (row >> 1) | ((row & 1) << 1);

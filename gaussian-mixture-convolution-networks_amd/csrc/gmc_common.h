@@ -641,17 +641,6 @@ __device__ __forceinline__ double row_sum_of_point(const double (&v)[D], int lan
 // a and b hold one value per lane each: afterwards the even rows (ROWS = 16) or the lower half (32) hold the sums of a over
 // the pairs of rows (halves), the others those of b
 template <int ROWS>
-__device__ __forceinline__ float swap_sum(float a, float b) {
-    const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
-    if constexpr (ROWS == 32) {
-        const auto r = __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
-        return __builtin_bit_cast(float, unsigned(r[0])) + __builtin_bit_cast(float, unsigned(r[1]));
-    } else {
-        const auto r = __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
-        return __builtin_bit_cast(float, unsigned(r[0])) + __builtin_bit_cast(float, unsigned(r[1]));
-    }
-}
-template <int ROWS>
 __device__ __forceinline__ double swap_sum(double a, double b) {
     const unsigned long long ua = __builtin_bit_cast(unsigned long long, a), ub = __builtin_bit_cast(unsigned long long, b);
     unsigned x[2], y[2];
@@ -671,10 +660,10 @@ __device__ __forceinline__ double swap_sum(double a, double b) {
 // NR = 10 or 6 values per lane summed over the four rows (lanes with the same lane & 15): row r holds the sums
 // 4 q + (r >> 1 | (r & 1) << 1) in w[q] for q < NR / 4; the last two sums are in w[NR / 4], the first of them in the rows 0 and 1
 // (the same in both), the second in the rows 2 and 3.
-template <typename T, int NR>
-__device__ __forceinline__ void sums_over_rows(const T (&v)[NR], T (&w)[NR / 4 + 1]) {
+template <int NR>
+__device__ __forceinline__ void sums_over_rows(const double (&v)[NR], double (&w)[NR / 4 + 1]) {
     static_assert(NR % 4 == 2, "pairs of pairs and one pair");
-    T h[NR / 2];
+    double h[NR / 2];
 #pragma unroll
     for (int i = 0; i < NR / 2; ++i) h[i] = swap_sum<32>(v[2 * i], v[2 * i + 1]);
 #pragma unroll

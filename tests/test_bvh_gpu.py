@@ -1017,3 +1017,29 @@ def test_pairs_outside_a_box_stay_out_of_the_gradients(dtype, D, need):
     near[:, :, 45:48] = False
     same(got[1], want[1], near)
     assert bool((got[1][:, :, 45:48] == 0).all())
+
+
+@pytest.mark.parametrize("D", [2, 3])
+def test_few_points_of_a_leaf_are_added_in_double(D):
+    """three points at one place in a leaf's box whose upstream gradients 2^24, 1, -2^24 (in every order) cancel: float32
+    sums of a leaf would lose the 1; the gradients are those of the point with the 1 alone"""
+    orders = [(24, 0, -24), (24, -24, 0), (0, 24, -24), (0, -24, 24), (-24, 0, 24), (-24, 24, 0)]
+    M, inside = 100, 21                                  # 63 points: one group; neighbours of the Morton order meet in one leaf
+    mix = torch.zeros(1, 1, M, 1 + D + D * D)
+    mix[..., 0] = torch.linspace(0.5, 2.0, M)
+    i = torch.arange(M)
+    mix[0, 0, :, 1], mix[0, 0, :, 2] = (i % 10).float(), (i // 10).float()
+    for d in range(D):
+        mix[..., 1 + D + d * (D + 1)] = 1e4 * (1 + 0.1 * d)                      # boxes that do not meet
+    at = mix[0, 0, :inside, 1:1 + D] + 0.004 * torch.tensor([1.0, -1.5, 0.7])[:D]
+    xes = at.repeat_interleave(3, 0)[None, None]
+    # sign and power of two of each upstream gradient; 0 stands for the 1
+    g = torch.tensor([[0.0 if p == 0 else float(np.sign(p)) * 2.0 ** abs(p) for p in orders[k % 6]] for k in range(inside)])
+    alone = torch.tensor([[1.0 if p == 0 else 0.0 for p in orders[k % 6]] for k in range(inside)])
+    g = (g + alone).view(1, 1, -1)
+    m, x = mix.to(DEV), xes.to(DEV)
+    bvh = _native.Bvh(m, x, 0.001, "tight")
+    _native.eval_bvh_fwd(m, x, bvh)
+    got, want = (_native.eval_bvh_bwd(v.to(DEV), m, x, bvh, True, True)[0][0, 0].cpu() for v in (g, alone.view(1, 1, -1)))
+    assert bool((want[:inside, 0] > 0).all()) and bool((want[inside:] == 0).all())
+    assert torch.allclose(got, want, rtol=1e-6, atol=0.0)
