@@ -1730,9 +1730,14 @@ __device__ __forceinline__ void group_boxes(const T (&x)[D], bool valid, int lan
 // mixture phase 2 turns round (evaluate_by_leaves, lanes = leaves): a lane keeps a candidate leaf and its ten sums in
 // registers and walks over the points, so a leaf's sums are reduced over four lanes once per 64 points instead of over
 // the wavefront or, hit by hit, with ten LDS atomics; of the pairs of a candidate a fifth (100000 points over
-// 16384 leaves on a surface) to a hundredth (1000 points) lie inside its box.  Measured, backward pass, lanes = points with reductions and LDS atomics / lanes = leaves:
-//   63 trees of 500 leaves, 4001 points each, float32 165 / 118 us;  one tree of 16384, 100000 points, float64 75 / 62,
-//   float32 67 / 48;  800 trees of 128 at 784 points, 2-D float32 138 / 106;  25 trees of 200 at 2000, float64 42 / 38
+// 16384 leaves on a surface) to a hundredth (1000 points) lie inside its box.  Measured, backward pass with its epilogue,
+// lanes = points with reductions and LDS atomics / lanes = leaves, us:
+//   63 trees of 500 leaves, 4001 points each, float32 166 / 120, float64 234 / 155;  one tree of 16384, 100000 points,
+//   float32 59 / 43, float64 77 / 52 (5000 points 79 / 73, 68 / 58; 1000 points 118 / 117, 126 / 104);  800 trees of 128 at
+//   784 points, 2-D, float32 137 / 107, float64 250 / 198;  25 trees of 200 at 2000 32 / 25, 42 / 30
+// In float64 the hits are taken lane by lane: with a step of the whole wavefront per point and row (and row sums of dL/dx)
+// the pass took 185, 65, 101, 193, 184, 41 us in this order.  (Both loops, chosen per 16 leaves by how many points lie inside:
+// 3 - 10 % slower than lane by lane in 3-D, 3 % faster where half of all pairs hit.)
 // Bound by vector issue (float32: 37 instructions and a row sum of six per four points and 16 leaves) and the fixed 5 us of a
 // workgroup.
 template <typename T, int D, int MODE, bool NEED_GM, bool NEED_GX>
@@ -2015,7 +2020,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
     // The backward pass with per-Gaussian sums: lanes = leaves.  The four rows of a wavefront hold the same 16 leaves of a
     // batch and walk over the 64 points of the group, a point per row and step, so the ten sums of a leaf stay in the
     // lane's registers, in double (over rows and, rounded, to memory once per batch), and only dL/dx of a point is added over the 16
-    // lanes of its row, four points at a time (row_sums_of_four).  Only pairs inside a box enter anything: upstream gradients,
+    // lanes of its row, four points at a time (row_sums_of_four; double: by additions in LDS).  Only pairs inside a box enter anything: upstream gradients,
     // amplitudes and, far away, t and u may be infinite or NaN, so the others are left out instead of multiplied by zero.
     auto evaluate_by_leaves = [&]() {
         const int row = lane >> 4, col = lane & 15;
@@ -2091,32 +2096,39 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
                     }
                 }
             } else {
-                // (more than one point at a time would not fit into the registers)
-#pragma unroll 1
+                // double: the box tests first, then every lane its own hits; a step of all lanes for every point, hit or not, took
+                // longer than lanes = points where few points meet many leaves (see above).  The lanes of a row start at different
+                // points, so that their additions to dL/dx seldom meet.
+                unsigned mine = 0u;
+#pragma unroll 8
                 for (int i = 0; i < kWave / 4; ++i) {
-                    T x[D], v[D];
+                    T x[D];
 #pragma unroll
-                    for (int d = 0; d < D; ++d) { x[d] = points[16 * i + d]; v[d] = T(0); }
-                    if (active & inside_box<T, D>(x, rec)) {
-                        T t[D];
-                        const T e = leaf_terms<T, D>(rec + 2 * D, exp2_tab, x, t, v);
-                        const T s = e * rec[kAmp], k0 = e * points[16 * i + D];
+                    for (int d = 0; d < D; ++d) x[d] = points[16 * i + d];
+                    mine |= (active & inside_box<T, D>(x, rec)) ? 1u << i : 0u;
+                }
+                mine = ((mine >> col) | (mine << (16 - col))) & 0xffffu;
+#pragma unroll 1
+                while (mine != 0u) {
+                    const int i = (__builtin_ctz(mine) + col) & 15;
+                    mine &= mine - 1u;
+                    T x[D], t[D], u[D];
 #pragma unroll
-                        for (int d = 0; d < D; ++d) v[d] *= s;
-                        rs[0] += k0;
-                        int at = 1 + D;
-#pragma unroll
-                        for (int a = 0; a < D; ++a) {
-                            const T kt = k0 * t[a];
-                            rs[1 + a] += kt;
-#pragma unroll
-                            for (int c = a; c < D; ++c) { rs[at] = fma_(kt, t[c], rs[at]); ++at; }
-                        }
-                    }
+                    for (int d = 0; d < D; ++d) x[d] = points[16 * i + d];
+                    const T e = leaf_terms<T, D>(rec + 2 * D, exp2_tab, x, t, u);
+                    const T s = e * rec[kAmp], k0 = e * points[16 * i + D];
                     if constexpr (NEED_GX) {
-                        const T w = row_sum_of_point<D>(v, lane);
-                        const int d = col == 0 ? 0 : col == 8 ? 1 : D == 3 && col == 4 ? 2 : -1;
-                        if (d >= 0) atomic_add(&result[gi][d][4 * i + row], w);
+#pragma unroll
+                        for (int d = 0; d < D; ++d) atomic_add(&result[gi][d][4 * i + row], double(s * u[d]));
+                    }
+                    rs[0] += k0;
+                    int at = 1 + D;
+#pragma unroll
+                    for (int a = 0; a < D; ++a) {
+                        const T kt = k0 * t[a];
+                        rs[1 + a] += kt;
+#pragma unroll
+                        for (int c = a; c < D; ++c) { rs[at] = fma_(kt, t[c], rs[at]); ++at; }
                     }
                 }
             }

@@ -622,22 +622,6 @@ __device__ __forceinline__ void row_sums_of_four(const float (&v)[4][2], float (
 }
 #undef GMC_ROR8
 #undef GMC_MIRROR
-// double: the D values of one point; the lanes 0, 8 and (D = 3) 4 of a row receive the sums of component 0, 1 and 2
-template <int D>
-__device__ __forceinline__ double row_sum_of_point(const double (&v)[D], int lane) {
-    const bool b3 = (lane & 8) != 0;
-    double k = (b3 ? v[1] : v[0]) + dpp_mov<0x128>(b3 ? v[0] : v[1]);            // row_ror:8
-    if constexpr (D == 3) {
-        const bool b2 = (lane & 4) != 0;
-        const double h = v[2] + dpp_mov<0x128>(v[2]);
-        k = (b2 ? h : k) + dpp_mov<0x141>(b2 ? k : h);                           // row_half_mirror
-    } else {
-        k += dpp_mov<0x141>(k);
-    }
-    k += dpp_mov<0x4e>(k);
-    return k + dpp_mov<0xb1>(k);
-}
-
 // a and b hold one value per lane each: afterwards the even rows (ROWS = 16) or the lower half (32) hold the sums of a over
 // the pairs of rows (halves), the others those of b
 template <int ROWS>

@@ -1043,3 +1043,39 @@ def test_few_points_of_a_leaf_are_added_in_double(D):
     got, want = (_native.eval_bvh_bwd(v.to(DEV), m, x, bvh, True, True)[0][0, 0].cpu() for v in (g, alone.view(1, 1, -1)))
     assert bool((want[:inside, 0] > 0).all()) and bool((want[inside:] == 0).all())
     assert torch.allclose(got, want, rtol=1e-6, atol=0.0)
+
+
+def test_backward_of_few_points_over_a_large_tree_in_double():
+    """1000 points over 16384 leaves on a surface: long lists, a pair in a hundred inside its box.  The float64 pass has to
+    leave the others out: it takes 0.9 times the float32 pass's time (1.65 times with every pair evaluated)"""
+    g = torch.Generator().manual_seed(5400)
+    M, N = 16384, 1000
+
+    def shell(n):
+        v = torch.randn(1, 1, n, 3, generator=g, dtype=torch.float64)
+        return v / v.norm(dim=-1, keepdim=True) + 0.01 * torch.randn(1, 1, n, 3, generator=g, dtype=torch.float64)
+    r = torch.linalg.qr(torch.randn(1, 1, M, 3, 3, generator=g, dtype=torch.float64))[0]
+    cov = (r * (1e-5 + 1e-3 * torch.rand(1, 1, M, 1, 3, generator=g, dtype=torch.float64))) @ r.transpose(-1, -2)
+    mix = torch.cat((torch.rand(1, 1, M, 1, generator=g, dtype=torch.float64), shell(M), torch.linalg.inv(cov).flatten(-2)), -1)
+    xes, gout = shell(N), torch.randn(1, 1, N, generator=g, dtype=torch.float64)
+    graphs, best = {}, {}
+    for dtype in (torch.float32, torch.float64):
+        m, x, go = (t.to(dtype).to(DEV) for t in (mix, xes, gout))
+        bvh = _native.Bvh(m, x, 0.001, "tight")
+        _native.eval_bvh_fwd(m, x, bvh)
+        _native.eval_bvh_bwd(go, m, x, bvh, True, True)
+        torch.cuda.synchronize()
+        graphs[dtype] = graph = torch.cuda.CUDAGraph()
+        graph.tensors = (m, x, go, bvh)
+        with torch.cuda.graph(graph):
+            for _ in range(5):
+                graph.result = _native.eval_bvh_bwd(go, m, x, bvh, True, True)
+    for _ in range(20):
+        for dtype, graph in graphs.items():
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            best[dtype] = min(best.get(dtype, 1e9), start.elapsed_time(end))
+    assert best[torch.float64] < 1.3 * best[torch.float32], best
