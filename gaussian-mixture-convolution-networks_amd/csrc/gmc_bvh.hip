@@ -1967,7 +1967,7 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
         for (int d = 0; d < D; ++d) gx[d] = T(0);
         while (cur_group == gi) {
-            const int cnt = cur_end - cur_base < kStageBatch ? cur_end - cur_base : kStageBatch;
+            const int cnt = cur_end - cur_base < kBatch ? cur_end - cur_base : kBatch;
 #pragma unroll
             for (int r = 0; r < kPre; ++r) {
                 const int s = lane + r * kWave;
@@ -2263,8 +2263,8 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
         for (int gi = 0; gi < groups; ++gi) {
             const int n_leaf = state[gi][0];
             left_on_stack |= state[gi][1] > 0;
-            if (NEED_GM || n_leaf == 0) continue;                       // uniform over the workgroup
-            evaluate_share(gi);
+            if constexpr (!NEED_GM)
+                if (n_leaf > 0) evaluate_share(gi);                     // uniform over the workgroup
         }
         if constexpr (NEED_GM) evaluate_by_leaves();
         if (MODE == 0) {
@@ -2832,7 +2832,7 @@ static int bvh_fwd_t(const T* xes, char* bvh, T* out, const gmc_shape& s, hipStr
     int chunks = (s.N + kWave * groups - 1) / (kWave * groups);
     // A launch that would leave resident slots empty is spread over all of them: workgroups whose last wavefront
     // finds no group left serve one group fewer (1563 groups: 512 workgroups of 3 or 4 instead of 391 of 4, 50.6 -> 46.5 us).
-    if (groups > 1 && BL * size_t(chunks) < size_t(kTravSlots)) {
+    if (groups > 1 && g_traversal_groups[0] == 0 && BL * size_t(chunks) < size_t(kTravSlots)) {
         const size_t per_mixture = (size_t(s.N) + kWave - 1) / kWave, fill = size_t(kTravSlots) / BL;
         chunks = int(fill < per_mixture ? fill : per_mixture);
     }
@@ -2883,7 +2883,8 @@ static int bvh_bwd_t(const T* grad_out, const T* mixture, const T* xes, char* bv
     }
     const int groups = traversal_groups(BL, s.M, s.N, true, gm);
     int chunks = (s.N + kWave * groups - 1) / (kWave * groups);
-    if (groups > 1 && BL * size_t(chunks) < size_t(kTravSlots)) {       // (as in the forward pass: no resident slot left empty)
+    // (as in the forward pass: no resident slot left empty)
+    if (groups > 1 && g_traversal_groups[1] == 0 && BL * size_t(chunks) < size_t(kTravSlots)) {
         const size_t per_mixture = (size_t(s.N) + kWave - 1) / kWave, fill = size_t(kTravSlots) / BL;
         chunks = int(fill < per_mixture ? fill : per_mixture);
     }

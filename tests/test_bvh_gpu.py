@@ -933,16 +933,47 @@ def test_step_is_capturable_in_a_hip_graph():
 @pytest.mark.parametrize("D", [2, 3])
 def test_backward_by_leaves_at_the_edges_of_its_batches(dtype, D):
     """the backward traversal keeps 16 candidate leaves per wavefront and walks over the 64 points of a group: leaf counts on
-    both sides of a batch, of the eight wavefronts and of several groups' batches dealt in turn; groups of 1 ... 64 points;
-    wide boxes, so that every leaf is a candidate of every group"""
+    both sides of a batch, of the eight wavefronts and, with two to four groups per workgroup, of several groups' batches dealt
+    in turn; groups of 1 ... 64 points; wide boxes, so that every leaf is a candidate of every group"""
     lib = _native.lib()
     lib.gmc_bvh_set_eval_path(1)
     try:
         for M, N in ((1, 1), (2, 65), (15, 64), (16, 63), (17, 130), (127, 64), (128, 257), (129, 300), (145, 1)):
             mix, xes, gout = _case(2, 2, M, N, D, 5000 + 10 * M + D, cov_radius=2.0)
-            _check_culled(mix, xes, gout, dtype, "tight", tag=f"{M} leaves, {N} points, {D}-D")
+            for groups in range(1, min(4, (N + 63) // 64) + 1):
+                lib.gmc_bvh_set_traversal_groups(0, groups)
+                _check_culled(mix, xes, gout, dtype, "tight", tag=f"{M} leaves, {N} points, {D}-D, {groups} groups")
     finally:
         lib.gmc_bvh_set_eval_path(0)
+        lib.gmc_bvh_set_traversal_groups(0, 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_batches_of_groups_with_lists_of_any_length(dtype):
+    """three groups of 64 points served by one workgroup, the middle one (or the first, or the last) without a candidate; the
+    lists of the others end just before, at and just behind a batch of 16 leaves, so that the wavefront that takes a group's
+    last batch and the one that takes the next group's first change"""
+    lib = _native.lib()
+    try:
+        for k, (first, last) in enumerate(((15, 16), (16, 17), (17, 15), (1, 33), (112, 1), (127, 129), (128, 128), (129, 127))):
+            for empty in range(3):
+                # clusters along the diagonal follow each other in Morton order: one group of 64 points at each
+                centre = [torch.tensor([c, c, c]) for c in (0.0, 10.0, 20.0)]
+                counts = [first, last]
+                counts.insert(empty, 0)
+                g = torch.Generator().manual_seed(5500 + 10 * k + empty)
+                mix = synthetic.random_inversed_mixture(1, 2, first + last, 3, g, pos_radius=1.0, cov_radius=0.3, dtype=torch.float64)
+                mix[..., 1:4] = mix[..., 1:4].clamp(-1, 1) + torch.cat([c.expand(n, 3) for c, n in zip(centre, counts)]).double()
+                xes = torch.cat([c + 2 * torch.rand(1, 2, 64, 3, generator=g, dtype=torch.float64) - 1 for c in centre], 2)
+                gout = torch.randn(1, 2, 192, generator=g, dtype=torch.float64)
+                for groups in (2, 3, 4):
+                    lib.gmc_bvh_set_eval_path(1)
+                    lib.gmc_bvh_set_traversal_groups(0, groups)
+                    out, _ = _check_culled(mix, xes, gout, dtype, "tight", tag=f"{counts} leaves, {groups} groups")
+                    assert not out[:, :, 64 * empty:64 * empty + 64].any()
+    finally:
+        lib.gmc_bvh_set_eval_path(0)
+        lib.gmc_bvh_set_traversal_groups(0, 0)
 
 
 def test_points_without_finite_coordinates_leave_the_gradients_of_the_others():
