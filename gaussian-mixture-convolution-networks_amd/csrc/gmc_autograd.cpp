@@ -17,6 +17,7 @@
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 
 #include "gmc_hip.h"
 
@@ -164,9 +165,13 @@ PyObject* evaluate(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// versions() -> ABI version of the header this file was built from, of the library it is linked to, version of torch's headers
+PyObject* versions(PyObject*, PyObject*) { return Py_BuildValue("iis", GMC_ABI_VERSION, gmc_abi_version(), TORCH_VERSION); }
+
 PyMethodDef methods[] = {
     {"evaluate", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(evaluate)), METH_FASTCALL,
      "evaluate(mixture, xes, covariance_form) -> values, or None for what is not a plain device tensor or not accepted"},
+    {"versions", versions, METH_NOARGS, "versions() -> (ABI version of the header, of the library, version of torch's headers)"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_gmc_autograd", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

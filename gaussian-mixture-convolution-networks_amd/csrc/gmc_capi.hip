@@ -39,7 +39,7 @@ int check_shape(const gmc_shape* s) {
 
 extern "C" {
 
-int gmc_abi_version(void) { return 12; }
+int gmc_abi_version(void) { return GMC_ABI_VERSION; }
 
 const char* gmc_error_string(int code) {
     switch (code) {

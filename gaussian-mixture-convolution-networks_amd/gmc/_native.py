@@ -39,14 +39,15 @@ def build(verbose: bool = False) -> str:
     """Compiles every HIP source of the library for gfx950 (hipcc cross-compiles without a GPU) and the C++ autograd of the
     dense evaluation for the torch of this interpreter."""
     out = None if verbose else subprocess.DEVNULL
-    subprocess.run(["make", "-B", "-j8", "-C", CSRC_DIR, f"PYTHON={sys.executable}", "_gmc_autograd.so"], check=True, stdout=out,
+    subprocess.run(["make", "-B", "-j8", "-C", CSRC_DIR, f"PYTHON={sys.executable}", "all"], check=True, stdout=out,
                    stderr=out)
-    global _lib
-    _lib = None
+    global _lib, native_evaluate
+    _lib = native_evaluate = None
     return LIB_PATH
 
 
 _lib = None
+native_evaluate = None      # evaluate() of _gmc_autograd.so or what stands in for it (cpp/extensions/evaluate_inversed)
 
 
 def lib() -> ctypes.CDLL:

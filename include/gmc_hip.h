@@ -42,7 +42,8 @@ typedef struct gmc_shape {
 } gmc_shape;
 
 const char* gmc_error_string(int code);
-/* ABI version of this header; bumps when a signature changes */
+/* ABI version of this header; bumps when a signature changes.  gmc_abi_version: of the header that the library was built from. */
+#define GMC_ABI_VERSION 12
 int gmc_abi_version(void);
 
 /* ---- dense all-pairs evaluation --------------------------------------------------------------------

@@ -268,3 +268,37 @@ def test_native_autograd_leaves_host_tensors_to_the_python_classes():
     for apply in (binding.apply, binding.apply_covariance):
         with pytest.raises(RuntimeError, match="AMD GPU only"):
             apply(m, x)
+
+
+def test_make_builds_both_libraries_by_default():
+    """what the build notes and the error of a missing library name: plain make builds the autograd extension too"""
+    commands = subprocess.run(["make", "-n", "-B", "-C", _native.CSRC_DIR], check=True, capture_output=True, text=True).stdout
+    assert "-o libgmc_hip.so" in commands and "-o _gmc_autograd.so" in commands
+
+
+def test_native_autograd_of_another_build_is_not_used(monkeypatch, tmp_path):
+    """an extension from another include/gmc_hip.h (its gmc_shape may be another) or another torch, or none: a warning, and every
+    call goes through the Python classes"""
+    _native.lib()
+
+    def refused(match):
+        with pytest.warns(UserWarning, match=match):
+            evaluate = ei._load_native_autograd()
+        assert evaluate(None, None, False) is None and evaluate.__module__ == ei.__name__
+    with monkeypatch.context() as m:
+        m.setattr(_native, "ABI_VERSION", _native.ABI_VERSION + 1)
+        refused("different include/gmc_hip.h")
+    with monkeypatch.context() as m:
+        m.setattr(torch, "__version__", "1.2.3")
+        refused("built for torch " + torch.version.__version__.split("+")[0])
+    with monkeypatch.context() as m:
+        m.setattr(_native, "CSRC_DIR", str(tmp_path))
+        refused("is missing")
+    assert getattr(ei._load_native_autograd(), "__module__", None) != ei.__name__
+    # a build replaces the choice that a process has made before it
+    with monkeypatch.context() as m:
+        m.setattr("subprocess.run", lambda *a, **k: None)
+        m.setattr(_native, "_lib", None)
+        m.setattr(_native, "native_evaluate", lambda *a: None)
+        _native.build()
+        assert _native.native_evaluate is None
