@@ -251,7 +251,8 @@ __device__ __forceinline__ void bwd_rc_pairs(const T* __restrict__ lds, const T*
                 if (idx >= 0 && k >= 0) {
                     // float: every wavefront meets every Gaussian of a tile once and has its own copy of the sums, so a
                     // plain store does (LDS float atomics are serialised lane by lane); double: one copy
-                    if constexpr (OWN_SUMS) block_sums[idx * NR + k] = total[0]; else atomic_add(&block_sums[idx * NR + k], total[0]);
+                    static_assert(OWN_SUMS, "");
+                    block_sums[idx * NR + k] = total[0];
                 }
             } else {
                 // two sums at a time: the halves of a row first exchange the sum they do not keep (lanes 0-7 keep the even

@@ -245,7 +245,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     using Tile = MTile<D, D, T>;
     constexpr int kSlots = Tile::kSlots;
     // 16-point groups whose exponentials are issued together: 2048 x 512 Gaussians at 8192 points in 3-D one 1743, two 1744,
-    // four 1773 us (1766 without the batch); 100 x 1280 at 10000 shared points in 2-D 241 / 250 / 258 (247)
+    // four 1773 us (1766 without the batch); 100 x 1280 at 10000 shared points in 2-D 241 / 250 / 258 (247).  The kernel alone;
+    // behind a backward pass that leaves a clock of 2190 instead of 2370 MHz the batch gains nothing (0.627 / 0.628 of peak at
+    // equal clock).
     constexpr int kBatch = 1;
     __shared__ Tile t;
 
