@@ -1733,13 +1733,13 @@ __device__ __forceinline__ void group_boxes(const T (&x)[D], bool valid, int lan
 // 16384 leaves on a surface) to a hundredth (1000 points) lie inside its box.  Measured, backward pass with its epilogue,
 // lanes = points with reductions and LDS atomics / lanes = leaves, us:
 //   63 trees of 500 leaves, 4001 points each, float32 166 / 120, float64 234 / 155;  one tree of 16384, 100000 points,
-//   float32 59 / 43, float64 77 / 52 (5000 points 79 / 73, 68 / 58; 1000 points 118 / 117, 126 / 104);  800 trees of 128 at
+//   float32 59 / 44, float64 77 / 51 (5000 points 78 / 73, 68 / 58; 1000 points 119 / 117, 126 / 104);  800 trees of 128 at
 //   784 points, 2-D, float32 137 / 107, float64 250 / 198;  25 trees of 200 at 2000 32 / 25, 42 / 30
 // In float64 the hits are taken lane by lane: with a step of the whole wavefront per point and row (and row sums of dL/dx)
 // the pass took 185, 65, 101, 193, 184, 41 us in this order.  (Both loops, chosen per 16 leaves by how many points lie inside:
 // 3 - 10 % slower than lane by lane in 3-D, 3 % faster where half of all pairs hit.)
-// Bound by vector issue (float32: 37 instructions and a row sum of six per four points and 16 leaves) and the fixed 5 us of a
-// workgroup.
+// Bound by vector issue (float32: every point of a group against every leaf of its list, and the sums of four points
+// widened to double) and, float64, by the box tests and the additions in LDS; the fixed 5 us of a workgroup.
 template <typename T, int D, int MODE, bool NEED_GM, bool NEED_GX>
 __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4))) void bvh_traverse_kernel(
         const T* __restrict__ xes, const int* __restrict__ p_order, const T* __restrict__ child_box,
@@ -2332,10 +2332,16 @@ __global__ __launch_bounds__(kTravBlock) __attribute__((amdgpu_waves_per_eu(4)))
 // 4096 points, forward / backward us without the tree against the traversal: 32 leaves 16 / 28 against 21 / 40 (6 % of
 // the pairs inside a box; the same ratio at 0.1 %), 64 leaves 25 / 44 against 23 / 49, and with a quarter of the pairs
 // inside (336 mixtures) 78 / 159 against 130 / 262; from 128 leaves on the traversal wins unless most boxes contain
-// most points (22 / 42 against 39 / 56 at 0.6 % inside).  With the traversal's backward pass on lanes = leaves, random
-// mixtures: 32 leaves in 3-D 14 / 33 against 20 / 33, 64 leaves 23 / 53 against 23 / 49 (336 mixtures: 72 / 127
-// against 88 / 170; in 2-D 46 / 78 against 74 / 110), 48 leaves (200 mixtures) 42 / 77 against 52 / 91: the line stays.  Mixtures of at most kAllPairsMax components are therefore
-// evaluated without the tree: the leaf records of the mixture (own box + evaluation record,
+// most points (22 / 42 against 39 / 56 at 0.6 % inside).  Those are figures of the traversal with lanes = points in the
+// backward pass.  With lanes = leaves the line depends on the number of mixtures (random mixtures, 4096 points each, tight
+// boxes, float32; forward / backward us without the tree | traversal):
+//   leaves       16 mixtures, 3-D         64, 3-D                  336, 3-D                   64, 2-D                  336, 2-D
+//   32           10 / 23 |  9 / 17        15 / 33 | 20 / 34        47 /  77 | 74 / 132        11 / 21 | 16 / 22        26 / 46 | 64 /  89
+//   48           13 / 32 | 10 / 18        19 / 43 | 22 / 41        61 / 101 | 81 / 146        15 / 30 | 18 / 25        37 / 62 | 69 / 103
+//   64           16 / 40 | 10 / 20        23 / 53 | 24 / 49        74 / 129 | 88 / 169        18 / 36 | 18 / 29        47 / 79 | 75 / 113
+// (float64 alike: 64 leaves 3-D 19 / 49 | 13 / 23, 34 / 81 | 33 / 62, 120 / 221 | 139 / 248).  The rule does not know it yet: it
+// is right for launches of hundreds of mixtures and costs up to half of the backward pass below 64.  Mixtures of at most
+// kAllPairsMax components are evaluated without the tree: the leaf records of the mixture (own box + evaluation record,
 // as the build left them) are staged in LDS, a wavefront owns P groups of 64 Morton-neighbouring points (lanes =
 // points), walks over ALL leaves and applies the per-point rule of lbvh/aabb.h:39-47 itself; a leaf is evaluated for a
 // group only when its box contains at least one of the group's points (one ballot: neighbouring points mostly agree).
@@ -2792,16 +2798,17 @@ static int bvh_build_t(const T* mixture, const T* xes, char* bvh, const gmc_shap
 // groups spread over exactly one round of resident workgroups are 3-6 % ahead at 1563 groups when the same backward
 // pass is repeated on one tree, and not ahead in a step that builds, traverses forward and backward: not taken.)  The
 // lists of many small trees are short and the fixed work of a workgroup weighs more: their backward launches take the
-// forward rule (64 trees of 512 leaves, 4096 groups: 72 us with 4 against 79 with 3 and 98 with 1; 256 trees of 200
-// leaves, 3328 groups: 44 us with 4, 46 with 2, 52 with 1).
+// forward rule (256 trees of 200 leaves, 3328 groups: 67 us with 4, 70 with 2, 80 with 1), and so does every backward pass with
+// lanes = leaves, where few groups per workgroup leave wavefronts without a batch of leaves: automatic (spread over the
+// resident slots) / 1 / 2 / 3 / 4 groups, us: one tree of 16384, 1563 groups, float64 51 / 63 / 58 / 63 / 57, float32
+// 42 / 51 / 46 / 50 / 47; four of 4096, 1876 groups, 68 / 74 / 69 / 71 / 65, 55 / 58 / 53 / 58 / 57; 64 of 512 leaves, 4096 groups,
+// 155 / 191 / 186 / 165 / 155, 126 / 141 / 136 / 132 / 128; four of 900, 1252 groups, float32 72 / 75 / 72 / 71 / 75.
 static int g_traversal_groups[2] = {0, 0};      // test knob (gmc_bvh_set_traversal_groups): forward, backward; 0 = automatic
 static int traversal_groups(size_t BL, int M, int N, bool backward, bool by_leaves = false) {
     const size_t per_mixture = (size_t(N) + kWave - 1) / kWave;
     const size_t total = BL * per_mixture, slots = size_t(kTravSlots);
     size_t g;
     if (g_traversal_groups[backward ? 1 : 0] > 0) g = size_t(g_traversal_groups[backward ? 1 : 0]);
-    // (lanes = leaves: few groups per workgroup leave wavefronts without a batch of leaves; one, two, three, four groups take 74,
-    // 69, 71, 62 us for 1563 groups of one tree of 16384 in float64, 82, 73, 81, 75 us for 1876 groups of four trees of 4096)
     else if (backward && !by_leaves && M > kSmallTreeMax) g = total < 4 * slots ? 1 : total < 8 * slots ? 2 : total < 16 * slots ? 3 : kGroupsMax;
     else g = total <= slots ? 1 : total <= 2 * slots ? 2 : kGroupsMax;
     if (g > per_mixture) g = per_mixture;

@@ -365,7 +365,8 @@ __device__ __forceinline__ T quad_form(const T* __restrict__ r, const T* __restr
 }
 
 // acc[p] += amplitude * exp2(-|y|^2) over the records begin, begin + STEP, ... of an LDS tile for the lane's P points.  float:
-// the exponentials of at least six pairs at once (pair_exp2_batch), of two Gaussians where a lane has few points.
+// the exponentials of all points of a lane at once (pair_exp2_batch), of two Gaussians with three to five points; one and two
+// points go one by one.
 template <typename T, int D, int P, int STEP, bool CENTRED>
 __device__ __forceinline__ void add_pairs(const T* __restrict__ lds, const T* __restrict__ tab, int begin, int end,
                                           const T (&x)[P][D], T (&acc)[P]) {
