@@ -207,8 +207,8 @@ template <int COUNT> __device__ __forceinline__ int cw_sum_index(int lane) {
 // point's dL/dx reduced over 64 lanes / now (us, float32, both gradients): 800 x 128 Gaussians at 784 points in 2-D
 // 128 / 102 (3.2 TB/s of grad_out), in 3-D 199 / 130; 20 x 512 at 4096 points 118 / 49 and 272 / 66; 1 x 2 mixtures of 4 at
 // 2 points 8.3 / 7.9.  At the first shape 31 instructions per 64 pairs take about 45 us of the 102, and grad_out is read at
-// 3.3 TB/s where the backward pass of the convolution reads its own at 4.9: bound by the wait for its reads, too few of
-// which are in flight, not by issue.
+// 3.3 TB/s where the backward pass of the convolution reads its own at 4.9: not bound by issue, and what holds its reads at
+// that rate is not shown (the next rows fetched ahead and batched exponentials change nothing).
 constexpr int kCwSteps = 4;        // points of a row per round
 
 template <typename T, int D, int Q, int WAVES, bool NEED_GM, bool NEED_GX>
